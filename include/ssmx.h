@@ -170,6 +170,69 @@ int ssmx_propagate(const ssmx_propagate_desc *desc, const int32_t *ell_col,
                    void *stream);
 
 /*
+ * Propagate n_inst instances whose exponents are A_j = h w_j C + f_j G with
+ * one constant matrix C (coefficient 1 at every node) and one driven matrix
+ * G, f_j = h sum_s w[j,s] c(t_s), w_j = sum_s w[j,s].
+ *
+ * Each exponential is applied as its power series in the drive alone,
+ *   exp(A_j) x = x + sum_k f_j^k E_k x,
+ * where E_0 = exp(h w_j C) - I and E_k holds everything of order k in G
+ * (all orders of C), computed once on the host.  C couples states within
+ * "sectors" and G couples each sector to one other (its opposite), so even
+ * orders act within a sector and odd orders across: row r of the kernel
+ * reads its own sector (`na` components, even orders 0, 2, .., 2 da) and
+ * the opposite one (`nb`, odd orders 1, 3, .., 2 db + 1).
+ *
+ * A wavefront holds `members` instances of `rows` rows each.  A member's
+ * components sit in LDS sector by sector, `sector` doubles apart.
+ *
+ * layout     int32 [rows][4]: per row its component's LDS position, the
+ *            start of its own sector, the start of the opposite sector
+ *            (both even) and its state index (0..n-1)
+ * state_pos  int32 [n]: LDS position of state s, or -1 if it stays zero
+ * table      double [sets][na (da + 1) + nb (db + 1)][rows]: entry
+ *            (s (da + 1) + k) is E_2k's coefficient of own-sector component
+ *            s, then (s (db + 1) + k) E_(2k+1)'s of the opposite one; one
+ *            set per distinct w_j (set min(j, n_exp - 1 - j))
+ * waves      ssmx_wave [ceil(n_inst / wave_group)]: instance i uses wave
+ *            i / wave_group, generator `gen`
+ * rho0       double [n_inst * n] (states without a row must be 0)
+ * obs        double [n_obs * n] readout rows (obs readouts)
+ * out        as ssmx_propagate (READ_FULL: standard state order, 0 for
+ *            states without a row)
+ *
+ * Replaces: generate_simulator.py:1945-2116, as ssmx_propagate.
+ */
+typedef struct ssmx_series_desc {
+    int32_t n;          /* states of an instance (rho0, obs, full readout) */
+    int32_t rows;       /* rows of an instance, 1..64 */
+    int32_t n_inst;
+    int32_t members;    /* instances per wavefront, members * rows <= 64 */
+    int32_t n_exp;      /* J */
+    int32_t n_node;     /* S */
+    int32_t fine;
+    int32_t n_out;
+    int32_t n_obs;      /* 1..2 for obs readouts */
+    int32_t flags;      /* SSMX_READ_FULL, SSMX_READ_INTEGRAL or 0 */
+    int32_t gen;        /* driven generator's index in ssmx_wave */
+    int32_t wave_group; /* instances that share one waveform, >= 1 */
+    int32_t na, da;     /* own-sector components and highest even order / 2 */
+    int32_t nb, db;     /* opposite components, (highest odd order - 1) / 2 */
+    int32_t sector;     /* LDS doubles per sector, even, >= na and nb */
+    int32_t sectors;    /* sectors per member */
+    double h;
+    double t0;
+    double dt;
+} ssmx_series_desc;
+
+int ssmx_propagate_series(const ssmx_series_desc *desc,
+                          const int32_t *layout, const int32_t *state_pos,
+                          const double *table, const double *cf_weights,
+                          const double *cf_nodes, const ssmx_wave *waves,
+                          const ssmx_segment *segments, const double *rho0,
+                          const double *obs, double *out, void *stream);
+
+/*
  * The reference's non-residual exponential (use_residual=False).
  *
  * Each exponential is (I + A / scale)^(2^squarings) with scale = 4^R and

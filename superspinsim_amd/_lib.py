@@ -91,6 +91,15 @@ class ChunkDesc(ctypes.Structure):
         "reserved")]
 
 
+class SeriesDesc(ctypes.Structure):
+    """Mirror of ``ssmx_series_desc`` (include/ssmx.h)."""
+    _fields_ = [(f, ctypes.c_int32) for f in (
+        "n", "rows", "n_inst", "members", "n_exp", "n_node", "fine", "n_out",
+        "n_obs", "flags", "gen", "wave_group", "na", "da", "nb", "db",
+        "sector", "sectors")] + [(f, ctypes.c_double) for f in (
+            "h", "t0", "dt")]
+
+
 class Segment(ctypes.Structure):
     """Mirror of ``ssmx_segment``."""
     _fields_ = [("t_start", ctypes.c_double), ("t_end", ctypes.c_double),
@@ -106,7 +115,8 @@ class Wave(ctypes.Structure):
 
 
 #: every symbol include/ssmx.h declares
-EXPORTS = ("ssmx_propagate", "ssmx_propagate_dense", "ssmx_chunk_combine",
+EXPORTS = ("ssmx_propagate", "ssmx_propagate_series",
+           "ssmx_propagate_dense", "ssmx_chunk_combine",
            "ssmx_propagate_queue",
            "ssmx_propagate_queue_noalloc", "ssmx_adjoint",
            "ssmx_adjoint_workspace_bytes", "ssmx_last_error", "ssmx_version",
@@ -138,6 +148,9 @@ def load():
     vp = ctypes.c_void_p
     lib.ssmx_propagate.argtypes = [ctypes.POINTER(PropagateDesc)] + [vp] * 13
     lib.ssmx_propagate.restype = ctypes.c_int
+    lib.ssmx_propagate_series.argtypes = [ctypes.POINTER(SeriesDesc)] + \
+        [vp] * 11
+    lib.ssmx_propagate_series.restype = ctypes.c_int
     lib.ssmx_propagate_queue.argtypes = (
         [ctypes.POINTER(PropagateDesc)] + [vp] * 13 +
         [ctypes.c_int32, ctypes.c_int32, vp, vp])

@@ -590,6 +590,21 @@ def coefficient_samples(cmin, cmax, count=48, seed=0):
     return np.array(out)
 
 
+def sample_exponents(mats, weights, coef_samples, h, rotating=False):
+    """Dense A_j for node-coefficient samples (count, S, K), all j, of
+    generators ``mats`` ((K, n, n), or (S, K, n, n) in the rotating frame)."""
+    out = []
+    for c in np.asarray(coef_samples, dtype=_f64):
+        for row in weights:
+            if rotating:
+                f = c * (h * row[:, None])                     # (S, K)
+                out.append(np.tensordot(f, mats, axes=([0, 1], [0, 1])))
+            else:
+                cw = row @ c                                   # (K,)
+                out.append(h * np.tensordot(cw, mats, axes=(0, 0)))
+    return out
+
+
 def taylor_plan(norm, tol=1e-17, max_taylor=_lib.MAX_TAYLOR):
     """Cheapest (m, s) with s * remainder(norm / s, m) <= tol.
 
@@ -915,17 +930,8 @@ class Propagator:
 
     def sample_exponents(self, coef_samples, h):
         """Dense A_j for node-coefficient samples (count, S, K), all j."""
-        out = []
-        mats = self._dense
-        for c in np.asarray(coef_samples, dtype=_f64):
-            for j in range(self.J):
-                if self.rotating:
-                    f = c * (h * self.weights[j][:, None])     # (S, K)
-                    out.append(np.tensordot(f, mats, axes=([0, 1], [0, 1])))
-                else:
-                    cw = self.weights[j] @ c                   # (K,)
-                    out.append(h * np.tensordot(cw, mats, axes=(0, 0)))
-        return out
+        return sample_exponents(self._dense, self.weights, coef_samples, h,
+                                self.rotating)
 
     def plan(self, coef_samples, h, tol=1e-17, max_substeps=1024,
              max_taylor=_lib.MAX_TAYLOR):

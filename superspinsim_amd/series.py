@@ -1,0 +1,346 @@
+"""Series-in-the-drive tables: plan and launch of ``ssmx_propagate_series``.
+
+An exponent ``h w C + f G`` with a constant matrix C and one driven matrix G
+is exponentiated as ``I + sum_k f^k E_k``, where ``E_k`` collects every term
+of order k in G (``coefficient_matrices``).  For the drives of magnetic
+resonance f G is small (1-norm about 1e-3 at 20 ps steps), so four or five
+orders reach the accuracy that takes a Taylor chain in the whole exponent
+11 products.
+
+``reachable`` finds the states a run can involve at all: those that the
+couplings connect to the initial states and to the readout.  The others stay
+exactly zero or are never read (a sweep that starts from populations never
+fills the coherences between the orbital blocks).
+"""
+
+import ctypes
+
+import numpy as np
+
+from superspinsim_amd import _lib
+from superspinsim_amd.propagator import _ptr, _torch, device_tensor
+
+_f64 = np.float64
+
+#: components per sector the kernels hold
+SIZES = (5, 11)
+#: (highest even order / 2, (highest odd order - 1) / 2), cheapest first
+ORDERS = ((1, 1), (2, 1), (2, 2))
+#: highest 1-norm of h w C (the series of E_0 then loses under one digit)
+MAX_NORM = 4.0
+
+
+def reachable(pattern, rho0, obs=None):
+    """Indices of the states a run can involve.
+
+    ``pattern[a, b]`` is set where some generator takes state b to state a;
+    ``rho0`` (instances, n) are the initial states.  States that no non-zero
+    initial component reaches stay zero; with readout rows ``obs`` those
+    that no read component depends on are left out as well.
+    """
+    def closure(adjacency, start):
+        seen = start.copy()
+        front = start
+        while front.any():
+            front = adjacency[:, front].any(axis=1) & ~seen
+            seen |= front
+        return seen
+
+    # a NaN or an infinite component counts as filled
+    keep = closure(pattern, np.any(rho0 != 0, axis=0))
+    if obs is not None:
+        keep &= closure(pattern.T, np.any(obs != 0, axis=0))
+    return np.flatnonzero(keep)
+
+
+def split_sectors(const, drive):
+    """(sector of each state, opposite sector of each sector) or None.
+
+    Sectors are the groups that ``const`` couples (in either direction);
+    ``drive`` must couple every state of a sector to states of one other
+    sector only, and that one back to it.  Sectors that the drive leaves
+    alone are their own opposite's empty partner (-1).
+    """
+    n = const.shape[0]
+    even = (const != 0) | (const.T != 0)
+    odd = (drive != 0) | (drive.T != 0)
+    # two-colour the connected components: even edges keep the colour, odd
+    # edges change it
+    comp = np.full(n, -1)
+    colour = np.zeros(n, dtype=np.int64)
+    count = 0
+    for s in range(n):
+        if comp[s] >= 0:
+            continue
+        comp[s], stack = count, [s]
+        while stack:
+            a = stack.pop()
+            for b in np.flatnonzero((even[a] | odd[a]) & (comp < 0)):
+                if even[a, b] and odd[a, b]:
+                    return None
+                comp[b] = count
+                colour[b] = colour[a] ^ int(odd[a, b])
+                stack.append(b)
+        count += 1
+    same = comp[:, None] == comp[None, :]
+    flip = colour[:, None] != colour[None, :]
+    if np.any(even & same & flip) or np.any(odd & ~flip):
+        return None
+    sector = 2 * comp + colour
+    names, sector = np.unique(sector, return_inverse=True)
+    index = {int(v): k for k, v in enumerate(names)}
+    opposite = np.array([index.get(int(v) ^ 1, -1) for v in names])
+    return sector, opposite
+
+
+def _dropped(count, da, db):
+    """Orders below ``count`` that the kernels' (da, db) leave out."""
+    return [k for k in range(count)
+            if k > (2 * da if k % 2 == 0 else 2 * db + 1)]
+
+
+def _sparse(mat):
+    """(columns, values) lists, slot by slot, of a matrix's rows."""
+    width = int(np.max(np.count_nonzero(mat, axis=1), initial=0))
+    n = mat.shape[0]
+    cols = np.zeros((width, n), dtype=np.int64)
+    vals = np.zeros((width, n), dtype=np.longdouble)
+    for r in range(n):
+        c = np.flatnonzero(mat[r])
+        cols[:c.size, r] = c
+        vals[:c.size, r] = mat[r, c]
+    return cols, vals
+
+
+def coefficient_matrices(const, drive, scale, orders):
+    """E_0 .. E_orders of exp(scale * const + f * drive) in powers of f.
+
+    E_0 has the identity taken off.  Summed in extended precision and
+    rounded once: the same E_k act at every step, so their rounding would
+    not average out.
+    """
+    n = const.shape[0]
+    cc, cv = _sparse(np.asarray(const, dtype=_f64))
+    dc, dv = _sparse(np.asarray(drive, dtype=_f64))
+    cv = cv * np.longdouble(scale)
+
+    def times(cols, vals, mat):
+        out = np.zeros_like(mat)
+        for c, v in zip(cols, vals):
+            out += v[:, None] * mat[c]
+        return out
+
+    zero = np.zeros((n, n), dtype=np.longdouble)
+    term = [np.eye(n, dtype=np.longdouble)] + [zero] * orders
+    total = [zero.copy() for _ in range(orders + 1)]
+    norm = float(np.abs(const).sum(axis=0).max(initial=0.0)) * abs(scale)
+    bound, t = 1.0, 0
+    # terms of order t in const fall like norm^t / t!, drive orders add to t
+    while bound > 1e-24 or t <= orders + 2:
+        t += 1
+        bound *= norm / max(t - orders, 1)
+        new = []
+        for k in range(orders + 1):
+            v = times(cc, cv, term[k])
+            if k:
+                v += times(dc, dv, term[k - 1])
+            new.append(v / t)
+        term = new
+        for k in range(orders + 1):
+            total[k] += term[k]
+    return [m.astype(_f64) for m in total]
+
+
+class SeriesModel:
+    """E_k and row layout of one (constant, drive) pair at one step size.
+
+    ``build`` returns None where the kernels do not apply: more than 64
+    states, states the drive couples within a sector, sectors of more than
+    ``SIZES`` components, a step whose constant part is large.
+    """
+
+    def __init__(self):
+        self._tables = None     # the last drive's
+
+    @classmethod
+    def build(cls, const, drive, weights, h):
+        n = const.shape[0]
+        J, S = weights.shape
+        sums = weights.sum(axis=1)
+        distinct = sums[:(J + 1) // 2]
+        if n > _lib.MAX_N or J not in (1, 2, 5) or \
+                (J <= 2 and S != J) or \
+                not np.allclose(sums, sums[::-1], rtol=1e-15, atol=1e-16):
+            return None
+        norm = float(np.abs(const).sum(axis=0).max()) * h * \
+            np.abs(sums).max()
+        if not norm <= MAX_NORM:
+            return None
+        found = split_sectors(const, drive)
+        if found is None:
+            return None
+        sector, opposite = found
+        counts = np.bincount(sector)
+        fit = [s for s in SIZES if s >= counts.max()]
+        if not fit or (J == 5 and fit[0] != SIZES[0]):
+            return None
+        self = cls()
+        self.n, self.size, self.h = n, fit[0], h
+        self.sector, self.opposite = sector, opposite
+        self.pad = fit[0] + 1                    # even
+        self.n_sectors = counts.size
+        self.weight = float(np.abs(weights).sum(axis=1).max())
+        self.nnz = int(np.count_nonzero((const != 0) | (drive != 0)))
+        top = 2 * ORDERS[-1][0] + 3
+        self.sets = [coefficient_matrices(const, drive, h * float(w), top)
+                     for w in distinct]
+        order = np.argsort(sector, kind="stable")
+        self.members = [order[np.searchsorted(sector[order], k):
+                              np.searchsorted(sector[order], k, "right")]
+                        for k in range(self.n_sectors)]
+        pos = np.empty(n, dtype=np.int32)
+        for k, states in enumerate(self.members):
+            pos[states] = k * self.pad + np.arange(states.size)
+        self.pos, self.order = pos, order
+        return self
+
+    def plan(self, drive_max, tol):
+        """(da, db, F) for drives |c(t)| <= ``drive_max``, or None.
+
+        F bounds the factors |f| and the kept orders are those of the
+        series in Chebyshev polynomials of f / F, whose order k is 2^(k-1)
+        smaller than the power series': what is left out must stay below
+        ``tol`` with the Taylor plans' margin (a factor of 8).
+        """
+        F = self.h * self.weight * float(drive_max)
+        worst = np.max([[np.abs(c).sum(axis=0).max() for c in cs]
+                        for cs in (self._chebyshev(es, F)
+                                   for es in self.sets)], axis=0)
+        if not np.all(np.isfinite(worst)):
+            return None
+        for da, db in ORDERS:
+            # (the orders beyond the last matrix are smaller than it)
+            if 8.0 * (worst[-1] + sum(worst[_dropped(worst.size, da, db)])) \
+                    <= tol:
+                return da, db, F
+        return None
+
+    @staticmethod
+    def _chebyshev(mats, F):
+        """Chebyshev coefficients in f / F of sum_k f^k E_k."""
+        out = [np.zeros_like(mats[0]) for _ in mats]
+        for k, m in enumerate(mats):
+            power = np.zeros(k + 1)
+            power[k] = F ** k
+            for j, c in enumerate(np.polynomial.chebyshev.poly2cheb(power)):
+                if c:
+                    out[j] += c * m
+        return out
+
+    def matrices(self, da, db, F):
+        """The kept E_k of every set, with the Chebyshev polynomials of the
+        orders left out taken off (so that they represent the truncated
+        Chebyshev series)."""
+        out = []
+        for mats in self.sets:
+            kept = [m.copy() for m in mats]
+            cheb = self._chebyshev(mats, F)
+            for j in _dropped(len(mats), da, db):
+                unit = np.zeros(j + 1)
+                unit[j] = 1.0
+                for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(
+                        unit)):
+                    # (an underflown power: its order is zero as well)
+                    if c and F ** k:
+                        kept[k] -= (c / F ** k) * cheb[j]
+            out.append(kept)
+        return out
+
+    def tables(self, da, db, F):
+        """Device (layout, table) of the kernel's rows."""
+        key = (da, db, F)
+        if self._tables is None or self._tables[0] != key:
+            n, size = self.n, self.size
+            layout = np.zeros((n, 4), dtype=np.int32)
+            own_w, opp_w = size * (da + 1), size * (db + 1)
+            sets = self.matrices(da, db, F)
+            table = np.zeros((len(sets), own_w + opp_w, n))
+            for r, state in enumerate(self.order):
+                k = self.sector[state]
+                o = self.opposite[k]
+                layout[r] = (self.pos[state], k * self.pad,
+                             (o if o >= 0 else k) * self.pad, state)
+                for e, mats in enumerate(sets):
+                    own = self.members[k]
+                    for a in range(da + 1):
+                        table[e, a:own.size * (da + 1):da + 1, r] = \
+                            mats[2 * a][state, own]
+                    if o < 0:
+                        continue
+                    opp = self.members[o]
+                    for a in range(db + 1):
+                        table[e, own_w + a:own_w + opp.size * (db + 1):
+                              db + 1, r] = mats[2 * a + 1][state, opp]
+            self._tables = (key, device_tensor(layout), device_tensor(table))
+        return self._tables[1:]
+
+
+class SeriesRun:
+    """Staged inputs of one run through ``ssmx_propagate_series``.
+
+    ``states`` are the caller's indices of the model's states; ``rho0``
+    (instances, n) and ``obs`` stay in the caller's order.  ``wave_group``
+    consecutive instances share one waveform.
+    """
+
+    def __init__(self, model, plan, states, members, weights, nodes, rho0,
+                 d_waves, d_segs, gen, fine, n_out, t0, dt, obs, read,
+                 wave_group=1):
+        torch = _torch()
+        n_inst, n = rho0.shape
+        flags = {"full": _lib.SSMX_READ_FULL, "obs": 0,
+                 "integral": _lib.SSMX_READ_INTEGRAL}[read]
+        n_obs = obs.shape[0] if obs is not None else 0
+        if read != "full" and not 1 <= n_obs <= _lib.MAX_OBS:
+            raise ValueError(f"{n_obs} readout rows outside 1.."
+                             f"{_lib.MAX_OBS}")
+        layout, table = model.tables(*plan)
+        local = model.order
+        # the kernel's state index is the caller's
+        self.layout = layout.clone()
+        self.layout[:, 3] = device_tensor(
+            np.asarray(states)[local].astype(np.int32))
+        where = np.full(n, -1, dtype=np.int32)
+        where[states] = model.pos
+        self.d_where = device_tensor(where)
+        self.table = table
+        self.d_w, self.d_nodes = device_tensor(weights), device_tensor(nodes)
+        self.d_rho0, self.d_waves, self.d_segs = (
+            device_tensor(np.ascontiguousarray(rho0, dtype=_f64)), d_waves,
+            d_segs)
+        self.d_obs = None if read == "full" else device_tensor(
+            np.ascontiguousarray(obs, dtype=_f64))
+        self.desc = _lib.SeriesDesc(
+            n=n, rows=model.n, n_inst=n_inst, members=members,
+            n_exp=weights.shape[0], n_node=weights.shape[1], fine=fine,
+            n_out=n_out, n_obs=n_obs, flags=flags, gen=gen,
+            wave_group=wave_group, na=model.size, da=plan[0],
+            nb=model.size, db=plan[1], sector=model.pad,
+            sectors=model.n_sectors, h=dt / fine, t0=t0, dt=dt)
+        shape = {"full": (n_inst, n_out, n), "obs": (n_inst, n_out, n_obs),
+                 "integral": (n_inst, n_obs)}[read]
+        self.out = torch.empty(shape, dtype=torch.float64, device="cuda")
+        self.k = members
+
+    def launch(self):
+        torch = _torch()
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(_lib.load().ssmx_propagate_series(
+            ctypes.byref(self.desc), _ptr(self.layout), _ptr(self.d_where),
+            _ptr(self.table), _ptr(self.d_w), _ptr(self.d_nodes),
+            _ptr(self.d_waves), _ptr(self.d_segs), _ptr(self.d_rho0),
+            _ptr(self.d_obs), _ptr(self.out), ctypes.c_void_p(stream)))
+        return self.out
+
+    def result(self):
+        return self.out

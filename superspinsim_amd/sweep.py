@@ -24,7 +24,8 @@ import numpy as np
 from superspinsim_amd import _lib, quadratures
 from superspinsim_amd.propagator import (
     Propagator, _ptr, coefficient_samples, device_tensor, eig_lane_factors,
-    rotating_tables)
+    rotating_tables, sample_exponents, taylor_plan_measured)
+from superspinsim_amd.series import SeriesModel, SeriesRun, reachable
 
 _f64 = np.float64
 
@@ -284,6 +285,12 @@ class BatchSimulator:
     small model (n <= 32, lab frame) into one block-diagonal system per
     wavefront (``pack_factor``); an integer asks for that many per system
     (within the kernel's limits) whatever the instance count.
+
+    ``run`` computes on the states the run can involve
+    (``series.reachable``).  A lab-frame run with one driven generator whose
+    model fits goes through the series in the drive (``series``), any other
+    through the Taylor action of the whole exponent; so does a run that
+    names a ``layout``, a Taylor degree or a substep count.
     """
 
     def __init__(self, generators, number_of_exponentials=2,
@@ -299,7 +306,10 @@ class BatchSimulator:
             number_of_exponentials)
         self.F = int(number_of_fine_divisions)
         self.rotating = bool(use_rotating)
+        self.scheme = number_of_exponentials
         self.tolerance = tolerance
+        self._reduced_cache = {}
+        self._series_cache = {}
         if self.rotating:
             self.V = np.asarray(vectors_real, dtype=_f64)
             self.Vinv = np.asarray(inv_vectors_real, dtype=_f64)
@@ -461,11 +471,149 @@ class BatchSimulator:
             out.append(nw)
         return out
 
+    # ------------------------------------------------------------------
+    def _reduced(self, states):
+        """This simulator on a subset of the states."""
+        if states.size == self.n:
+            return self
+        key = states.tobytes()
+        if key not in self._reduced_cache:
+            self._reduced_cache[key] = BatchSimulator(
+                self.gens[:, states][:, :, states], self.scheme, self.F,
+                tolerance=self.tolerance, layout=self.layout,
+                pack=self.pack)
+        sub = self._reduced_cache[key]
+        sub.tolerance, sub.pack = self.tolerance, self.pack
+        return sub
+
+    def involved(self, active, rho0, obs=None):
+        """States a run over the ``active`` generators involves
+        (``series.reachable``); every state where none is left or the frame
+        is not the lab's."""
+        every = np.arange(self.n)
+        if self.rotating or self.layout != "auto":
+            return every
+        pattern = np.any(self.gens[list(active)] != 0, axis=0)
+        states = reachable(pattern, rho0, obs)
+        return states if states.size else every
+
+    def folded(self, const):
+        """Sum of the generators with constant coefficients."""
+        return sum((v * self.gens[g] for g, v in const.items()),
+                   np.zeros((self.n, self.n)))
+
+    def series_plan(self, waves, const, program, time_step):
+        """(model, plan) of the series in the drive, or None."""
+        varying = [g for g in program if g is not None]
+        if self.rotating or self.layout != "auto" or len(varying) > 1:
+            return None
+        h = time_step / self.F
+        key = (tuple(varying), tuple(sorted(const.items())), h)
+        if key not in self._series_cache:
+            drive = self.gens[varying[0]] if varying else \
+                np.zeros((self.n, self.n))
+            self._series_cache[key] = SeriesModel.build(
+                self.folded(const), drive, self.weights, h)
+        model = self._series_cache[key]
+        if model is None:
+            return None
+        drive_max = max(w.abs_max()[varying[0]] for w in waves) \
+            if varying else 0.0
+        plan = model.plan(drive_max, self.tolerance)
+        return None if plan is None else (model, plan)
+
+    def series_members(self, n_inst, rows):
+        """Instances per wavefront of a series run.
+
+        A SIMD's time goes with the wavefronts it holds, each costing the
+        same whatever its lanes do, so the smallest count that minimises the
+        wavefronts on the fullest SIMD (4096 instances of 19 rows: 2 per
+        wavefront, 2 wavefronts per SIMD)."""
+        limit = min(_lib.MAX_N // rows, _lib.MAX_N // self.weights.shape[0])
+        if not self.pack or n_inst < 2:
+            return 1
+        if self.pack is not True:
+            return max(1, min(limit, int(self.pack)))
+        torch = __import__("torch")
+        simds = 4 * torch.cuda.get_device_properties(
+            0).multi_processor_count
+        return min(range(1, limit + 1), key=lambda k: (
+            -(-(-(-n_inst // k)) // simds), k))
+
+    def _prepare_series(self, found, states, n, waves, program, rho0, obs,
+                        read, time_start, time_step, N, wave_group=1):
+        """``SeriesRun`` of this (reduced) simulator; ``states`` are its
+        states among the caller's ``n``."""
+        model, plan = found
+        kwaves = self.kernel_waves(waves, program)
+        d_waves, d_segs = pack_waveforms(kwaves, len(program))
+        gen = next((k for k, g in enumerate(program) if g is not None), 0)
+        members = self.series_members(rho0.shape[0], model.n)
+        return SeriesRun(model, plan, states, members, self.weights,
+                         self.nodes, rho0, d_waves, d_segs, gen, self.F, N,
+                         time_start, time_step, obs, read,
+                         wave_group=wave_group)
+
     def prepare(self, waves, rho0, time_start, time_end, time_step,
                 obs=None, read="obs", taylor=None, substeps=None):
-        """Plan, pack and stage one ``run`` on the device; returns a
-        ``PreparedRun`` whose ``launch`` only enqueues the kernel."""
+        """Plan, pack and stage one ``run`` on the device; returns an
+        object whose ``launch`` only enqueues the kernel and whose
+        ``result`` is the output of the last launch, one row per instance
+        (``SeriesRun``, ``PreparedRun`` or ``ReducedRun``)."""
         N = int((time_end - time_start) / time_step)
+        n_inst = len(waves)
+        rho0 = np.atleast_2d(np.asarray(rho0, dtype=_f64))
+        if rho0.shape[0] == 1 and n_inst > 1:
+            rho0 = np.repeat(rho0, n_inst, axis=0)
+        if obs is not None:
+            obs = np.atleast_2d(np.asarray(obs, dtype=_f64))
+        if taylor is None and substeps is None and \
+                rho0.shape == (n_inst, self.n) and (
+                    read == "full" if obs is None else
+                    obs.shape[1] == self.n and
+                    1 <= obs.shape[0] <= _lib.MAX_OBS):
+            active, const, program = self.program(waves)
+            states = self.involved(active, rho0,
+                                   None if read == "full" else obs)
+            sub = self._reduced(states)
+            found = sub.series_plan(waves, const, program, time_step)
+            if found is not None:
+                run = sub._prepare_series(
+                    found, states, self.n, waves, program, rho0, obs, read,
+                    time_start, time_step, N)
+                m, s = sub.taylor_plan(waves, active, const, program,
+                                       time_step)
+                model, plan = found
+                self.last_plan = dict(
+                    taylor=m, substeps=s, slots=2 * model.size,
+                    nnz=model.nnz, active=program, n_out=N,
+                    steps=N * self.F, n=self.n, packed=run.k,
+                    involved=model.n, series=plan[:2])
+                return run
+            if sub is not self:
+                run = sub._prepare_taylor(
+                    waves, rho0[:, states], time_start, time_step, N,
+                    None if obs is None else obs[:, states], read, None,
+                    None)
+                self.last_plan = dict(sub.last_plan, n=self.n,
+                                      involved=int(states.size))
+                return ReducedRun(run, states, self.n) if read == "full" \
+                    else run
+        return self._prepare_taylor(waves, rho0, time_start, time_step, N,
+                                    obs, read, taylor, substeps)
+
+    def taylor_plan(self, waves, active, const, program, time_step):
+        """(degree, substeps) of the Taylor action for a lab-frame batch."""
+        mats = ([self.folded(const)[None]] if None in program else []) + \
+            [self.gens[[g for g in program if g is not None]]]
+        return taylor_plan_measured(sample_exponents(
+            np.concatenate(mats), self.weights,
+            self.coefficient_box(waves, program), time_step / self.F),
+            tol=self.tolerance)
+
+    def _prepare_taylor(self, waves, rho0, time_start, time_step, N, obs,
+                        read, taylor, substeps):
+        """``prepare`` through the Taylor action on every state."""
         prop0, program, m, s = self.plan(waves, time_step)
         prop = prop0
         if taylor is not None:
@@ -473,13 +621,9 @@ class BatchSimulator:
         if substeps is not None:
             s = substeps
         n_inst = len(waves)
-        rho0 = np.atleast_2d(np.asarray(rho0, dtype=_f64))
-        if rho0.shape[0] == 1 and n_inst > 1:
-            rho0 = np.repeat(rho0, n_inst, axis=0)
         x0 = rho0 @ self.Vinv.T if self.rotating else rho0
         obs_eff = None
         if obs is not None:
-            obs = np.atleast_2d(np.asarray(obs, dtype=_f64))
             obs_eff = obs @ self.V if self.rotating else obs
         n_obs = obs_eff.shape[0] if obs_eff is not None else 0
         k = self.pack_factor(n_inst, program, read, n_obs)
@@ -683,6 +827,24 @@ class ChunkedRun:
 
     def result(self):
         return self.out
+
+
+class ReducedRun:
+    """A full-state run on part of the states: ``result`` fills the others
+    with zeros."""
+
+    def __init__(self, run, states, n):
+        self.run, self.n, self.k = run, n, run.k
+        self.states = device_tensor(np.asarray(states, dtype=np.int64))
+
+    def launch(self):
+        return self.run.launch()
+
+    def result(self):
+        part = self.run.result()
+        out = part.new_zeros(part.shape[:-1] + (self.n,))
+        out[..., self.states] = part
+        return out
 
 
 class PreparedRun:

@@ -1,0 +1,123 @@
+"""Series-in-the-drive kernel against the Taylor kernels (GPU).
+
+Both propagate the same exponentials to 1e-16, so over the few thousand
+exponentials of each case they differ by rounding only: at most one ulp of
+the state per exponential, i.e. 4000 x 1.1e-16 = 4.4e-13 relative to the
+largest value; 1e-12 is the bar.  ``taylor=17`` asks for the Taylor path on
+every state.
+"""
+
+import numpy as np
+import pytest
+
+from superspinsim_amd import configs
+from superspinsim_amd.sweep import BatchSimulator, Waveform
+
+pytestmark = pytest.mark.gpu
+
+SAME = 1e-12
+
+
+def _model(name):
+    if name == "nv3":
+        return configs.odmr3(1)
+    return configs.odmr7(1, use_incoherent=name == "nv7c")
+
+
+def _waves(wl, points, rabi, gated=False):
+    b1 = configs.drive_amplitude(rabi)
+    out = []
+    for k in range(points):
+        w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, wl.excitation])
+        f = 2.80e9 + 1.4e8 * k / max(points - 1, 1)
+        if gated:
+            w.add(1, 1e-9, 5e-9 + 1e-10 * (k % 40), b1, 2 * np.pi * f, 0.3)
+            w.add(1, 9e-9, 2e-8, -b1, 2 * np.pi * f, 0.1 * k)
+        else:
+            w.tone(1, b1, f)
+        out.append(w)
+    return out
+
+
+@pytest.mark.parametrize("name,points,exps,fine,rabi,read,pack,orders", [
+    ("nv7", 1, 2, 7, 3e6, "obs", True, (2, 1)),
+    ("nv7", 5, 2, 16, 5e5, "integral", 3, (1, 1)),
+    ("nv7", 4, 2, 33, 2.5e7, "full", 2, (2, 2)),
+    ("nv7c", 7, 1, 20, 1.2e7, "full", 3, (2, 2)),
+    ("nv7c", 2, 1, 50, 5e5, "obs", True, (1, 1)),
+    ("nv3", 9, 2, 17, 5e6, "full", 7, (2, 1)),
+    ("nv3", 15, 5, 11, 5e6, "obs", 7, (2, 1)),
+    ("nv3", 3, 5, 10, 3e7, "integral", 2, (2, 2)),
+    ("nv3", 3, 5, 10, 1e6, "integral", 2, (1, 1)),
+    ("nv3", 3, 1, 10, 1e7, "obs", 5, (2, 2)),
+    ("nv3", 65, 2, 10, 1e6, "obs", 7, (1, 1)),
+])
+def test_series_equals_taylor(gpu, name, points, exps, fine, rabi, read,
+                              pack, orders):
+    wl = _model(name)
+    sim = BatchSimulator(wl.generators, exps, fine, pack=pack)
+    dt = fine * 20e-12
+    n_out = 1000 // fine
+    args = (_waves(wl, points, rabi, gated=points > 4), wl.rho0, 3e-10,
+            3e-10 + n_out * dt * (1 + 1e-9), dt)
+    obs = None if read == "full" else wl.obs
+    if points > 4 and obs is not None:
+        obs = np.concatenate([obs, np.roll(obs, -1, axis=1)])
+    print(f"{name} x {points}, {exps} exponentials, {read}", flush=True)
+    got = sim.run(*args, obs=obs, read=read).cpu().numpy()
+    assert sim.last_plan["series"] == orders, sim.last_plan
+    want = sim.run(*args, obs=obs, read=read, taylor=17).cpu().numpy()
+    assert got.shape == want.shape
+    err = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    print(f"  {err:.1e}")
+    assert err <= SAME
+
+
+def test_every_state_and_own_initial_states(gpu):
+    """Initial coherences everywhere: all 49 states in one wavefront, with a
+    different state per instance; some sectors have no opposite."""
+    wl = configs.odmr7(1)
+    rng = np.random.default_rng(3)
+    rho = rng.standard_normal((3, wl.n))
+    sim = BatchSimulator(wl.generators, 2, 20)
+    args = (_waves(wl, 3, 3e6), rho, 0.0, 20 * 4e-10 * (1 + 1e-9), 4e-10)
+    got = sim.run(*args, read="full").cpu().numpy()
+    assert sim.last_plan["involved"] == 49 and "series" in sim.last_plan
+    want = sim.run(*args, read="full", taylor=17).cpu().numpy()
+    assert np.max(np.abs(got - want)) / np.max(np.abs(want)) <= SAME
+
+
+def test_undriven_run_and_non_finite_neighbour(gpu):
+    """No driven generator at all; and an instance whose input is NaN leaves
+    the instances that share its wavefront alone."""
+    wl = configs.odmr7(1, use_incoherent=True)
+    sim = BatchSimulator(wl.generators, 2, 10)
+    free = [Waveform(5, base=[1.0, 0.0, 0.0, 0.0, wl.excitation])] * 3
+    args = (0.0, 5 * 2e-10 * (1 + 1e-9), 2e-10)
+    got = sim.run(free, wl.rho0, *args, read="full").cpu().numpy()
+    assert "series" in sim.last_plan
+    want = sim.run(free, wl.rho0, *args, read="full",
+                   taylor=17).cpu().numpy()
+    assert np.max(np.abs(got - want)) <= SAME
+    rho = np.repeat(wl.rho0[None], 3, axis=0)
+    rho[1, 2] = np.nan
+    sim.pack = 3
+    waves = _waves(wl, 3, 3e6)
+    bad = sim.run(waves, rho, *args, obs=wl.obs).cpu().numpy()
+    good = sim.run(waves, wl.rho0, *args, obs=wl.obs).cpu().numpy()
+    assert np.all(np.isnan(bad[1])) and np.array_equal(bad[::2], good[::2])
+
+
+def test_reduced_wide_states(gpu):
+    """21 levels: the 171 involved states of 441, zeros elsewhere."""
+    wl = configs.odmr21(2)
+    sim = wl.simulator()
+    waves = wl.waveforms()
+    args = (waves, wl.rho0, 0.0, 2 * wl.time_step * (1 + 1e-9),
+            wl.time_step)
+    got = sim.run(*args, read="full").cpu().numpy()
+    assert sim.last_plan["involved"] == 171
+    want = sim.run(*args, read="full", taylor=11).cpu().numpy()
+    assert np.max(np.abs(got - want)) / np.max(np.abs(want)) <= SAME
+    obs = sim.run(*args, obs=wl.obs).cpu().numpy()[:, :, 0]
+    assert np.max(np.abs(obs - got @ wl.obs[0])) <= 1e-15

@@ -1,0 +1,105 @@
+"""Series in the drive: tables and the choice of states (no GPU needed).
+
+The E_k are compared with the whole exponent's Taylor series in extended
+precision (scipy's expm is off by 2e-14 at the longer step), the omitted
+orders with the plan's tolerance; ``reachable`` with brute-force
+propagation; models the kernels do not cover must be refused.
+"""
+
+import numpy as np
+import pytest
+from scipy.linalg import expm
+
+from superspinsim_amd import configs, quadratures
+from superspinsim_amd.series import (
+    SeriesModel, coefficient_matrices, reachable, split_sectors)
+
+H = 20e-12
+
+
+def _pair(wl):
+    return (wl.generators[0] + wl.excitation * wl.generators[4],
+            wl.generators[1])
+
+
+def _exponential(a):
+    a = a.astype(np.longdouble)
+    term = total = np.eye(a.shape[0], dtype=np.longdouble)
+    for k in range(1, 60):
+        term = term @ a / k
+        total = total + term
+    return total
+
+
+@pytest.mark.parametrize("wl", [configs.odmr3(1),
+                                configs.odmr7(1, use_incoherent=True)])
+@pytest.mark.parametrize("scale", [H / 2, 2e-10])
+def test_matrices_sum_to_the_exponential(wl, scale):
+    const, drive = _pair(wl)
+    mats = coefficient_matrices(const, drive, scale, 7)
+    for f in (0.0, 1e-14, -wl.b1 * H):
+        total = np.eye(wl.n) + sum(f ** k * m for k, m in enumerate(mats))
+        want = _exponential(scale * const + f * drive)
+        # rounding: a few ulp of the entries
+        assert np.max(np.abs(total - want)) < 5e-15
+
+
+@pytest.mark.parametrize("rabi,orders", [(5e5, (1, 1)), (3e6, (2, 1)),
+                                         (2.5e7, (2, 2)), (1e9, None)])
+def test_orders_meet_the_tolerance(rabi, orders):
+    wl = configs.odmr7(1, use_incoherent=True)
+    const, drive = _pair(wl)
+    _, weights, _ = quadratures.scheme(2)
+    model = SeriesModel.build(const, drive, weights, H)
+    plan = model.plan(configs.drive_amplitude(rabi), 1e-16)
+    assert (plan and plan[:2]) == orders
+    if plan is None:
+        return
+    da, db, F = plan
+    mats, = model.matrices(*plan)
+    for f in F * np.linspace(-1, 1, 9):
+        kept = np.eye(wl.n, dtype=np.longdouble) + sum(
+            np.longdouble(f) ** k * m for k, m in enumerate(mats)
+            if k <= (2 * da if k % 2 == 0 else 2 * db + 1))
+        want = _exponential(H * weights[0].sum() * const + f * drive)
+        # truncation 1e-16 / 8, and the tables' own rounding: half an ulp
+        # of entries below 0.25 (1.4e-17 each, at most 11 in a column)
+        assert np.abs(kept - want).sum(axis=0).max() <= 1.7e-16
+
+
+def test_reachable_states_of_the_sweep():
+    wl = configs.odmr7(1)
+    const, drive = _pair(wl)
+    pattern = (const != 0) | (drive != 0)
+    states = reachable(pattern, wl.rho0[None], wl.obs)
+    assert states.size == 19
+    step = expm(H * const + wl.b1 * H * drive)
+    x = np.linalg.matrix_power(step, 50) @ wl.rho0
+    others = np.setdiff1d(np.arange(wl.n), states)
+    assert np.all(x[others] == 0) and np.all(x[states] != 0)
+    # a filled coherence brings its block in; a NaN counts as filled
+    for value in (0.1, np.nan):
+        rho = wl.rho0.copy()
+        rho[others[0]] = value
+        assert reachable(pattern, rho[None]).size > 19
+    # nothing reaches the readout
+    assert reachable(pattern, wl.rho0[None], np.zeros((1, wl.n))).size == 0
+
+
+def test_uncovered_models_are_refused():
+    _, weights, _ = quadratures.scheme(2)
+    wl = configs.odmr7(1, use_incoherent=True)
+    const, drive = _pair(wl)
+    # a drive along the field couples within a sector
+    assert SeriesModel.build(const, wl.generators[3], weights, H) is None
+    # a transverse static field joins the sectors
+    assert split_sectors(const + 1e-3 * drive, drive) is None
+    # a long step
+    assert SeriesModel.build(const, drive, weights, 1e-9) is None
+    # five exponentials need three sets of tables
+    _, w5, _ = quadratures.scheme(5)
+    assert SeriesModel.build(const, drive, w5, H) is None
+    _, w3, _ = quadratures.scheme(3)
+    assert SeriesModel.build(const, drive, w3, H) is None
+    small = _pair(configs.odmr3(1))
+    assert len(SeriesModel.build(*small, w5, H).sets) == 3
