@@ -220,6 +220,10 @@ typedef struct ssmx_series_desc {
     int32_t nb, db;     /* opposite components, (highest odd order - 1) / 2 */
     int32_t sector;     /* LDS doubles per sector, even, >= na and nb */
     int32_t sectors;    /* sectors per member */
+    int32_t sector_rows; /* > 0: at most two sectors, the first of this many
+                            rows (rows 0..), the second the opposite one; the
+                            kernel may then exchange by row broadcasts */
+    int32_t reserved;   /* 0 */
     double h;
     double t0;
     double dt;

@@ -96,8 +96,8 @@ class SeriesDesc(ctypes.Structure):
     _fields_ = [(f, ctypes.c_int32) for f in (
         "n", "rows", "n_inst", "members", "n_exp", "n_node", "fine", "n_out",
         "n_obs", "flags", "gen", "wave_group", "na", "da", "nb", "db",
-        "sector", "sectors")] + [(f, ctypes.c_double) for f in (
-            "h", "t0", "dt")]
+        "sector", "sectors", "sector_rows", "reserved")] + [
+            (f, ctypes.c_double) for f in ("h", "t0", "dt")]
 
 
 class Segment(ctypes.Structure):

@@ -18,6 +18,15 @@
 // doubles), forms its row of the exponential by Horner in f^2, and
 // multiplies it by the two sectors read from LDS in 16-byte reads, which all
 // lanes of a sector read at one address.
+//
+// What bounds it (4096 points of the 7-level sweep, n = 19, two instances per
+// wavefront, two wavefronts per SIMD, 99,900 steps): the Taylor kernel took
+// 260 ms on all 49 states. With the exchange through LDS the sweep takes 68
+// ms, bound by LDS (24 16-byte reads per wavefront and step at 8 CU-cycles);
+// with the broadcast exchange of series_row_kernel 57-61 ms, bound by VALU
+// issue (135 VALU instructions per wavefront and step, 110 of them the
+// multiply-adds). A wavefront alone on its SIMD issues a 64-bit multiply-add
+// every 8 cycles, two together one every 4.
 #include "ssmx_common.h"
 
 namespace {
@@ -26,7 +35,6 @@ using ssmx::kWave;
 using ssmx::node_time;
 using ssmx::set_error;
 using ssmx::swap_pair;
-using ssmx::wave_coef;
 using ssmx::wave_exchange;
 
 struct SParams {
@@ -50,6 +58,91 @@ constexpr int set_of(int j)
 {
     return j < J - 1 - j ? j : J - 1 - j;
 }
+
+// Drive factors of a wavefront's members, lane-parallel: entry
+// (b * members + member) * J + j of `fbuf` holds f_j of step b of the batch.
+// The lane's waveform segment stays in registers between batches (node
+// times only increase), and output and fine index come from the batch's
+// first step by one 32-bit division: a batch of 16 steps is otherwise a tenth
+// of the wavefront's instructions.
+template <int J>
+struct DriveFactors {
+    int MJ, B, my_b, my_j, cursor, begin, count;
+    double base;
+    ssmx_segment seg;
+
+    __device__ DriveFactors(const SParams &p, long sys, int members, int lane)
+    {
+        MJ = members * J;
+        B = kWave / MJ;
+        my_b = lane / MJ;
+        my_j = lane % J;
+        long wi = sys * members + (lane / J) % members;
+        if (wi >= p.d.n_inst)
+            wi = p.d.n_inst - 1;
+        const ssmx_wave *wv = p.waves + wi / p.d.wave_group;
+        base = wv->base[p.d.gen];
+        begin = wv->seg_begin[p.d.gen];
+        count = wv->seg_count[p.d.gen];
+        cursor = 0;
+        if (count > 0)
+            seg = p.segs[begin];
+    }
+
+    // wave_coef for times that only increase
+    __device__ double coefficient(const SParams &p, double t)
+    {
+#pragma clang fp contract(off)
+        while (cursor < count && !(t < seg.t_end)) {
+            ++cursor;
+            if (cursor < count)
+                seg = p.segs[begin + cursor];
+        }
+        double c = base;
+        if (cursor < count && !(t < seg.t_start))
+            c += seg.amp * cos(seg.omega * t + seg.phase);
+        return c;
+    }
+
+    // Steps i fine + k .. of the batch.
+    __device__ void fill(const SParams &p, int i, int k, int lane,
+                         double *fbuf)
+    {
+        const ssmx_series_desc &d = p.d;
+        const unsigned ahead = (unsigned)k + (unsigned)my_b;
+        const unsigned di = ahead / (unsigned)d.fine;
+        const int r = (int)(ahead - di * (unsigned)d.fine);
+        const long out = (long)i + di;
+        const bool on = my_b < B && out < d.n_out;
+        double f;
+        if constexpr (J <= 2) {
+            // schemes with as many nodes as exponentials: each lane
+            // evaluates one node, pairs of lanes exchange theirs
+            double c = 0.0;
+            if (on)
+                c = coefficient(p, node_time(d.t0, d.dt, d.fine, r, out,
+                                             p.nodes[my_j]));
+            if constexpr (J == 2) {
+                const double o = swap_pair(c);
+                const double c0 = my_j == 0 ? c : o;
+                const double c1 = my_j == 0 ? o : c;
+                f = fma(p.w[my_j * 2 + 1], c1, fma(p.w[my_j * 2], c0, 0.0));
+            } else {
+                f = fma(p.w[0], c, 0.0);
+            }
+        } else {
+            f = 0.0;
+            if (on)
+                for (int s = 0; s < d.n_node; ++s)
+                    f = fma(p.w[my_j * d.n_node + s],
+                            coefficient(p, node_time(d.t0, d.dt, d.fine, r,
+                                                     out, p.nodes[s])),
+                            f);
+        }
+        fbuf[lane] = d.h * f;
+        wave_exchange();
+    }
+};
 
 // One instance per `rows` lanes.  J = n_exp.
 template <int NA, int DA, int NB, int DB, int J>
@@ -126,58 +219,8 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
         wave_exchange();
     };
 
-    // drive factors, lane-parallel: entry (b * members + member) * J + j
-    // holds f_j of step b of the batch
-    const int MJ = d.members * J;
-    const int B = kWave / MJ;
-    const int my_b = lane / MJ;
-    const int my_j = lane % J;
-    const long total = (long)d.n_out * d.fine;
-    const ssmx_wave *wv;
-    {
-        long wi = sys * d.members + (lane / J) % d.members;
-        if (wi >= d.n_inst)
-            wi = d.n_inst - 1;
-        wv = p.waves + wi / d.wave_group;
-    }
-    int cursor = 0;
-    auto fill = [&](long first) {
-        const long mine = first + my_b;
-        const bool on = my_b < B && mine < total;
-        const long i = on ? mine / d.fine : 0;
-        const int rr = on ? (int)(mine - i * d.fine) : 0;
-        double f;
-        if constexpr (J <= 2) {
-            // schemes with as many nodes as exponentials: each lane
-            // evaluates one node, pairs of lanes exchange theirs
-            double c = 0.0;
-            if (on)
-                c = wave_coef(wv, p.segs, d.gen,
-                              node_time(d.t0, d.dt, d.fine, rr, i,
-                                        p.nodes[my_j]),
-                              cursor);
-            if constexpr (J == 2) {
-                const double o = swap_pair(c);
-                const double c0 = my_j == 0 ? c : o;
-                const double c1 = my_j == 0 ? o : c;
-                f = fma(p.w[my_j * 2 + 1], c1, fma(p.w[my_j * 2], c0, 0.0));
-            } else {
-                f = fma(p.w[0], c, 0.0);
-            }
-        } else {
-            f = 0.0;
-            if (on)
-                for (int s = 0; s < d.n_node; ++s)
-                    f = fma(p.w[my_j * d.n_node + s],
-                            wave_coef(wv, p.segs, d.gen,
-                                      node_time(d.t0, d.dt, d.fine, rr, i,
-                                                p.nodes[s]),
-                                      cursor),
-                            f);
-        }
-        fbuf[lane] = d.h * f;
-        wave_exchange();
-    };
+    DriveFactors<J> drive(p, sys, d.members, lane);
+    const int MJ = drive.MJ, B = drive.B;
 
     double xint = 0.0;
     const double half_h = 0.5 * d.h;
@@ -186,13 +229,12 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
     for (int j = 0; j < J; ++j)
         fc[j] = 0.0;
     wave_exchange();
-    long step = 0;
     int b = B;
     for (int i = 0; i < d.n_out; ++i) {
-        for (int k = 0; k < d.fine; ++k, ++step) {
+        for (int k = 0; k < d.fine; ++k) {
             if (b == B) {
                 b = 0;
-                fill(step);
+                drive.fill(p, i, k, lane, fbuf);
 #pragma unroll
                 for (int j = 0; j < J; ++j)
                     fc[j] = fbuf[q * J + j];
@@ -287,6 +329,201 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
     }
 }
 
+// a += wa[k] x(lane K + k), b += wb[k] x(lane K + k) for the lanes of each
+// 16-lane row, x broadcast within the row by the multiply-add's own DPP
+// operand (row_newbcast).  One block per group: a DPP operand may be read two
+// wait states after a VALU write, which the leading s_nop covers whatever
+// the compiler places in front; nothing in the block writes x.
+#define SSMX_BCAST(K, A, B)                                                 \
+    "v_fmac_f64_dpp %0, %2, " A " row_newbcast:" #K                         \
+    " row_mask:0xf bank_mask:0xf\n\t"                                       \
+    "v_fmac_f64_dpp %1, %2, " B " row_newbcast:" #K                         \
+    " row_mask:0xf bank_mask:0xf\n\t"
+
+__device__ __forceinline__ void bcast_0_3(double &a, double &b, double x,
+                                          const double *wa, const double *wb)
+{
+    asm("s_nop 1\n\t" SSMX_BCAST(0, "%3", "%7") SSMX_BCAST(1, "%4", "%8")
+            SSMX_BCAST(2, "%5", "%9") SSMX_BCAST(3, "%6", "%10")
+        : "+v"(a), "+v"(b)
+        : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wa[3]), "v"(wb[0]),
+          "v"(wb[1]), "v"(wb[2]), "v"(wb[3]));
+}
+
+__device__ __forceinline__ void bcast_4_7(double &a, double &b, double x,
+                                          const double *wa, const double *wb)
+{
+    asm("s_nop 1\n\t" SSMX_BCAST(4, "%3", "%7") SSMX_BCAST(5, "%4", "%8")
+            SSMX_BCAST(6, "%5", "%9") SSMX_BCAST(7, "%6", "%10")
+        : "+v"(a), "+v"(b)
+        : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wa[3]), "v"(wb[0]),
+          "v"(wb[1]), "v"(wb[2]), "v"(wb[3]));
+}
+
+__device__ __forceinline__ void bcast_8_10(double &a, double &b, double x,
+                                           const double *wa, const double *wb)
+{
+    asm("s_nop 1\n\t" SSMX_BCAST(8, "%3", "%6") SSMX_BCAST(9, "%4", "%7")
+            SSMX_BCAST(10, "%5", "%8")
+        : "+v"(a), "+v"(b)
+        : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wb[0]), "v"(wb[1]),
+          "v"(wb[2]));
+}
+#undef SSMX_BCAST
+
+// v of the lane 16 further or back, i.e. of the other row of its pair.
+__device__ __forceinline__ double swap_rows(double v, bool odd_row)
+{
+    const auto lo = __builtin_amdgcn_permlane16_swap(
+        __double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(
+        __double2hiint(v), __double2hiint(v), false, false);
+    // result 0 holds the even rows' values in both rows, result 1 the odd
+    // rows'
+    return odd_row ? __hiloint2double(hi[0], lo[0])
+                   : __hiloint2double(hi[1], lo[1]);
+}
+
+// The same exponentials for models of one sector pair, without LDS in the
+// exchange: a pair of 16-lane rows holds an instance, each row one sector.
+// A lane multiplies its row's broadcast components into two sums, its own
+// component's (own-sector coefficients) and that of the opposite sector's
+// component with its index, and the rows exchange the second sums.  Two
+// instances per wavefront.
+template <int N, int DA, int DB, int J>
+__global__ __launch_bounds__(kWave)
+__attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
+{
+    static_assert(N == 11, "the broadcast groups cover 11 components");
+    __shared__ double fbuf[kWave], red[kWave];
+    const ssmx_series_desc &d = p.d;
+    const int lane = threadIdx.x;
+    const int q = lane / 32, i16 = lane % 16;
+    const bool odd_row = (lane & 16) != 0;
+    const int rows = d.rows;
+    const int first = d.sectors > 1 ? d.sector_rows : rows;
+    const int own_rows = odd_row ? rows - first : first;
+    const int row0 = odd_row ? first : 0;
+    const int other_rows = rows - own_rows, other0 = odd_row ? 0 : first;
+    const bool has = q < d.members && i16 < own_rows;
+    const bool other = q < d.members && i16 < other_rows;
+
+    double ca[N][DA + 1], cb[N][DB + 1];
+#pragma unroll
+    for (int e = 0; e < N * (DA + 1); ++e)
+        ca[e / (DA + 1)][e % (DA + 1)] =
+            has ? p.table[(size_t)e * rows + row0 + i16] : 0.0;
+#pragma unroll
+    for (int e = 0; e < N * (DB + 1); ++e)
+        cb[e / (DB + 1)][e % (DB + 1)] =
+            other ? p.table[(size_t)(N * (DA + 1) + e) * rows + other0 + i16]
+                  : 0.0;
+
+    const long sys = blockIdx.x;
+    const long inst = sys * d.members + q;
+    const bool live = has && inst < d.n_inst;
+    const int state = has ? p.layout[4 * (row0 + i16) + 3] : 0;
+    double x = live ? p.rho0[(size_t)inst * d.n + state] : 0.0;
+    const bool read_full = (d.flags & SSMX_READ_FULL) != 0;
+    const bool read_int = (d.flags & SSMX_READ_INTEGRAL) != 0;
+    double ob0 = 0.0, ob1 = 0.0;
+    if (!read_full && live) {
+        ob0 = p.obs[state];
+        if (d.n_obs > 1)
+            ob1 = p.obs[d.n + state];
+    }
+    // sum over the member's 32 lanes (idle ones hold 0)
+    auto observe = [&](double v, long index) {
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1)
+            v += __shfl_xor(v, off, kWave);
+        if (live && lane % 32 == 0)
+            p.out[index] = v;
+    };
+
+    DriveFactors<J> drive(p, sys, d.members, lane);
+    const int MJ = drive.MJ, B = drive.B;
+    const int qf = q < d.members ? q : 0;
+    double xint = 0.0;
+    const double half_h = 0.5 * d.h;
+    double fc[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+        fc[j] = 0.0;
+    int b = B;
+    for (int i = 0; i < d.n_out; ++i) {
+        for (int k = 0; k < d.fine; ++k) {
+            if (b == B) {
+                b = 0;
+                drive.fill(p, i, k, lane, fbuf);
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+                    fc[j] = fbuf[qf * J + j];
+            }
+            double fn[J];
+            const int nb = b + 1 < B ? b + 1 : b;
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                fn[j] = fbuf[nb * MJ + qf * J + j];
+            const double before = x;
+#pragma unroll
+            for (int j = J - 1; j >= 0; --j) {
+                const double f = fc[j], u = f * f;
+                double wa[N], wb[N];
+#pragma unroll
+                for (int s = 0; s < N; ++s) {
+                    wa[s] = ca[s][DA];
+#pragma unroll
+                    for (int o = DA - 1; o >= 0; --o)
+                        wa[s] = fma(u, wa[s], ca[s][o]);
+                    wb[s] = cb[s][DB];
+#pragma unroll
+                    for (int o = DB - 1; o >= 0; --o)
+                        wb[s] = fma(u, wb[s], cb[s][o]);
+                }
+                double ya = 0.0, yb = 0.0;
+                bcast_0_3(ya, yb, x, wa, wb);
+                bcast_4_7(ya, yb, x, wa + 4, wb + 4);
+                bcast_8_10(ya, yb, x, wa + 8, wb + 8);
+                x += fma(f, swap_rows(yb, odd_row), ya);
+            }
+            if (read_int) {
+                ssmx::keep_branch();
+                xint = fma(half_h, before + x, xint);
+            }
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                fc[j] = fn[j];
+            ++b;
+        }
+        if (read_full) {
+            // components to LDS, then states in standard order
+            red[lane] = x;
+            wave_exchange();
+            for (int e = lane; e < d.members * d.n; e += kWave) {
+                const int m = e / d.n, s = e - m * d.n;
+                const long to = sys * d.members + m;
+                const int sp = p.state_pos[s];
+                if (to < d.n_inst)
+                    p.out[((size_t)to * d.n_out + i) * d.n + s] =
+                        sp < 0 ? 0.0
+                               : red[32 * m + 16 * (sp / d.sector) +
+                                     sp % d.sector];
+            }
+            wave_exchange();
+        } else if (!read_int) {
+            observe(ob0 * x, ((size_t)inst * d.n_out + i) * d.n_obs);
+            if (d.n_obs > 1)
+                observe(ob1 * x, ((size_t)inst * d.n_out + i) * d.n_obs + 1);
+        }
+    }
+    if (read_int) {
+        observe(ob0 * xint, (size_t)inst * d.n_obs);
+        if (d.n_obs > 1)
+            observe(ob1 * xint, (size_t)inst * d.n_obs + 1);
+    }
+}
+
 template <int NA, int DA, int NB, int DB, int J>
 int launch(const SParams &p, hipStream_t stream)
 {
@@ -294,6 +531,17 @@ int launch(const SParams &p, hipStream_t stream)
     const size_t lds = ((size_t)d.members * d.sectors * d.sector + 2 +
                         2 * kWave) * sizeof(double);
     const int systems = (d.n_inst + d.members - 1) / d.members;
+    if constexpr (NA == 11 && J <= 2) {
+        if (d.sector_rows > 0 && d.members <= 2) {
+            hipLaunchKernelGGL((series_row_kernel<NA, DA, DB, J>),
+                               dim3(systems), dim3(kWave), 0, stream, p);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess)
+                return set_error(SSMX_ELAUNCH, "series launch: %s",
+                                 hipGetErrorString(e));
+            return SSMX_OK;
+        }
+    }
     hipLaunchKernelGGL((series_kernel<NA, DA, NB, DB, J>), dim3(systems),
                        dim3(kWave), lds, stream, p);
     const hipError_t e = hipGetLastError();
@@ -362,6 +610,13 @@ int validate(const ssmx_series_desc *d)
         (d->sector & 1) || d->sectors < 1 || d->sectors > 2 * d->rows)
         return set_error(SSMX_EINVAL, "na=%d, nb=%d, %d sectors of %d",
                          d->na, d->nb, d->sectors, d->sector);
+    if (d->sector_rows < 0 || d->sector_rows > d->na ||
+        (d->sector_rows > 0 &&
+         (d->sectors > 2 || d->rows - d->sector_rows > d->na ||
+          d->rows < d->sector_rows ||
+          (d->sectors == 1 && d->rows != d->sector_rows))))
+        return set_error(SSMX_EINVAL, "sector_rows=%d of %d rows, %d sectors",
+                         d->sector_rows, d->rows, d->sectors);
     if (!(d->h > 0.0) || !(d->dt > 0.0))
         return set_error(SSMX_EINVAL, "h and dt must be positive");
     if ((size_t)d->members * d->sectors * d->sector * 8 > 48 * 1024)

@@ -326,7 +326,9 @@ class SeriesRun:
             n_out=n_out, n_obs=n_obs, flags=flags, gen=gen,
             wave_group=wave_group, na=model.size, da=plan[0],
             nb=model.size, db=plan[1], sector=model.pad,
-            sectors=model.n_sectors, h=dt / fine, t0=t0, dt=dt)
+            sectors=model.n_sectors,
+            sector_rows=model.members[0].size if model.n_sectors <= 2 else 0,
+            reserved=0, h=dt / fine, t0=t0, dt=dt)
         shape = {"full": (n_inst, n_out, n), "obs": (n_inst, n_out, n_obs),
                  "integral": (n_inst, n_obs)}[read]
         self.out = torch.empty(shape, dtype=torch.float64, device="cuda")

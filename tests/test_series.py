@@ -6,11 +6,15 @@ orders with the plan's tolerance; ``reachable`` with brute-force
 propagation; models the kernels do not cover must be refused.
 """
 
+import ctypes
+import os
+import subprocess
+
 import numpy as np
 import pytest
 from scipy.linalg import expm
 
-from superspinsim_amd import configs, quadratures
+from superspinsim_amd import _lib, configs, quadratures
 from superspinsim_amd.series import (
     SeriesModel, coefficient_matrices, reachable, split_sectors)
 
@@ -103,3 +107,28 @@ def test_uncovered_models_are_refused():
     assert SeriesModel.build(const, drive, w3, H) is None
     small = _pair(configs.odmr3(1))
     assert len(SeriesModel.build(*small, w5, H).sets) == 3
+
+
+def test_descriptor_layout_matches_header(tmp_path):
+    include = os.path.join(os.path.dirname(os.path.dirname(
+        os.path.abspath(__file__))), "include")
+    (tmp_path / "p.c").write_text(r'''
+#include <stddef.h>
+#include <stdio.h>
+#include "ssmx.h"
+int main(void) {
+  printf("%zu %zu %zu %zu\n", sizeof(ssmx_series_desc),
+         offsetof(ssmx_series_desc, wave_group),
+         offsetof(ssmx_series_desc, sector_rows),
+         offsetof(ssmx_series_desc, h));
+  return 0;
+}
+''')
+    exe = str(tmp_path / "p")
+    subprocess.run(["gcc", "-I", include, "-o", exe, str(tmp_path / "p.c")],
+                   check=True)
+    got = subprocess.run([exe], capture_output=True, text=True, check=True)
+    D = _lib.SeriesDesc
+    assert [int(v) for v in got.stdout.split()] == [
+        ctypes.sizeof(D), D.wave_group.offset, D.sector_rows.offset,
+        D.h.offset]
