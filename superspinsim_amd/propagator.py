@@ -592,17 +592,17 @@ def coefficient_samples(cmin, cmax, count=48, seed=0):
 
 def sample_exponents(mats, weights, coef_samples, h, rotating=False):
     """Dense A_j for node-coefficient samples (count, S, K), all j, of
-    generators ``mats`` ((K, n, n), or (S, K, n, n) in the rotating frame)."""
-    out = []
-    for c in np.asarray(coef_samples, dtype=_f64):
-        for row in weights:
-            if rotating:
-                f = c * (h * row[:, None])                     # (S, K)
-                out.append(np.tensordot(f, mats, axes=([0, 1], [0, 1])))
-            else:
-                cw = row @ c                                   # (K,)
-                out.append(h * np.tensordot(cw, mats, axes=(0, 0)))
-    return out
+    generators ``mats`` ((K, n, n), or (S, K, n, n) in the rotating frame):
+    (count * J, n, n)."""
+    c = np.asarray(coef_samples, dtype=_f64)
+    weights = np.asarray(weights, dtype=_f64)
+    n = mats.shape[-1]
+    if rotating:
+        f = c[:, None] * (h * weights[None, :, :, None])   # (count, J, S, K)
+    else:
+        f = h * np.matmul(weights, c)                      # (count, J, K)
+    f = f.reshape(f.shape[0] * weights.shape[0], -1)
+    return (f @ mats.reshape(f.shape[1], n * n)).reshape(-1, n, n)
 
 
 def taylor_plan(norm, tol=1e-17, max_taylor=_lib.MAX_TAYLOR):
@@ -628,6 +628,32 @@ def taylor_plan(norm, tol=1e-17, max_taylor=_lib.MAX_TAYLOR):
     return best
 
 
+def _power_norms(exps):
+    """1-norms of the exponents, then of their powers 2, 3, ..: yields
+    (count,) arrays.  Wide exponents (n > 64) are multiplied on the device,
+    where a power of the whole sample takes about a millisecond."""
+    if exps.shape[-1] > _lib.MAX_N:
+        torch = __import__("torch")
+        if torch.cuda.is_available():
+            dev = power = torch.from_numpy(exps).cuda()
+            while True:
+                yield power.abs().sum(dim=1).amax(dim=1).cpu().numpy()
+                power = torch.bmm(power, dev)
+    power = exps
+    while True:
+        yield np.abs(power).sum(axis=1).max(axis=1)
+        power = np.matmul(power, exps)
+
+
+def _truncation(norms, powers, m, fact):
+    """Largest bound of the terms beyond degree m over the samples (those
+    that are not NaN)."""
+    if np.any(norms >= m + 2):
+        return math.inf
+    return float(np.fmax.reduce(powers / fact / (1 - norms / (m + 2)),
+                                initial=0.0))
+
+
 def taylor_degrees_measured(exponents, tols, safety=8.0, max_taylor=None):
     """Least degree m with one substep meeting each tolerance of ``tols``.
 
@@ -640,21 +666,13 @@ def taylor_degrees_measured(exponents, tols, safety=8.0, max_taylor=None):
     if max_taylor is None:
         max_taylor = [_lib.MAX_TAYLOR] * len(tols)
     max_taylor = [int(m) for m in max_taylor]
-    exps = [np.asarray(a, dtype=_f64) for a in exponents]
-    norms = [float(np.abs(b).sum(axis=0).max()) for b in exps]
-    powers = [b.copy() for b in exps]
+    series = _power_norms(np.asarray(exponents, dtype=_f64))
+    norms = next(series)
     degrees = [None] * len(tols)
     fact = 1.0
     for m in range(1, max(max_taylor) + 1):
         fact *= (m + 1)
-        worst = 0.0
-        for k, b in enumerate(exps):
-            powers[k] = powers[k] @ b          # B^(m+1), every sample
-            if norms[k] >= m + 2:
-                worst = math.inf
-            elif worst < math.inf:
-                pn = float(np.abs(powers[k]).sum(axis=0).max())
-                worst = max(worst, pn / fact / (1 - norms[k] / (m + 2)))
+        worst = _truncation(norms, next(series), m, fact)
         for i, tol in enumerate(tols):
             if degrees[i] is None and m <= max_taylor[i] and \
                     safety * worst <= tol:
@@ -678,27 +696,31 @@ def taylor_plan_measured(exponents, tol=1e-17, safety=8.0,
     ||B||^i); ``safety`` covers coefficients between the samples.  Returns
     the cheapest (m * s) plan meeting ``tol`` with s <= ``max_substeps``.
     """
-    exps = [np.asarray(a, dtype=_f64) for a in exponents]
+    exps = np.asarray(exponents, dtype=_f64)
+    # the powers of A / s are those of A over s^k: one pass serves every s
+    series = _power_norms(exps)
+    powers = [next(series)]
+
+    def power(k):
+        while len(powers) < k:
+            powers.append(next(series))
+        return powers[k - 1]
+
     best = None
     s = 1
     while s <= max_substeps:
-        scaled = [a / s for a in exps]
-        norms = [float(np.abs(b).sum(axis=0).max()) for b in scaled]
-        powers = [b.copy() for b in scaled]
+        norms = powers[0] / s
         fact = 1.0
         for m in range(1, max_taylor + 1):
+            if best is not None and m * s >= best[0] * best[1]:
+                break                   # no longer cheaper
             fact *= (m + 1)
-            worst = 0.0
-            for k, b in enumerate(scaled):
-                powers[k] = powers[k] @ b          # B^(m+1), every sample
-                if norms[k] >= m + 2:
-                    worst = math.inf
-                elif worst < math.inf:
-                    pn = float(np.abs(powers[k]).sum(axis=0).max())
-                    worst = max(worst, pn / fact / (1 - norms[k] / (m + 2)))
-            if s * safety * worst <= tol:
-                if best is None or m * s < best[0] * best[1]:
-                    best = (m, s)
+            if np.any(norms >= m + 2):
+                continue
+            scale = float(s) ** (m + 1)
+            if s * safety * _truncation(norms, power(m + 1) / scale, m,
+                                        fact) <= tol:
+                best = (m, s)
                 break
         s *= 2
         if best is not None and best[0] * best[1] <= s:

@@ -264,14 +264,54 @@ def waveform_records(waves, n_gen, with_tags=False):
     return recs, seg_arr, index, scale
 
 
-def pack_waveforms(waves, n_gen):
-    """Device buffers (ssmx_wave array, ssmx_segment array) for instances."""
-    recs, seg_arr = waveform_records(waves, n_gen)
+def program_records(waves, program):
+    """``waveform_records`` of the waveforms over a kernel's generator list
+    (None: coefficient 1), generator by generator: the instances' segments
+    of one generator lie together."""
+    n_inst = len(waves)
+    recs = np.zeros(n_inst, dtype=WAVE_DTYPE)
+    base = np.array([w.base for w in waves])
+    parts = [np.zeros((1, 5), dtype=_f64)]      # never empty
+    at = 1
+    for k, g in enumerate(program):
+        recs["base"][:, k] = 1.0 if g is None else base[:, g]
+        recs["seg_begin"][:, k] = at
+        if g is None:
+            continue
+        rows = [w.segment_arrays(g)[0] for w in waves]
+        count = np.array([r.shape[0] for r in rows])
+        seg = np.concatenate(rows)
+        start = np.cumsum(count) - count
+        # rows of one instance in strictly ascending t_start, ends before the
+        # next one's start: else sorted and checked instance by instance
+        own = np.ones(max(seg.shape[0] - 1, 0), dtype=bool)
+        inner = start[(start > 0) & (start < seg.shape[0])]
+        own[inner - 1] = False
+        if not np.all((seg[1:, 0] > seg[:-1, 0])[own]):
+            rows = [r[np.lexsort(r.T[::-1])] for r in rows]
+            seg = np.concatenate(rows)
+        late = np.flatnonzero((seg[1:, 0] < seg[:-1, 1]) & own)
+        if late.size:
+            i = int(np.searchsorted(start, late[0], side="right")) - 1
+            raise ValueError(f"overlapping segments on generator {k} of "
+                             f"instance {i}")
+        recs["seg_begin"][:, k] = at + start
+        recs["seg_count"][:, k] = count
+        parts.append(seg)
+        at += seg.shape[0]
+    return recs, np.concatenate(parts)
+
+
+def stage_records(recs, seg_arr):
+    """Device buffers (ssmx_wave array, ssmx_segment array)."""
     torch = __import__("torch")
     rec_bytes = np.frombuffer(recs.tobytes(), dtype=np.uint8).copy()
-    d_waves = torch.from_numpy(rec_bytes).to("cuda")
-    d_segs = device_tensor(seg_arr)
-    return d_waves, d_segs
+    return torch.from_numpy(rec_bytes).to("cuda"), device_tensor(seg_arr)
+
+
+def pack_waveforms(waves, n_gen):
+    """Device buffers (ssmx_wave array, ssmx_segment array) for instances."""
+    return stage_records(*waveform_records(waves, n_gen))
 
 
 class BatchSimulator:
@@ -425,26 +465,26 @@ class BatchSimulator:
         matrix list: None for the folded sum of constant generators
         (coefficient 1), an int for a varying generator.
         """
-        amax = np.max([w.abs_max() for w in waves], axis=0)
+        base = np.array([w.base for w in waves])
+        amp = np.array([w._amplitude_max() for w in waves])
+        amax = np.max(np.abs(base) + amp, axis=0)
         active = [g for g in range(self.G) if amax[g] != 0] or [0]
         const = {}
         for g in active:
-            bases = {float(w.base[g]) for w in waves}
-            if len(bases) == 1 and not any(w.segment_count(g)
-                                           for w in waves):
-                const[g] = bases.pop()
+            if np.all(base[:, g] == base[0, g]) and not any(
+                    w.segment_count(g) for w in waves):
+                const[g] = float(base[0, g])
         program = ([None] if const else []) + \
             [g for g in active if g not in const]
         return active, const, program
 
     def coefficient_box(self, waves, program):
         """Node-coefficient samples (count, S, K) covering the batch."""
-        lo = np.array([1.0 if g is None else
-                       np.min([w.bounds()[0][g] for w in waves])
-                       for g in program])
-        hi = np.array([1.0 if g is None else
-                       np.max([w.bounds()[1][g] for w in waves])
-                       for g in program])
+        base = np.array([w.base for w in waves])
+        amp = np.array([w._amplitude_max() for w in waves])
+        low, high = (base - amp).min(axis=0), (base + amp).max(axis=0)
+        lo = np.array([1.0 if g is None else low[g] for g in program])
+        hi = np.array([1.0 if g is None else high[g] for g in program])
         S = self.nodes.size
         return coefficient_samples(np.broadcast_to(lo, (S, lo.size)),
                                    np.broadcast_to(hi, (S, hi.size)))
@@ -545,8 +585,7 @@ class BatchSimulator:
         """``SeriesRun`` of this (reduced) simulator; ``states`` are its
         states among the caller's ``n``."""
         model, plan = found
-        kwaves = self.kernel_waves(waves, program)
-        d_waves, d_segs = pack_waveforms(kwaves, len(program))
+        d_waves, d_segs = stage_records(*program_records(waves, program))
         gen = next((k for k, g in enumerate(program) if g is not None), 0)
         members = self.series_members(rho0.shape[0], model.n)
         return SeriesRun(model, plan, states, members, self.weights,
@@ -627,8 +666,8 @@ class BatchSimulator:
             obs_eff = obs @ self.V if self.rotating else obs
         n_obs = obs_eff.shape[0] if obs_eff is not None else 0
         k = self.pack_factor(n_inst, program, read, n_obs)
-        kwaves = self.kernel_waves(waves, program)
         if k > 1:
+            kwaves = self.kernel_waves(waves, program)
             # systems of k consecutive instances; the last is filled up with
             # copies of the last instance, whose results are dropped
             n_sys = -(-n_inst // k)
@@ -646,7 +685,9 @@ class BatchSimulator:
                     blk[j * n_obs:(j + 1) * n_obs,
                         j * self.n:(j + 1) * self.n] = obs_eff
                 obs_eff = blk
-        d_waves, d_segs = pack_waveforms(kwaves, kwaves[0].n_gen)
+            d_waves, d_segs = pack_waveforms(kwaves, kwaves[0].n_gen)
+        else:
+            d_waves, d_segs = stage_records(*program_records(waves, program))
         run = PreparedRun(self, prop, k, n_inst, read, N, m, s, time_start,
                           time_step, device_tensor(x0), d_waves, d_segs,
                           obs_eff)
