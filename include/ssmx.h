@@ -237,6 +237,63 @@ int ssmx_propagate_series(const ssmx_series_desc *desc,
                           const double *obs, double *out, void *stream);
 
 /*
+ * Uneven protocols through the series in the drive: instance i is the runs
+ * run_begin[i] .. run_begin[i + 1] - 1 in order of time, and writes the
+ * trapezoid integral of its readout rows over the runs with `read` set:
+ *   out[i][o] = sum over their steps k of (h/2) obs_o . (x_k + x_k+1).
+ * Node times are those of ssmx_propagate_queue (t0 + dt k + dt c_s).
+ *
+ * kind  SSMX_RUN_DRIVEN: `count` steps from step `first` with table set
+ *       set0 for every exponential and the drive from the waveform;
+ *       SSMX_RUN_SPLIT: the same with set0 for exponential 0 and set1 for
+ *       exponential 1 (a constant part that changes between the nodes);
+ *       SSMX_RUN_FREE: `count` steps without drive through the powers of
+ *       power set set0.
+ * Both halves of the wavefront hold the state, 16-lane row 0 (and 2) the
+ * first sector, row 1 (and 3) the second, component i in lane i; half 0
+ * multiplies the components 0..5 of a row, half 1 the components 6..10.
+ * lanes   int32 [64]: state of the lane's component, -1 in idle lanes
+ * table   double [sets][6 (da + 1) + 6 (db + 1)][64]: entry
+ *       (s (da + 1) + k) is E_2k's coefficient of the half's component s of
+ *       the lane's sector in the lane's own component, then
+ *       (s (db + 1) + k) E_(2k+1)'s of the same component in the opposite
+ *       sector's component of the lane's index; 0 where there is none
+ * powers  double [power sets][levels][2][6][64]: E^(2^b) - I of the undriven
+ *       step E, then (h/2) sum_{k < 2^b} (E^k + E^(k+1)), laid out as the
+ *       own-sector coefficients; count < 2^levels
+ * desc    n_inst protocols; fine, members, wave_group 1; flags
+ *       SSMX_READ_INTEGRAL; n_exp 1..2, na = nb = 11, at most two sectors
+ *       (sector_rows > 0); n_out unused
+ * order, counter, n_waves, waves_per_block  as ssmx_propagate_queue;
+ *       counter NULL: wavefront w runs entries w, w + n_waves, ..
+ * waves, segments, rho0, obs  as ssmx_propagate_series
+ *
+ * No counterpart in the reference (one simulate call per protocol).
+ */
+#define SSMX_RUN_DRIVEN 0
+#define SSMX_RUN_SPLIT 1
+#define SSMX_RUN_FREE 2
+
+typedef struct ssmx_run {
+    int64_t first;
+    int64_t count;
+    int32_t kind;
+    int32_t set0;
+    int32_t set1;
+    int32_t read;
+} ssmx_run;
+
+int ssmx_series_queue(const ssmx_series_desc *desc, const int32_t *lanes,
+                      const double *table, const double *powers,
+                      int32_t levels, const double *cf_weights,
+                      const double *cf_nodes, const ssmx_wave *waves,
+                      const ssmx_segment *segments, const double *rho0,
+                      const double *obs, const ssmx_run *runs,
+                      const int32_t *run_begin, const int32_t *order,
+                      int32_t *counter, int32_t n_waves,
+                      int32_t waves_per_block, double *out, void *stream);
+
+/*
  * The reference's non-residual exponential (use_residual=False).
  *
  * Each exponential is (I + A / scale)^(2^squarings) with scale = 4^R and

@@ -115,7 +115,7 @@ class Wave(ctypes.Structure):
 
 
 #: every symbol include/ssmx.h declares
-EXPORTS = ("ssmx_propagate", "ssmx_propagate_series",
+EXPORTS = ("ssmx_propagate", "ssmx_propagate_series", "ssmx_series_queue",
            "ssmx_propagate_dense", "ssmx_chunk_combine",
            "ssmx_propagate_queue",
            "ssmx_propagate_queue_noalloc", "ssmx_adjoint",
@@ -151,6 +151,10 @@ def load():
     lib.ssmx_propagate_series.argtypes = [ctypes.POINTER(SeriesDesc)] + \
         [vp] * 11
     lib.ssmx_propagate_series.restype = ctypes.c_int
+    lib.ssmx_series_queue.argtypes = (
+        [ctypes.POINTER(SeriesDesc)] + [vp] * 3 + [ctypes.c_int32] +
+        [vp] * 10 + [ctypes.c_int32, ctypes.c_int32, vp, vp])
+    lib.ssmx_series_queue.restype = ctypes.c_int
     lib.ssmx_propagate_queue.argtypes = (
         [ctypes.POINTER(PropagateDesc)] + [vp] * 13 +
         [ctypes.c_int32, ctypes.c_int32, vp, vp])

@@ -91,9 +91,12 @@ def tune(batch, trial_steps=20000, repeats=2, use_cache=True, verbose=False):
     torch = _torch()
     cache = _load_cache() if use_cache else {}
     key = problem_key(batch)
-    samples = batch.sim.coefficient_box(batch.waves_host,
-                                        batch.program)
-    plans = plan_candidates(batch, samples)
+    if batch.series is not None:
+        # runs of the series in the drive: only the grid's shape is open
+        plans = [tuple(batch.plan_default)]
+    else:
+        plans = plan_candidates(batch, batch.sim.coefficient_box(
+            batch.waves_host, batch.program))
     if use_cache and key in cache:
         best = cache[key]
         if (best["taylor"], best["substeps"]) in [tuple(p) for p in plans]:

@@ -59,6 +59,13 @@ constexpr int set_of(int j)
     return j < J - 1 - j ? j : J - 1 - j;
 }
 
+// Node times and weights of a run.
+struct Clock {
+    double t0, dt, h;
+    int fine, n_node;
+    const double *nodes, *w;
+};
+
 // Drive factors of a wavefront's members, lane-parallel: entry
 // (b * members + member) * J + j of `fbuf` holds f_j of step b of the batch.
 // The lane's waveform segment stays in registers between batches (node
@@ -71,32 +78,30 @@ struct DriveFactors {
     double base;
     ssmx_segment seg;
 
-    __device__ DriveFactors(const SParams &p, long sys, int members, int lane)
+    // `wv` is the waveform of the lane's entry (member (lane / J) % members)
+    __device__ DriveFactors(const ssmx_wave *wv, const ssmx_segment *segs,
+                            int gen, int members, int lane)
     {
         MJ = members * J;
         B = kWave / MJ;
         my_b = lane / MJ;
         my_j = lane % J;
-        long wi = sys * members + (lane / J) % members;
-        if (wi >= p.d.n_inst)
-            wi = p.d.n_inst - 1;
-        const ssmx_wave *wv = p.waves + wi / p.d.wave_group;
-        base = wv->base[p.d.gen];
-        begin = wv->seg_begin[p.d.gen];
-        count = wv->seg_count[p.d.gen];
+        base = wv->base[gen];
+        begin = wv->seg_begin[gen];
+        count = wv->seg_count[gen];
         cursor = 0;
         if (count > 0)
-            seg = p.segs[begin];
+            seg = segs[begin];
     }
 
     // wave_coef for times that only increase
-    __device__ double coefficient(const SParams &p, double t)
+    __device__ double coefficient(const ssmx_segment *segs, double t)
     {
 #pragma clang fp contract(off)
         while (cursor < count && !(t < seg.t_end)) {
             ++cursor;
             if (cursor < count)
-                seg = p.segs[begin + cursor];
+                seg = segs[begin + cursor];
         }
         double c = base;
         if (cursor < count && !(t < seg.t_start))
@@ -104,45 +109,60 @@ struct DriveFactors {
         return c;
     }
 
-    // Steps i fine + k .. of the batch.
-    __device__ void fill(const SParams &p, int i, int k, int lane,
-                         double *fbuf)
+    // The steps from output i, fine step k on, `left` at most.
+    __device__ void fill(const Clock &c, const ssmx_segment *segs, long i,
+                         int k, long left, int lane, double *fbuf)
     {
-        const ssmx_series_desc &d = p.d;
         const unsigned ahead = (unsigned)k + (unsigned)my_b;
-        const unsigned di = ahead / (unsigned)d.fine;
-        const int r = (int)(ahead - di * (unsigned)d.fine);
-        const long out = (long)i + di;
-        const bool on = my_b < B && out < d.n_out;
+        const unsigned di = ahead / (unsigned)c.fine;
+        const int r = (int)(ahead - di * (unsigned)c.fine);
+        const long out = i + di;
+        const bool on = my_b < B && my_b < left;
         double f;
         if constexpr (J <= 2) {
             // schemes with as many nodes as exponentials: each lane
             // evaluates one node, pairs of lanes exchange theirs
-            double c = 0.0;
+            double v = 0.0;
             if (on)
-                c = coefficient(p, node_time(d.t0, d.dt, d.fine, r, out,
-                                             p.nodes[my_j]));
+                v = coefficient(segs, node_time(c.t0, c.dt, c.fine, r, out,
+                                                c.nodes[my_j]));
             if constexpr (J == 2) {
-                const double o = swap_pair(c);
-                const double c0 = my_j == 0 ? c : o;
-                const double c1 = my_j == 0 ? o : c;
-                f = fma(p.w[my_j * 2 + 1], c1, fma(p.w[my_j * 2], c0, 0.0));
+                const double o = swap_pair(v);
+                const double c0 = my_j == 0 ? v : o;
+                const double c1 = my_j == 0 ? o : v;
+                f = fma(c.w[my_j * 2 + 1], c1, fma(c.w[my_j * 2], c0, 0.0));
             } else {
-                f = fma(p.w[0], c, 0.0);
+                f = fma(c.w[0], v, 0.0);
             }
         } else {
             f = 0.0;
             if (on)
-                for (int s = 0; s < d.n_node; ++s)
-                    f = fma(p.w[my_j * d.n_node + s],
-                            coefficient(p, node_time(d.t0, d.dt, d.fine, r,
-                                                     out, p.nodes[s])),
+                for (int s = 0; s < c.n_node; ++s)
+                    f = fma(c.w[my_j * c.n_node + s],
+                            coefficient(segs, node_time(c.t0, c.dt, c.fine,
+                                                        r, out,
+                                                        c.nodes[s])),
                             f);
         }
-        fbuf[lane] = d.h * f;
+        fbuf[lane] = c.h * f;
         wave_exchange();
     }
 };
+
+// Waveform of a lane's drive-factor entry in a sweep.
+template <int J>
+__device__ const ssmx_wave *entry_wave(const SParams &p, long sys, int lane)
+{
+    long wi = sys * p.d.members + (lane / J) % p.d.members;
+    if (wi >= p.d.n_inst)
+        wi = p.d.n_inst - 1;
+    return p.waves + wi / p.d.wave_group;
+}
+
+__device__ __forceinline__ Clock clock_of(const SParams &p)
+{
+    return Clock{p.d.t0, p.d.dt, p.d.h, p.d.fine, p.d.n_node, p.nodes, p.w};
+}
 
 // One instance per `rows` lanes.  J = n_exp.
 template <int NA, int DA, int NB, int DB, int J>
@@ -219,7 +239,10 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
         wave_exchange();
     };
 
-    DriveFactors<J> drive(p, sys, d.members, lane);
+    const Clock clk = clock_of(p);
+    DriveFactors<J> drive(entry_wave<J>(p, sys, lane), p.segs, d.gen,
+                          d.members, lane);
+    const long total = (long)d.n_out * d.fine;
     const int MJ = drive.MJ, B = drive.B;
 
     double xint = 0.0;
@@ -234,7 +257,8 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
         for (int k = 0; k < d.fine; ++k) {
             if (b == B) {
                 b = 0;
-                drive.fill(p, i, k, lane, fbuf);
+                drive.fill(clk, p.segs, i, k,
+                           total - ((long)i * d.fine + k), lane, fbuf);
 #pragma unroll
                 for (int j = 0; j < J; ++j)
                     fc[j] = fbuf[q * J + j];
@@ -329,47 +353,73 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
     }
 }
 
-// a += wa[k] x(lane K + k), b += wb[k] x(lane K + k) for the lanes of each
-// 16-lane row, x broadcast within the row by the multiply-add's own DPP
-// operand (row_newbcast).  One block per group: a DPP operand may be read two
-// wait states after a VALU write, which the leading s_nop covers whatever
-// the compiler places in front; nothing in the block writes x.
+// a += wa[k] x(lane K0 + k), b += wb[k] x(lane K0 + k), k < N, for the lanes
+// of each 16-lane row: x is broadcast within the row by the multiply-add's own
+// DPP operand (row_newbcast).  One block per group of up to four: a DPP operand
+// may be read two wait states after a VALU write, which the leading s_nop
+// covers whatever the compiler places in front; nothing in the block writes
+// x.
 #define SSMX_BCAST(K, A, B)                                                 \
-    "v_fmac_f64_dpp %0, %2, " A " row_newbcast:" #K                         \
+    "v_fmac_f64_dpp %0, %2, " A " row_newbcast:" K                          \
     " row_mask:0xf bank_mask:0xf\n\t"                                       \
-    "v_fmac_f64_dpp %1, %2, " B " row_newbcast:" #K                         \
+    "v_fmac_f64_dpp %1, %2, " B " row_newbcast:" K                          \
     " row_mask:0xf bank_mask:0xf\n\t"
 
-__device__ __forceinline__ void bcast_0_3(double &a, double &b, double x,
+template <int K0, int N>
+__device__ __forceinline__ void bcast_fma(double &a, double &b, double x,
                                           const double *wa, const double *wb)
 {
-    asm("s_nop 1\n\t" SSMX_BCAST(0, "%3", "%7") SSMX_BCAST(1, "%4", "%8")
-            SSMX_BCAST(2, "%5", "%9") SSMX_BCAST(3, "%6", "%10")
-        : "+v"(a), "+v"(b)
-        : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wa[3]), "v"(wb[0]),
-          "v"(wb[1]), "v"(wb[2]), "v"(wb[3]));
-}
-
-__device__ __forceinline__ void bcast_4_7(double &a, double &b, double x,
-                                          const double *wa, const double *wb)
-{
-    asm("s_nop 1\n\t" SSMX_BCAST(4, "%3", "%7") SSMX_BCAST(5, "%4", "%8")
-            SSMX_BCAST(6, "%5", "%9") SSMX_BCAST(7, "%6", "%10")
-        : "+v"(a), "+v"(b)
-        : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wa[3]), "v"(wb[0]),
-          "v"(wb[1]), "v"(wb[2]), "v"(wb[3]));
-}
-
-__device__ __forceinline__ void bcast_8_10(double &a, double &b, double x,
-                                           const double *wa, const double *wb)
-{
-    asm("s_nop 1\n\t" SSMX_BCAST(8, "%3", "%6") SSMX_BCAST(9, "%4", "%7")
-            SSMX_BCAST(10, "%5", "%8")
-        : "+v"(a), "+v"(b)
-        : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wb[0]), "v"(wb[1]),
-          "v"(wb[2]));
+    if constexpr (N >= 4) {
+        asm("s_nop 1\n\t" SSMX_BCAST("%11", "%3", "%7")
+                SSMX_BCAST("%12", "%4", "%8") SSMX_BCAST("%13", "%5", "%9")
+                    SSMX_BCAST("%14", "%6", "%10")
+            : "+v"(a), "+v"(b)
+            : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wa[3]),
+              "v"(wb[0]), "v"(wb[1]), "v"(wb[2]), "v"(wb[3]), "n"(K0),
+              "n"(K0 + 1), "n"(K0 + 2), "n"(K0 + 3));
+        bcast_fma<K0 + 4, N - 4>(a, b, x, wa + 4, wb + 4);
+    } else if constexpr (N >= 2) {
+        asm("s_nop 1\n\t" SSMX_BCAST("%7", "%3", "%5")
+                SSMX_BCAST("%8", "%4", "%6")
+            : "+v"(a), "+v"(b)
+            : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wb[0]), "v"(wb[1]),
+              "n"(K0), "n"(K0 + 1));
+        bcast_fma<K0 + 2, N - 2>(a, b, x, wa + 2, wb + 2);
+    } else if constexpr (N == 1) {
+        asm("s_nop 1\n\t" SSMX_BCAST("%5", "%3", "%4")
+            : "+v"(a), "+v"(b)
+            : "v"(x), "v"(wa[0]), "v"(wb[0]), "n"(K0));
+    }
 }
 #undef SSMX_BCAST
+
+// a += w[k] x(lane K0 + k), k < N.
+template <int K0, int N>
+__device__ __forceinline__ void bcast_fma1(double &a, double x,
+                                           const double *w)
+{
+    if constexpr (N >= 1) {
+        asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3"
+            " row_mask:0xf bank_mask:0xf"
+            : "+v"(a)
+            : "v"(x), "v"(w[0]), "n"(K0));
+        bcast_fma1<K0 + 1, N - 1>(a, x, w + 1);
+    }
+}
+
+// Coefficients of one exponential for one lane: P_s(u) = sum_o c[s][o] u^o.
+template <int N, int D>
+__device__ __forceinline__ void horner(double (&w)[N],
+                                       const double (&c)[N][D + 1], double u)
+{
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+        w[s] = c[s][D];
+#pragma unroll
+        for (int o = D - 1; o >= 0; --o)
+            w[s] = fma(u, w[s], c[s][o]);
+    }
+}
 
 // v of the lane 16 further or back, i.e. of the other row of its pair.
 __device__ __forceinline__ double swap_rows(double v, bool odd_row)
@@ -394,7 +444,6 @@ template <int N, int DA, int DB, int J>
 __global__ __launch_bounds__(kWave)
 __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
 {
-    static_assert(N == 11, "the broadcast groups cover 11 components");
     __shared__ double fbuf[kWave], red[kWave];
     const ssmx_series_desc &d = p.d;
     const int lane = threadIdx.x;
@@ -441,7 +490,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
             p.out[index] = v;
     };
 
-    DriveFactors<J> drive(p, sys, d.members, lane);
+    const Clock clk = clock_of(p);
+    DriveFactors<J> drive(entry_wave<J>(p, sys, lane), p.segs, d.gen,
+                          d.members, lane);
+    const long total = (long)d.n_out * d.fine;
     const int MJ = drive.MJ, B = drive.B;
     const int qf = q < d.members ? q : 0;
     double xint = 0.0;
@@ -455,7 +507,8 @@ __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
         for (int k = 0; k < d.fine; ++k) {
             if (b == B) {
                 b = 0;
-                drive.fill(p, i, k, lane, fbuf);
+                drive.fill(clk, p.segs, i, k,
+                           total - ((long)i * d.fine + k), lane, fbuf);
 #pragma unroll
                 for (int j = 0; j < J; ++j)
                     fc[j] = fbuf[qf * J + j];
@@ -470,21 +523,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
             for (int j = J - 1; j >= 0; --j) {
                 const double f = fc[j], u = f * f;
                 double wa[N], wb[N];
-#pragma unroll
-                for (int s = 0; s < N; ++s) {
-                    wa[s] = ca[s][DA];
-#pragma unroll
-                    for (int o = DA - 1; o >= 0; --o)
-                        wa[s] = fma(u, wa[s], ca[s][o]);
-                    wb[s] = cb[s][DB];
-#pragma unroll
-                    for (int o = DB - 1; o >= 0; --o)
-                        wb[s] = fma(u, wb[s], cb[s][o]);
-                }
+                horner<N, DA>(wa, ca, u);
+                horner<N, DB>(wb, cb, u);
                 double ya = 0.0, yb = 0.0;
-                bcast_0_3(ya, yb, x, wa, wb);
-                bcast_4_7(ya, yb, x, wa + 4, wb + 4);
-                bcast_8_10(ya, yb, x, wa + 8, wb + 8);
+                bcast_fma<0, N>(ya, yb, x, wa, wb);
                 x += fma(f, swap_rows(yb, odd_row), ya);
             }
             if (read_int) {
@@ -521,6 +563,228 @@ __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
         observe(ob0 * xint, (size_t)inst * d.n_obs);
         if (d.n_obs > 1)
             observe(ob1 * xint, (size_t)inst * d.n_obs + 1);
+    }
+}
+
+// Sum of v over the wavefront's halves (lane, lane ^ 32), in every lane.
+__device__ __forceinline__ double sum_halves(double v)
+{
+    const auto lo = __builtin_amdgcn_permlane32_swap(
+        __double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(
+        __double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
+// One instance on the whole wavefront: both halves hold the state (rows as
+// in series_row_kernel); the first half multiplies the first S = ceil(N / 2)
+// components of its rows, the second half the others, which a rotation within
+// the row brings to the same lanes.
+template <int N>
+struct Halves {
+    static constexpr int S = (N + 1) / 2;
+
+    // x in the first half, x of lane + S (of the row) in the second
+    static __device__ __forceinline__ double shifted(double x)
+    {
+        constexpr int kRotate = 0x120 + 16 - S;     // row_ror
+        const int lo = __double2loint(x), hi = __double2hiint(x);
+        return __hiloint2double(
+            __builtin_amdgcn_update_dpp(hi, hi, kRotate, 0xC, 0xF, false),
+            __builtin_amdgcn_update_dpp(lo, lo, kRotate, 0xC, 0xF, false));
+    }
+
+    // x <- exp(A) x
+    template <int DA, int DB>
+    static __device__ __forceinline__ void exponential(
+        double &x, double f, const double (&ca)[S][DA + 1],
+        const double (&cb)[S][DB + 1], bool odd_row)
+    {
+        const double u = f * f;
+        double wa[S], wb[S];
+        horner<S, DA>(wa, ca, u);
+        horner<S, DB>(wb, cb, u);
+        double ya = 0.0, yb = 0.0;
+        bcast_fma<0, S>(ya, yb, shifted(x), wa, wb);
+        x += sum_halves(fma(f, swap_rows(yb, odd_row), ya));
+    }
+
+    // M x for a matrix within the sectors
+    static __device__ __forceinline__ double within(double xs,
+                                                    const double (&m)[S])
+    {
+        double y = 0.0;
+        bcast_fma1<0, S>(y, xs, m);
+        return sum_halves(y);
+    }
+};
+
+struct QSParams {
+    ssmx_series_desc d;
+    const int32_t *lanes;
+    const double *table;
+    const double *powers;
+    const double *w;
+    const double *nodes;
+    const ssmx_wave *waves;
+    const ssmx_segment *segs;
+    const double *rho0;
+    const double *obs;
+    const ssmx_run *runs;
+    const int32_t *run_begin;
+    const int32_t *order;
+    int32_t *counter;
+    double *out;
+    int32_t levels;
+    int32_t n_waves;
+};
+
+// Uneven protocols, one per wavefront at a time (ssmx_series_queue).
+//
+// A protocol is a list of runs.  Driven runs go step by step.  In a free run
+// every step is the same matrix, so its 2^b-th powers (formed on the host) take
+// the state through it in one product per set bit of the step count, and the
+// readout integral over 2^b steps is a matrix as well: the 100,000s of steps
+// of free precession and the readout window become some twenty products.
+// 2,048 protocols of 58k-742k steps (at most 200k of them driven) took 1046 ms
+// step by step with the Taylor action, 68 ms so: the driven steps at two
+// wavefronts per SIMD, 105 VALU instructions each.
+template <int N, int DA, int DB, int J>
+__global__ __launch_bounds__(kWave * 8) __attribute__((
+    amdgpu_waves_per_eu(2))) void series_queue_kernel(QSParams p)
+{
+    constexpr int S = Halves<N>::S;
+    constexpr int kEntries = S * (DA + 1) + S * (DB + 1);
+    __shared__ double fbufs[8][kWave];
+    const ssmx_series_desc &d = p.d;
+    const int lane = threadIdx.x % kWave;
+    double *fbuf = fbufs[threadIdx.x / kWave];
+    const bool odd_row = (lane & 16) != 0;
+    const int state = p.lanes[lane];
+    const bool has = state >= 0;
+    const double ob0 = has ? p.obs[state] : 0.0;
+    const double ob1 = has && d.n_obs > 1 ? p.obs[d.n + state] : 0.0;
+    const Clock clk{d.t0, d.dt, d.h, 1, d.n_node, p.nodes, p.w};
+    const double half_h = 0.5 * d.h;
+
+    // The opaque lane offset keeps the table addresses out of the run loop's
+    // registers (they would be hoisted and spill).
+    double ca[S][DA + 1], cb[S][DB + 1];
+    auto load_set = [&](int set) {
+        int at = lane;
+        asm volatile("" : "+v"(at));
+        const double *t = p.table + (size_t)set * kEntries * kWave;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+#pragma unroll
+            for (int o = 0; o <= DA; ++o)
+                ca[s][o] = t[(s * (DA + 1) + o) * kWave + at];
+#pragma unroll
+            for (int o = 0; o <= DB; ++o)
+                cb[s][o] = t[(S * (DA + 1) + s * (DB + 1) + o) * kWave + at];
+        }
+    };
+    auto load_power = [&](double (&m)[S], int set, int level, int which) {
+        int at = lane;
+        asm volatile("" : "+v"(at));
+        const double *t =
+            p.powers +
+            (((size_t)set * p.levels + level) * 2 + which) * S * kWave;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            m[s] = t[s * kWave + at];
+    };
+
+    int entry = (int)(blockIdx.x * (blockDim.x / kWave) +
+                      threadIdx.x / kWave);
+    if (entry >= p.n_waves)
+        return;
+    for (;;) {
+        if (p.counter) {
+            int got = 0;
+            if (lane == 0)
+                got = atomicAdd(p.counter, 1);
+            entry = __builtin_amdgcn_readfirstlane(got);
+        }
+        if (entry >= d.n_inst)
+            return;
+        const int inst = __builtin_amdgcn_readfirstlane(p.order[entry]);
+        DriveFactors<J> drive(p.waves + inst, p.segs, d.gen, 1, lane);
+        const int B = drive.B;
+        double x = has ? p.rho0[(size_t)inst * d.n + state] : 0.0;
+        double xint = 0.0;
+        int loaded = -1;
+        const int end = p.run_begin[inst + 1];
+        for (int ri = p.run_begin[inst]; ri < end; ++ri) {
+            const ssmx_run run = p.runs[ri];
+            const bool reads = run.read != 0;
+            if (run.kind == SSMX_RUN_FREE) {
+                long left = run.count;
+                for (int level = 0; left > 0; ++level, left >>= 1) {
+                    if (!(left & 1))
+                        continue;
+                    double m[S];
+                    const double xs = Halves<N>::shifted(x);
+                    if (reads) {
+                        load_power(m, run.set0, level, 1);
+                        xint += Halves<N>::within(xs, m);
+                    }
+                    load_power(m, run.set0, level, 0);
+                    x += Halves<N>::within(xs, m);
+                }
+                continue;
+            }
+            for (long done = 0; done < run.count;) {
+                const long left = run.count - done;
+                drive.fill(clk, p.segs, run.first + done, 0, left, lane,
+                           fbuf);
+                const int steps = left < B ? (int)left : B;
+                double fc[J];
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+                    fc[j] = fbuf[j];
+                for (int b = 0; b < steps; ++b) {
+                    // the next step's factors, read while this runs
+                    const int nb = b + 1 < B ? b + 1 : b;
+                    double fn[J];
+#pragma unroll
+                    for (int j = 0; j < J; ++j)
+                        fn[j] = fbuf[nb * J + j];
+                    const double before = x;
+#pragma unroll
+                    for (int j = J - 1; j >= 0; --j) {
+                        // (set1 differs from set0 in split runs only)
+                        const int set = j == 0 ? run.set0 : run.set1;
+                        if (set != loaded) {
+                            load_set(set);
+                            loaded = set;
+                        }
+                        Halves<N>::template exponential<DA, DB>(
+                            x, fc[j], ca, cb, odd_row);
+                    }
+                    if (reads) {
+                        ssmx::keep_branch();
+                        xint = fma(half_h, before + x, xint);
+                    }
+#pragma unroll
+                    for (int j = 0; j < J; ++j)
+                        fc[j] = fn[j];
+                }
+                wave_exchange();
+                done += steps;
+            }
+        }
+        for (int o = 0; o < d.n_obs; ++o) {
+            double v = (o == 0 ? ob0 : ob1) * xint;
+#pragma unroll
+            for (int off = 16; off > 0; off >>= 1)
+                v += __shfl_xor(v, off, kWave);
+            if (lane == 0)
+                p.out[(size_t)inst * d.n_obs + o] = v;
+        }
+        if (!p.counter) {
+            entry += p.n_waves;
+        }
     }
 }
 
@@ -626,6 +890,89 @@ int validate(const ssmx_series_desc *d)
 }
 
 }  // namespace
+
+namespace {
+
+template <int DA, int DB, int J>
+int launch_queue(const QSParams &p, int waves_per_block, hipStream_t stream)
+{
+    const int blocks = (p.n_waves + waves_per_block - 1) / waves_per_block;
+    hipLaunchKernelGGL((series_queue_kernel<11, DA, DB, J>), dim3(blocks),
+                       dim3(kWave * waves_per_block), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return set_error(SSMX_ELAUNCH, "series queue launch: %s",
+                         hipGetErrorString(e));
+    return SSMX_OK;
+}
+
+template <int DA, int DB>
+int launch_queue_scheme(const QSParams &p, int waves_per_block,
+                        hipStream_t stream)
+{
+    return p.d.n_exp == 1 ? launch_queue<DA, DB, 1>(p, waves_per_block, stream)
+                          : launch_queue<DA, DB, 2>(p, waves_per_block,
+                                                    stream);
+}
+
+}  // namespace
+
+extern "C" int ssmx_series_queue(
+    const ssmx_series_desc *desc, const int32_t *lanes, const double *table,
+    const double *powers, int32_t levels, const double *cf_weights,
+    const double *cf_nodes, const ssmx_wave *waves,
+    const ssmx_segment *segments, const double *rho0, const double *obs,
+    const ssmx_run *runs, const int32_t *run_begin, const int32_t *order,
+    int32_t *counter, int32_t n_waves, int32_t waves_per_block, double *out,
+    void *stream)
+{
+    ssmx::error_buffer()[0] = '\0';
+    const int rc = validate(desc);
+    if (rc)
+        return rc;
+    if (desc->flags != SSMX_READ_INTEGRAL || desc->na != 11 ||
+        desc->n_exp > 2 || desc->sector_rows < 1 || desc->members != 1 ||
+        desc->wave_group != 1 || desc->fine != 1)
+        return set_error(SSMX_EINVAL, "series queue: flags=%d, na=%d, "
+                         "n_exp=%d, sector_rows=%d, members=%d",
+                         desc->flags, desc->na, desc->n_exp,
+                         desc->sector_rows, desc->members);
+    if (n_waves < 1 || waves_per_block < 1 || waves_per_block > 8 ||
+        levels < 0 || levels > 62)
+        return set_error(SSMX_EINVAL, "n_waves=%d, waves_per_block=%d, "
+                         "levels=%d", n_waves, waves_per_block, levels);
+    if (!lanes || !table || !powers || !cf_weights || !cf_nodes || !waves ||
+        !segments || !rho0 || !obs || !runs || !run_begin || !order || !out)
+        return set_error(SSMX_EINVAL, "null required pointer");
+    QSParams p;
+    p.d = *desc;
+    p.lanes = lanes;
+    p.table = table;
+    p.powers = powers;
+    p.w = cf_weights;
+    p.nodes = cf_nodes;
+    p.waves = waves;
+    p.segs = segments;
+    p.rho0 = rho0;
+    p.obs = obs;
+    p.runs = runs;
+    p.run_begin = run_begin;
+    p.order = order;
+    p.counter = counter;
+    p.out = out;
+    p.levels = levels;
+    p.n_waves = n_waves;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int da = desc->da, db = desc->db;
+    if (da == 1 && db == 1)
+        return launch_queue_scheme<1, 1>(p, waves_per_block, s);
+    if (da == 2 && db == 1)
+        return launch_queue_scheme<2, 1>(p, waves_per_block, s);
+    if (da == 2 && db == 2)
+        return launch_queue_scheme<2, 2>(p, waves_per_block, s);
+    return set_error(SSMX_EINVAL, "no series kernel for orders da=%d, db=%d",
+                     da, db);
+}
 
 extern "C" int ssmx_propagate_series(
     const ssmx_series_desc *desc, const int32_t *layout,

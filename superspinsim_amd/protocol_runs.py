@@ -1,0 +1,309 @@
+"""Protocols as runs of the series in the drive (``ssmx_series_queue``).
+
+A pulsed protocol drives one generator with tones for short pulses and
+switches others (the readout laser) between constant values.  Its steps fall
+into runs: *driven* ones go step by step with the tables of their switch
+values; in *free* ones every step is the same matrix, whose 2^b-th powers take
+the state through any number of steps; a step in which a switch falls
+between the quadrature nodes is *split*, with tables of its own for each
+exponential.
+"""
+
+import ctypes
+
+import numpy as np
+
+from superspinsim_amd import _lib
+from superspinsim_amd.propagator import _ptr, _torch, device_tensor
+from superspinsim_amd.series import SeriesModel, coefficient_matrices
+
+_f64 = np.float64
+
+RUN_DTYPE = np.dtype([("first", np.int64), ("count", np.int64),
+                      ("kind", np.int32), ("set0", np.int32),
+                      ("set1", np.int32), ("read", np.int32)])
+DRIVEN, SPLIT, FREE = 0, 1, 2
+
+#: most distinct combinations of switch values, and most (run, segment)
+#: pairs looked at while the runs are laid out
+MAX_SETS = 32
+MAX_PAIRS = 1 << 26
+
+
+def _times(k, h, c):
+    """Node times of steps ``k`` in the kernels' operations (t0 = 0,
+    dt = h, one fine step): (t0 + dt k) + dt c."""
+    return (0.0 + h * k) + (h * c) / 1
+
+
+def _first_steps(edges, h, c, limit):
+    """Smallest step whose node lies at or after each edge (0 .. limit)."""
+    guess = np.clip((edges - h * c) / h, -1.0, float(limit) + 1.0)
+    k = np.clip(np.ceil(guess), 0, limit).astype(np.int64)
+    for _ in range(2):
+        k = np.where((k > 0) & (_times(k - 1, h, c) >= edges), k - 1, k)
+    for _ in range(2):
+        k = np.where((k < limit) & (_times(k, h, c) < edges), k + 1, k)
+    return k
+
+
+def _padded(waves, g):
+    """Segments of generator g, (instances, most, 5); empty rows at the end
+    of time."""
+    rows = [w.segment_arrays(g)[0] for w in waves]
+    out = np.full((len(rows), max(r.shape[0] for r in rows), 5), 0.0)
+    out[:, :, :2] = np.inf
+    for i, r in enumerate(rows):
+        out[i, :r.shape[0]] = r
+    return out
+
+
+class ProtocolRuns:
+    """Run lists, tables and launch of one protocol batch, or None from
+    ``build`` where the batch does not fit: more than one generator with
+    tones, too many switch values, a model the kernel does not cover."""
+
+    @classmethod
+    def build(cls, sim, waves, const, program, steps, read_from, h,
+              drive_max_of, tolerance):
+        varying = [g for g in program if g is not None]
+        J, S = sim.weights.shape
+        if sim.rotating or J > 2 or S != J:
+            return None
+        toned = [g for g in varying
+                 if any(np.any(w.segment_arrays(g)[0][:, 3] != 0)
+                        for w in waves)]
+        if len(toned) > 1:
+            return None
+        drive = toned[0] if toned else None
+        switched = [g for g in varying if g != drive]
+        segs = {g: _padded(waves, g) for g in varying}
+        base = np.array([w.base for w in waves])
+        if not all(np.all(np.isfinite(s[:, :, 2:])) and
+                   not np.any(np.isnan(s[:, :, :2])) for s in segs.values()) \
+                or not np.all(np.isfinite(base[:, varying])):
+            return None
+        n_inst = len(waves)
+        runs = cls._layout(segs, base, drive, switched, sim.nodes, steps,
+                           read_from, h)
+        if runs is None:
+            return None
+        self = cls()
+        first, count, read, values, driven, inst = runs
+        # sets: the switch values at every node, alike or not
+        flat = values.reshape(values.shape[0], -1)
+        kinds, index = (np.unique(flat, axis=0, return_inverse=True)
+                        if flat.shape[1] else
+                        (np.zeros((1, 0)), np.zeros(len(flat), np.int64)))
+        index = index.reshape(-1)
+        if kinds.shape[0] > MAX_SETS:
+            return None
+        folded = sim.folded(const)
+        weights = sim.weights
+        sets, where, pure = [], [], []
+        for row in kinds:
+            v = row.reshape(S, -1)              # (node, switched)
+            same = bool(np.all(v == v[0]))
+            pure.append(same)
+            ids = []
+            for j in range(1 if same else J):
+                terms = [(folded, h * float(weights[j].sum()))]
+                for k, g in enumerate(switched):
+                    scale = float(weights[j].sum()) * v[0, k] if same else \
+                        float(weights[j] @ v[:, k])
+                    if scale != 0:
+                        terms.append((sim.gens[g], h * scale))
+                ids.append(len(sets))
+                sets.append(terms)
+            where.append((ids[0], ids[-1]))
+        sums = weights.sum(axis=1)
+        if not np.allclose(sums, sums[::-1], rtol=1e-15, atol=1e-16):
+            return None
+        gen = sim.gens[drive] if drive is not None else \
+            np.zeros((sim.n, sim.n))
+        model = SeriesModel.of_sets(sets, gen, weights, h)
+        if model is None or model.n_sectors > 2 or \
+                max(s.size for s in model.members) > 11:
+            return None
+        plan = model.plan(drive_max_of(drive), tolerance)
+        if plan is None:
+            return None
+        pure = np.array(pure)[index]
+        free = pure & ~driven
+        rec = np.zeros(first.size, dtype=RUN_DTYPE)
+        rec["first"], rec["count"], rec["read"] = first, count, read
+        ids = np.array(where, dtype=np.int32)[index]
+        rec["set0"], rec["set1"] = ids[:, 0], ids[:, 1]
+        rec["kind"] = np.where(free, FREE, np.where(pure, DRIVEN, SPLIT))
+        # powers of the undriven steps that some free run uses
+        used = np.unique(index[free])
+        power_of = {int(k): p for p, k in enumerate(used)}
+        if used.size:
+            rec["set0"][free] = [power_of[int(k)] for k in index[free]]
+        levels = int(count[free].max()).bit_length() if used.size else 0
+        self.levels = levels
+        lanes, own, opp = cls._lanes(model)
+        self.d_lanes = device_tensor(lanes)
+        self.d_table = device_tensor(np.array(
+            [cls._rows(m, own, opp, plan[0], plan[1])
+             for m in model.matrices(*plan)]))
+        powers = np.zeros((max(used.size, 1), max(levels, 1), 2, 6, 64))
+        for k in used:
+            v = kinds[k].reshape(S, -1)[0] if switched else []
+            terms = [(folded, h)] + [(sim.gens[g], h * float(x))
+                                     for g, x in zip(switched, v)]
+            for b, (step, read_mat) in enumerate(
+                    cls._powers(terms, sim.n, h, levels)):
+                powers[power_of[int(k)], b, 0] = cls._own(step, own)
+                powers[power_of[int(k)], b, 1] = cls._own(read_mat, own)
+        self.d_powers = device_tensor(powers)
+        begin = np.zeros(n_inst + 1, dtype=np.int32)
+        np.cumsum(np.bincount(inst, minlength=n_inst), out=begin[1:])
+        self.d_begin = device_tensor(begin)
+        raw = rec.tobytes() or bytes(RUN_DTYPE.itemsize)
+        self.d_runs = _torch().from_numpy(
+            np.frombuffer(raw, dtype=np.uint8).copy()).to("cuda")
+        # a free run costs about as much as twenty steps per power
+        cost = np.where(free, 40, count + 20)
+        self.cost = np.bincount(inst, weights=cost, minlength=n_inst)
+        self.model, self.plan, self.h = model, plan, h
+        self.gen = program.index(drive) if drive is not None else 0
+        return self
+
+    @staticmethod
+    def _layout(segs, base, drive, switched, nodes, steps, read_from, h):
+        """(first, count, read, values (runs, S, switched), driven, instance)
+        of every run, instance by instance in order of time."""
+        n_inst, S = steps.size, nodes.size
+        limit = int(steps.max(initial=0))
+        edges = [s[:, :, k] for s in segs.values() for k in (0, 1)]
+        edges = np.concatenate(edges, axis=1) if edges else \
+            np.zeros((n_inst, 0))
+        if n_inst * (edges.shape[1] * S + 2) * max(1, edges.shape[1]) > \
+                MAX_PAIRS:
+            return None
+        cuts = [_first_steps(edges, h, c, limit) for c in nodes]
+        cuts = np.concatenate(
+            cuts + [np.zeros((n_inst, 1), np.int64), steps[:, None],
+                    np.minimum(read_from, steps)[:, None]], axis=1)
+        cuts = np.sort(np.minimum(cuts, steps[:, None]), axis=1)
+        inst, at = np.nonzero(cuts[:, 1:] > cuts[:, :-1])
+        first = cuts[inst, at]
+        count = cuts[inst, at + 1] - first
+
+        def inside(g, t):
+            s = segs[g]
+            for m in range(s.shape[1]):
+                row = s[inst, m]
+                yield row, (row[:, 0] <= t) & (t < row[:, 1])
+
+        values = np.zeros((first.size, S, len(switched)))
+        driven = np.zeros(first.size, dtype=bool)
+        for s, c in enumerate(nodes):
+            t = _times(first, h, c)
+            for k, g in enumerate(switched):
+                values[:, s, k] = base[inst, g]
+                for row, on in inside(g, t):
+                    values[:, s, k] += np.where(
+                        on, row[:, 2] * np.cos(row[:, 4]), 0.0)
+            if drive is not None:
+                driven |= base[inst, drive] != 0
+                for row, on in inside(drive, t):
+                    driven |= on
+        return (first, count, (first >= read_from[inst]).astype(np.int32),
+                values, driven, inst)
+
+    @staticmethod
+    def _lanes(model):
+        """(state per lane, own components, opposite rows): the matrix entry
+        [target state, source state] of each lane's six own-sector slots,
+        and of the slots it multiplies for the opposite sector's row."""
+        lanes = np.full(64, -1, dtype=np.int32)
+        own, opp = [], []
+        pair = [model.members[0], model.members[1]
+                if model.n_sectors > 1 else np.zeros(0, dtype=np.int64)]
+        linked = model.n_sectors > 1 and model.opposite[0] == 1
+        for lane in range(64):
+            half, row, i = lane // 32, (lane // 16) % 2, lane % 16
+            mine, other = pair[row], pair[1 - row]
+            if i < mine.size:
+                lanes[lane] = mine[i]
+            for s in range(6 if half == 0 else 5):
+                k = s + 6 * half
+                if k >= mine.size:
+                    continue
+                if i < mine.size:
+                    own.append((s, lane, mine[i], mine[k]))
+                if linked and i < other.size:
+                    opp.append((s, lane, other[i], mine[k]))
+        return lanes, np.array(own).reshape(-1, 4), \
+            np.array(opp, dtype=np.int64).reshape(-1, 4)
+
+    @staticmethod
+    def _own(mat, own):
+        out = np.zeros((6, 64))
+        out[own[:, 0], own[:, 1]] = mat[own[:, 2], own[:, 3]]
+        return out
+
+    @staticmethod
+    def _rows(mats, own, opp, da, db):
+        """One set's lane table."""
+        out = np.zeros((6 * (da + 1) + 6 * (db + 1), 64))
+        for k in range(da + 1):
+            out[own[:, 0] * (da + 1) + k, own[:, 1]] = \
+                mats[2 * k][own[:, 2], own[:, 3]]
+        for k in range(db + 1):
+            out[6 * (da + 1) + opp[:, 0] * (db + 1) + k, opp[:, 1]] = \
+                mats[2 * k + 1][opp[:, 2], opp[:, 3]]
+        return out
+
+    @staticmethod
+    def _powers(terms, n, h, levels):
+        """(E^(2^b) - I, (h/2) sum_{k<2^b} (E^k + E^(k+1))), b < levels, of
+        E = exp(sum of terms), squared up in extended precision."""
+        d = coefficient_matrices(terms, np.zeros((n, n)), 0,
+                                 extended=True)[0]
+        half = np.longdouble(h) / 2
+        read = half * (2 * np.eye(n, dtype=np.longdouble) + d)
+        for _ in range(levels):
+            yield d.astype(_f64), read.astype(_f64)
+            read = 2 * read + read @ d
+            d = 2 * d + d @ d
+
+    def stage(self, sim, states, rho0, obs, d_waves, d_segs):
+        """Device copies of the caller's states and readout."""
+        n = rho0.shape[1]
+        lanes = self.d_lanes.cpu().numpy()
+        self.d_lanes = device_tensor(np.where(
+            lanes >= 0, np.asarray(states)[np.maximum(lanes, 0)],
+            -1).astype(np.int32))
+        self.d_rho0 = device_tensor(np.ascontiguousarray(rho0))
+        self.d_obs = device_tensor(np.ascontiguousarray(obs))
+        self.d_w = device_tensor(sim.weights)
+        self.d_nodes = device_tensor(sim.nodes)
+        self.d_waves, self.d_segs = d_waves, d_segs
+        m = self.model
+        self.desc = _lib.SeriesDesc(
+            n=n, rows=m.n, n_inst=rho0.shape[0], members=1,
+            n_exp=sim.weights.shape[0], n_node=sim.weights.shape[1], fine=1,
+            n_out=0, n_obs=obs.shape[0], flags=_lib.SSMX_READ_INTEGRAL,
+            gen=self.gen, wave_group=1, na=11, da=self.plan[0], nb=11,
+            db=self.plan[1], sector=12, sectors=m.n_sectors,
+            sector_rows=m.members[0].size, reserved=0, h=self.h, t0=0.0,
+            dt=self.h)
+
+    def launch(self, d_order, counter, n_waves, waves_per_block, out,
+               stream):
+        _lib.check(_lib.load().ssmx_series_queue(
+            ctypes.byref(self.desc), _ptr(self.d_lanes),
+            _ptr(self.d_table), _ptr(self.d_powers),
+            ctypes.c_int32(max(self.levels, 1)), _ptr(self.d_w),
+            _ptr(self.d_nodes), _ptr(self.d_waves), _ptr(self.d_segs),
+            _ptr(self.d_rho0), _ptr(self.d_obs), _ptr(self.d_runs),
+            _ptr(self.d_begin), _ptr(d_order), _ptr(counter),
+            ctypes.c_int32(n_waves), ctypes.c_int32(waves_per_block),
+            _ptr(out), ctypes.c_void_p(stream)))
+        return out
+
+
+__all__ = ["ProtocolRuns"]

@@ -7,9 +7,12 @@ and reports the trapezoid integral of its readout rows over steps
 ``read_from[i] .. steps[i]`` (e.g. the fluorescence collected during a final
 optical readout window).
 
-The launch is ``ssmx_propagate_queue``: a grid of about as many wavefronts as
-the device holds, each taking the next instance from an atomic counter.
-Instances are queued longest first (greedy longest-processing-time), so the
+A batch with one toned generator and switched others runs as driven and free
+runs of the series in the drive (``protocol_runs``, ``ssmx_series_queue``); any
+other, and one prepared with a Taylor plan, step by step through
+``ssmx_propagate_queue``.  Either way a grid of about as many wavefronts as
+the device holds takes the instances from an atomic counter, queued longest
+first (greedy longest-processing-time), so the
 tail of the launch is filled with short protocols.  ``capture`` records the
 counter reset and the launch in a HIP graph (``torch.cuda.CUDAGraph``) for
 repeated replay; the reset is a fill kernel, not a memset node.
@@ -25,7 +28,9 @@ import numpy as np
 
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
-from superspinsim_amd.sweep import BatchSimulator, waveform_records
+from superspinsim_amd.protocol_runs import ProtocolRuns
+from superspinsim_amd.sweep import (
+    BatchSimulator, program_records, stage_records, waveform_records)
 
 _f64 = np.float64
 
@@ -73,29 +78,34 @@ class ProtocolBatch:
             raise ValueError("negative step counts")
         self.h = float(time_step)
         self.waves_host = waves
-        prop, program, m, s = self.sim.plan(waves, self.h)
-        self.prop = prop
-        self.program = program
-        self.plan_default = (m, s)
-        self.taylor = int(taylor if taylor is not None else m)
-        self.substeps = int(substeps if substeps is not None else s)
-        kwaves = self.sim.kernel_waves(waves, program)
-        recs, seg_arr = waveform_records(kwaves, len(program))
-        self.d_waves = torch.from_numpy(np.frombuffer(
-            recs.tobytes(), dtype=np.uint8).copy()).to("cuda")
-        self.d_segs = device_tensor(seg_arr)
         rho0 = np.atleast_2d(np.asarray(rho0, dtype=_f64))
         if rho0.shape[0] == 1 and n_inst > 1:
             rho0 = np.repeat(rho0, n_inst, axis=0)
-        self.d_rho0 = device_tensor(rho0[:, prop.perm])
         obs = np.atleast_2d(np.asarray(obs, dtype=_f64))
-        rows = np.zeros((obs.shape[0], 64), dtype=_f64)
-        rows[:, :prop.n] = obs[:, prop.perm]
+        self._inputs = (rho0, obs)
+        self._prop = None
+        self.series = None
+        self.d_rho0 = None
+        active, const, program = self.sim.program(waves)
+        self.program = program
+        if taylor is None and substeps is None and \
+                rho0.shape == (n_inst, self.sim.n) and \
+                obs.shape[1] == self.sim.n and \
+                obs.shape[0] <= _lib.MAX_OBS:
+            self._plan_series(active, const, rho0, obs, steps, read_from)
+        if self.series is None:
+            self.plan_default = self.sim.plan(waves, self.h)[2:]
+        m, s = self.plan_default
+        self.taylor = int(taylor if taylor is not None else m)
+        self.substeps = int(substeps if substeps is not None else s)
+        if self.series is None:
+            self._stage_taylor()
         self.n_obs = obs.shape[0]
-        self.d_obs = device_tensor(rows)
         self.steps = steps
         self.read_from = read_from
-        self.order = np.argsort(-steps, kind="stable").astype(np.int32)
+        self.order = np.argsort(
+            -steps if self.series is None else -self.series.cost,
+            kind="stable").astype(np.int32)
         self.d_order = device_tensor(self.order)
         self.d_steps = device_tensor(steps)
         self.d_read_from = device_tensor(read_from)
@@ -107,6 +117,59 @@ class ProtocolBatch:
         self.n_waves = int(n_waves or min(n_inst, resident_wavefronts()))
         self.prepared = True
         return self
+
+    def _plan_series(self, active, const, rho0, obs, steps, read_from):
+        """Lay the batch out as runs of the series in the drive, on the
+        states it involves, where it fits."""
+        waves, program = self.waves_host, self.program
+        states = self.sim.involved(active, rho0, obs)
+        sub = self.sim._reduced(states)
+        if self.sim.layout != "auto":
+            return
+        runs = ProtocolRuns.build(
+            sub, waves, const, program, steps, read_from, self.h,
+            lambda g: 0.0 if g is None else
+            max(w.abs_max()[g] for w in waves), self.tolerance)
+        if runs is None:
+            return
+        d_waves, d_segs = stage_records(*program_records(waves, program))
+        runs.stage(sub, states, rho0, obs, d_waves, d_segs)
+        self.series = runs
+        self.plan_default = sub.taylor_plan(waves, active, const, program,
+                                            self.h)
+
+    @property
+    def prop(self):
+        """Propagator of the Taylor action (built when first needed)."""
+        if self._prop is None:
+            self._prop = self.sim._propagator(
+                *self.sim.program(self.waves_host)[:2], self.h)
+        return self._prop
+
+    def _stage_taylor(self):
+        """Device inputs of the Taylor queue kernel."""
+        torch = _torch()
+        prop = self.prop
+        rho0, obs = self._inputs
+        kwaves = self.sim.kernel_waves(self.waves_host, self.program)
+        recs, seg_arr = waveform_records(kwaves, len(self.program))
+        self.d_waves = torch.from_numpy(np.frombuffer(
+            recs.tobytes(), dtype=np.uint8).copy()).to("cuda")
+        self.d_segs = device_tensor(seg_arr)
+        self.d_rho0 = device_tensor(rho0[:, prop.perm])
+        rows = np.zeros((obs.shape[0], 64), dtype=_f64)
+        rows[:, :prop.n] = obs[:, prop.perm]
+        self.d_obs = device_tensor(rows)
+
+    def _runs_series(self):
+        """Whether launches go through the series: planned so, and the
+        Taylor plan not changed since."""
+        if self.series is not None and \
+                (self.taylor, self.substeps) == tuple(self.plan_default):
+            return True
+        if self.d_rho0 is None:
+            self._stage_taylor()
+        return False
 
     def total_steps(self):
         return int(self.steps.sum())
@@ -134,6 +197,10 @@ class ProtocolBatch:
             # the kernel could read the previous launch's final count
             with torch.cuda.stream(torch.cuda.ExternalStream(stream)):
                 self.counter.zero_()
+        if self._runs_series():
+            return self.series.launch(self.d_order, self.counter,
+                                      self.n_waves, self.waves_per_block,
+                                      self.out, stream)
         desc = self._desc()
         prop = self.prop
         rc = _lib.load().ssmx_propagate_queue(
@@ -156,6 +223,10 @@ class ProtocolBatch:
         torch = _torch()
         if stream is None:
             stream = torch.cuda.current_stream().cuda_stream
+        if self._runs_series():
+            # no queue: wavefront w runs entries w, w + n_waves, ..
+            return self.series.launch(self.d_order, None, self.n_waves,
+                                      self.waves_per_block, self.out, stream)
         desc = self._desc()
         prop = self.prop
         rc = _lib.load().ssmx_propagate_queue_noalloc(

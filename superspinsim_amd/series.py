@@ -112,17 +112,19 @@ def _sparse(mat):
     return cols, vals
 
 
-def coefficient_matrices(const, drive, scale, orders):
-    """E_0 .. E_orders of exp(scale * const + f * drive) in powers of f.
+def coefficient_matrices(terms, drive, orders, extended=False):
+    """E_0 .. E_orders of exp(sum_k scale_k M_k + f * drive) in powers of f
+    for ``terms`` [(M_k, scale_k)].
 
     E_0 has the identity taken off.  Summed in extended precision and
-    rounded once: the same E_k act at every step, so their rounding would
-    not average out.
+    rounded once (not at all with ``extended``): the same E_k act at every
+    step, so their rounding would not average out.
     """
+    const = sum(np.asarray(m, dtype=np.longdouble) * np.longdouble(s)
+                for m, s in terms)
     n = const.shape[0]
-    cc, cv = _sparse(np.asarray(const, dtype=_f64))
+    cc, cv = _sparse(const)
     dc, dv = _sparse(np.asarray(drive, dtype=_f64))
-    cv = cv * np.longdouble(scale)
 
     def times(cols, vals, mat):
         out = np.zeros_like(mat)
@@ -133,7 +135,7 @@ def coefficient_matrices(const, drive, scale, orders):
     zero = np.zeros((n, n), dtype=np.longdouble)
     term = [np.eye(n, dtype=np.longdouble)] + [zero] * orders
     total = [zero.copy() for _ in range(orders + 1)]
-    norm = float(np.abs(const).sum(axis=0).max(initial=0.0)) * abs(scale)
+    norm = float(np.abs(const).sum(axis=0).max(initial=0.0))
     bound, t = 1.0, 0
     # terms of order t in const fall like norm^t / t!, drive orders add to t
     while bound > 1e-24 or t <= orders + 2:
@@ -148,7 +150,7 @@ def coefficient_matrices(const, drive, scale, orders):
         term = new
         for k in range(orders + 1):
             total[k] += term[k]
-    return [m.astype(_f64) for m in total]
+    return total if extended else [m.astype(_f64) for m in total]
 
 
 class SeriesModel:
@@ -164,25 +166,41 @@ class SeriesModel:
 
     @classmethod
     def build(cls, const, drive, weights, h):
-        n = const.shape[0]
+        """Model of the exponents h (w_j const + sum_s w_js c_s drive); one
+        set of matrices per distinct w_j."""
         J, S = weights.shape
         sums = weights.sum(axis=1)
-        distinct = sums[:(J + 1) // 2]
-        if n > _lib.MAX_N or J not in (1, 2, 5) or \
-                (J <= 2 and S != J) or \
+        if J not in (1, 2, 5) or (J <= 2 and S != J) or \
                 not np.allclose(sums, sums[::-1], rtol=1e-15, atol=1e-16):
             return None
-        norm = float(np.abs(const).sum(axis=0).max()) * h * \
-            np.abs(sums).max()
-        if not norm <= MAX_NORM:
+        self = cls.of_sets([[(const, h * float(w))]
+                            for w in sums[:(J + 1) // 2]], drive, weights, h)
+        if self is not None and J == 5 and self.size != SIZES[0]:
             return None
-        found = split_sectors(const, drive)
+        return self
+
+    @classmethod
+    def of_sets(cls, sets, drive, weights, h):
+        """Model with one set of matrices per element of ``sets`` (terms of
+        ``coefficient_matrices``) on common sectors."""
+        n = drive.shape[0]
+        if n > _lib.MAX_N:
+            return None
+        pattern = np.zeros((n, n))
+        for terms in sets:
+            norm = sum(abs(s) * np.abs(m).sum(axis=0).max()
+                       for m, s in terms)
+            if not norm <= MAX_NORM:
+                return None
+            for m, _ in terms:
+                pattern[m != 0] = 1.0
+        found = split_sectors(pattern, drive)
         if found is None:
             return None
         sector, opposite = found
         counts = np.bincount(sector)
         fit = [s for s in SIZES if s >= counts.max()]
-        if not fit or (J == 5 and fit[0] != SIZES[0]):
+        if not fit:
             return None
         self = cls()
         self.n, self.size, self.h = n, fit[0], h
@@ -190,10 +208,10 @@ class SeriesModel:
         self.pad = fit[0] + 1                    # even
         self.n_sectors = counts.size
         self.weight = float(np.abs(weights).sum(axis=1).max())
-        self.nnz = int(np.count_nonzero((const != 0) | (drive != 0)))
+        self.nnz = int(np.count_nonzero((pattern != 0) | (drive != 0)))
         top = 2 * ORDERS[-1][0] + 3
-        self.sets = [coefficient_matrices(const, drive, h * float(w), top)
-                     for w in distinct]
+        self.sets = [coefficient_matrices(terms, drive, top)
+                     for terms in sets]
         order = np.argsort(sector, kind="stable")
         self.members = [order[np.searchsorted(sector[order], k):
                               np.searchsorted(sector[order], k, "right")]

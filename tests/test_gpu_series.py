@@ -121,3 +121,61 @@ def test_reduced_wide_states(gpu):
     assert np.max(np.abs(got - want)) / np.max(np.abs(want)) <= SAME
     obs = sim.run(*args, obs=wl.obs).cpu().numpy()[:, :, 0]
     assert np.max(np.abs(obs - got @ wl.obs[0])) <= 1e-15
+
+
+def _protocols(seed, count, exps=2, early=False):
+    """Pulses, waits and switched light with edges anywhere in a step; light
+    and drive overlap in some."""
+    wl = configs.odmr7(1, use_incoherent=seed % 2 == 1)
+    rng = np.random.default_rng(seed)
+    b1 = configs.drive_amplitude(3e6)
+    waves, steps, read_from = [], [], []
+    for k in range(count):
+        w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0,
+                              0.01 if early else 0.0])
+        t = np.cumsum(rng.uniform(0.05, 3.0, 6)) * 1e-9
+        w.add(1, t[0], t[1], b1, 2 * np.pi * 2.87e9, 0.2)
+        w.add(1, t[2], t[3], -b1, 2 * np.pi * 2.74e9, 0.0)
+        w.add(4, t[3] - (0.5e-9 if k % 2 else 0.0), t[5],
+              wl.excitation if k % 3 else 2 * wl.excitation)
+        waves.append(w)
+        steps.append(int(np.ceil(t[5] / 20e-12)) + 3 * (k % 2))
+        read_from.append(int(t[2 + k % 3] / 20e-12))
+    steps[0], read_from[1] = 0, steps[1] + 5
+    batch = configs.ProtocolWorkload(
+        "protocols", wl.generators, waves, wl.rho0, wl.obs, 20e-12,
+        np.array(steps), np.array(read_from), {})
+    return wl, batch, exps
+
+
+@pytest.mark.parametrize("seed,count,exps,early", [
+    (2, 7, 2, False), (3, 40, 2, True), (4, 5, 1, False)])
+def test_protocol_runs_equal_steps(gpu, seed, count, exps, early):
+    """Runs against the trapezoid of every step of a sweep through the Taylor
+    kernel at degree 17 (at most 1,000 steps; a free run is at least as
+    accurate as its steps)."""
+    from superspinsim_amd.protocols import ProtocolBatch, trapezoid_window
+    wl, pw, exps = _protocols(seed, count, exps, early)
+    obs = np.concatenate([wl.obs, np.roll(wl.obs, 1, axis=1)])
+    rng = np.random.default_rng(seed)
+    rho = np.abs(rng.standard_normal((count, wl.n))) * (wl.rho0 != 0)
+    b = ProtocolBatch(pw.generators, exps).prepare(
+        pw.waves, rho, 20e-12, pw.steps, pw.read_from, obs)
+    assert b.series is not None
+    print(f"{count} protocols", flush=True)
+    got = b.run().cpu().numpy().copy()
+    last = int(pw.steps.max())
+    trace = BatchSimulator(pw.generators, exps, 1).run(
+        pw.waves, rho, 0.0, last * 20e-12 * (1 + 1e-12), 20e-12, obs=obs,
+        taylor=17).cpu().numpy()
+    assert trace.shape[1] == last
+    want = np.stack([trapezoid_window(
+        np.concatenate([(rho @ row)[:, None], trace[:, :, k]], axis=1),
+        pw.read_from, pw.steps, 20e-12) for k, row in enumerate(obs)], axis=1)
+    assert np.all(got[:2] == 0) and np.all(want[:2] == 0)
+    err = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    print(f"  {err:.1e}")
+    assert err <= SAME
+    # without the counter
+    b.out.fill_(np.nan)
+    assert np.array_equal(b.launch_noalloc().cpu().numpy(), got)

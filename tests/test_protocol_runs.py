@@ -1,0 +1,82 @@
+"""Run lists and powers of the protocol series (no GPU needed).
+
+The run list must cover every step once, in order, and agree with the
+waveform at each node of each step; the powers must equal step-by-step
+products.
+"""
+
+import numpy as np
+import pytest
+
+from superspinsim_amd import configs, quadratures
+from superspinsim_amd.protocol_runs import ProtocolRuns, _padded, _times
+from superspinsim_amd.sweep import Waveform
+
+H = 20e-12
+
+
+def _waves(rng, count):
+    out = []
+    for _ in range(count):
+        w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, 0.1])
+        t = np.sort(rng.uniform(0, 60, 6)) * H
+        t[1] = 7 * H                       # an edge on a step's start
+        t = np.sort(t)
+        w.add(1, t[0], t[1], 2.0, 3e9, 0.1)
+        w.add(1, t[2], t[3], 1.0, 3e9)
+        w.add(4, t[1], t[4], 0.5, 0.0, 0.0)
+        if rng.random() < 0.5:
+            w.add(4, t[4], np.inf, -0.3)
+        out.append(w)
+    return out
+
+
+@pytest.mark.parametrize("scheme", [1, 2])
+def test_runs_agree_with_the_waveforms(scheme):
+    rng = np.random.default_rng(scheme)
+    waves = _waves(rng, 12)
+    nodes, _, _ = quadratures.scheme(scheme)
+    steps = rng.integers(0, 70, 12)
+    steps[3] = 0
+    read_from = rng.integers(0, 60, 12)
+    segs = {g: _padded(waves, g) for g in (1, 4)}
+    base = np.array([w.base for w in waves])
+    first, count, read, values, driven, inst = ProtocolRuns._layout(
+        segs, base, 1, [4], nodes, steps, read_from, H)
+    for i, w in enumerate(waves):
+        mine = np.flatnonzero(inst == i)
+        covered = [k for r in mine for k in range(first[r],
+                                                  first[r] + count[r])]
+        assert covered == list(range(steps[i]))
+        for r in mine:
+            for k in range(first[r], first[r] + count[r]):
+                assert read[r] == (k >= read_from[i])
+                on = False
+                for s, c in enumerate(nodes):
+                    at = w(float(_times(k, H, c)))
+                    assert at[4] == values[r, s, 0]
+                    on |= at[1] != 0
+                assert driven[r] or not on
+    # undriven runs exist, and steps split between the nodes (two nodes)
+    assert np.any(~driven)
+    assert np.any(np.ptp(values[:, :, 0], axis=1) != 0) == (scheme == 2)
+
+
+def test_powers_equal_steps():
+    wl = configs.odmr7(1, use_incoherent=True)
+    const = wl.generators[0] + wl.excitation * wl.generators[4]
+    n = wl.n
+    powers = list(ProtocolRuns._powers([(const, H)], n, H, 9))
+    step = np.eye(n) + powers[0][0]
+    x0 = np.random.default_rng(0).standard_normal(n)
+    x, xint = x0.copy(), np.zeros(n)
+    for k in range(256):
+        after = x + powers[0][0] @ x
+        xint += 0.5 * H * (x + after)
+        x = after
+    d, read = powers[8]
+    # rounding of 256 steps, half an ulp each
+    assert np.max(np.abs(x0 + d @ x0 - x)) < 256 * 1.2e-16 * np.abs(x).max()
+    assert np.max(np.abs(read @ x0 - xint)) < \
+        256 * 1.2e-16 * np.abs(xint).max()
+    assert np.max(np.abs(step @ step - np.eye(n) - powers[1][0])) < 1e-15

@@ -40,7 +40,7 @@ def _exponential(a):
 @pytest.mark.parametrize("scale", [H / 2, 2e-10])
 def test_matrices_sum_to_the_exponential(wl, scale):
     const, drive = _pair(wl)
-    mats = coefficient_matrices(const, drive, scale, 7)
+    mats = coefficient_matrices([(const, scale)], drive, 7)
     for f in (0.0, 1e-14, -wl.b1 * H):
         total = np.eye(wl.n) + sum(f ** k * m for k, m in enumerate(mats))
         want = _exponential(scale * const + f * drive)
