@@ -106,9 +106,11 @@ typedef struct ssmx_propagate_desc {
                          row (exchanged by DPP instead of ds_bpermute) */
     int32_t ckpt_every; /* K > 0: state_out receives checkpoints (the state
                            before steps 0, K, 2K, ...); 0: the final state */
-    int32_t reserved;   /* 0 */
-    int64_t coef_inst_stride; /* table mode: doubles between instances;
-                                 0 = one table shared by all instances */
+    int32_t reserved;   /* ssmx_propagate, table mode, n <= 64: instances in a
+                           row that share one coefficient table (0 = 1);
+                           else 0 */
+    int64_t coef_inst_stride; /* table mode: doubles between instances (or
+                                 groups); 0 = one table for all */
     double h;         /* propagator step dt / F (s) */
     double t0;        /* start time (s) */
     double dt;        /* output step (s) */

@@ -35,7 +35,8 @@ import numpy as np
 
 from superspinsim_amd import _lib, quadratures
 from superspinsim_amd.propagator import (
-    Propagator, _ptr, device_tensor, eig_lane_factors, rotating_tables)
+    Propagator, _ptr, device_tensor, eig_lane_factors, rotating_tables,
+    sample_exponents, taylor_plan_measured)
 
 _f64 = np.float64
 
@@ -115,6 +116,103 @@ def plan_steps(flat, gen_norms, count=48):
     return np.unique(np.concatenate([
         np.argsort(bound, kind="stable")[-count:],
         np.linspace(0, flat.shape[0] - 1, count).astype(np.int64)]))
+
+
+#: microseconds of one wavefront per product and per matrix assembled in an
+#: exponential, and of one link of the chain of chunks (measured)
+PRODUCT_US, ASSEMBLY_US, LINK_US = 0.2, 0.2, 4.0
+#: wavefronts one launch of chunks may hold (four per SIMD)
+MAX_CHUNK_WAVES = 4096
+#: doubles of chunk propagators one run may hold
+MAX_CHUNK_DOUBLES = 1 << 27
+
+
+def time_chunks(n_out, fine, n, J, products, matrices, pairs=False):
+    """(a, P, L, pack) of a run of one system cut in time, or None.
+
+    One system's steps follow each other on one wavefront.  Cut into P
+    chunks, each carries the n basis vectors, all chunks run side by side,
+    and the chunk propagators are chained: n times the work on thousands of
+    wavefronts.  P balances a chunk's length against the chain's links.
+    Every output interval counts as ``a`` intervals of fine / a steps (a
+    divides fine), so that chunks may end inside one; a chunk holds L of
+    these.  ``pack`` basis vectors share a wavefront (``pairs``: rows 2k,
+    2k + 1 belong together, so an odd n is not packed).  None where one
+    wavefront is as quick.
+    """
+    if n > _lib.MAX_N:
+        return None
+    step = J * (products * PRODUCT_US + matrices * ASSEMBLY_US)
+    steps = n_out * fine
+    pack = 1 if pairs and n % 2 else max(
+        k for k in range(1, n + 1)
+        if k == 1 or (n % k == 0 and k * n <= _lib.MAX_N))
+    most = max(1, MAX_CHUNK_WAVES // (n // pack))
+    want = max(1, min(most, int((steps * step / LINK_US) ** 0.5)))
+    a = 1
+    if n_out < want:
+        a = next(d for d in range(1, fine + 1)
+                 if fine % d == 0 and (n_out * d >= want or d == fine))
+    while a > 1 and n_out * a * n * n > MAX_CHUNK_DOUBLES:
+        a = next(d for d in range(a - 1, 0, -1) if fine % d == 0)
+    total = n_out * a
+    if total * n * n > MAX_CHUNK_DOUBLES:
+        return None
+    L = -(-total // min(want, total))
+    P = -(-total // L)
+    # the chain writes 256 / n outputs at a time
+    links = P + total * n / 256
+    if P < 2 or L * (fine // a) * step + links * LINK_US > \
+            0.7 * steps * step:
+        return None
+    return a, P, L, pack
+
+
+def _blocks(mats, k):
+    """Each matrix repeated on the diagonal k times."""
+    eye = np.eye(k)
+    out = np.einsum("ab,...ij->...aibj", eye, mats)
+    size = k * mats.shape[-1]
+    return out.reshape(mats.shape[:-2] + (size, size))
+
+
+def _chunked_states(mats, weights, nodes, rotating, eig, coef, x0, h, m, s,
+                    N, F, split):
+    """States (1, N, n) of one system run by time chunks."""
+    torch = __import__("torch")
+    a, P, L, pack = split
+    n = mats.shape[-1]
+    fine = F // a
+    if eig is not None:
+        # the eigen-step's row factors, repeated for each packed column
+        half = eig.size // 2
+        wide = np.zeros((2, _lib.MAX_N))
+        wide[:, :pack * n] = np.tile(np.stack([eig[:n], eig[half:half + n]]),
+                                     pack)
+        eig = wide.ravel()
+    prop = Propagator(_blocks(mats, pack) if pack > 1 else mats, weights,
+                      nodes, rotating=rotating, eig=eig)
+    flat = coef.reshape(N * F, -1)
+    table = np.zeros((P * L * fine, flat.shape[1]))
+    table[:flat.shape[0]] = flat        # beyond the end: no coefficients
+    systems = P * (n // pack)
+    basis = np.tile(np.eye(n), (P, 1)).reshape(systems, pack * n)
+    ops = prop.run(n_inst=systems, fine=fine, n_out=L, h=h, t0=0.0,
+                   dt=h * fine, rho0=device_tensor(basis),
+                   coef=device_tensor(table),
+                   coef_inst_stride=L * fine * flat.shape[1],
+                   coef_group=n // pack, taylor=m, substeps=s, read="full")
+    ops = ops.contiguous()
+    total = N * a
+    out = torch.empty((1, total, n), dtype=torch.float64, device="cuda")
+    desc = _lib.ChunkDesc(n=n, n_inst=1, n_chunks=P, chunk_out=L,
+                          n_out=total, pack=pack, n_obs=0, reserved=0)
+    d_rho = device_tensor(x0)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(_lib.load().ssmx_chunk_combine(
+        ctypes.byref(desc), _ptr(ops), _ptr(d_rho), None, _ptr(out),
+        ctypes.c_void_p(stream)))
+    return out[:, a - 1::a].cpu().numpy()
 
 
 def generate_simulator(
@@ -225,12 +323,18 @@ def generate_simulator(
         ones = [np.ones(coef.shape[:-1] + (1,))] if const else []
         coef = np.ascontiguousarray(np.concatenate(
             ones + [coef[..., varying]], axis=-1))
-        prop = Propagator(mats, weights, nodes, rotating=use_rotating,
-                          eig=eig)
+
+        def propagator():
+            return Propagator(mats, weights, nodes, rotating=use_rotating,
+                              eig=eig)
+
         flat = coef.reshape(-1, coef.shape[2], coef.shape[3])  # (N*F, S, K)
-        pick = plan_steps(flat, prop.gen_norms)
-        m, s = prop.plan(flat[pick], h, tol=tolerance)
+        pick = plan_steps(flat, np.abs(mats).sum(axis=-2).max(axis=-1))
+        m, s = taylor_plan_measured(
+            sample_exponents(mats, weights, flat[pick], h, use_rotating),
+            tol=tolerance)
         if verbose:
+            prop = propagator()
             print(f"Taylor degree {m}, {s} substeps, {prop.ell.slots} ELL "
                   f"slots, nnz {prop.ell.nnz}")
 
@@ -239,6 +343,19 @@ def generate_simulator(
         x0 = _initial_rows(rho_flat, n, use_rotating, inv_vectors_real,
                            use_kernel, image_projection, use_unitary)
         n_inst = x0.shape[0]
+        split = None if n_inst > 1 else time_chunks(
+            N, F, mats.shape[-1], J=weights.shape[0], products=m * s,
+            matrices=mats.shape[0] if not use_rotating else
+            mats.shape[0] * mats.shape[1], pairs=use_rotating)
+        if split is not None:
+            states = _chunked_states(mats, weights, nodes, use_rotating, eig,
+                                     coef, x0, h, m, s, N, F, split)
+            return time, _finish(states, n, rho_flat, vmap, use_hermitian,
+                                 hilbert, use_rotating, vectors_real,
+                                 inv_vectors_real, use_kernel,
+                                 image_projection, use_unitary, elimination,
+                                 duplication)
+        prop = propagator()
         d_rho = device_tensor(x0)
         d_coef = device_tensor(coef)
         out = prop.run(n_inst=n_inst, fine=F, n_out=N, h=h, t0=time_start,

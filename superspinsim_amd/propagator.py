@@ -986,10 +986,12 @@ class Propagator:
             coef_inst_stride=0, waves=None, segments=None, taylor=None,
             substeps=1, read="full", obs=None, obs_offset=None, out=None,
             state_out=None, ckpt_every=0, first_out=0, stream=None,
-            store_inputs=False):
+            store_inputs=False, coef_group=0):
         """Launch one propagation; returns the output tensor.
 
-        ``rho0`` (n_inst, n) device tensor.  Coefficients: ``coef`` device
+        ``coef_group`` consecutive instances share one coefficient table
+        (``coef_inst_stride`` doubles apart).  ``rho0`` (n_inst, n) device
+        tensor.  Coefficients: ``coef`` device
         table (..., n_out*fine*S*K) or ``waves``/``segments`` device buffers
         of ``ssmx_wave``/``ssmx_segment`` bytes.  ``read`` is "full",
         "obs" or "integral".  ``state_out`` (device, float64) receives the
@@ -1033,7 +1035,7 @@ class Propagator:
             taylor=int(taylor), substeps=int(substeps), n_obs=max(n_obs, 1),
             flags=flags, first_out=int(first_out),
             partner=1 if self.ell.partner else 0,
-            ckpt_every=int(ckpt_every), reserved=0,
+            ckpt_every=int(ckpt_every), reserved=int(coef_group),
             coef_inst_stride=int(coef_inst_stride), h=float(h),
             t0=float(t0), dt=float(dt))
         obs_rows = None

@@ -25,7 +25,8 @@ from superspinsim_amd import _lib, quadratures
 from superspinsim_amd.propagator import (
     Propagator, _ptr, coefficient_samples, device_tensor, eig_lane_factors,
     rotating_tables, sample_exponents, taylor_plan_measured)
-from superspinsim_amd.series import SeriesModel, SeriesRun, reachable
+from superspinsim_amd.series import (
+    SIZES, SeriesModel, SeriesRun, reachable)
 
 _f64 = np.float64
 
@@ -731,7 +732,7 @@ class BatchSimulator:
     # ------------------------------------------------------------------
     # time-chunked runs (small systems, few instances)
 
-    def chunk_plan(self, n_inst, N, resident=None):
+    def chunk_plan(self, n_inst, N, resident=None, pack=None):
         """(chunks P, outputs per chunk L, pack k) of a chunked run.
 
         Every instance's N outputs are cut into P chunks of L; each chunk
@@ -741,7 +742,7 @@ class BatchSimulator:
         """
         if self.rotating or self.n > 32:
             raise ValueError("chunked runs need the lab frame and n <= 32")
-        k = max(1, min(_lib.MAX_N // self.n, _lib.MAX_GEN - 1))
+        k = pack or max(1, min(_lib.MAX_N // self.n, _lib.MAX_GEN - 1))
         if resident is None:
             torch = __import__("torch")
             resident = 16 * torch.cuda.get_device_properties(
@@ -773,31 +774,59 @@ class BatchSimulator:
             raise ValueError("chunked runs read out 'obs' or 'full'")
         N = int((time_end - time_start) / time_step)
         n_inst = len(waves)
-        if chunks is None:
-            P, L, k = self.chunk_plan(n_inst, N)
-        else:
-            P = max(1, min(int(chunks), N))
-            L = -(-N // P)
-            P = -(-N // L)
-            k = max(1, min(_lib.MAX_N // self.n, _lib.MAX_GEN - 1))
         n = self.n
-        members = []
-        for w in waves:
-            for p in range(P):
-                shifted = w.shifted(time_start + p * L * time_step)
-                members.extend([shifted] * n)
-        basis = np.tile(np.eye(n), (n_inst * P, 1))
-        saved = self.pack
-        self.pack = k
-        try:
-            run = self.prepare(members, basis, 0.0,
-                               L * time_step * (1 + 1e-12), time_step,
-                               read="full")
-        finally:
-            self.pack = saved
         rho0 = np.atleast_2d(np.asarray(rho0, dtype=_f64))
         if rho0.shape[0] == 1 and n_inst > 1:
             rho0 = np.repeat(rho0, n_inst, axis=0)
+        found = None
+        if self.n <= 32 and rho0.shape == (n_inst, n):
+            active, const, program = self.program(waves)
+            found = self.series_plan(waves, const, program, time_step)
+        if found is not None:
+            # the series kernel: as many columns per wavefront as fit, 3 (or
+            # 2 for the larger tables) wavefronts per SIMD
+            torch = __import__("torch")
+            simds = 4 * torch.cuda.get_device_properties(
+                0).multi_processor_count
+            small = found[0].size == SIZES[0]
+            k = max(1, min(_lib.MAX_N // n,
+                           _lib.MAX_N // self.weights.shape[0],
+                           _lib.MAX_N if small else 2))
+            P, L, k = self.chunk_plan(n_inst, N, simds * (3 if small else 2),
+                                      k)
+        if chunks is not None:
+            P = max(1, min(int(chunks), N))
+            L = -(-N // P)
+            P = -(-N // L)
+            if found is None:
+                k = max(1, min(_lib.MAX_N // n, _lib.MAX_GEN - 1))
+        elif found is None:
+            P, L, k = self.chunk_plan(n_inst, N)
+        shifted = [w.shifted(time_start + p * L * time_step)
+                   for w in waves for p in range(P)]
+        basis = np.tile(np.eye(n), (n_inst * P, 1))
+        if found is not None:
+            model, plan = found
+            d_waves, d_segs = stage_records(*program_records(shifted,
+                                                             program))
+            gen = next((i for i, g in enumerate(program) if g is not None),
+                       0)
+            run = SeriesRun(model, plan, np.arange(n), k, self.weights,
+                            self.nodes, basis, d_waves, d_segs, gen, self.F,
+                            L, 0.0, time_step, None, "full", wave_group=n)
+            m, s = self.taylor_plan(waves, active, const, program, time_step)
+            self.last_plan = dict(
+                taylor=m, substeps=s, slots=2 * model.size, nnz=model.nnz,
+                active=program, n=n, packed=k, involved=n, series=plan[:2])
+        else:
+            members = [w for w in shifted for _ in range(n)]
+            saved = self.pack
+            self.pack = k
+            try:
+                run = self._prepare_taylor(members, basis, 0.0, time_step, L,
+                                           None, "full", None, None)
+            finally:
+                self.pack = saved
         obs_rows = None
         if read == "obs":
             obs_rows = np.atleast_2d(np.asarray(obs, dtype=_f64))
@@ -806,7 +835,7 @@ class BatchSimulator:
                               chunk_pack=run.k)
         return ChunkedRun(run, n_inst, N, P, L, device_tensor(rho0),
                           None if obs_rows is None else
-                          device_tensor(obs_rows))
+                          device_tensor(obs_rows), n)
 
     def run_chunked(self, waves, rho0, time_start, time_end, time_step,
                     obs=None, read="obs", chunks=None):
@@ -838,15 +867,17 @@ class ChunkedRun:
     """Device inputs of a time-chunked run (``prepare_chunked``): ``launch``
     propagates every chunk's basis vectors, then chains the chunks."""
 
-    def __init__(self, chunk_run, n_inst, N, P, L, d_rho0, d_obs):
+    def __init__(self, chunk_run, n_inst, N, P, L, d_rho0, d_obs, n):
         torch = __import__("torch")
         self.chunk_run, self.n_inst, self.N = chunk_run, n_inst, N
         self.P, self.L = P, L
         self.d_rho0, self.d_obs = d_rho0, d_obs
-        n = chunk_run.sim.n
         n_obs = 0 if d_obs is None else d_obs.shape[0]
+        # the series kernel writes column by column, the Taylor kernel by
+        # packed system
+        pack = 1 if isinstance(chunk_run, SeriesRun) else chunk_run.k
         self.desc = _lib.ChunkDesc(n=n, n_inst=n_inst, n_chunks=P,
-                                   chunk_out=L, n_out=N, pack=chunk_run.k,
+                                   chunk_out=L, n_out=N, pack=pack,
                                    n_obs=n_obs, reserved=0)
         shape = (n_inst, N, n_obs if n_obs else n)
         self.out = torch.empty(shape, dtype=torch.float64, device="cuda")

@@ -7,6 +7,8 @@ largest value; 1e-12 is the bar.  ``taylor=17`` asks for the Taylor path on
 every state.
 """
 
+import importlib
+
 import numpy as np
 import pytest
 
@@ -179,3 +181,74 @@ def test_protocol_runs_equal_steps(gpu, seed, count, exps, early):
     # without the counter
     b.out.fill_(np.nan)
     assert np.array_equal(b.launch_noalloc().cpu().numpy(), got)
+
+
+@pytest.mark.parametrize("rotating,n,F,N,schemes", [
+    (False, 3, 12, 30, 2), (True, 3, 12, 30, 5), (True, 4, 30, 7, 2),
+    (False, 9, 7, 41, 3), (True, 19, 10, 20, 5), (False, 40, 50, 2, 1)])
+def test_time_chunked_drop_in_equals_one_wavefront(gpu, monkeypatch,
+                                                   rotating, n, F, N,
+                                                   schemes):
+    """One system cut in time against the same run on one wavefront: the
+    chunk propagators hold n columns each, so the bar is that of the other
+    comparisons times the chain's rounding (SAME x 4)."""
+    gs = importlib.import_module("superspinsim_amd.generate_simulator")
+    rng = np.random.default_rng(n)
+    gens = rng.standard_normal((3, n, n)) * 1e9 / n
+    gens[0] -= 2e9 * np.eye(n)
+    kw = {}
+    if rotating:
+        nd = n // 2
+        kw = dict(use_rotating=True, vectors_real=np.eye(n),
+                  inv_vectors_real=np.eye(n),
+                  doubles=np.stack([-rng.uniform(1e6, 1e8, nd),
+                                    rng.uniform(-2e9, 2e9, nd)], axis=1),
+                  singles=-rng.uniform(1e6, 1e7, n - 2 * nd))
+        gens = gens[1:]
+
+    def sampler(t, row):
+        row[0] = np.cos(3e9 * t) if rotating else 1.0
+        row[1] = np.sin(2e9 * t)
+        if not rotating:
+            row[2] = 0.3 * np.cos(1e9 * t)
+
+    hil = 8                          # n rows of an 8 x 8 density
+    vmap = np.array([(k // 8, k % 8, 0) if k // 8 <= k % 8 else
+                     (k % 8, k // 8, 1) for k in range(n)])
+    rho = rng.standard_normal((hil, hil))
+    sim = gs.generate_simulator(sampler, gens, vmap,
+                                number_of_exponentials=schemes,
+                                number_of_fine_divisions=F, **kw)
+    args = (rho, 1e-9, 1e-9 + N * F * 2e-11 * (1 + 1e-9), F * 2e-11)
+    plans = []
+    plan = gs.time_chunks
+    monkeypatch.setattr(gs, "time_chunks", lambda *a, **k: (
+        plans.append(plan(*a, **k)), plans[-1])[1])
+    t1, got = sim(*args)
+    assert plans and plans[0] is not None, plans
+    monkeypatch.setattr(gs, "time_chunks", lambda *a, **k: None)
+    t2, want = sim(*args)
+    assert np.array_equal(t1, t2) and got.shape == want.shape
+    err = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    print(f"n={n} chunks {plans[0]}: {err:.1e}", flush=True)
+    assert err <= 4 * SAME
+
+
+@pytest.mark.parametrize("name,exps,read", [
+    ("nv3", 2, "full"), ("nv3", 5, "obs"), ("nv7c", 2, "obs")])
+def test_chunked_series_equals_run(gpu, name, exps, read):
+    wl = _model(name)
+    sim = BatchSimulator(wl.generators, exps, 20)
+    dt = 20 * 20e-12
+    args = (_waves(wl, 3, 3e6), wl.rho0, 2e-9, 2e-9 + 50 * dt * (1 + 1e-9),
+            dt)
+    obs = None if read == "full" else wl.obs
+    want = sim.run(*args, obs=obs, read=read).cpu().numpy()
+    got = sim.run_chunked(*args, obs=obs, read=read, chunks=7).cpu().numpy()
+    assert sim.last_plan["chunks"] == 7
+    assert ("series" in sim.last_plan) == (exps == 2 or name == "nv3")
+    err = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    print(f"{name}: {err:.1e}", flush=True)
+    # node times counted from a chunk's start move by rounding: 4e-24 s in
+    # phases of 2e10 rad/s, far below the state's own rounding
+    assert err <= SAME
