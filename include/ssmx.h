@@ -296,6 +296,50 @@ int ssmx_series_queue(const ssmx_series_desc *desc, const int32_t *lanes,
                       int32_t waves_per_block, double *out, void *stream);
 
 /*
+ * ssmx_propagate_series with one instance on a whole wavefront (members 1,
+ * na = nb = 11, n_exp 1..2, at most two sectors, sector_rows > 0).
+ *
+ * lanes, table  as ssmx_series_queue, with one set
+ * store   double [n_inst][n_out * fine][n_exp][32] (or NULL): the input of
+ *         every exponential for ssmx_series_adjoint, exponential n_exp - 1
+ *         first, component of lane l (< 32) at l
+ * out     READ_FULL: states without a lane are not written
+ */
+int ssmx_propagate_series_wave(const ssmx_series_desc *desc,
+                               const int32_t *lanes, const double *table,
+                               const double *cf_weights,
+                               const double *cf_nodes, const ssmx_wave *waves,
+                               const ssmx_segment *segments,
+                               const double *rho0, const double *obs,
+                               double *out, double *store, void *stream);
+
+/*
+ * Gradient of the integrated readout of ssmx_propagate_series_wave
+ * (SSMX_READ_INTEGRAL), as ssmx_adjoint's: dLoss/dtheta, dLoss/d(segment
+ * amplitude) of the driven generator's records, dLoss/drho0.
+ *
+ * table    as the forward's with the transposed matrices: entry
+ *          (s (da + 1) + k) is E_2k[row s of the half's][lane's component],
+ *          row s in the lane's sector, then (s (db + 1) + k)
+ *          E_(2k+1)[row s][lane's component], row s in the opposite sector
+ * dtable   double [n_theta][2][6][4][64]: d E_k / d theta, k = 0..3, at the
+ *          same rows and columns, own sector then opposite sector
+ * store    the forward's
+ * seed     double [n_inst * n_obs] dLoss/dF; obs double [n_obs * n]
+ * grad_theta  double [n_inst * n_theta]; grad_seg double [records],
+ *          accumulated (or NULL: no amplitude gradients); lambda_out double
+ *          [n_inst * n], states with a lane only (or NULL)
+ */
+int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
+                        const double *table, const double *dtable,
+                        int32_t n_theta, const double *cf_weights,
+                        const double *cf_nodes, const ssmx_wave *waves,
+                        const ssmx_segment *segments, const double *store,
+                        const double *obs, const double *seed,
+                        double *grad_theta, double *grad_seg,
+                        double *lambda_out, void *stream);
+
+/*
  * The reference's non-residual exponential (use_residual=False).
  *
  * Each exponential is (I + A / scale)^(2^squarings) with scale = 4^R and

@@ -116,6 +116,7 @@ class Wave(ctypes.Structure):
 
 #: every symbol include/ssmx.h declares
 EXPORTS = ("ssmx_propagate", "ssmx_propagate_series", "ssmx_series_queue",
+           "ssmx_propagate_series_wave", "ssmx_series_adjoint",
            "ssmx_propagate_dense", "ssmx_chunk_combine",
            "ssmx_propagate_queue",
            "ssmx_propagate_queue_noalloc", "ssmx_adjoint",
@@ -151,6 +152,13 @@ def load():
     lib.ssmx_propagate_series.argtypes = [ctypes.POINTER(SeriesDesc)] + \
         [vp] * 11
     lib.ssmx_propagate_series.restype = ctypes.c_int
+    lib.ssmx_propagate_series_wave.argtypes = \
+        [ctypes.POINTER(SeriesDesc)] + [vp] * 11
+    lib.ssmx_propagate_series_wave.restype = ctypes.c_int
+    lib.ssmx_series_adjoint.argtypes = (
+        [ctypes.POINTER(SeriesDesc)] + [vp] * 3 + [ctypes.c_int32] +
+        [vp] * 11)
+    lib.ssmx_series_adjoint.restype = ctypes.c_int
     lib.ssmx_series_queue.argtypes = (
         [ctypes.POINTER(SeriesDesc)] + [vp] * 3 + [ctypes.c_int32] +
         [vp] * 10 + [ctypes.c_int32, ctypes.c_int32, vp, vp])

@@ -34,7 +34,10 @@ import ctypes
 import numpy as np
 
 from superspinsim_amd import _lib
-from superspinsim_amd.propagator import _bank_slots, _ptr, _torch, device_tensor
+from superspinsim_amd.propagator import (
+    _bank_slots, _ptr, _torch, device_tensor, sample_exponents,
+    taylor_degrees_measured)
+from superspinsim_amd.series_gradient import SeriesGradient
 from superspinsim_amd.sweep import BatchSimulator, waveform_records
 
 _f64 = np.float64
@@ -192,6 +195,26 @@ def wide_adjoint_ell(ell, mats, dmats):
     return col_e, val_e, col_t, dval_e, ell.slots
 
 
+class GradientState(dict):
+    """A parameter point set up for ``forward`` and ``backward``.  The Taylor
+    kernels' tables are built when first asked for where the series in the
+    drive serves the point (``series``)."""
+
+    later = None
+
+    def complete(self):
+        later, self.later = self.later, None
+        if later is not None:
+            for key, value in later().items():
+                self.setdefault(key, value)
+
+    def __missing__(self, key):
+        if self.later is None:
+            raise KeyError(key)
+        self.complete()
+        return self[key]
+
+
 class GradientProblem:
     """Batch of parametrised instances with an integrated readout."""
 
@@ -299,12 +322,7 @@ class GradientProblem:
         sim = BatchSimulator(gens, self.J, self.F, tolerance=self.tolerance,
                              layout="plain")
         active, const, program = sim.program(waves)
-        prop = sim._propagator(active, const, self.dt)
         h = self.dt / self.F
-        samples = sim.coefficient_box(waves, program)
-        m, ma = prop.plan_degrees(
-            samples, h, (self.tolerance, self.adjoint_tolerance),
-            max_taylor=(_lib.MAX_TAYLOR, _lib.ADJ_MAX_TAYLOR))
 
         # derivative tables of the folded constant matrix
         dgen = self.derivative_generators(theta) \
@@ -335,12 +353,55 @@ class GradientProblem:
         grad_gen = tagged[0] if tagged else -1
         recs, seg_arr, tag_index, tag_scale = waveform_records(
             kwaves, len(program), with_tags=True)
+        torch = _torch()
+        series = None
+        if self.store_inputs == "auto" and \
+                self.rho0.shape[-1] == gens.shape[1] == self.obs.shape[1]:
+            series = SeriesGradient.build(
+                sim, const, program, waves, dconst, np.atleast_2d(self.rho0),
+                self.obs, h, self.tolerance, self.adjoint_tolerance)
+            if series is not None and grad_gen not in (-1, series.gen):
+                series = None
+        state = GradientState(
+            theta=theta, amplitudes=amplitudes, program=program,
+            derivatives=bool(derivatives), series=series,
+            theta_gen=theta_gen, grad_gen=grad_gen,
+            n_theta=dconst.shape[0] if theta_gen >= 0 else 0,
+            d_waves=torch.from_numpy(np.frombuffer(
+                recs.tobytes(), dtype=np.uint8).copy()).to("cuda"),
+            d_segs=device_tensor(seg_arr),
+            tag_index=tag_index, tag_scale=tag_scale,
+            n_records=seg_arr.shape[0], n_inst=len(waves), dconst=dconst,
+            kernel_waves=kwaves)
+        state.later = lambda: self._taylor_tables(
+            sim, waves, active, const, program, dconst, derivatives, grad_gen)
+        if series is None:
+            state.complete()
+        else:
+            # the degrees the Taylor kernels would run at (a point beyond
+            # them is refused as ever)
+            sub = sim.gens[:, series.states][:, :, series.states]
+            mats = np.stack([sum(c * sub[g] for g, c in const.items()),
+                             sub[varying[0]]])
+            state["taylor"], state["taylor_adj"] = taylor_degrees_measured(
+                sample_exponents(mats, sim.weights,
+                                 sim.coefficient_box(waves, program), h),
+                (self.tolerance, self.adjoint_tolerance),
+                max_taylor=(_lib.MAX_TAYLOR, _lib.ADJ_MAX_TAYLOR))
+        return state
 
+    def _taylor_tables(self, sim, waves, active, const, program, dconst,
+                       derivatives, grad_gen):
+        """Plan and device tables of the Taylor kernels."""
+        prop = sim._propagator(active, const, self.dt)
+        m, ma = prop.plan_degrees(
+            sim.coefficient_box(waves, program), self.dt / self.F,
+            (self.tolerance, self.adjoint_tolerance),
+            max_taylor=(_lib.MAX_TAYLOR, _lib.ADJ_MAX_TAYLOR))
         perm = prop.perm
         mats = prop._dense                                   # (M, n, n)
         mp = mats[:, perm][:, :, perm]
         dp = dconst[:, perm][:, :, perm]
-        torch = _torch()
         if not derivatives:
             # forward only: the adjoint's tables (whose pattern may exceed
             # the adjoint kernels' limits where the forward's does not) are
@@ -380,18 +441,7 @@ class GradientProblem:
                 d_col_t=device_tensor(col_t), d_val_t=device_tensor(val_t),
                 d_dval_t=device_tensor(dval_t) if dconst.shape[0] else None,
                 slots=prop.ell.slots, slots_t=col_t.shape[0], slots_f=0)
-        state = dict(
-            theta=theta, amplitudes=amplitudes, prop=prop, program=program,
-            derivatives=bool(derivatives),
-            taylor=m, taylor_adj=ma, theta_gen=theta_gen, grad_gen=grad_gen,
-            n_theta=dconst.shape[0] if theta_gen >= 0 else 0,
-            d_waves=torch.from_numpy(np.frombuffer(
-                recs.tobytes(), dtype=np.uint8).copy()).to("cuda"),
-            d_segs=device_tensor(seg_arr),
-            tag_index=tag_index, tag_scale=tag_scale,
-            n_records=seg_arr.shape[0], n_inst=len(waves), dconst=dconst,
-            kernel_waves=kwaves, **tables)
-        return state
+        return dict(tables, prop=prop, taylor=m, taylor_adj=ma)
 
     # ------------------------------------------------------------------
     def forward(self, theta, amplitudes, state=None):
@@ -399,13 +449,22 @@ class GradientProblem:
         torch = _torch()
         if state is None:
             state = self.setup(theta, amplitudes)
-        prop = state["prop"]
         n_inst = state["n_inst"]
         rho0 = np.atleast_2d(self.rho0)
         if rho0.shape[0] == 1 and n_inst > 1:
             rho0 = np.repeat(rho0, n_inst, axis=0)
         total = self.n_out * self.F
         P = (total + self.K - 1) // self.K
+        series = state.get("series")
+        if series is not None and rho0.shape[0] == n_inst and total > 0:
+            store = self._series_store(state, series, total)
+            if store is not False:
+                out = series.forward(self, state, rho0, store)
+                state.update(ckpt=store, inputs=store, n_ckpt=P,
+                             stored=store is not None, by_series=True)
+                return out, state
+        state["by_series"] = False
+        prop = state["prop"]
         stored = self._use_stored_inputs(state)
         if stored:
             # every exponential's input (the backward's forward terms start
@@ -432,6 +491,26 @@ class GradientProblem:
         state["n_ckpt"] = P
         state["stored"] = stored
         return out, state
+
+    def _series_store(self, state, series, total):
+        """Buffer of the exponentials' inputs for the series backward (None
+        for a forward-only state, False if it does not fit in 80 % of the
+        free device memory); reused across calls."""
+        if not state["derivatives"]:
+            return None
+        torch = _torch()
+        shape = (state["n_inst"], total, series.d_w.shape[0], 32)
+        have = state.get("inputs")
+        if have is not None and tuple(have.shape) == shape:
+            return have
+        state.pop("inputs", None)
+        state.pop("ckpt", None)
+        have = None
+        free, _ = torch.cuda.mem_get_info()
+        free += torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
+        if series.store_bytes(shape[0], total, shape[2]) > 0.8 * free:
+            return False
+        return torch.empty(shape, dtype=torch.float64, device="cuda")
 
     def adjoint_desc(self, state):
         prop = state["prop"]
@@ -462,39 +541,22 @@ class GradientProblem:
                              "(setup(..., derivatives=False) or readout); "
                              "use forward(theta, amplitudes) for gradients")
         torch = _torch()
-        prop = state["prop"]
         n_inst = state["n_inst"]
-        desc = self.adjoint_desc(state)
-        lib = _lib.load()
-        nbytes = ctypes.c_uint64(0)
-        _lib.check(lib.ssmx_adjoint_workspace_bytes(ctypes.byref(desc),
-                                                   ctypes.byref(nbytes)))
-        work = torch.empty(int(nbytes.value) // 8, dtype=torch.float64,
-                           device="cuda")
         seed = torch.as_tensor(seed, dtype=torch.float64).to("cuda")
         seed = seed.reshape(n_inst, self.obs.shape[0]).contiguous()
-        rows = np.zeros((self.obs.shape[0], prop.ell.npad), dtype=_f64)
-        rows[:, :prop.n] = self.obs[:, prop.perm]
-        d_obs = device_tensor(rows)
         n_theta = int(state["n_theta"])
         g_theta = torch.zeros((n_inst, max(n_theta, 1)), dtype=torch.float64,
                               device="cuda")
         g_seg = torch.zeros(state["n_records"], dtype=torch.float64,
                             device="cuda")
-        lam = torch.empty((n_inst, prop.n), dtype=torch.float64,
+        lam = torch.empty((n_inst, self.rho0.shape[-1]), dtype=torch.float64,
                           device="cuda") if lambda_out else None
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.ssmx_adjoint(
-            ctypes.byref(desc), _ptr(state["d_col"]), _ptr(state["d_val_f"]),
-            _ptr(state["d_col_t"]), _ptr(state["d_val_t"]),
-            _ptr(state["d_dval_t"]), _ptr(prop.d_w), _ptr(prop.d_nodes),
-            _ptr(state["d_waves"]), _ptr(state["d_segs"]),
-            _ptr(state["ckpt"]), _ptr(d_obs), _ptr(seed), _ptr(work),
-            _ptr(g_theta) if n_theta else None,
-            _ptr(g_seg) if state["grad_gen"] >= 0 else None,
-            _ptr(lam), ctypes.c_void_p(stream))
-        _lib.check(rc)
-        self._keep = (work, d_obs, seed)
+        if state.get("by_series"):
+            state["series"].backward(
+                self, state, seed, g_theta if n_theta else None,
+                g_seg if state["grad_gen"] >= 0 else None, lam)
+        else:
+            self._backward_taylor(state, seed, n_theta, g_theta, g_seg, lam)
         result = dict(theta=g_theta[:, :n_theta], records=g_seg)
         n_amp = state["amplitudes"].size
         if "amp_sum" not in state:
@@ -516,8 +578,35 @@ class GradientProblem:
             g_amp = torch.zeros(n_amp, dtype=torch.float64, device="cuda")
         result["amplitudes"] = g_amp
         if lambda_out:
-            result["lambda"] = lam[:, prop.d_inv_perm]
+            result["lambda"] = lam if state.get("by_series") else \
+                lam[:, state["prop"].d_inv_perm]
         return result
+
+    def _backward_taylor(self, state, seed, n_theta, g_theta, g_seg, lam):
+        torch = _torch()
+        prop = state["prop"]
+        desc = self.adjoint_desc(state)
+        lib = _lib.load()
+        nbytes = ctypes.c_uint64(0)
+        _lib.check(lib.ssmx_adjoint_workspace_bytes(ctypes.byref(desc),
+                                                   ctypes.byref(nbytes)))
+        work = torch.empty(int(nbytes.value) // 8, dtype=torch.float64,
+                           device="cuda")
+        rows = np.zeros((self.obs.shape[0], prop.ell.npad), dtype=_f64)
+        rows[:, :prop.n] = self.obs[:, prop.perm]
+        d_obs = device_tensor(rows)
+        stream = torch.cuda.current_stream().cuda_stream
+        rc = lib.ssmx_adjoint(
+            ctypes.byref(desc), _ptr(state["d_col"]), _ptr(state["d_val_f"]),
+            _ptr(state["d_col_t"]), _ptr(state["d_val_t"]),
+            _ptr(state["d_dval_t"]), _ptr(prop.d_w), _ptr(prop.d_nodes),
+            _ptr(state["d_waves"]), _ptr(state["d_segs"]),
+            _ptr(state["ckpt"]), _ptr(d_obs), _ptr(seed), _ptr(work),
+            _ptr(g_theta) if n_theta else None,
+            _ptr(g_seg) if state["grad_gen"] >= 0 else None,
+            _ptr(lam), ctypes.c_void_p(stream))
+        _lib.check(rc)
+        self._keep = (work, d_obs, seed)
 
     # ------------------------------------------------------------------
     def readout(self, theta, amplitudes):

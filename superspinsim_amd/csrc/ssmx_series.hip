@@ -27,14 +27,18 @@
 // issue (135 VALU instructions per wavefront and step, 110 of them the
 // multiply-adds). A wavefront alone on its SIMD issues a 64-bit multiply-add
 // every 8 cycles, two together one every 4.
-#include "ssmx_common.h"
+#include "ssmx_series_dev.h"
 
 namespace {
 
+using ssmx::bcast_fma;
+using ssmx::Clock;
+using ssmx::DriveFactors;
+using ssmx::Halves;
+using ssmx::horner;
 using ssmx::kWave;
-using ssmx::node_time;
 using ssmx::set_error;
-using ssmx::swap_pair;
+using ssmx::swap_rows;
 using ssmx::wave_exchange;
 
 struct SParams {
@@ -58,96 +62,6 @@ constexpr int set_of(int j)
 {
     return j < J - 1 - j ? j : J - 1 - j;
 }
-
-// Node times and weights of a run.
-struct Clock {
-    double t0, dt, h;
-    int fine, n_node;
-    const double *nodes, *w;
-};
-
-// Drive factors of a wavefront's members, lane-parallel: entry
-// (b * members + member) * J + j of `fbuf` holds f_j of step b of the batch.
-// The lane's waveform segment stays in registers between batches (node
-// times only increase), and output and fine index come from the batch's
-// first step by one 32-bit division: a batch of 16 steps is otherwise a tenth
-// of the wavefront's instructions.
-template <int J>
-struct DriveFactors {
-    int MJ, B, my_b, my_j, cursor, begin, count;
-    double base;
-    ssmx_segment seg;
-
-    // `wv` is the waveform of the lane's entry (member (lane / J) % members)
-    __device__ DriveFactors(const ssmx_wave *wv, const ssmx_segment *segs,
-                            int gen, int members, int lane)
-    {
-        MJ = members * J;
-        B = kWave / MJ;
-        my_b = lane / MJ;
-        my_j = lane % J;
-        base = wv->base[gen];
-        begin = wv->seg_begin[gen];
-        count = wv->seg_count[gen];
-        cursor = 0;
-        if (count > 0)
-            seg = segs[begin];
-    }
-
-    // wave_coef for times that only increase
-    __device__ double coefficient(const ssmx_segment *segs, double t)
-    {
-#pragma clang fp contract(off)
-        while (cursor < count && !(t < seg.t_end)) {
-            ++cursor;
-            if (cursor < count)
-                seg = segs[begin + cursor];
-        }
-        double c = base;
-        if (cursor < count && !(t < seg.t_start))
-            c += seg.amp * cos(seg.omega * t + seg.phase);
-        return c;
-    }
-
-    // The steps from output i, fine step k on, `left` at most.
-    __device__ void fill(const Clock &c, const ssmx_segment *segs, long i,
-                         int k, long left, int lane, double *fbuf)
-    {
-        const unsigned ahead = (unsigned)k + (unsigned)my_b;
-        const unsigned di = ahead / (unsigned)c.fine;
-        const int r = (int)(ahead - di * (unsigned)c.fine);
-        const long out = i + di;
-        const bool on = my_b < B && my_b < left;
-        double f;
-        if constexpr (J <= 2) {
-            // schemes with as many nodes as exponentials: each lane
-            // evaluates one node, pairs of lanes exchange theirs
-            double v = 0.0;
-            if (on)
-                v = coefficient(segs, node_time(c.t0, c.dt, c.fine, r, out,
-                                                c.nodes[my_j]));
-            if constexpr (J == 2) {
-                const double o = swap_pair(v);
-                const double c0 = my_j == 0 ? v : o;
-                const double c1 = my_j == 0 ? o : v;
-                f = fma(c.w[my_j * 2 + 1], c1, fma(c.w[my_j * 2], c0, 0.0));
-            } else {
-                f = fma(c.w[0], v, 0.0);
-            }
-        } else {
-            f = 0.0;
-            if (on)
-                for (int s = 0; s < c.n_node; ++s)
-                    f = fma(c.w[my_j * c.n_node + s],
-                            coefficient(segs, node_time(c.t0, c.dt, c.fine,
-                                                        r, out,
-                                                        c.nodes[s])),
-                            f);
-        }
-        fbuf[lane] = c.h * f;
-        wave_exchange();
-    }
-};
 
 // Waveform of a lane's drive-factor entry in a sweep.
 template <int J>
@@ -353,87 +267,6 @@ __attribute__((amdgpu_waves_per_eu(NA > 6 || J > 2 ? 2 : 3))) void series_kernel
     }
 }
 
-// a += wa[k] x(lane K0 + k), b += wb[k] x(lane K0 + k), k < N, for the lanes
-// of each 16-lane row: x is broadcast within the row by the multiply-add's own
-// DPP operand (row_newbcast).  One block per group of up to four: a DPP operand
-// may be read two wait states after a VALU write, which the leading s_nop
-// covers whatever the compiler places in front; nothing in the block writes
-// x.
-#define SSMX_BCAST(K, A, B)                                                 \
-    "v_fmac_f64_dpp %0, %2, " A " row_newbcast:" K                          \
-    " row_mask:0xf bank_mask:0xf\n\t"                                       \
-    "v_fmac_f64_dpp %1, %2, " B " row_newbcast:" K                          \
-    " row_mask:0xf bank_mask:0xf\n\t"
-
-template <int K0, int N>
-__device__ __forceinline__ void bcast_fma(double &a, double &b, double x,
-                                          const double *wa, const double *wb)
-{
-    if constexpr (N >= 4) {
-        asm("s_nop 1\n\t" SSMX_BCAST("%11", "%3", "%7")
-                SSMX_BCAST("%12", "%4", "%8") SSMX_BCAST("%13", "%5", "%9")
-                    SSMX_BCAST("%14", "%6", "%10")
-            : "+v"(a), "+v"(b)
-            : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wa[2]), "v"(wa[3]),
-              "v"(wb[0]), "v"(wb[1]), "v"(wb[2]), "v"(wb[3]), "n"(K0),
-              "n"(K0 + 1), "n"(K0 + 2), "n"(K0 + 3));
-        bcast_fma<K0 + 4, N - 4>(a, b, x, wa + 4, wb + 4);
-    } else if constexpr (N >= 2) {
-        asm("s_nop 1\n\t" SSMX_BCAST("%7", "%3", "%5")
-                SSMX_BCAST("%8", "%4", "%6")
-            : "+v"(a), "+v"(b)
-            : "v"(x), "v"(wa[0]), "v"(wa[1]), "v"(wb[0]), "v"(wb[1]),
-              "n"(K0), "n"(K0 + 1));
-        bcast_fma<K0 + 2, N - 2>(a, b, x, wa + 2, wb + 2);
-    } else if constexpr (N == 1) {
-        asm("s_nop 1\n\t" SSMX_BCAST("%5", "%3", "%4")
-            : "+v"(a), "+v"(b)
-            : "v"(x), "v"(wa[0]), "v"(wb[0]), "n"(K0));
-    }
-}
-#undef SSMX_BCAST
-
-// a += w[k] x(lane K0 + k), k < N.
-template <int K0, int N>
-__device__ __forceinline__ void bcast_fma1(double &a, double x,
-                                           const double *w)
-{
-    if constexpr (N >= 1) {
-        asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3"
-            " row_mask:0xf bank_mask:0xf"
-            : "+v"(a)
-            : "v"(x), "v"(w[0]), "n"(K0));
-        bcast_fma1<K0 + 1, N - 1>(a, x, w + 1);
-    }
-}
-
-// Coefficients of one exponential for one lane: P_s(u) = sum_o c[s][o] u^o.
-template <int N, int D>
-__device__ __forceinline__ void horner(double (&w)[N],
-                                       const double (&c)[N][D + 1], double u)
-{
-#pragma unroll
-    for (int s = 0; s < N; ++s) {
-        w[s] = c[s][D];
-#pragma unroll
-        for (int o = D - 1; o >= 0; --o)
-            w[s] = fma(u, w[s], c[s][o]);
-    }
-}
-
-// v of the lane 16 further or back, i.e. of the other row of its pair.
-__device__ __forceinline__ double swap_rows(double v, bool odd_row)
-{
-    const auto lo = __builtin_amdgcn_permlane16_swap(
-        __double2loint(v), __double2loint(v), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap(
-        __double2hiint(v), __double2hiint(v), false, false);
-    // result 0 holds the even rows' values in both rows, result 1 the odd
-    // rows'
-    return odd_row ? __hiloint2double(hi[0], lo[0])
-                   : __hiloint2double(hi[1], lo[1]);
-}
-
 // The same exponentials for models of one sector pair, without LDS in the
 // exchange: a pair of 16-lane rows holds an instance, each row one sector.
 // A lane multiplies its row's broadcast components into two sums, its own
@@ -566,58 +399,131 @@ __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
     }
 }
 
-// Sum of v over the wavefront's halves (lane, lane ^ 32), in every lane.
-__device__ __forceinline__ double sum_halves(double v)
-{
-    const auto lo = __builtin_amdgcn_permlane32_swap(
-        __double2loint(v), __double2loint(v), false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap(
-        __double2hiint(v), __double2hiint(v), false, false);
-    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
-}
-
-// One instance on the whole wavefront: both halves hold the state (rows as
-// in series_row_kernel); the first half multiplies the first S = ceil(N / 2)
-// components of its rows, the second half the others, which a rotation within
-// the row brings to the same lanes.
-template <int N>
-struct Halves {
-    static constexpr int S = (N + 1) / 2;
-
-    // x in the first half, x of lane + S (of the row) in the second
-    static __device__ __forceinline__ double shifted(double x)
-    {
-        constexpr int kRotate = 0x120 + 16 - S;     // row_ror
-        const int lo = __double2loint(x), hi = __double2hiint(x);
-        return __hiloint2double(
-            __builtin_amdgcn_update_dpp(hi, hi, kRotate, 0xC, 0xF, false),
-            __builtin_amdgcn_update_dpp(lo, lo, kRotate, 0xC, 0xF, false));
-    }
-
-    // x <- exp(A) x
-    template <int DA, int DB>
-    static __device__ __forceinline__ void exponential(
-        double &x, double f, const double (&ca)[S][DA + 1],
-        const double (&cb)[S][DB + 1], bool odd_row)
-    {
-        const double u = f * f;
-        double wa[S], wb[S];
-        horner<S, DA>(wa, ca, u);
-        horner<S, DB>(wb, cb, u);
-        double ya = 0.0, yb = 0.0;
-        bcast_fma<0, S>(ya, yb, shifted(x), wa, wb);
-        x += sum_halves(fma(f, swap_rows(yb, odd_row), ya));
-    }
-
-    // M x for a matrix within the sectors
-    static __device__ __forceinline__ double within(double xs,
-                                                    const double (&m)[S])
-    {
-        double y = 0.0;
-        bcast_fma1<0, S>(y, xs, m);
-        return sum_halves(y);
-    }
+// Sweeps of one instance per wavefront (Halves): fewer instructions per
+// step than two instances on a wavefront, for launches that do not fill the
+// SIMDs (64 points of the 7-level sweep: 344 ns a step in series_row_kernel).
+// With p.store every exponential's input is kept for the adjoint: at J = 2
+// half 0 of the wavefront's 64 doubles per step holds the input of
+// exponential 1 and half 1 that of exponential 0, one coalesced store.
+struct HParams {
+    ssmx_series_desc d;
+    const int32_t *lanes;
+    const double *table;
+    const double *w;
+    const double *nodes;
+    const ssmx_wave *waves;
+    const ssmx_segment *segs;
+    const double *rho0;
+    const double *obs;
+    double *out;
+    double *store;
 };
+
+template <int N, int DA, int DB, int J, bool STORE>
+__global__ __launch_bounds__(kWave)
+__attribute__((amdgpu_waves_per_eu(2))) void series_half_kernel(HParams p)
+{
+    constexpr int S = Halves<N>::S;
+    __shared__ double fbuf[kWave];
+    const ssmx_series_desc &d = p.d;
+    const int lane = threadIdx.x;
+    const bool odd_row = (lane & 16) != 0;
+    const int state = p.lanes[lane];
+    const bool has = state >= 0;
+    const long inst = blockIdx.x;
+    double ca[S][DA + 1], cb[S][DB + 1];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+        for (int o = 0; o <= DA; ++o)
+            ca[s][o] = p.table[(s * (DA + 1) + o) * kWave + lane];
+#pragma unroll
+        for (int o = 0; o <= DB; ++o)
+            cb[s][o] =
+                p.table[(S * (DA + 1) + s * (DB + 1) + o) * kWave + lane];
+    }
+    double x = has ? p.rho0[(size_t)inst * d.n + state] : 0.0;
+    const bool read_full = (d.flags & SSMX_READ_FULL) != 0;
+    const bool read_int = (d.flags & SSMX_READ_INTEGRAL) != 0;
+    const double ob0 = !read_full && has ? p.obs[state] : 0.0;
+    const double ob1 =
+        !read_full && has && d.n_obs > 1 ? p.obs[d.n + state] : 0.0;
+    // sum over the first half's lanes (idle ones hold 0)
+    auto observe = [&](double v, long index) {
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1)
+            v += __shfl_xor(v, off, kWave);
+        if (lane == 0)
+            p.out[index] = v;
+    };
+    const Clock clk{d.t0, d.dt, d.h, d.fine, d.n_node, p.nodes, p.w};
+    DriveFactors<J> drive(p.waves + inst / d.wave_group, p.segs, d.gen, 1,
+                          lane);
+    const int B = drive.B;
+    const long total = (long)d.n_out * d.fine;
+    double *store = STORE ? p.store + (size_t)inst * total * 32 * J : nullptr;
+    double xint = 0.0;
+    const double half_h = 0.5 * d.h;
+    double fc[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+        fc[j] = 0.0;
+    int b = B;
+    long step = 0;
+    for (int i = 0; i < d.n_out; ++i) {
+        for (int k = 0; k < d.fine; ++k, ++step) {
+            if (b == B) {
+                b = 0;
+                drive.fill(clk, p.segs, i, k, total - step, lane, fbuf);
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+                    fc[j] = fbuf[j];
+            }
+            double fn[J];
+            const int nb = b + 1 < B ? b + 1 : b;
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                fn[j] = fbuf[nb * J + j];
+            const double before = x;
+#pragma unroll
+            for (int j = J - 1; j >= 0; --j) {
+                if constexpr (STORE && J == 2) {
+                    if (j == 0)
+                        store[(size_t)step * 64 + lane] =
+                            lane < 32 ? before : x;
+                }
+                if constexpr (STORE && J == 1) {
+                    if (lane < 32)
+                        store[(size_t)step * 32 + lane] = x;
+                }
+                Halves<N>::template exponential<DA, DB>(x, fc[j], ca, cb,
+                                                        odd_row);
+            }
+            if (read_int) {
+                ssmx::keep_branch();
+                xint = fma(half_h, before + x, xint);
+            }
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                fc[j] = fn[j];
+            ++b;
+        }
+        if (read_full) {
+            // (the host clears the states without a lane)
+            if (has && lane < 32)
+                p.out[((size_t)inst * d.n_out + i) * d.n + state] = x;
+        } else if (!read_int) {
+            observe(ob0 * x, ((size_t)inst * d.n_out + i) * d.n_obs);
+            if (d.n_obs > 1)
+                observe(ob1 * x, ((size_t)inst * d.n_out + i) * d.n_obs + 1);
+        }
+    }
+    if (read_int) {
+        observe(ob0 * xint, (size_t)inst * d.n_obs);
+        if (d.n_obs > 1)
+            observe(ob1 * xint, (size_t)inst * d.n_obs + 1);
+    }
+}
 
 struct QSParams {
     ssmx_series_desc d;
@@ -970,6 +876,76 @@ extern "C" int ssmx_series_queue(
         return launch_queue_scheme<2, 1>(p, waves_per_block, s);
     if (da == 2 && db == 2)
         return launch_queue_scheme<2, 2>(p, waves_per_block, s);
+    return set_error(SSMX_EINVAL, "no series kernel for orders da=%d, db=%d",
+                     da, db);
+}
+
+namespace {
+
+template <int DA, int DB, int J>
+int launch_half(const HParams &p, hipStream_t stream)
+{
+    if (p.store)
+        hipLaunchKernelGGL((series_half_kernel<11, DA, DB, J, true>),
+                           dim3(p.d.n_inst), dim3(kWave), 0, stream, p);
+    else
+        hipLaunchKernelGGL((series_half_kernel<11, DA, DB, J, false>),
+                           dim3(p.d.n_inst), dim3(kWave), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return set_error(SSMX_ELAUNCH, "series launch: %s",
+                         hipGetErrorString(e));
+    return SSMX_OK;
+}
+
+template <int DA, int DB>
+int launch_half_scheme(const HParams &p, hipStream_t stream)
+{
+    return p.d.n_exp == 1 ? launch_half<DA, DB, 1>(p, stream)
+                          : launch_half<DA, DB, 2>(p, stream);
+}
+
+}  // namespace
+
+extern "C" int ssmx_propagate_series_wave(
+    const ssmx_series_desc *desc, const int32_t *lanes, const double *table,
+    const double *cf_weights, const double *cf_nodes, const ssmx_wave *waves,
+    const ssmx_segment *segments, const double *rho0, const double *obs,
+    double *out, double *store, void *stream)
+{
+    ssmx::error_buffer()[0] = '\0';
+    const int rc = validate(desc);
+    if (rc)
+        return rc;
+    if (desc->na != 11 || desc->n_exp > 2 || desc->sector_rows < 1 ||
+        desc->members != 1)
+        return set_error(SSMX_EINVAL, "one instance per wavefront: na=%d, "
+                         "n_exp=%d, sector_rows=%d, members=%d", desc->na,
+                         desc->n_exp, desc->sector_rows, desc->members);
+    if (!lanes || !table || !cf_weights || !cf_nodes || !waves ||
+        !segments || !rho0 || !out ||
+        (!(desc->flags & SSMX_READ_FULL) && !obs))
+        return set_error(SSMX_EINVAL, "null required pointer");
+    HParams p;
+    p.d = *desc;
+    p.lanes = lanes;
+    p.table = table;
+    p.w = cf_weights;
+    p.nodes = cf_nodes;
+    p.waves = waves;
+    p.segs = segments;
+    p.rho0 = rho0;
+    p.obs = obs;
+    p.out = out;
+    p.store = store;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int da = desc->da, db = desc->db;
+    if (da == 1 && db == 1)
+        return launch_half_scheme<1, 1>(p, s);
+    if (da == 2 && db == 1)
+        return launch_half_scheme<2, 1>(p, s);
+    if (da == 2 && db == 2)
+        return launch_half_scheme<2, 2>(p, s);
     return set_error(SSMX_EINVAL, "no series kernel for orders da=%d, db=%d",
                      da, db);
 }

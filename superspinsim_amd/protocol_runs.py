@@ -15,7 +15,8 @@ import numpy as np
 
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
-from superspinsim_amd.series import SeriesModel, coefficient_matrices
+from superspinsim_amd.series import (
+    SeriesModel, coefficient_matrices, lane_entries, lane_table)
 
 _f64 = np.float64
 
@@ -122,8 +123,7 @@ class ProtocolRuns:
         gen = sim.gens[drive] if drive is not None else \
             np.zeros((sim.n, sim.n))
         model = SeriesModel.of_sets(sets, gen, weights, h)
-        if model is None or model.n_sectors > 2 or \
-                max(s.size for s in model.members) > 11:
+        if model is None or not model.one_pair():
             return None
         plan = model.plan(drive_max_of(drive), tolerance)
         if plan is None:
@@ -142,10 +142,10 @@ class ProtocolRuns:
             rec["set0"][free] = [power_of[int(k)] for k in index[free]]
         levels = int(count[free].max()).bit_length() if used.size else 0
         self.levels = levels
-        lanes, own, opp = cls._lanes(model)
+        lanes, own, opp = lane_entries(model)
         self.d_lanes = device_tensor(lanes)
         self.d_table = device_tensor(np.array(
-            [cls._rows(m, own, opp, plan[0], plan[1])
+            [lane_table(m, own, opp, plan[0], plan[1])
              for m in model.matrices(*plan)]))
         powers = np.zeros((max(used.size, 1), max(levels, 1), 2, 6, 64))
         for k in used:
@@ -214,47 +214,9 @@ class ProtocolRuns:
                 values, driven, inst)
 
     @staticmethod
-    def _lanes(model):
-        """(state per lane, own components, opposite rows): the matrix entry
-        [target state, source state] of each lane's six own-sector slots,
-        and of the slots it multiplies for the opposite sector's row."""
-        lanes = np.full(64, -1, dtype=np.int32)
-        own, opp = [], []
-        pair = [model.members[0], model.members[1]
-                if model.n_sectors > 1 else np.zeros(0, dtype=np.int64)]
-        linked = model.n_sectors > 1 and model.opposite[0] == 1
-        for lane in range(64):
-            half, row, i = lane // 32, (lane // 16) % 2, lane % 16
-            mine, other = pair[row], pair[1 - row]
-            if i < mine.size:
-                lanes[lane] = mine[i]
-            for s in range(6 if half == 0 else 5):
-                k = s + 6 * half
-                if k >= mine.size:
-                    continue
-                if i < mine.size:
-                    own.append((s, lane, mine[i], mine[k]))
-                if linked and i < other.size:
-                    opp.append((s, lane, other[i], mine[k]))
-        return lanes, np.array(own).reshape(-1, 4), \
-            np.array(opp, dtype=np.int64).reshape(-1, 4)
-
-    @staticmethod
     def _own(mat, own):
         out = np.zeros((6, 64))
         out[own[:, 0], own[:, 1]] = mat[own[:, 2], own[:, 3]]
-        return out
-
-    @staticmethod
-    def _rows(mats, own, opp, da, db):
-        """One set's lane table."""
-        out = np.zeros((6 * (da + 1) + 6 * (db + 1), 64))
-        for k in range(da + 1):
-            out[own[:, 0] * (da + 1) + k, own[:, 1]] = \
-                mats[2 * k][own[:, 2], own[:, 3]]
-        for k in range(db + 1):
-            out[6 * (da + 1) + opp[:, 0] * (db + 1) + k, opp[:, 1]] = \
-                mats[2 * k + 1][opp[:, 2], opp[:, 3]]
         return out
 
     @staticmethod
@@ -287,10 +249,8 @@ class ProtocolRuns:
             n=n, rows=m.n, n_inst=rho0.shape[0], members=1,
             n_exp=sim.weights.shape[0], n_node=sim.weights.shape[1], fine=1,
             n_out=0, n_obs=obs.shape[0], flags=_lib.SSMX_READ_INTEGRAL,
-            gen=self.gen, wave_group=1, na=11, da=self.plan[0], nb=11,
-            db=self.plan[1], sector=12, sectors=m.n_sectors,
-            sector_rows=m.members[0].size, reserved=0, h=self.h, t0=0.0,
-            dt=self.h)
+            gen=self.gen, wave_group=1, **m.shape(self.plan, whole=True),
+            reserved=0, h=self.h, t0=0.0, dt=self.h)
 
     def launch(self, d_order, counter, n_waves, waves_per_block, out,
                stream):

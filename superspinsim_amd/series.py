@@ -22,6 +22,11 @@ from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 
 _f64 = np.float64
 
+def simd_count():
+    """SIMDs of the device (four per CU)."""
+    return 4 * _torch().cuda.get_device_properties(0).multi_processor_count
+
+
 #: components per sector the kernels hold
 SIZES = (5, 11)
 #: (highest even order / 2, (highest odd order - 1) / 2), cheapest first
@@ -222,6 +227,12 @@ class SeriesModel:
         self.pos, self.order = pos, order
         return self
 
+    def one_pair(self):
+        """Whether one sector pair holds every state, so that a wavefront's
+        lane rows can exchange without LDS."""
+        return self.n_sectors <= 2 and \
+            max(s.size for s in self.members) <= 11
+
     def plan(self, drive_max, tol):
         """(da, db, F) for drives |c(t)| <= ``drive_max``, or None.
 
@@ -302,6 +313,70 @@ class SeriesModel:
             self._tables = (key, device_tensor(layout), device_tensor(table))
         return self._tables[1:]
 
+    def lane_tables(self, da, db, F, states):
+        """Device (state per lane, table) of one instance per wavefront;
+        ``states`` are the caller's indices of the model's."""
+        lanes, own, opp = lane_entries(self)
+        mats, = self.matrices(da, db, F)
+        return (device_tensor(np.where(
+            lanes >= 0, states[np.maximum(lanes, 0)], -1).astype(np.int32)),
+            device_tensor(lane_table(mats, own, opp, da, db)))
+
+    def shape(self, plan, whole=False):
+        """The model's fields of ``ssmx_series_desc``; ``whole``: for the
+        kernels of one instance per wavefront."""
+        size = 11 if whole else self.size
+        return dict(
+            na=size, da=plan[0], nb=size, db=plan[1],
+            sector=12 if whole else self.pad, sectors=self.n_sectors,
+            sector_rows=self.members[0].size if self.n_sectors <= 2 else 0)
+
+
+def lane_entries(model, transposed=False):
+    """(state per lane, own entries, opposite entries) of one instance on a
+    whole wavefront (``ssmx_series_queue``).
+
+    An entry (slot, lane, row, column) names the matrix element the lane
+    multiplies in that slot: of the own-sector tables, and of the tables
+    that couple to the opposite sector.  ``transposed``: those of
+    ``ssmx_series_adjoint``, whose lanes own columns.
+    """
+    lanes = np.full(64, -1, dtype=np.int32)
+    own, opp = [], []
+    pair = [model.members[0], model.members[1]
+            if model.n_sectors > 1 else np.zeros(0, dtype=np.int64)]
+    linked = model.n_sectors > 1 and model.opposite[0] == 1
+    for lane in range(64):
+        half, row, i = lane // 32, (lane // 16) % 2, lane % 16
+        mine, other = pair[row], pair[1 - row]
+        if i < mine.size:
+            lanes[lane] = mine[i]
+        for s in range(6 if half == 0 else 5):
+            k = s + 6 * half
+            if i < mine.size and k < mine.size:
+                own.append((s, lane, mine[k], mine[i]) if transposed else
+                           (s, lane, mine[i], mine[k]))
+            if not linked:
+                continue
+            if transposed and i < mine.size and k < other.size:
+                opp.append((s, lane, other[k], mine[i]))
+            if not transposed and i < other.size and k < mine.size:
+                opp.append((s, lane, other[i], mine[k]))
+    return lanes, np.array(own, dtype=np.int64).reshape(-1, 4), \
+        np.array(opp, dtype=np.int64).reshape(-1, 4)
+
+
+def lane_table(mats, own, opp, da, db):
+    """One set's table over ``lane_entries``."""
+    out = np.zeros((6 * (da + 1) + 6 * (db + 1), 64))
+    for k in range(da + 1):
+        out[own[:, 0] * (da + 1) + k, own[:, 1]] = \
+            mats[2 * k][own[:, 2], own[:, 3]]
+    for k in range(db + 1):
+        out[6 * (da + 1) + opp[:, 0] * (db + 1) + k, opp[:, 1]] = \
+            mats[2 * k + 1][opp[:, 2], opp[:, 3]]
+    return out
+
 
 class SeriesRun:
     """Staged inputs of one run through ``ssmx_propagate_series``.
@@ -322,16 +397,23 @@ class SeriesRun:
         if read != "full" and not 1 <= n_obs <= _lib.MAX_OBS:
             raise ValueError(f"{n_obs} readout rows outside 1.."
                              f"{_lib.MAX_OBS}")
-        layout, table = model.tables(*plan)
-        local = model.order
-        # the kernel's state index is the caller's
-        self.layout = layout.clone()
-        self.layout[:, 3] = device_tensor(
-            np.asarray(states)[local].astype(np.int32))
-        where = np.full(n, -1, dtype=np.int32)
-        where[states] = model.pos
-        self.d_where = device_tensor(where)
-        self.table = table
+        # a launch that leaves SIMDs idle spreads each instance over a whole
+        # wavefront: 64 points of the 7-level sweep 344 -> 270 ns a step;
+        # from two wavefronts per SIMD on, two instances to one are quicker
+        self.whole = members == 1 and model.one_pair() and \
+            weights.shape[0] <= 2 and n_inst <= simd_count()
+        states = np.asarray(states)
+        if self.whole:
+            self.layout, self.table = model.lane_tables(*plan, states)
+        else:
+            layout, self.table = model.tables(*plan)
+            # the kernel's state index is the caller's
+            self.layout = layout.clone()
+            self.layout[:, 3] = device_tensor(
+                states[model.order].astype(np.int32))
+            where = np.full(n, -1, dtype=np.int32)
+            where[states] = model.pos
+            self.d_where = device_tensor(where)
         self.d_w, self.d_nodes = device_tensor(weights), device_tensor(nodes)
         self.d_rho0, self.d_waves, self.d_segs = (
             device_tensor(np.ascontiguousarray(rho0, dtype=_f64)), d_waves,
@@ -342,10 +424,7 @@ class SeriesRun:
             n=n, rows=model.n, n_inst=n_inst, members=members,
             n_exp=weights.shape[0], n_node=weights.shape[1], fine=fine,
             n_out=n_out, n_obs=n_obs, flags=flags, gen=gen,
-            wave_group=wave_group, na=model.size, da=plan[0],
-            nb=model.size, db=plan[1], sector=model.pad,
-            sectors=model.n_sectors,
-            sector_rows=model.members[0].size if model.n_sectors <= 2 else 0,
+            wave_group=wave_group, **model.shape(plan, self.whole),
             reserved=0, h=dt / fine, t0=t0, dt=dt)
         shape = {"full": (n_inst, n_out, n), "obs": (n_inst, n_out, n_obs),
                  "integral": (n_inst, n_obs)}[read]
@@ -355,6 +434,17 @@ class SeriesRun:
     def launch(self):
         torch = _torch()
         stream = torch.cuda.current_stream().cuda_stream
+        if self.whole:
+            if self.desc.flags & _lib.SSMX_READ_FULL and \
+                    self.desc.rows < self.desc.n:
+                self.out.zero_()
+            _lib.check(_lib.load().ssmx_propagate_series_wave(
+                ctypes.byref(self.desc), _ptr(self.layout),
+                _ptr(self.table), _ptr(self.d_w), _ptr(self.d_nodes),
+                _ptr(self.d_waves), _ptr(self.d_segs), _ptr(self.d_rho0),
+                _ptr(self.d_obs), _ptr(self.out), None,
+                ctypes.c_void_p(stream)))
+            return self.out
         _lib.check(_lib.load().ssmx_propagate_series(
             ctypes.byref(self.desc), _ptr(self.layout), _ptr(self.d_where),
             _ptr(self.table), _ptr(self.d_w), _ptr(self.d_nodes),

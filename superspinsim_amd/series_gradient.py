@@ -1,0 +1,174 @@
+"""Gradients through the series in the drive (``ssmx_series_adjoint``).
+
+``SeriesGradient`` holds the tables of one parameter point of a
+``GradientProblem``: the forward's, their transposes, and d E_k / d theta.
+"""
+
+import ctypes
+
+import numpy as np
+
+from superspinsim_amd import _lib
+from superspinsim_amd.propagator import _ptr, _torch, device_tensor
+from superspinsim_amd.series import (
+    SeriesModel, lane_entries, lane_table, reachable)
+
+_f64 = np.float64
+
+#: moments of orders 0 .. ORDERS - 1 are kept by the kernel
+ORDERS = 4
+
+
+def derivative_matrices(const, drive, dconst, orders):
+    """d E_k of exp(const + f drive) in each direction dconst[i]:
+    (orders + 1, directions, n, n)."""
+    n = const.shape[0]
+    m = dconst.shape[0]
+    term = np.zeros((orders + 1, n, n))
+    term[0] = np.eye(n)
+    dterm = np.zeros((orders + 1, m, n, n))
+    total = np.zeros_like(dterm)
+    norm = float(np.abs(const).sum(axis=0).max(initial=0.0))
+    bound, t = 1.0, 0
+    while bound > 1e-22 or t <= orders + 2:
+        t += 1
+        bound *= norm / max(t - orders - 1, 1)
+        new = np.matmul(const, dterm) + np.matmul(dconst[None],
+                                                  term[:, None])
+        new[1:] += np.matmul(drive, dterm[:-1])
+        step = np.matmul(const, term)
+        step[1:] += np.matmul(drive, term[:-1])
+        term, dterm = step / t, new / t
+        total += dterm
+    return total
+
+
+class SeriesGradient:
+    """Forward and backward tables of one parameter point, or None from
+    ``build`` where the kernels do not apply."""
+
+    @classmethod
+    def build(cls, sim, const, program, waves, dconst, rho0, obs, h, tol,
+              adjoint_tol):
+        """``sim`` holds every state; ``dconst`` (directions, n, n) are the
+        derivatives of the folded constant matrix."""
+        varying = [g for g in program if g is not None]
+        if len(varying) != 1 or None not in program or sim.rotating or \
+                sim.weights.shape[0] > 2:
+            return None
+        folded, drive = sim.folded(const), sim.gens[varying[0]]
+        pattern = (folded != 0) | (drive != 0)
+        # a gradient needs the states the run reaches and those the readout
+        # depends on: a parameter may join one to the other
+        forward = reachable(pattern, rho0)
+        back = reachable(pattern.T, np.atleast_2d(obs))
+        states = np.union1d(forward, back)
+        if states.size == 0 or states.size > _lib.MAX_N:
+            return None
+        at = np.ix_(states, states)
+        c, g = folded[at], drive[at]
+        model = SeriesModel.build(c, g, sim.weights, h)
+        if model is None or len(model.sets) != 1 or not model.one_pair():
+            return None
+        plan = model.plan(max(w.abs_max()[varying[0]] for w in waves), tol)
+        if plan is None:
+            return None
+        self = cls()
+        da, db, F = plan
+        self.model, self.plan, self.states, self.h = model, plan, states, h
+        self.gen = program.index(varying[0])
+        self.d_lanes, self.d_table = model.lane_tables(*plan, states)
+        _, own, opp = lane_entries(model, transposed=True)
+        mats, = model.matrices(*plan)
+        self.d_back = device_tensor(lane_table(mats, own, opp, da, db))
+        dc = dconst[:, at[0], at[1]]
+        self.n_theta = dc.shape[0]
+        scale = h * float(sim.weights[0].sum())
+        dmats = derivative_matrices(scale * c, g, scale * dc, 7)
+        kept = cls._kept(dmats, F, adjoint_tol)
+        if kept is None:
+            return None
+        # [theta][own, opposite][slot][order][lane]
+        table = np.zeros((self.n_theta, 2, 6, ORDERS, 64))
+        for which, entries in enumerate((own, opp)):
+            s, lane, row, col = entries.T
+            for k in range(ORDERS):
+                table[:, which, s, k, lane] = kept[k][:, row, col]
+        self.d_dtable = device_tensor(table)
+        self.d_w, self.d_nodes = (device_tensor(sim.weights),
+                                  device_tensor(sim.nodes))
+        return self
+
+    @staticmethod
+    def _kept(dmats, F, tol):
+        """Orders 0 .. ORDERS - 1 of the derivatives as series in Chebyshev
+        polynomials of f / F cut there; None if more than ``tol`` of a
+        direction is cut off."""
+        count = dmats.shape[0]
+        cheb = SeriesModel._chebyshev(list(dmats), F)
+        size = np.array([np.abs(c).sum(axis=1).max(axis=1) for c in cheb])
+        if size.shape[1] and np.any(
+                size[ORDERS:].sum(axis=0) + size[-1] > tol * size.max(axis=0)):
+            return None
+        kept = [m.copy() for m in dmats[:ORDERS]]
+        for j in range(ORDERS, count):
+            unit = np.zeros(j + 1)
+            unit[j] = 1.0
+            for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(
+                    unit)[:ORDERS]):
+                if c and F ** k:
+                    kept[k] -= (c / F ** k) * cheb[j]
+        return kept
+
+    def store_bytes(self, n_inst, steps, J):
+        return n_inst * steps * J * 32 * 8
+
+    def _desc(self, problem, n_inst, n, J, S):
+        m = self.model
+        return _lib.SeriesDesc(
+            n=n, rows=m.n, n_inst=n_inst, members=1, n_exp=J, n_node=S,
+            fine=problem.F, n_out=problem.n_out, n_obs=problem.obs.shape[0],
+            flags=_lib.SSMX_READ_INTEGRAL, gen=self.gen, wave_group=1,
+            **m.shape(self.plan, whole=True), reserved=0,
+            h=problem.dt / problem.F, t0=problem.t0, dt=problem.dt)
+
+    def forward(self, problem, state, rho0, store):
+        """Integrated readouts (n_inst, n_obs); ``store`` keeps the inputs
+        of every exponential (or None)."""
+        torch = _torch()
+        n_inst, n = rho0.shape
+        J, S = self.d_w.shape
+        out = torch.empty((n_inst, problem.obs.shape[0]),
+                          dtype=torch.float64, device="cuda")
+        d_rho, d_obs = device_tensor(rho0), device_tensor(problem.obs)
+        desc = self._desc(problem, n_inst, n, J, S)
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(_lib.load().ssmx_propagate_series_wave(
+            ctypes.byref(desc), _ptr(self.d_lanes), _ptr(self.d_table),
+            _ptr(self.d_w), _ptr(self.d_nodes), _ptr(state["d_waves"]),
+            _ptr(state["d_segs"]), _ptr(d_rho), _ptr(d_obs), _ptr(out),
+            _ptr(store), ctypes.c_void_p(stream)))
+        self._keep = (d_rho, d_obs)
+        return out
+
+    def backward(self, problem, state, seed, g_theta, g_seg, lam):
+        torch = _torch()
+        n_inst = seed.shape[0]
+        n = problem.rho0.shape[-1]
+        J, S = self.d_w.shape
+        desc = self._desc(problem, n_inst, n, J, S)
+        d_obs = device_tensor(problem.obs)
+        if lam is not None:
+            lam.zero_()
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(_lib.load().ssmx_series_adjoint(
+            ctypes.byref(desc), _ptr(self.d_lanes), _ptr(self.d_back),
+            _ptr(self.d_dtable), ctypes.c_int32(self.n_theta),
+            _ptr(self.d_w), _ptr(self.d_nodes), _ptr(state["d_waves"]),
+            _ptr(state["d_segs"]), _ptr(state["inputs"]), _ptr(d_obs),
+            _ptr(seed), _ptr(g_theta), _ptr(g_seg), _ptr(lam),
+            ctypes.c_void_p(stream)))
+        self._keep_back = (d_obs, seed)
+
+
+__all__ = ["SeriesGradient", "derivative_matrices"]

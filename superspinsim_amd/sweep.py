@@ -26,7 +26,7 @@ from superspinsim_amd.propagator import (
     Propagator, _ptr, coefficient_samples, device_tensor, eig_lane_factors,
     rotating_tables, sample_exponents, taylor_plan_measured)
 from superspinsim_amd.series import (
-    SIZES, SeriesModel, SeriesRun, reachable)
+    SIZES, SeriesModel, SeriesRun, reachable, simd_count)
 
 _f64 = np.float64
 
@@ -575,9 +575,7 @@ class BatchSimulator:
             return 1
         if self.pack is not True:
             return max(1, min(limit, int(self.pack)))
-        torch = __import__("torch")
-        simds = 4 * torch.cuda.get_device_properties(
-            0).multi_processor_count
+        simds = simd_count()
         return min(range(1, limit + 1), key=lambda k: (
             -(-(-(-n_inst // k)) // simds), k))
 
@@ -785,9 +783,7 @@ class BatchSimulator:
         if found is not None:
             # the series kernel: as many columns per wavefront as fit, 3 (or
             # 2 for the larger tables) wavefronts per SIMD
-            torch = __import__("torch")
-            simds = 4 * torch.cuda.get_device_properties(
-                0).multi_processor_count
+            simds = simd_count()
             small = found[0].size == SIZES[0]
             k = max(1, min(_lib.MAX_N // n,
                            _lib.MAX_N // self.weights.shape[0],

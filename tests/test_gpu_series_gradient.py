@@ -1,0 +1,91 @@
+"""Gradients through the series in the drive against the Frechet chain (GPU).
+
+``store_inputs=False`` takes the Taylor forward and the checkpointed Frechet
+adjoint (degree 10, 1e-13 per exponential here); the default takes the
+series. Both are exact to their truncation, which is relative to each
+exponential: the parameter gradients differ by at most a few 1e-12 of their
+own size plus the cancellation floor 1e-12 F / theta_scale that the oracle
+comparison of the Frechet adjoint uses, over a thousand steps.
+"""
+
+import numpy as np
+import pytest
+
+from superspinsim_amd import configs
+from superspinsim_amd.adjoint import GradientProblem
+from superspinsim_amd.sweep import Waveform
+
+pytestmark = pytest.mark.gpu
+
+
+def _problem(exps, incoherent, points, outputs, fine, rabi, store, two_rows,
+             seed=5):
+    wl = configs.odmr7(1, use_incoherent=incoherent)
+    rng = np.random.default_rng(seed)
+    scale = configs.drive_amplitude(1.0)
+    h = 20e-12 if exps == 2 else 10e-12
+    end = outputs * fine * h
+    # segments with gaps, an edge on a step, edges inside steps
+    edges = np.array([0.0, 0.13, 0.2, 0.3703, 0.37045, 0.9]) * end
+    edges[2] = round(0.2 * end / h) * h
+    freqs = rng.uniform(2.70e9, 2.76e9, points)
+
+    def waveforms(amps):
+        out = []
+        for f in freqs:
+            w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, wl.excitation])
+            for k, (a, b) in enumerate(((0, 1), (2, 3), (4, 5))):
+                w.add(1, edges[a], edges[b], scale * amps[k],
+                      2 * np.pi * f, 0.3 * k, param=k, dparam=scale)
+            # an untagged segment between tagged ones
+            w.add(1, edges[3], edges[4], scale * rabi, 2 * np.pi * f, 0.0)
+            out.append(w)
+        return out
+
+    rho = np.array([1.0 if (y, x) == (1, 1) else 0.0
+                    for y, x, _ in wl.vmap])
+    obs = wl.obs
+    if two_rows:
+        obs = np.concatenate([obs, rho[None]])
+    problem = GradientProblem(
+        lambda th: configs.nv7_generators(th, use_incoherent=incoherent),
+        waveforms, rho, obs, 1e-10, 1e-10 + end * (1 + 1e-9), fine * h, fine,
+        exps, 300, adjoint_tolerance=1e-13 if not store else 1e-12,
+        theta_scale=configs.THETA_SCALE,
+        store_inputs=False if not store else "auto")
+    theta = configs.nv7_theta0() * (1 + 0.01 * rng.standard_normal(9))
+    amps = rng.normal(rabi, rabi / 6, 3)
+    seeds = rng.uniform(0.5, 1.5, (points, obs.shape[0]))
+    return problem, theta, amps, seeds
+
+
+@pytest.mark.parametrize("exps,incoherent,points,outputs,fine,rabi,two", [
+    (2, False, 3, 10, 100, 3e6, False), (2, True, 5, 7, 61, 8e6, True),
+    (2, True, 1, 1, 3, 3e5, False), (1, True, 2, 30, 33, 3e6, False)])
+def test_series_gradient_equals_frechet(gpu, exps, incoherent, points,
+                                        outputs, fine, rabi, two):
+    res = {}
+    for store in (True, False):
+        problem, theta, amps, seeds = _problem(
+            exps, incoherent, points, outputs, fine, rabi, store, two)
+        out, state = problem.forward(theta, amps)
+        assert state["by_series"] == store
+        back = problem.backward(state, seeds, lambda_out=True)
+        res[store] = (out.cpu().numpy(),
+                      {k: v.cpu().numpy() for k, v in back.items()})
+    (fa, a), (fb, b) = res[True], res[False]
+    assert np.max(np.abs(fa - fb)) <= 1e-12 * np.max(np.abs(fb))
+    weight = (np.abs(fb) * seeds).sum(axis=1)
+    err = np.abs(a["theta"] - b["theta"])
+    floor = 1e-12 * weight[:, None] / configs.THETA_SCALE[None]
+    size = np.abs(b["theta"])
+    print("theta", (err / (1e-11 * size + floor)).max(axis=0), flush=True)
+    assert np.all(err <= 1e-11 * size + floor)
+    for key in ("records", "amplitudes"):
+        # (all zero where three steps are too short for any effect)
+        e, most = np.max(np.abs(a[key] - b[key])), np.max(np.abs(b[key]))
+        print(key, f"{e:.1e} of {most:.1e}")
+        assert e <= 1e-10 * most
+    e = np.max(np.abs(a["lambda"] - b["lambda"])) / \
+        np.max(np.abs(b["lambda"]))
+    assert e <= 1e-12

@@ -132,3 +132,23 @@ int main(void) {
     assert [int(v) for v in got.stdout.split()] == [
         ctypes.sizeof(D), D.wave_group.offset, D.sector_rows.offset,
         D.h.offset]
+
+
+def test_derivative_matrices_match_differences():
+    """Central differences of the extended-precision E_k with a step of
+    1e-5: truncation of order 1e-10 of the entries."""
+    from superspinsim_amd.series_gradient import derivative_matrices
+    rng = np.random.default_rng(2)
+    wl = configs.odmr3(1)
+    const, drive = _pair(wl)
+    const = const * (H / 2)
+    dirs = rng.standard_normal((3,) + const.shape)
+    got = derivative_matrices(const, drive, dirs, 5)
+    for i, d in enumerate(dirs):
+        up = coefficient_matrices([(const, 1.0), (d, 1e-5)], drive, 5, True)
+        down = coefficient_matrices([(const, 1.0), (d, -1e-5)], drive, 5,
+                                    True)
+        for k in range(6):
+            want = (up[k] - down[k]) / 2e-5
+            assert np.max(np.abs(got[k, i] - want)) <= \
+                1e-9 * np.max(np.abs(want))
