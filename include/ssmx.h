@@ -340,6 +340,43 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
                         double *lambda_out, void *stream);
 
 /*
+ * ssmx_propagate_series for models of more rows than a wavefront (at most
+ * 256), one workgroup of n_blocks (at most 12) wavefronts per instance;
+ * n_exp = n_node = 2, da = db = 1; members, na, nb, sector fields unused.
+ *
+ * Rows are taken in pairs of one sector. A pair's columns are spread over
+ * `lanes` (8 or 16) consecutive lanes of its wavefront; every lane of
+ * wavefront b holds blocks[b].slots (4..7) columns of the pair's own sector
+ * and as many of the opposite one (padded with coefficient 0). The lower half
+ * of the lanes keeps the pair's first row, the upper half the second.
+ * blocks   ssmx_series_block [n_blocks]
+ * states   int32 [n_blocks][64][2]: the lane's row (0..255, -1 idle) and its
+ *          state index (idle lanes 0)
+ * columns  int32 from blocks[b].columns: [2 slots][64] rows (0..255) of the
+ *          own-sector columns, then of the opposite ones
+ * table    double from blocks[b].table: [2 slots][4][64], entry 2 o + i of
+ *          column s the coefficient of row i of the pair, order 2 o (own
+ *          sector; E_0 without the identity) or 2 o + 1 (opposite sector)
+ * READ_FULL: states without a row are not written.
+ */
+typedef struct ssmx_series_block {
+    int32_t slots;
+    int32_t lanes;
+    int32_t columns;
+    int32_t table;
+} ssmx_series_block;
+
+int ssmx_propagate_series_wide(const ssmx_series_desc *desc,
+                               const ssmx_series_block *blocks,
+                               int32_t n_blocks, const int32_t *states,
+                               const int32_t *columns, const double *table,
+                               const double *cf_weights,
+                               const double *cf_nodes, const ssmx_wave *waves,
+                               const ssmx_segment *segments,
+                               const double *rho0, const double *obs,
+                               double *out, void *stream);
+
+/*
  * The reference's non-residual exponential (use_residual=False).
  *
  * Each exponential is (I + A / scale)^(2^squarings) with scale = 4^R and

@@ -116,7 +116,8 @@ class Wave(ctypes.Structure):
 
 #: every symbol include/ssmx.h declares
 EXPORTS = ("ssmx_propagate", "ssmx_propagate_series", "ssmx_series_queue",
-           "ssmx_propagate_series_wave", "ssmx_series_adjoint",
+           "ssmx_propagate_series_wave", "ssmx_propagate_series_wide",
+           "ssmx_series_adjoint",
            "ssmx_propagate_dense", "ssmx_chunk_combine",
            "ssmx_propagate_queue",
            "ssmx_propagate_queue_noalloc", "ssmx_adjoint",
@@ -155,6 +156,9 @@ def load():
     lib.ssmx_propagate_series_wave.argtypes = \
         [ctypes.POINTER(SeriesDesc)] + [vp] * 11
     lib.ssmx_propagate_series_wave.restype = ctypes.c_int
+    lib.ssmx_propagate_series_wide.argtypes = \
+        [ctypes.POINTER(SeriesDesc), vp, ctypes.c_int32] + [vp] * 11
+    lib.ssmx_propagate_series_wide.restype = ctypes.c_int
     lib.ssmx_series_adjoint.argtypes = (
         [ctypes.POINTER(SeriesDesc)] + [vp] * 3 + [ctypes.c_int32] +
         [vp] * 11)

@@ -1,0 +1,308 @@
+// ssmx_series_wide.hip - the series in the drive for models of more rows than
+// a wavefront (the 21-level NV + 14N model, 171 involved states).
+//
+// The Taylor kernel for such models (ssmx_wide.hip) pays 11 exchanges across
+// the workgroup's wavefronts per exponential, each about 430 cycles of LDS
+// round trip and barrier for some 10 multiply-adds a row. The series reads
+// every component that a row depends on once: about 70 a row here (the E_k
+// fill in, entries far below the tolerance are left out), one barrier per
+// exponential.
+//
+// Split. Two rows with nearly the same columns share 8 lanes (16 for the widest
+// pairs): a lane gathers each of its columns once for both rows, the lanes
+// add their parts by DPP. Pairs are sorted by width, and each wavefront runs
+// code for its own entries per lane (C own-sector and C opposite-sector
+// columns, coefficients and LDS addresses in registers). 171 rows take 12
+// wavefronts, three per SIMD. One wavefront, the last and narrowest,
+// evaluates the drive for all; the first one adds up readouts.
+//
+// Measured, 25,000 steps of 512 points: Taylor 4.6 us a step and round of
+// 256 workgroups, series 1.17.
+#include "ssmx_series_dev.h"
+
+namespace {
+
+using ssmx::Clock;
+using ssmx::DriveFactors;
+using ssmx::kWave;
+using ssmx::quad_perm;
+using ssmx::set_error;
+
+constexpr int kMaxWaves = 12;
+constexpr int kMaxRows = 256;
+
+typedef __attribute__((address_space(3))) double lds_double;
+
+struct WSParams {
+    ssmx_series_desc d;
+    const ssmx_series_block *blocks;
+    const int32_t *states;
+    const int32_t *columns;
+    const double *table;
+    const double *w;
+    const double *nodes;
+    const ssmx_wave *waves;
+    const ssmx_segment *segs;
+    const double *rho0;
+    const double *obs;
+    double *out;
+};
+
+// The sum of a pair's rows over its 8 or 16 lanes: that of row a in its lower
+// half, of row b in its upper half.
+__device__ __forceinline__ double sum_pair(double a, double b, bool sixteen,
+                                           bool upper)
+{
+    const double keep = upper ? b : a, give = upper ? a : b;
+    double v;
+    if (sixteen) {
+        v = keep + quad_perm<0x140>(give);      // row_mirror
+        v += quad_perm<0x141>(v);               // row_half_mirror
+    } else {
+        v = keep + quad_perm<0x141>(give);
+    }
+    v += quad_perm<0xB1>(v);                    // lane ^ 1
+    v += quad_perm<0x4E>(v);                    // lane ^ 2
+    return v;
+}
+
+// Readouts of the components in `x` (LDS) by one wavefront.
+__device__ __forceinline__ void observe(const WSParams &p, const double *x,
+                                        const double *obs, long index,
+                                        int lane)
+{
+    double v[kMaxRows / kWave];
+#pragma unroll
+    for (int k = 0; k < kMaxRows / kWave; ++k)
+        v[k] = x[k * kWave + lane];
+    for (int o = 0; o < p.d.n_obs; ++o) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < kMaxRows / kWave; ++k)
+            s = fma(obs[o * kMaxRows + k * kWave + lane], v[k], s);
+        s = ssmx::wave_sum(s);
+        if (lane == 0)
+            p.out[index * p.d.n_obs + o] = s;
+    }
+}
+
+// One wavefront's part of its workgroup's instance: C own-sector and C
+// opposite-sector columns per lane. FILL: this wavefront evaluates the drive.
+template <int C, bool FILL>
+__device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
+                                         double *fbuf, const double *obs,
+                                         const ssmx_series_block &blk,
+                                         int wave, int lane, long inst)
+{
+    constexpr int J = 2, B = kWave / J;
+    const ssmx_series_desc &d = p.d;
+    const int row = p.states[2 * (wave * kWave + lane)];
+    const int state = p.states[2 * (wave * kWave + lane) + 1];
+    const bool sixteen = blk.lanes == 16;
+    const int half = blk.lanes / 2;
+    const bool upper = (lane & half) != 0;
+    const bool leader = row >= 0 && lane % half == 0;
+    const double *t = p.table + blk.table + lane;
+    const int32_t *col = p.columns + blk.columns + lane;
+    // [column][order][row of the pair]
+    double ca[C][2][2], cb[C][2][2];
+    lds_double *xa[C], *xb[C];
+#pragma unroll
+    for (int s = 0; s < C; ++s) {
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            ca[s][o / 2][o % 2] = t[(s * 4 + o) * kWave];
+            cb[s][o / 2][o % 2] = t[((C + s) * 4 + o) * kWave];
+        }
+        xa[s] = (lds_double *)xbuf + col[s * kWave];
+        xb[s] = (lds_double *)xbuf + col[(C + s) * kWave];
+    }
+    double x = row >= 0 ? p.rho0[(size_t)inst * d.n + state] : 0.0;
+    if (leader)
+        xbuf[row] = x;
+    const bool read_full = (d.flags & SSMX_READ_FULL) != 0;
+    const bool read_int = (d.flags & SSMX_READ_INTEGRAL) != 0;
+    const Clock clk{d.t0, d.dt, d.h, d.fine, d.n_node, p.nodes, p.w};
+    DriveFactors<J> drive(p.waves + inst / d.wave_group, p.segs, d.gen, 1,
+                          lane);
+    const long total = (long)d.n_out * d.fine;
+    if constexpr (FILL)
+        drive.fill(clk, p.segs, 0, 0, total, lane, fbuf);
+    double xint = 0.0;
+    const double half_h = 0.5 * d.h;
+    __syncthreads();
+    int b = 0;
+    long step = 0;
+    double *fcur = fbuf;
+    for (int i = 0; i < d.n_out; ++i) {
+        for (int k = 0; k < d.fine; ++k, ++step) {
+            const double fc[J] = {fcur[b * J], fcur[b * J + 1]};
+            if (++b == B) {
+                // the next batch: read from the next step on, two barriers
+                // from here; its buffer was last read a batch ago
+                fcur = fcur == fbuf ? fbuf + kWave : fbuf;
+                b = 0;
+                if constexpr (FILL)
+                    drive.fill(clk, p.segs, i, k + 1, total - step - 1, lane,
+                               fcur);
+            }
+            const double before = x;
+#pragma unroll
+            for (int j = J - 1; j >= 0; --j) {
+                // the first exponential reads buffer 0 and writes buffer 1,
+                // the second goes back: a wavefront that still reads a buffer
+                // is one barrier ahead of any that writes it
+                const int from = j == 1 ? 0 : kMaxRows;
+                const int to = j == 1 ? kMaxRows : 0;
+                double va[C], vb[C];
+#pragma unroll
+                for (int s = 0; s < C; ++s)
+                    va[s] = xa[s][from];
+#pragma unroll
+                for (int s = 0; s < C; ++s)
+                    vb[s] = xb[s][from];
+                const double f = fc[j], u = f * f;
+                double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+#pragma unroll
+                for (int s = 0; s < C; ++s) {
+                    a0 = fma(fma(u, ca[s][1][0], ca[s][0][0]), va[s], a0);
+                    a1 = fma(fma(u, ca[s][1][1], ca[s][0][1]), va[s], a1);
+                }
+#pragma unroll
+                for (int s = 0; s < C; ++s) {
+                    b0 = fma(fma(u, cb[s][1][0], cb[s][0][0]), vb[s], b0);
+                    b1 = fma(fma(u, cb[s][1][1], cb[s][0][1]), vb[s], b1);
+                }
+                x += sum_pair(fma(f, b0, a0), fma(f, b1, a1), sixteen, upper);
+                if (leader)
+                    xbuf[to + row] = x;
+                __syncthreads();
+            }
+            if (read_int) {
+                ssmx::keep_branch();
+                xint = fma(half_h, before + x, xint);
+            }
+        }
+        if (read_full) {
+            if (leader)
+                p.out[((size_t)inst * d.n_out + i) * d.n + state] = x;
+        } else if (!read_int && wave == 0) {
+            observe(p, xbuf, obs, inst * d.n_out + i, lane);
+        }
+    }
+    if (read_int) {
+        // (buffer 1 was last read before the last barrier)
+        if (leader)
+            xbuf[kMaxRows + row] = xint;
+        __syncthreads();
+        if (wave == 0)
+            observe(p, xbuf + kMaxRows, obs, inst, lane);
+    }
+}
+
+template <int C>
+__device__ __forceinline__ void run_class(const WSParams &p, double *xbuf,
+                                          double *fbuf, const double *obs,
+                                          const ssmx_series_block &blk,
+                                          int wave, int lane, long inst,
+                                          bool fill)
+{
+    if (fill)
+        run_wave<C, true>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+    else
+        run_wave<C, false>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+}
+
+__global__ __launch_bounds__(kWave *kMaxWaves)
+__attribute__((amdgpu_waves_per_eu(3))) void series_wide_kernel(WSParams p)
+{
+    __shared__ double xbuf[2 * kMaxRows];
+    __shared__ double fbuf[2 * kWave];
+    __shared__ double obs[SSMX_MAX_OBS * kMaxRows];
+    const int lane = threadIdx.x % kWave;
+    const int wave =
+        __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const ssmx_series_block blk = p.blocks[wave];
+    const long inst = blockIdx.x;
+    const bool fill = wave == (int)(blockDim.x / kWave) - 1;
+    for (int k = threadIdx.x; k < 2 * kMaxRows; k += blockDim.x)
+        xbuf[k] = 0.0;
+    for (int k = threadIdx.x; k < p.d.n_obs * kMaxRows; k += blockDim.x)
+        obs[k] = 0.0;
+    __syncthreads();
+    const int row = p.states[2 * (wave * kWave + lane)];
+    if (row >= 0)
+        for (int o = 0; o < p.d.n_obs; ++o)
+            obs[o * kMaxRows + row] =
+                p.obs[o * p.d.n + p.states[2 * (wave * kWave + lane) + 1]];
+    // every wavefront meets the same barriers whatever its class
+    switch (blk.slots) {
+    case 4:
+        run_class<4>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        break;
+    case 5:
+        run_class<5>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        break;
+    case 6:
+        run_class<6>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        break;
+    default:
+        run_class<7>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+    }
+}
+
+}  // namespace
+
+extern "C" int ssmx_propagate_series_wide(
+    const ssmx_series_desc *desc, const ssmx_series_block *blocks,
+    int32_t n_blocks, const int32_t *states, const int32_t *columns,
+    const double *table, const double *cf_weights, const double *cf_nodes,
+    const ssmx_wave *waves, const ssmx_segment *segments, const double *rho0,
+    const double *obs, double *out, void *stream)
+{
+    ssmx::error_buffer()[0] = '\0';
+    if (!desc)
+        return set_error(SSMX_EINVAL, "null descriptor");
+    const ssmx_series_desc &d = *desc;
+    const bool full = (d.flags & SSMX_READ_FULL) != 0;
+    if (d.n < 1 || d.n > SSMX_MAX_N_WIDE || d.rows < 1 ||
+        d.rows > kMaxRows || d.n_inst < 1 || d.n_exp != 2 ||
+        d.n_node != 2 || d.da != 1 || d.db != 1 || d.fine < 1 ||
+        d.n_out < 0 || d.wave_group < 1 || d.gen < 0 ||
+        d.gen >= SSMX_MAX_GEN || !(d.h > 0.0) || !(d.dt > 0.0) ||
+        (d.flags & ~(SSMX_READ_FULL | SSMX_READ_INTEGRAL)) != 0 ||
+        (full && (d.flags & SSMX_READ_INTEGRAL)) ||
+        (!full && (d.n_obs < 1 || d.n_obs > SSMX_MAX_OBS)))
+        return set_error(SSMX_EINVAL, "wide series: n=%d, rows=%d, "
+                         "n_inst=%d, n_exp=%d, da=%d, db=%d, fine=%d, "
+                         "n_out=%d, n_obs=%d, flags=%d", d.n, d.rows, d.n_inst,
+                         d.n_exp, d.da, d.db, d.fine, d.n_out, d.n_obs,
+                         d.flags);
+    if (n_blocks < 1 || n_blocks > kMaxWaves)
+        return set_error(SSMX_EINVAL, "%d wavefronts outside 1..%d",
+                         n_blocks, kMaxWaves);
+    if (!blocks || !states || !columns || !table || !cf_weights ||
+        !cf_nodes || !waves || !segments || !rho0 || !out || (!full && !obs))
+        return set_error(SSMX_EINVAL, "null required pointer");
+    WSParams p;
+    p.d = d;
+    p.blocks = blocks;
+    p.states = states;
+    p.columns = columns;
+    p.table = table;
+    p.w = cf_weights;
+    p.nodes = cf_nodes;
+    p.waves = waves;
+    p.segs = segments;
+    p.rho0 = rho0;
+    p.obs = obs;
+    p.out = out;
+    hipLaunchKernelGGL(series_wide_kernel, dim3(d.n_inst),
+                       dim3(kWave * n_blocks), 0,
+                       static_cast<hipStream_t>(stream), p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return set_error(SSMX_ELAUNCH, "wide series launch: %s",
+                         hipGetErrorString(e));
+    return SSMX_OK;
+}

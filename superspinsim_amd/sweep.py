@@ -27,6 +27,7 @@ from superspinsim_amd.propagator import (
     rotating_tables, sample_exponents, taylor_plan_measured)
 from superspinsim_amd.series import (
     SIZES, SeriesModel, SeriesRun, reachable, simd_count)
+from superspinsim_amd.series_wide import WideModel, WideRun
 
 _f64 = np.float64
 
@@ -553,7 +554,9 @@ class BatchSimulator:
         if key not in self._series_cache:
             drive = self.gens[varying[0]] if varying else \
                 np.zeros((self.n, self.n))
-            self._series_cache[key] = SeriesModel.build(
+            build = SeriesModel.build if self.n <= _lib.MAX_N else \
+                WideModel.build
+            self._series_cache[key] = build(
                 self.folded(const), drive, self.weights, h)
         model = self._series_cache[key]
         if model is None:
@@ -581,11 +584,16 @@ class BatchSimulator:
 
     def _prepare_series(self, found, states, n, waves, program, rho0, obs,
                         read, time_start, time_step, N, wave_group=1):
-        """``SeriesRun`` of this (reduced) simulator; ``states`` are its
-        states among the caller's ``n``."""
+        """``SeriesRun`` (``WideRun`` above a wavefront's rows) of this
+        (reduced) simulator; ``states`` are its states among the caller's
+        ``n``."""
         model, plan = found
         d_waves, d_segs = stage_records(*program_records(waves, program))
         gen = next((k for k, g in enumerate(program) if g is not None), 0)
+        if model.n > _lib.MAX_N:
+            return WideRun(model, plan, states, self.weights, self.nodes,
+                           rho0, d_waves, d_segs, gen, self.F, N, time_start,
+                           time_step, obs, read)
         members = self.series_members(rho0.shape[0], model.n)
         return SeriesRun(model, plan, states, members, self.weights,
                          self.nodes, rho0, d_waves, d_segs, gen, self.F, N,
@@ -597,7 +605,8 @@ class BatchSimulator:
         """Plan, pack and stage one ``run`` on the device; returns an
         object whose ``launch`` only enqueues the kernel and whose
         ``result`` is the output of the last launch, one row per instance
-        (``SeriesRun``, ``PreparedRun`` or ``ReducedRun``)."""
+        (``SeriesRun``, ``WideRun``, ``PreparedRun`` or
+        ``ReducedRun``)."""
         N = int((time_end - time_start) / time_step)
         n_inst = len(waves)
         rho0 = np.atleast_2d(np.asarray(rho0, dtype=_f64))
