@@ -344,11 +344,12 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
  * 256), one workgroup of n_blocks (at most 12) wavefronts per instance;
  * n_exp = n_node = 2, da = db = 1; members, na, nb, sector fields unused.
  *
- * Rows are taken in pairs of one sector. A pair's columns are spread over
- * `lanes` (8 or 16) consecutive lanes of its wavefront; every lane of
- * wavefront b holds blocks[b].slots (4..7) columns of the pair's own sector
- * and as many of the opposite one (padded with coefficient 0). The lower half
- * of the lanes keeps the pair's first row, the upper half the second.
+ * Rows are taken in pairs of one sector. The columns of pair g of wavefront b
+ * are spread over its `lanes` (8 or 16) lanes 32 v + g lanes / 2 + (0 ..
+ * lanes / 2 - 1), v = 0, 1; every lane holds blocks[b].slots (4..7) columns of
+ * the pair's own sector and as many of the opposite one (padded with
+ * coefficient 0). Lanes below 32 keep the pair's first row, the others the
+ * second.
  * blocks   ssmx_series_block [n_blocks]
  * states   int32 [n_blocks][64][2]: the lane's row (0..255, -1 idle) and its
  *          state index (idle lanes 0)

@@ -9,15 +9,22 @@
 // exponential.
 //
 // Split. Two rows with nearly the same columns share 8 lanes (16 for the widest
-// pairs): a lane gathers each of its columns once for both rows, the lanes
-// add their parts by DPP. Pairs are sorted by width, and each wavefront runs
+// pairs), half of them in either half of the wavefront: a lane gathers each of
+// its columns once for both rows, a swap of the halves leaves each half one
+// row to add up by DPP. Pairs are sorted by width, and each wavefront runs
 // code for its own entries per lane (C own-sector and C opposite-sector
 // columns, coefficients and LDS addresses in registers). 171 rows take 12
 // wavefronts, three per SIMD. One wavefront, the last and narrowest,
 // evaluates the drive for all; the first one adds up readouts.
 //
-// Measured, 25,000 steps of 512 points: Taylor 4.6 us a step and round of
-// 256 workgroups, series 1.17.
+// What bounds it: VALU issue, about 700 of 1,130 cycles per exponential (134
+// gathers with four multiply-adds each over the workgroup); the rest is the
+// latency from the barrier to the first gathers and that of the sum. Measured,
+// 512 points (two rounds of 256 workgroups), per step of a round: Taylor
+// 2.35 us, series 1.05; 1.17 with rows in pair order in LDS (2.4 ways of bank
+// conflict a gather instead of 1.8) and pairs on consecutive lanes (selects
+// and a DPP step where the half swap is). Coefficients evaluated ahead of the
+// gathers gained 1% and spilled.
 #include "ssmx_series_dev.h"
 
 namespace {
@@ -48,19 +55,18 @@ struct WSParams {
     double *out;
 };
 
-// The sum of a pair's rows over its 8 or 16 lanes: that of row a in its lower
-// half, of row b in its upper half.
-__device__ __forceinline__ double sum_pair(double a, double b, bool sixteen,
-                                           bool upper)
+// The sum of a pair's rows over its lanes: that of row a in the lanes of the
+// wavefront's lower half, of row b in those of its upper half.
+__device__ __forceinline__ double sum_pair(double a, double b, bool sixteen)
 {
-    const double keep = upper ? b : a, give = upper ? a : b;
-    double v;
-    if (sixteen) {
-        v = keep + quad_perm<0x140>(give);      // row_mirror
+    // the upper half of a for the lower one of b
+    const auto lo = __builtin_amdgcn_permlane32_swap(
+        __double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(
+        __double2hiint(a), __double2hiint(b), false, false);
+    double v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    if (sixteen)
         v += quad_perm<0x141>(v);               // row_half_mirror
-    } else {
-        v = keep + quad_perm<0x141>(give);
-    }
     v += quad_perm<0xB1>(v);                    // lane ^ 1
     v += quad_perm<0x4E>(v);                    // lane ^ 2
     return v;
@@ -99,9 +105,7 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
     const int row = p.states[2 * (wave * kWave + lane)];
     const int state = p.states[2 * (wave * kWave + lane) + 1];
     const bool sixteen = blk.lanes == 16;
-    const int half = blk.lanes / 2;
-    const bool upper = (lane & half) != 0;
-    const bool leader = row >= 0 && lane % half == 0;
+    const bool leader = row >= 0 && lane % (blk.lanes / 2) == 0;
     const double *t = p.table + blk.table + lane;
     const int32_t *col = p.columns + blk.columns + lane;
     // [column][order][row of the pair]
@@ -173,7 +177,7 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
                     b0 = fma(fma(u, cb[s][1][0], cb[s][0][0]), vb[s], b0);
                     b1 = fma(fma(u, cb[s][1][1], cb[s][0][1]), vb[s], b1);
                 }
-                x += sum_pair(fma(f, b0, a0), fma(f, b1, a1), sixteen, upper);
+                x += sum_pair(fma(f, b0, a0), fma(f, b1, a1), sixteen);
                 if (leader)
                     xbuf[to + row] = x;
                 __syncthreads();

@@ -173,12 +173,10 @@ class WideModel:
         waves = self._waves(widest[rank])
         if waves is None:
             return None
-        pos = np.full(self.n, -1, dtype=np.int32)
-        for k, p in enumerate(rank):
-            a, b = pairs[p]
-            pos[a] = 2 * k
-            if b >= 0:
-                pos[b] = 2 * k + 1
+        # LDS positions by sector: the lanes of a pair then read runs of
+        # neighbours, and pairs with common columns the same ones
+        pos = np.empty(self.n, dtype=np.int32)
+        pos[np.argsort(self.sector, kind="stable")] = np.arange(self.n)
         blocks = np.zeros((len(waves), 4), dtype=np.int32)
         states = np.zeros((len(waves), 64, 2), dtype=np.int32)
         states[:, :, 0] = -1
@@ -192,17 +190,17 @@ class WideModel:
                 if first + g >= len(pairs):
                     break
                 p = rank[first + g]
-                at = g * lanes
-                c[:, at:at + lanes] = pos[pairs[p][0]]
+                h = lanes // 2
+                mine = 32 * np.arange(2)[:, None] + g * h + np.arange(h)
+                c[:, mine.ravel()] = pos[pairs[p][0]]
                 for i, r in enumerate(pairs[p]):
                     if r < 0:
                         continue
-                    half = slice(at + i * lanes // 2,
-                                 at + (i + 1) * lanes // 2)
-                    states[w, half, 0], states[w, half, 1] = pos[r], r
+                    states[w, mine[i], 0], states[w, mine[i], 1] = pos[r], r
                 for part in (0, 1):
                     e = np.arange(cols[p][part].size)
-                    slot, lane = part * slots + e // lanes, at + e % lanes
+                    slot = part * slots + e // lanes
+                    lane = mine.ravel()[e % lanes]
                     c[slot, lane] = pos[cols[p][part]]
                     for i, r in enumerate(pairs[p]):
                         for o in (0, 1):
