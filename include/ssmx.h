@@ -358,6 +358,10 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
  * table    double from blocks[b].table: [2 slots][4][64], entry 2 o + i of
  *          column s the coefficient of row i of the pair, order 2 o (own
  *          sector; E_0 without the identity) or 2 o + 1 (opposite sector)
+ * store    double [n_inst][n_out fine][2][16 ceil(rows / 16)] or null: every
+ *          exponential's input by row (padding not written); rows are then
+ *          below desc->rows
+ * factors  double [n_inst][n_out fine][2], their factors f (with store)
  * READ_FULL: states without a row are not written.
  */
 typedef struct ssmx_series_block {
@@ -375,7 +379,54 @@ int ssmx_propagate_series_wide(const ssmx_series_desc *desc,
                                const double *cf_nodes, const ssmx_wave *waves,
                                const ssmx_segment *segments,
                                const double *rho0, const double *obs,
-                               double *out, void *stream);
+                               double *out, double *store, double *factors,
+                               void *stream);
+
+/*
+ * Cotangents of a wide series run in reverse, for integrated readouts
+ * (READ_INTEGRAL). Tables hold the transposed matrices on the same rows,
+ * factors what the forward run left; states, obs as forward.
+ * seed        double [n_inst][n_obs], cotangents of the readouts
+ * store       receives the cotangent of every exponential's result, laid out
+ *             as the forward's
+ * lambda_out  double [n_inst][n], cotangents of rho0 (states without a row
+ *             are not written); may be null
+ */
+int ssmx_series_wide_adjoint(const ssmx_series_desc *desc,
+                             const ssmx_series_block *blocks,
+                             int32_t n_blocks, const int32_t *states,
+                             const int32_t *columns, const double *table,
+                             const double *factors, const double *obs,
+                             const double *seed, double *store,
+                             double *lambda_out, void *stream);
+
+/*
+ * dE_0 .. dE_3 of exp(A + f G) = sum f^k E_k in n_theta directions dA, to
+ * `terms` terms of the exponential's series; n at most 192.
+ * col_*, val_*  [slots][n] columns and values of A and G, [n_theta][slots][n]
+ *               of dA (padding: value 0)
+ * out           double [n_theta][4][npad][npad], npad = 16 ceil(n / 16)
+ */
+int ssmx_series_derivatives(int32_t n, int32_t n_theta, int32_t terms,
+                            int32_t slots_a, const int32_t *col_a,
+                            const double *val_a, int32_t slots_g,
+                            const int32_t *col_g, const double *val_g,
+                            int32_t slots_d, const int32_t *col_d,
+                            const double *val_d, double *out, void *stream);
+
+/*
+ * grad_theta[inst][theta] = sum over the instance's `exps` exponentials and
+ * k < 4 of f^k mu^T dE_k y.
+ * y, mu    double [n_inst][exps][npad] inputs and cotangents of the results
+ * factors  double [n_inst][exps]
+ * dtable   as ssmx_series_derivatives' out
+ * work     double [n_inst][ssmx_series_moment_groups(n)][n_theta]
+ */
+int ssmx_series_moments(int32_t n, int32_t n_inst, int32_t exps,
+                        int32_t n_theta, const double *y, const double *mu,
+                        const double *factors, const double *dtable,
+                        double *work, double *grad_theta, void *stream);
+int ssmx_series_moment_groups(int32_t n);
 
 /*
  * The reference's non-residual exponential (use_residual=False).

@@ -117,6 +117,8 @@ class Wave(ctypes.Structure):
 #: every symbol include/ssmx.h declares
 EXPORTS = ("ssmx_propagate", "ssmx_propagate_series", "ssmx_series_queue",
            "ssmx_propagate_series_wave", "ssmx_propagate_series_wide",
+           "ssmx_series_wide_adjoint", "ssmx_series_derivatives",
+           "ssmx_series_moments", "ssmx_series_moment_groups",
            "ssmx_series_adjoint",
            "ssmx_propagate_dense", "ssmx_chunk_combine",
            "ssmx_propagate_queue",
@@ -157,8 +159,19 @@ def load():
         [ctypes.POINTER(SeriesDesc)] + [vp] * 11
     lib.ssmx_propagate_series_wave.restype = ctypes.c_int
     lib.ssmx_propagate_series_wide.argtypes = \
-        [ctypes.POINTER(SeriesDesc), vp, ctypes.c_int32] + [vp] * 11
+        [ctypes.POINTER(SeriesDesc), vp, ctypes.c_int32] + [vp] * 13
     lib.ssmx_propagate_series_wide.restype = ctypes.c_int
+    lib.ssmx_series_wide_adjoint.argtypes = \
+        [ctypes.POINTER(SeriesDesc), vp, ctypes.c_int32] + [vp] * 8
+    lib.ssmx_series_wide_adjoint.restype = ctypes.c_int
+    i32 = ctypes.c_int32
+    lib.ssmx_series_derivatives.argtypes = [i32] * 3 + [i32, vp, vp] * 3 + \
+        [vp] * 2
+    lib.ssmx_series_derivatives.restype = ctypes.c_int
+    lib.ssmx_series_moments.argtypes = [i32] * 4 + [vp] * 7
+    lib.ssmx_series_moments.restype = ctypes.c_int
+    lib.ssmx_series_moment_groups.argtypes = [i32]
+    lib.ssmx_series_moment_groups.restype = ctypes.c_int
     lib.ssmx_series_adjoint.argtypes = (
         [ctypes.POINTER(SeriesDesc)] + [vp] * 3 + [ctypes.c_int32] +
         [vp] * 11)

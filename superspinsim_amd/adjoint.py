@@ -30,6 +30,7 @@ The reference has no gradients; this differentiates the path that
 """
 
 import ctypes
+import math
 
 import numpy as np
 
@@ -38,6 +39,7 @@ from superspinsim_amd.propagator import (
     _bank_slots, _ptr, _torch, device_tensor, sample_exponents,
     taylor_degrees_measured)
 from superspinsim_amd.series_gradient import SeriesGradient
+from superspinsim_amd.series_wide_gradient import WideGradient
 from superspinsim_amd.sweep import BatchSimulator, waveform_records
 
 _f64 = np.float64
@@ -357,11 +359,14 @@ class GradientProblem:
         series = None
         if self.store_inputs == "auto" and \
                 self.rho0.shape[-1] == gens.shape[1] == self.obs.shape[1]:
-            series = SeriesGradient.build(
-                sim, const, program, waves, dconst, np.atleast_2d(self.rho0),
-                self.obs, h, self.tolerance, self.adjoint_tolerance)
+            point = (sim, const, program, waves, dconst,
+                     np.atleast_2d(self.rho0), self.obs, h, self.tolerance,
+                     self.adjoint_tolerance)
+            series = SeriesGradient.build(*point)
             if series is not None and grad_gen not in (-1, series.gen):
                 series = None
+            if series is None and grad_gen < 0:
+                series = WideGradient.build(*point)
         state = GradientState(
             theta=theta, amplitudes=amplitudes, program=program,
             derivatives=bool(derivatives), series=series,
@@ -375,7 +380,9 @@ class GradientProblem:
             kernel_waves=kwaves)
         state.later = lambda: self._taylor_tables(
             sim, waves, active, const, program, dconst, derivatives, grad_gen)
-        if series is None:
+        if series is None or isinstance(series, WideGradient):
+            # (at once for a wide model: patterns beyond the Taylor adjoint's
+            # limits are refused as ever)
             state.complete()
         else:
             # the degrees the Taylor kernels would run at (a point beyond
@@ -499,7 +506,8 @@ class GradientProblem:
         if not state["derivatives"]:
             return None
         torch = _torch()
-        shape = (state["n_inst"], total, series.d_w.shape[0], 32)
+        shape = series.store_shape(state["n_inst"], total,
+                                   series.d_w.shape[0])
         have = state.get("inputs")
         if have is not None and tuple(have.shape) == shape:
             return have
@@ -508,7 +516,7 @@ class GradientProblem:
         have = None
         free, _ = torch.cuda.mem_get_info()
         free += torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
-        if series.store_bytes(shape[0], total, shape[2]) > 0.8 * free:
+        if 8 * math.prod(shape) > 0.8 * free:
             return False
         return torch.empty(shape, dtype=torch.float64, device="cuda")
 

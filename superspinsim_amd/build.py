@@ -17,7 +17,7 @@ OBJ_DIR = os.path.join(LIB_DIR, "_obj")
 SOURCES = ["ssmx_propagate.hip", "ssmx_adjoint.hip", "ssmx_queue.hip",
            "ssmx_wide.hip", "ssmx_adjoint_wide.hip", "ssmx_dense.hip",
            "ssmx_chunks.hip", "ssmx_series.hip", "ssmx_series_adjoint.hip",
-           "ssmx_series_wide.hip"]
+           "ssmx_series_wide.hip", "ssmx_series_moments.hip"]
 
 # -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (some of their forms
 # have given wrong results on MI355X without any error); the host pass warns

@@ -37,6 +37,7 @@ using ssmx::set_error;
 
 constexpr int kMaxWaves = 12;
 constexpr int kMaxRows = 256;
+enum { kRun, kStore, kBack };
 
 typedef __attribute__((address_space(3))) double lds_double;
 
@@ -53,6 +54,12 @@ struct WSParams {
     const double *rho0;
     const double *obs;
     double *out;
+    // gradients (null otherwise): every exponential's input (forward) or its
+    // result's cotangent (reverse), [instance][step][j][pad]; its factor
+    double *store;
+    double *factors;
+    const double *seed;
+    int pad;
 };
 
 // The sum of a pair's rows over its lanes: that of row a in the lanes of the
@@ -92,9 +99,42 @@ __device__ __forceinline__ void observe(const WSParams &p, const double *x,
     }
 }
 
+// What an exponential of factor f adds to the lane's row, from the components
+// at `from` in LDS.
+template <int C>
+__device__ __forceinline__ double
+exponential(const double (&ca)[C][2][2], const double (&cb)[C][2][2],
+            lds_double *const (&xa)[C], lds_double *const (&xb)[C], int from,
+            double f, bool sixteen)
+{
+    double va[C], vb[C];
+#pragma unroll
+    for (int s = 0; s < C; ++s)
+        va[s] = xa[s][from];
+#pragma unroll
+    for (int s = 0; s < C; ++s)
+        vb[s] = xb[s][from];
+    const double u = f * f;
+    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+#pragma unroll
+    for (int s = 0; s < C; ++s) {
+        a0 = fma(fma(u, ca[s][1][0], ca[s][0][0]), va[s], a0);
+        a1 = fma(fma(u, ca[s][1][1], ca[s][0][1]), va[s], a1);
+    }
+#pragma unroll
+    for (int s = 0; s < C; ++s) {
+        b0 = fma(fma(u, cb[s][1][0], cb[s][0][0]), vb[s], b0);
+        b1 = fma(fma(u, cb[s][1][1], cb[s][0][1]), vb[s], b1);
+    }
+    return sum_pair(fma(f, b0, a0), fma(f, b1, a1), sixteen);
+}
+
 // One wavefront's part of its workgroup's instance: C own-sector and C
 // opposite-sector columns per lane. FILL: this wavefront evaluates the drive.
-template <int C, bool FILL>
+// M is kRun, kStore (a run that keeps every exponential's input and factor) or
+// kBack: the cotangents of an integrated readout in reverse, with transposed
+// matrices and the factors that kStore left.
+template <int C, bool FILL, int M>
 __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
                                          double *fbuf, const double *obs,
                                          const ssmx_series_block &blk,
@@ -121,19 +161,64 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
         xa[s] = (lds_double *)xbuf + col[s * kWave];
         xb[s] = (lds_double *)xbuf + col[(C + s) * kWave];
     }
-    double x = row >= 0 ? p.rho0[(size_t)inst * d.n + state] : 0.0;
+    const double half_h = 0.5 * d.h;
+    double x = 0.0, source = 0.0;
+    if constexpr (M == kBack) {
+        if (row >= 0)
+            for (int o = 0; o < d.n_obs; ++o)
+                source = fma(p.seed[inst * d.n_obs + o],
+                             p.obs[o * d.n + state], source);
+        x = half_h * source;
+    } else if (row >= 0) {
+        x = p.rho0[(size_t)inst * d.n + state];
+    }
     if (leader)
         xbuf[row] = x;
     const bool read_full = (d.flags & SSMX_READ_FULL) != 0;
     const bool read_int = (d.flags & SSMX_READ_INTEGRAL) != 0;
+    const long total = (long)d.n_out * d.fine;
+    double *store = nullptr;
+    if (M != kRun && leader)
+        store = p.store + (size_t)inst * total * J * p.pad + row;
+    if constexpr (M == kBack) {
+        const double *factors = p.factors + (size_t)inst * total * J;
+        __syncthreads();
+        double n0 = factors[(total - 1) * J], n1 = factors[total * J - 1];
+        for (long step = total - 1; step >= 0; --step) {
+            const double fc[J] = {n0, n1};
+            const long next = step > 0 ? step - 1 : 0;
+            n0 = factors[next * J];
+            n1 = factors[next * J + 1];
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                if (leader)
+                    store[(step * J + j) * p.pad] = x;
+                x += exponential<C>(ca, cb, xa, xb, j == 0 ? 0 : kMaxRows,
+                                    fc[j], sixteen);
+                // readouts after the step before and before this one
+                if (j == J - 1)
+                    x = fma(step == 0 ? half_h : d.h, source, x);
+                if (leader)
+                    xbuf[(j == 0 ? kMaxRows : 0) + row] = x;
+                __syncthreads();
+            }
+        }
+        if (p.out && leader)
+            p.out[(size_t)inst * d.n + state] = x;
+        return;
+    }
     const Clock clk{d.t0, d.dt, d.h, d.fine, d.n_node, p.nodes, p.w};
     DriveFactors<J> drive(p.waves + inst / d.wave_group, p.segs, d.gen, 1,
                           lane);
-    const long total = (long)d.n_out * d.fine;
+    // the drive factors from output i, step k on
+    auto fill = [&](long i, int k, long step, double *f) {
+        drive.fill(clk, p.segs, i, k, total - step, lane, f);
+        if (M == kStore && step * J + lane < total * J)
+            p.factors[(inst * total + step) * J + lane] = f[lane];
+    };
     if constexpr (FILL)
-        drive.fill(clk, p.segs, 0, 0, total, lane, fbuf);
+        fill(0, 0, 0, fbuf);
     double xint = 0.0;
-    const double half_h = 0.5 * d.h;
     __syncthreads();
     int b = 0;
     long step = 0;
@@ -147,8 +232,7 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
                 fcur = fcur == fbuf ? fbuf + kWave : fbuf;
                 b = 0;
                 if constexpr (FILL)
-                    drive.fill(clk, p.segs, i, k + 1, total - step - 1, lane,
-                               fcur);
+                    fill(i, k + 1, step + 1, fcur);
             }
             const double before = x;
 #pragma unroll
@@ -158,26 +242,9 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
                 // is one barrier ahead of any that writes it
                 const int from = j == 1 ? 0 : kMaxRows;
                 const int to = j == 1 ? kMaxRows : 0;
-                double va[C], vb[C];
-#pragma unroll
-                for (int s = 0; s < C; ++s)
-                    va[s] = xa[s][from];
-#pragma unroll
-                for (int s = 0; s < C; ++s)
-                    vb[s] = xb[s][from];
-                const double f = fc[j], u = f * f;
-                double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
-#pragma unroll
-                for (int s = 0; s < C; ++s) {
-                    a0 = fma(fma(u, ca[s][1][0], ca[s][0][0]), va[s], a0);
-                    a1 = fma(fma(u, ca[s][1][1], ca[s][0][1]), va[s], a1);
-                }
-#pragma unroll
-                for (int s = 0; s < C; ++s) {
-                    b0 = fma(fma(u, cb[s][1][0], cb[s][0][0]), vb[s], b0);
-                    b1 = fma(fma(u, cb[s][1][1], cb[s][0][1]), vb[s], b1);
-                }
-                x += sum_pair(fma(f, b0, a0), fma(f, b1, a1), sixteen);
+                if (M == kStore && leader)
+                    store[(step * J + j) * p.pad] = x;
+                x += exponential<C>(ca, cb, xa, xb, from, fc[j], sixteen);
                 if (leader)
                     xbuf[to + row] = x;
                 __syncthreads();
@@ -204,19 +271,22 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
     }
 }
 
-template <int C>
+template <int C, int M>
 __device__ __forceinline__ void run_class(const WSParams &p, double *xbuf,
                                           double *fbuf, const double *obs,
                                           const ssmx_series_block &blk,
                                           int wave, int lane, long inst,
                                           bool fill)
 {
-    if (fill)
-        run_wave<C, true>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+    if constexpr (M == kBack)
+        run_wave<C, false, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+    else if (fill)
+        run_wave<C, true, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
     else
-        run_wave<C, false>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+        run_wave<C, false, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
 }
 
+template <int M>
 __global__ __launch_bounds__(kWave *kMaxWaves)
 __attribute__((amdgpu_waves_per_eu(3))) void series_wide_kernel(WSParams p)
 {
@@ -235,39 +305,28 @@ __attribute__((amdgpu_waves_per_eu(3))) void series_wide_kernel(WSParams p)
         obs[k] = 0.0;
     __syncthreads();
     const int row = p.states[2 * (wave * kWave + lane)];
-    if (row >= 0)
+    if (M != kBack && row >= 0)
         for (int o = 0; o < p.d.n_obs; ++o)
             obs[o * kMaxRows + row] =
                 p.obs[o * p.d.n + p.states[2 * (wave * kWave + lane) + 1]];
     // every wavefront meets the same barriers whatever its class
     switch (blk.slots) {
     case 4:
-        run_class<4>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<4, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
         break;
     case 5:
-        run_class<5>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<5, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
         break;
     case 6:
-        run_class<6>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<6, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
         break;
     default:
-        run_class<7>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<7, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
     }
 }
 
-}  // namespace
-
-extern "C" int ssmx_propagate_series_wide(
-    const ssmx_series_desc *desc, const ssmx_series_block *blocks,
-    int32_t n_blocks, const int32_t *states, const int32_t *columns,
-    const double *table, const double *cf_weights, const double *cf_nodes,
-    const ssmx_wave *waves, const ssmx_segment *segments, const double *rho0,
-    const double *obs, double *out, void *stream)
+int check(const ssmx_series_desc &d, int32_t n_blocks, const char *what)
 {
-    ssmx::error_buffer()[0] = '\0';
-    if (!desc)
-        return set_error(SSMX_EINVAL, "null descriptor");
-    const ssmx_series_desc &d = *desc;
     const bool full = (d.flags & SSMX_READ_FULL) != 0;
     if (d.n < 1 || d.n > SSMX_MAX_N_WIDE || d.rows < 1 ||
         d.rows > kMaxRows || d.n_inst < 1 || d.n_exp != 2 ||
@@ -277,19 +336,52 @@ extern "C" int ssmx_propagate_series_wide(
         (d.flags & ~(SSMX_READ_FULL | SSMX_READ_INTEGRAL)) != 0 ||
         (full && (d.flags & SSMX_READ_INTEGRAL)) ||
         (!full && (d.n_obs < 1 || d.n_obs > SSMX_MAX_OBS)))
-        return set_error(SSMX_EINVAL, "wide series: n=%d, rows=%d, "
-                         "n_inst=%d, n_exp=%d, da=%d, db=%d, fine=%d, "
-                         "n_out=%d, n_obs=%d, flags=%d", d.n, d.rows, d.n_inst,
+        return set_error(SSMX_EINVAL, "%s: n=%d, rows=%d, n_inst=%d, "
+                         "n_exp=%d, da=%d, db=%d, fine=%d, n_out=%d, "
+                         "n_obs=%d, flags=%d", what, d.n, d.rows, d.n_inst,
                          d.n_exp, d.da, d.db, d.fine, d.n_out, d.n_obs,
                          d.flags);
     if (n_blocks < 1 || n_blocks > kMaxWaves)
         return set_error(SSMX_EINVAL, "%d wavefronts outside 1..%d",
                          n_blocks, kMaxWaves);
+    return SSMX_OK;
+}
+
+template <int M>
+int launch(const WSParams &p, int n_blocks, void *stream, const char *what)
+{
+    hipLaunchKernelGGL(series_wide_kernel<M>, dim3(p.d.n_inst),
+                       dim3(kWave * n_blocks), 0,
+                       static_cast<hipStream_t>(stream), p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return set_error(SSMX_ELAUNCH, "%s launch: %s", what,
+                         hipGetErrorString(e));
+    return SSMX_OK;
+}
+
+}  // namespace
+
+extern "C" int ssmx_propagate_series_wide(
+    const ssmx_series_desc *desc, const ssmx_series_block *blocks,
+    int32_t n_blocks, const int32_t *states, const int32_t *columns,
+    const double *table, const double *cf_weights, const double *cf_nodes,
+    const ssmx_wave *waves, const ssmx_segment *segments, const double *rho0,
+    const double *obs, double *out, double *store, double *factors,
+    void *stream)
+{
+    ssmx::error_buffer()[0] = '\0';
+    if (!desc)
+        return set_error(SSMX_EINVAL, "null descriptor");
+    const int rc = check(*desc, n_blocks, "wide series");
+    if (rc != SSMX_OK)
+        return rc;
     if (!blocks || !states || !columns || !table || !cf_weights ||
-        !cf_nodes || !waves || !segments || !rho0 || !out || (!full && !obs))
+        !cf_nodes || !waves || !segments || !rho0 || !out ||
+        (!(desc->flags & SSMX_READ_FULL) && !obs) || !store != !factors)
         return set_error(SSMX_EINVAL, "null required pointer");
-    WSParams p;
-    p.d = d;
+    WSParams p{};
+    p.d = *desc;
     p.blocks = blocks;
     p.states = states;
     p.columns = columns;
@@ -301,12 +393,42 @@ extern "C" int ssmx_propagate_series_wide(
     p.rho0 = rho0;
     p.obs = obs;
     p.out = out;
-    hipLaunchKernelGGL(series_wide_kernel, dim3(d.n_inst),
-                       dim3(kWave * n_blocks), 0,
-                       static_cast<hipStream_t>(stream), p);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
-        return set_error(SSMX_ELAUNCH, "wide series launch: %s",
-                         hipGetErrorString(e));
-    return SSMX_OK;
+    p.store = store;
+    p.factors = factors;
+    p.pad = (desc->rows + 15) / 16 * 16;
+    return store ? launch<kStore>(p, n_blocks, stream, "wide series")
+                 : launch<kRun>(p, n_blocks, stream, "wide series");
+}
+
+extern "C" int ssmx_series_wide_adjoint(
+    const ssmx_series_desc *desc, const ssmx_series_block *blocks,
+    int32_t n_blocks, const int32_t *states, const int32_t *columns,
+    const double *table, const double *factors, const double *obs,
+    const double *seed, double *store, double *lambda_out, void *stream)
+{
+    ssmx::error_buffer()[0] = '\0';
+    if (!desc)
+        return set_error(SSMX_EINVAL, "null descriptor");
+    const int rc = check(*desc, n_blocks, "wide series adjoint");
+    if (rc != SSMX_OK)
+        return rc;
+    if (desc->n_out < 1 || desc->n_obs < 1)
+        return set_error(SSMX_EINVAL, "wide series adjoint: n_out=%d, "
+                         "n_obs=%d", desc->n_out, desc->n_obs);
+    if (!blocks || !states || !columns || !table || !factors || !obs ||
+        !seed || !store)
+        return set_error(SSMX_EINVAL, "null required pointer");
+    WSParams p{};
+    p.d = *desc;
+    p.blocks = blocks;
+    p.states = states;
+    p.columns = columns;
+    p.table = table;
+    p.factors = const_cast<double *>(factors);
+    p.obs = obs;
+    p.seed = seed;
+    p.out = lambda_out;
+    p.store = store;
+    p.pad = (desc->rows + 15) / 16 * 16;
+    return launch<kBack>(p, n_blocks, stream, "wide series adjoint");
 }

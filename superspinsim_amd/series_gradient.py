@@ -120,8 +120,9 @@ class SeriesGradient:
                     kept[k] -= (c / F ** k) * cheb[j]
         return kept
 
-    def store_bytes(self, n_inst, steps, J):
-        return n_inst * steps * J * 32 * 8
+    def store_shape(self, n_inst, steps, J):
+        """Inputs of every exponential."""
+        return n_inst, steps, J, 32
 
     def _desc(self, problem, n_inst, n, J, S):
         m = self.model

@@ -118,6 +118,10 @@ class WideModel:
         self = cls()
         self.n, self.h = n, h
         self.sector = found[0]
+        # LDS rows by sector: the lanes of a pair then read runs of
+        # neighbours, and pairs with common columns the same ones
+        self.pos = np.empty(n, dtype=np.int32)
+        self.pos[np.argsort(self.sector, kind="stable")] = np.arange(n)
         self.size = int(np.bincount(self.sector).max())
         self.weight = float(np.abs(weights).sum(axis=1).max())
         self.nnz = int(np.count_nonzero((const != 0) | (drive != 0)))
@@ -148,7 +152,11 @@ class WideModel:
                             tuple(device_tensor(a) for a in arrays))
         return self._layout[1]
 
-    def _arrays(self, F, budget):
+    def transposed(self, plan):
+        """``layout`` of the transposed matrices, on the host."""
+        return self._arrays(*plan[2:], transpose=True)
+
+    def _arrays(self, F, budget, transpose=False):
         kept = [m.copy() for m in self.mats[:4]]
         # the dropped order's Chebyshev polynomial taken off
         # (T_4 = 8 u^4 - 8 u^2 + 1: its lower coefficients stay with E_0, E_2)
@@ -156,6 +164,8 @@ class WideModel:
         if F ** 2 > 0.0:
             kept[0] -= top
             kept[2] += (8.0 / F ** 2) * top
+        if transpose:
+            kept = [np.ascontiguousarray(m.T) for m in kept]
         size = sum(F ** k * np.abs(m) for k, m in enumerate(kept))
         order = np.argsort(size, axis=0, kind="stable")
         keep = np.empty(size.shape, dtype=bool)
@@ -173,10 +183,7 @@ class WideModel:
         waves = self._waves(widest[rank])
         if waves is None:
             return None
-        # LDS positions by sector: the lanes of a pair then read runs of
-        # neighbours, and pairs with common columns the same ones
-        pos = np.empty(self.n, dtype=np.int32)
-        pos[np.argsort(self.sector, kind="stable")] = np.arange(self.n)
+        pos = self.pos
         blocks = np.zeros((len(waves), 4), dtype=np.int32)
         states = np.zeros((len(waves), 64, 2), dtype=np.int32)
         states[:, :, 0] = -1
@@ -278,7 +285,7 @@ class WideRun:
             self.blocks.shape[0], _ptr(self.states), _ptr(self.columns),
             _ptr(self.table), _ptr(self.d_w), _ptr(self.d_nodes),
             _ptr(self.d_waves), _ptr(self.d_segs), _ptr(self.d_rho0),
-            _ptr(self.d_obs), _ptr(self.out), ctypes.c_void_p(
+            _ptr(self.d_obs), _ptr(self.out), None, None, ctypes.c_void_p(
                 _torch().cuda.current_stream().cuda_stream)))
         return self.out
 
