@@ -401,32 +401,37 @@ int ssmx_series_wide_adjoint(const ssmx_series_desc *desc,
                              double *lambda_out, void *stream);
 
 /*
- * dE_0 .. dE_3 of exp(A + f G) = sum f^k E_k in n_theta directions dA, to
- * `terms` terms of the exponential's series; n at most 192.
+ * dE_k, k < orders (3 or 4), of exp(A + f G) = sum f^k E_k in n_theta
+ * directions dA, to `terms` terms of the exponential's series; n at most 192.
+ * With three orders the fourth is economised: for |f| <= drive_max it is
+ * taken as the linear term that leaves a quarter of it.
  * col_*, val_*  [slots][n] columns and values of A and G, [n_theta][slots][n]
  *               of dA (padding: value 0)
- * out           double [n_theta][4][npad][npad], npad = 16 ceil(n / 16)
+ * out           double [n_theta][orders][npad][npad], npad = 16 ceil(n/16)
  */
 int ssmx_series_derivatives(int32_t n, int32_t n_theta, int32_t terms,
-                            int32_t slots_a, const int32_t *col_a,
-                            const double *val_a, int32_t slots_g,
+                            int32_t orders, double drive_max, int32_t slots_a,
+                            const int32_t *col_a, const double *val_a,
+                            int32_t slots_g,
                             const int32_t *col_g, const double *val_g,
                             int32_t slots_d, const int32_t *col_d,
                             const double *val_d, double *out, void *stream);
 
 /*
  * grad_theta[inst][theta] = sum over the instance's `exps` exponentials and
- * k < 4 of f^k mu^T dE_k y.
+ * k < orders (3 or 4) of f^k mu^T dE_k y.
  * y, mu    double [n_inst][exps][npad] inputs and cotangents of the results
  * factors  double [n_inst][exps]
  * dtable   as ssmx_series_derivatives' out
- * work     double [n_inst][ssmx_series_moment_groups(n)][n_theta]
+ * work     double [n_inst][ssmx_series_moment_groups(n, orders)]
+ *          [n_theta]
  */
 int ssmx_series_moments(int32_t n, int32_t n_inst, int32_t exps,
-                        int32_t n_theta, const double *y, const double *mu,
-                        const double *factors, const double *dtable,
-                        double *work, double *grad_theta, void *stream);
-int ssmx_series_moment_groups(int32_t n);
+                        int32_t orders, int32_t n_theta, const double *y,
+                        const double *mu, const double *factors,
+                        const double *dtable, double *work,
+                        double *grad_theta, void *stream);
+int ssmx_series_moment_groups(int32_t n, int32_t orders);
 
 /*
  * The reference's non-residual exponential (use_residual=False).

@@ -165,12 +165,12 @@ def load():
         [ctypes.POINTER(SeriesDesc), vp, ctypes.c_int32] + [vp] * 8
     lib.ssmx_series_wide_adjoint.restype = ctypes.c_int
     i32 = ctypes.c_int32
-    lib.ssmx_series_derivatives.argtypes = [i32] * 3 + [i32, vp, vp] * 3 + \
-        [vp] * 2
+    lib.ssmx_series_derivatives.argtypes = [i32] * 4 + [ctypes.c_double] + \
+        [i32, vp, vp] * 3 + [vp] * 2
     lib.ssmx_series_derivatives.restype = ctypes.c_int
-    lib.ssmx_series_moments.argtypes = [i32] * 4 + [vp] * 7
+    lib.ssmx_series_moments.argtypes = [i32] * 5 + [vp] * 7
     lib.ssmx_series_moments.restype = ctypes.c_int
-    lib.ssmx_series_moment_groups.argtypes = [i32]
+    lib.ssmx_series_moment_groups.argtypes = [i32] * 2
     lib.ssmx_series_moment_groups.restype = ctypes.c_int
     lib.ssmx_series_adjoint.argtypes = (
         [ctypes.POINTER(SeriesDesc)] + [vp] * 3 + [ctypes.c_int32] +

@@ -25,6 +25,11 @@
 // conflict a gather instead of 1.8) and pairs on consecutive lanes (selects
 // and a DPP step where the half swap is). Coefficients evaluated ahead of the
 // gathers gained 1% and spilled.
+//
+// Gradients store the inputs of all exponentials forward and the cotangents of
+// their results in reverse (kStore, kBack); ssmx_series_moments.hip contracts
+// the two. 128 points x 5,000 steps, 12 parameters: 5.9 + 5.9 + 4.9 ms; Taylor
+// forward 22 and Frechet adjoint 77.
 #include "ssmx_series_dev.h"
 
 namespace {

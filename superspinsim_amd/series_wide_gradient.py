@@ -18,10 +18,8 @@ from superspinsim_amd.series_wide import WideModel
 
 _f64 = np.float64
 
-#: rows of the moment kernel; moments of orders 0..3 are kept
+#: rows of the moment kernel
 MAX_ROWS = 192
-#: instances of one launch (a grid dimension)
-MAX_INST = 65535
 
 
 def row_lists(mats):
@@ -49,7 +47,7 @@ class WideGradient:
         """Arguments as ``SeriesGradient.build``."""
         varying = [g for g in program if g is not None]
         if len(varying) != 1 or None not in program or sim.rotating or \
-                len(waves) > MAX_INST or sim.n <= _lib.MAX_N:
+                sim.n <= _lib.MAX_N:
             return None
         folded, drive = sim.folded(const), sim.gens[varying[0]]
         pattern = (folded != 0) | (drive != 0)
@@ -70,12 +68,20 @@ class WideGradient:
         scale = h * float(sim.weights[0].sum())
         norm = scale * float(np.abs(c).sum(axis=0).max())
         # order k of a derivative is at most F^k |G|^k / k! e^norm |dA|, the
-        # whole at least about e^-norm |dA|
+        # whole at least about e^-norm |dA|; four orders are kept, or three
+        # where the quarter of the fourth that Chebyshev polynomials leave is
+        # below the tolerance (a quarter less of the moments' work)
         b = plan[2] * float(np.abs(g).sum(axis=0).max())
-        if not b ** 4 / 24.0 * math.exp(b + 2.0 * norm) <= adjoint_tol:
+        spread = math.exp(b + 2.0 * norm)
+        if b ** 3 / 24.0 * spread <= adjoint_tol:
+            orders = 3
+        elif b ** 4 / 24.0 * spread <= adjoint_tol:
+            orders = 4
+        else:
             return None
         self = cls()
         self.model, self.plan, self.states = model, plan, states
+        self.orders = orders
         self.gen = program.index(varying[0])
         self.npad = -(-model.n // 16) * 16
         self.d_w, self.d_nodes = (device_tensor(sim.weights),
@@ -96,7 +102,7 @@ class WideGradient:
                 size *= norm / (terms - 4)
             self.dtable = self._derivatives(
                 scale * c[rows], g[rows],
-                scale * dc[:, rows[0], rows[1]], terms)
+                scale * dc[:, rows[0], rows[1]], terms, plan[2])
         return self
 
     @staticmethod
@@ -116,8 +122,8 @@ class WideGradient:
                 tuple(device_tensor(a) for a in arrays), self.index)
         return self.back
 
-    def _derivatives(self, a, g, da, terms):
-        """d E_0 .. d E_3 in every direction, by row position."""
+    def _derivatives(self, a, g, da, terms, drive_max):
+        """d E_k in every direction, by row position."""
         torch = _torch()
         n = a.shape[0]
         lists = []
@@ -125,12 +131,12 @@ class WideGradient:
             col, val = row_lists(mats)
             lists.append((col.shape[1], device_tensor(col),
                           device_tensor(val)))
-        out = torch.empty((da.shape[0], 4, self.npad, self.npad),
+        out = torch.empty((da.shape[0], self.orders, self.npad, self.npad),
                           dtype=torch.float64, device="cuda")
         args = [v for s, col, val in lists
                 for v in (ctypes.c_int32(s), _ptr(col), _ptr(val))]
         _lib.check(_lib.load().ssmx_series_derivatives(
-            n, da.shape[0], terms, *args, _ptr(out),
+            n, da.shape[0], terms, self.orders, drive_max, *args, _ptr(out),
             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
         return out
 
@@ -194,12 +200,12 @@ class WideGradient:
         work = None
         if g_theta is not None and self.n_theta:
             work = torch.empty(
-                (n_inst, lib.ssmx_series_moment_groups(self.model.n),
-                 self.n_theta), dtype=torch.float64, device="cuda")
+                (n_inst, lib.ssmx_series_moment_groups(
+                    self.model.n, self.orders), self.n_theta), dtype=torch.float64, device="cuda")
             _lib.check(lib.ssmx_series_moments(
-                self.model.n, n_inst, exps, self.n_theta, _ptr(store[0]),
-                _ptr(store[1]), _ptr(factors), _ptr(self.dtable),
-                _ptr(work), _ptr(g_theta), stream))
+                self.model.n, n_inst, exps, self.orders, self.n_theta,
+                _ptr(store[0]), _ptr(store[1]), _ptr(factors),
+                _ptr(self.dtable), _ptr(work), _ptr(g_theta), stream))
         self._keep_back = (d_obs, seed, work)
 
 

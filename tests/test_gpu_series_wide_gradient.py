@@ -17,10 +17,10 @@ from superspinsim_amd.sweep import Waveform
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,points,exps,thetas", [
-    (65, 1, 2, 1), (80, 3, 6, 2), (81, 2, 40, 3), (171, 2, 101, 12),
-    (192, 1, 4, 1)])
-def test_moments_equal_numpy(gpu, n, points, exps, thetas):
+@pytest.mark.parametrize("n,points,exps,thetas,orders", [
+    (65, 1, 2, 1, 4), (80, 9, 6, 2, 3), (81, 2, 40, 3, 4),
+    (171, 2, 101, 12, 3), (171, 11, 10, 1, 4), (192, 1, 4, 1, 3)])
+def test_moments_equal_numpy(gpu, n, points, exps, thetas, orders):
     """Sums of exps n^2 products in another order: exps n^2 / 2^53 of the sum
     of magnitudes at the very most, a thousandth of that in practice; the
     bar is 1e-13 of that sum.  The padding holds NaN."""
@@ -31,18 +31,19 @@ def test_moments_equal_numpy(gpu, n, points, exps, thetas):
     y[..., :n] = rng.standard_normal((points, exps, n))
     mu[..., :n] = rng.standard_normal((points, exps, n))
     f = rng.uniform(-1, 1, (points, exps))
-    table = np.zeros((thetas, 4, npad, npad))
-    table[:, :, :n, :n] = rng.standard_normal((thetas, 4, n, n))
+    table = np.zeros((thetas, orders, npad, npad))
+    table[:, :, :n, :n] = rng.standard_normal((thetas, orders, n, n))
     lib = _lib.load()
-    work = torch.empty((points, lib.ssmx_series_moment_groups(n), thetas),
+    work = torch.empty((points, lib.ssmx_series_moment_groups(n, orders),
+                        thetas),
                        dtype=torch.float64, device="cuda")
     got = torch.empty((points, thetas), dtype=torch.float64, device="cuda")
     d = [device_tensor(a) for a in (y, mu, f, table)]
     _lib.check(lib.ssmx_series_moments(
-        n, points, exps, thetas, *[_ptr(a) for a in d], _ptr(work),
+        n, points, exps, orders, thetas, *[_ptr(a) for a in d], _ptr(work),
         _ptr(got), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
     want, size = 0.0, 0.0
-    for k in range(4):
+    for k in range(orders):
         m = np.einsum("pe,per,pec->prc", f ** k, mu[..., :n], y[..., :n])
         t = table[:, k, :n, :n]
         want = want + np.einsum("prc,trc->pt", m, t)
@@ -52,10 +53,11 @@ def test_moments_equal_numpy(gpu, n, points, exps, thetas):
     assert np.all(err <= 1e-13)
 
 
-@pytest.mark.parametrize("n,thetas", [(65, 1), (171, 3)])
-def test_derivatives_equal_numpy(gpu, n, thetas):
+@pytest.mark.parametrize("n,thetas,orders", [(65, 1, 4), (171, 3, 4),
+                                             (80, 2, 3)])
+def test_derivatives_equal_numpy(gpu, n, thetas, orders):
     """The same recurrence in another order of summation: 1e-14 of each
-    order's largest element."""
+    order's largest element.  f^3 is F^3 / 4 T_3(f / F) + 3 / 4 F^2 f."""
     rng = np.random.default_rng(n)
     far = np.abs(np.arange(n)[:, None] - np.arange(n)[None])
     a = rng.standard_normal((n, n)) * (far <= 3) * 0.05
@@ -63,10 +65,13 @@ def test_derivatives_equal_numpy(gpu, n, thetas):
     da = rng.standard_normal((thetas, n, n)) * (far % 7 == 0)
     self = WideGradient()
     self.npad = -(-n // 16) * 16
-    got = self._derivatives(a, g, da, 30).cpu().numpy()
+    self.orders = orders
+    got = self._derivatives(a, g, da, 30, 0.25).cpu().numpy()
     assert np.all(got[:, :, n:] == 0) and np.all(got[:, :, :, n:] == 0)
     want = derivative_matrices(a, g, da, 3)
-    for k in range(4):
+    if orders == 3:
+        want[1] += 0.75 * 0.25 ** 2 * want[3]
+    for k in range(orders):
         err = np.max(np.abs(got[:, k, :n, :n] - want[k]))
         assert err <= 1e-14 * np.max(np.abs(want[k])), k
 
