@@ -12,18 +12,18 @@ per-instance inputs uploaded from pinned host memory before each launch.
 
 The gradient leg runs the 1024-point version of the sweep with a
 200-segment microwave amplitude: a forward that keeps every exponential's
-input in HBM (105 GB), then the adjoint (forward terms from the stored
-inputs + reverse sweep) for the squared error against targets simulated at
+input in HBM, then the reverse run of the cotangents and the parameter
+moments, for the squared error against targets simulated at
 parameters perturbed by up to 2 %; the ratio is (forward with stored inputs
 + backward) / plain forward, wall time.
 
 The protocol leg runs 16384 pulsed Ramsey / Hahn-echo protocols of 58k-742k
-steps in one persistent work-queue launch (autotuned shape, replayed from a
-HIP graph) and reports propagator steps/s over the whole batch.
+steps in one persistent work-queue launch (driven stretches step by step,
+waits by powers of their exponential; replayed from a HIP graph) and reports propagator steps/s over the whole batch.
 
 The hyperfine leg runs the 21-level NV + 14N sweep (512 points, 250,000
 steps each, fluorescence every 2 ns) at n = 441 and at n = 171 through the
-wide propagator (several wavefronts per instance), with a bounded CPU sample
+wide series kernel (several wavefronts per instance), with a bounded CPU sample
 of the reference algorithm at n = 441.  The hyperfine gradient leg runs the
 n = 441 sweep forward with checkpoints and then the adjoint, for gradients
 of the integrated fluorescence over 12 parameters (the 7-level set and the
@@ -222,11 +222,10 @@ def adjoint_leg(args):
         "checkpoint_every": pb.K,
         "taylor_degree": int(state["taylor"]),
         "adjoint_degree": int(state["taylor_adj"]),
-        "ell_slots": int(state["prop"].ell.slots),
-        "ell_slots_adjoint": int(state["slots_t"]),
+        "series": bool(st["by_series"]),
         "setup_s": setup_s,
         "stored_inputs": bool(st.get("stored")),
-        "stored_input_bytes": pb.stored_input_bytes(state["n_inst"])
+        "stored_input_bytes": st["inputs"].numel() * 8
         if st.get("stored") else 0,
         "forward_s": med["forward"],
         "forward_ckpt_s": med["forward_ckpt"],
@@ -269,7 +268,6 @@ def protocol_leg(args):
     wall = (time.perf_counter() - t0) / args.protocol_steps
     kernel_s = ev[0].elapsed_time(ev[1]) / 1e3 / args.protocol_steps
     out = batch.out.cpu().numpy()
-    flops = batch.step_flops() * total
     return {
         "workload": wl.name,
         "protocols": batch.n_inst,
@@ -285,18 +283,15 @@ def protocol_leg(args):
         "s_per_batch": wall,
         "kernel_s": kernel_s,
         "steps_per_s": total / wall,
-        "achieved_tflops": flops / kernel_s / 1e12,
         "finite": bool(np.all(np.isfinite(out))),
     }
 
 
 def hyperfine_leg(args):
-    """21-level NV + 14N sweep (n = 441 and 171) through the wide kernel."""
+    """21-level NV + 14N sweep (n = 441 and 171) through the wide series."""
     import numpy as np
     import torch
     from superspinsim_amd import configs
-    from superspinsim_amd.propagator import device_tensor
-    from superspinsim_amd.sweep import pack_waveforms
     legs = {}
     for inc in (False, True):
         wl = configs.odmr21(args.hyperfine_instances, use_incoherent=inc)
@@ -306,26 +301,15 @@ def hyperfine_leg(args):
         sim = wl.simulator()
         waves = wl.waveforms()
         n_inst = len(waves)
-        # plan and device tables from a one-interval run (untimed)
-        sim.run(waves, wl.rho0, 0.0, wl.time_step * (1 + 1e-12),
-                wl.time_step, obs=wl.obs, read="obs")
+        # staged on the device (untimed)
+        run = sim.prepare(waves, wl.rho0, 0.0,
+                          wl.n_out * wl.time_step * (1 + 1e-12),
+                          wl.time_step, obs=wl.obs, read="obs")
         plan = dict(sim.last_plan)
-        prop, program, m, sub = sim.plan(waves, wl.time_step)
-        d_waves, d_segs = pack_waveforms(sim.kernel_waves(waves, program),
-                                         len(program))
-        d_rho = device_tensor(np.repeat(wl.rho0[None], n_inst, axis=0))
-        out = torch.empty((n_inst, wl.n_out, 1), dtype=torch.float64,
-                          device="cuda")
-
-        def launch():
-            prop.run(n_inst=n_inst, fine=wl.fine, n_out=wl.n_out,
-                     h=wl.time_step / wl.fine, t0=0.0, dt=wl.time_step,
-                     rho0=d_rho, waves=d_waves, segments=d_segs, taylor=m,
-                     substeps=sub, read="obs", obs=wl.obs, out=out)
-
+        out, launch = run.result(), run.launch
         steps = wl.n_out * wl.fine
         print(f"hyperfine workload {wl.name}: {n_inst} x {steps} steps, "
-              f"n={wl.n}, m={m}, s={sub}, slots={plan['slots']}",
+              f"n={wl.n}, {plan['involved']} involved",
               file=sys.stderr, flush=True)
         launch()                                    # warm
         torch.cuda.synchronize()
@@ -338,7 +322,6 @@ def hyperfine_leg(args):
         torch.cuda.synchronize()
         wall = time.perf_counter() - t0
         kernel_s = ev[0].elapsed_time(ev[1]) / 1e3
-        plan["steps"] = steps
         flops = sim.step_flops(plan) * n_inst * steps
         fl = out[:, :, 0].cpu().numpy()
         print(f"  {wall:.3f} s, {n_inst * steps / wall:.3e} steps/s",
@@ -347,9 +330,8 @@ def hyperfine_leg(args):
             "instances": n_inst,
             "superoperator_n": wl.n,
             "steps_per_instance": steps,
-            "taylor_degree": m,
-            "substeps": sub,
-            "ell_slots": plan["slots"],
+            "involved_states": plan["involved"],
+            "series_orders": list(plan["series"]),
             "nnz": plan["nnz"],
             "s_per_sweep": wall,
             "kernel_s": kernel_s,
@@ -417,15 +399,16 @@ def secondary_leg(name):
         extra = {"time_chunks": plan["chunks"],
                  "outputs_per_chunk": plan["chunk_out"],
                  "basis_vectors_per_wavefront": plan["chunk_pack"],
-                 "launch": "chunk propagators (ssmx_propagate, n basis "
-                           "vectors per chunk) + ssmx_chunk_combine",
+                 "launch": "chunk propagators (ssmx_propagate_series, n "
+                           "basis vectors per chunk) + ssmx_chunk_combine",
                  "executed_member_steps": executed,
                  "executed_tflops":
                      sim.step_flops(plan) * executed / seconds / 1e12}
     return {"workload": wl.name, "instances": n_inst,
             "superoperator_n": wl.n,
             "steps_per_instance": wl.steps_per_instance(),
-            "taylor_degree": plan["taylor"], "ell_slots": plan["slots"],
+            "involved_states": plan["involved"],
+            "series_orders": list(plan["series"]),
             "instances_per_wavefront": plan["packed"], **extra,
             "s_per_sweep": wall, "steps_per_s": steps / wall,
             "achieved_tflops": flops / 1e12,
@@ -480,6 +463,7 @@ def hyperfine_adjoint_leg(args):
         "slots_matrix_transposed_extended": [int(state["slots_f"]),
                                              int(state["slots_t"]),
                                              int(state["slots"])],
+        "series": bool(st["by_series"]),
         "setup_s": setup_s,
         "forward_s": fwd,
         "forward_ckpt_s": fwd_ckpt,
@@ -498,7 +482,6 @@ def main():
         sys.exit(2)
     import numpy as np
     import torch
-    from superspinsim_amd.propagator import device_tensor  # noqa: F401
 
     if args.copy_calibration:
         nbytes = 1 << 30
@@ -538,28 +521,17 @@ def main():
         return sim.run(waves, wl.rho0, wl.time_start, wl.time_end,
                        wl.time_step, obs=wl.obs, read="obs")
 
-    # warmup (also builds device tables and the Taylor plan)
+    # warmup (also builds device tables and the plan)
     for _ in range(max(args.warmup, 1)):
         out = one_sweep()
     torch.cuda.synchronize()
     plan = dict(sim.last_plan)
 
-    # Pre-pack so the timed region is launch + kernel only.
-    prop, program, m, s = sim.plan(waves, wl.time_step)
-    from superspinsim_amd.sweep import pack_waveforms
-    d_waves, d_segs = pack_waveforms(sim.kernel_waves(waves, program),
-                                     len(program))
-    from superspinsim_amd.propagator import device_tensor as dt_
-    d_rho = dt_(np.repeat(wl.rho0[None], n_inst, axis=0))
-    out = torch.empty((n_inst, wl.n_out, 1), dtype=torch.float64,
-                      device="cuda")
-
-    def launch():
-        prop.run(n_inst=n_inst, fine=wl.fine, n_out=wl.n_out,
-                 h=wl.time_step / wl.fine, t0=wl.time_start,
-                 dt=wl.time_step, rho0=d_rho, waves=d_waves,
-                 segments=d_segs, taylor=m, substeps=s, read="obs",
-                 obs=wl.obs, out=out)
+    # staged on the device, so the timed region is launch + kernel only
+    run = sim.prepare(waves, wl.rho0, wl.time_start, wl.time_end,
+                      wl.time_step, obs=wl.obs, read="obs")
+    out = run.result()
+    launch = run.launch
 
     # the fluorescence readout comes back to pinned host memory every step
     host_out = torch.empty(out.shape, dtype=out.dtype, pin_memory=True)
@@ -586,7 +558,7 @@ def main():
     # per-instance inputs (waveform records, segments, initial states) are
     # uploaded from pinned host memory before each launch
     staged = [(t, torch.empty(t.shape, dtype=t.dtype, pin_memory=True))
-              for t in (d_waves, d_segs, d_rho)]
+              for t in (run.d_waves, run.d_segs, run.d_rho0)]
     for dev, host in staged:
         host.copy_(dev)
     torch.cuda.synchronize()
@@ -631,27 +603,25 @@ def main():
             "h_s": wl.time_step / wl.fine,
             "scheme": "CF4:2",
             "readout": "fluorescence every output interval",
-            "taylor_degree": plan["taylor"],
-            "substeps": plan["substeps"],
-            "ell_slots": plan["slots"],
+            "involved_states": plan["involved"],
+            "series_orders": list(plan["series"]),
             "nnz": plan["nnz"],
-            "parallelism": "one instance per wavefront",
+            "parallelism": f"{plan['packed']} instances per wavefront",
         },
         "value_pcie_inclusive": n_inst * wl.steps_per_instance()
         * args.steps / wall_pcie,
         "roofline": {
             "bound": "valu",
-            "bound_detail": "FP64 VALU and LDS instruction issue of the "
-                            "sparse Taylor action (no MFMA); priced against "
-                            "the FP64 vector peak, equal to the FP64 matrix "
-                            "peak on MI355X",
+            "bound_detail": "FP64 VALU issue of the series in the drive "
+                            "(no MFMA: its FP64 rate is the vector's); "
+                            "priced against the FP64 vector peak",
             "achieved": achieved,
             "peak": PEAK_FP64_TFLOPS,
             "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP64_TFLOPS,
             "traffic": MEASURED_TRAFFIC.get(
                 (wl.name, n_inst, wl.steps_per_instance())),
-            "kernel": "propagate_kernel",
+            "kernel": "series_row_kernel",
             "kernel_ms": avg_kernel_s * 1e3,
             "flops_per_step": flops_step,
         },

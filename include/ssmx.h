@@ -342,11 +342,14 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
 /*
  * ssmx_propagate_series for models of more rows than a wavefront (at most
  * 256), one workgroup of n_blocks (at most 12) wavefronts per instance;
- * n_exp = n_node = 2, da = db = 1; members, na, nb, sector fields unused.
+ * n_exp = n_node = 2, (da, db) = (1, 1), (2, 1) or (2, 2); na the sum over the
+ * wavefronts of (da + db - 2) slots + 4 max(0, slots - 7), the KB of LDS for
+ * the coefficients that registers don't hold (at most 150); members, nb,
+ * sector fields unused.
  *
  * Rows are taken in pairs of one sector. The columns of pair g of wavefront b
  * are spread over its `lanes` (8 or 16) lanes 32 v + g lanes / 2 + (0 ..
- * lanes / 2 - 1), v = 0, 1; every lane holds blocks[b].slots (4..7) columns of
+ * lanes / 2 - 1), v = 0, 1; every lane holds blocks[b].slots (4..8) columns of
  * the pair's own sector and as many of the opposite one (padded with
  * coefficient 0). Lanes below 32 keep the pair's first row, the others the
  * second.
@@ -355,9 +358,14 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
  *          state index (idle lanes 0)
  * columns  int32 from blocks[b].columns: [2 slots][64] rows (0..255) of the
  *          own-sector columns, then of the opposite ones
- * table    double from blocks[b].table: [2 slots][4][64], entry 2 o + i of
- *          column s the coefficient of row i of the pair, order 2 o (own
- *          sector; E_0 without the identity) or 2 o + 1 (opposite sector)
+ * table    double from blocks[b].table, r = min(slots, 7):
+ *          [2 r][4][64], entry 2 o + i of the first r own-sector columns, then
+ *          of the first r opposite ones: the coefficient of row i of the pair,
+ *          order 2 o (own sector; E_0 without the identity) or 2 o + 1;
+ *          [da + db - 2][slots][64][2], both rows' coefficients of order 4
+ *          (own sector), with (2, 2) of order 5 (opposite sector);
+ *          [slots - r][4][64][2], both rows' coefficients of orders 0, 2, 1, 3
+ *          of the other columns
  * store    double [n_inst][n_out fine][2][16 ceil(rows / 16)] or null: every
  *          exponential's input by row (padding not written); rows are then
  *          below desc->rows

@@ -20,11 +20,14 @@
 // What bounds it: VALU issue, about 700 of 1,130 cycles per exponential (134
 // gathers with four multiply-adds each over the workgroup); the rest is the
 // latency from the barrier to the first gathers and that of the sum. Measured,
-// 512 points (two rounds of 256 workgroups), per step of a round: Taylor
-// 2.35 us, series 1.05; 1.17 with rows in pair order in LDS (2.4 ways of bank
-// conflict a gather instead of 1.8) and pairs on consecutive lanes (selects
-// and a DPP step where the half swap is). Coefficients evaluated ahead of the
-// gathers gained 1% and spilled.
+// us per step of 256 points (512): orders (1, 1) 1.15 (2.1), Taylor 4.4 (4.7);
+// orders (2, 1) 1.45 to 1.7. 1.3 with rows in pair order in LDS (2.4 ways of
+// bank conflict a gather instead of 1.8) and pairs on consecutive lanes
+// (selects and a DPP step where the half swap is). Coefficients evaluated ahead
+// of the gathers gained 1% and spilled.
+//
+// Orders 4 and 5 do not fit the registers: their coefficients are read from
+// LDS, as are all of an eighth column per lane.
 //
 // Gradients store the inputs of all exponentials forward and the cotangents of
 // their results in reverse (kStore, kBack); ssmx_series_moments.hip contracts
@@ -42,6 +45,10 @@ using ssmx::set_error;
 
 constexpr int kMaxWaves = 12;
 constexpr int kMaxRows = 256;
+// LDS for the coefficients that registers don't hold, and for one column of them
+constexpr int kHighBytes = 150 * 1024;
+constexpr int kColumnBytes = kWave * sizeof(double2);
+constexpr int kRegSlots = 7, kMaxSlots = 8;
 enum { kRun, kStore, kBack };
 
 typedef __attribute__((address_space(3))) double lds_double;
@@ -104,13 +111,24 @@ __device__ __forceinline__ void observe(const WSParams &p, const double *x,
     }
 }
 
+extern __shared__ double2 high_orders[];
+
+// Columns of `slots` slots in LDS: of the orders above 3, and four for each slot
+// beyond the registers'.
+__host__ __device__ constexpr int high_columns(int slots, int hi)
+{
+    return hi * slots + 4 * (slots > kRegSlots ? slots - kRegSlots : 0);
+}
+
 // What an exponential of factor f adds to the lane's row, from the components
-// at `from` in LDS.
-template <int C>
+// at `from` in LDS. Registers hold orders 0..3 of up to kRegSlots columns;
+// coefficients of E_4 (HI >= 1), E_5 (HI 2) and of the columns beyond come from
+// `high` in LDS, for both rows.
+template <int C, int HI, int R>
 __device__ __forceinline__ double
-exponential(const double (&ca)[C][2][2], const double (&cb)[C][2][2],
+exponential(const double (&ca)[R][2][2], const double (&cb)[R][2][2],
             lds_double *const (&xa)[C], lds_double *const (&xb)[C], int from,
-            double f, bool sixteen)
+            const double2 *high, double f, bool sixteen)
 {
     double va[C], vb[C];
 #pragma unroll
@@ -123,13 +141,49 @@ exponential(const double (&ca)[C][2][2], const double (&cb)[C][2][2],
     double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
 #pragma unroll
     for (int s = 0; s < C; ++s) {
-        a0 = fma(fma(u, ca[s][1][0], ca[s][0][0]), va[s], a0);
-        a1 = fma(fma(u, ca[s][1][1], ca[s][0][1]), va[s], a1);
+        double w0, w1, v0, v1;
+        if (s < R) {
+            w0 = ca[s < R ? s : 0][1][0];
+            w1 = ca[s < R ? s : 0][1][1];
+            v0 = ca[s < R ? s : 0][0][0];
+            v1 = ca[s < R ? s : 0][0][1];
+        } else {
+            const double2 *more = high + (HI * C + (s - R) * 4) * kWave;
+            w0 = more[kWave].x;
+            w1 = more[kWave].y;
+            v0 = more[0].x;
+            v1 = more[0].y;
+        }
+        if constexpr (HI >= 1) {
+            const double2 c = high[s * kWave];
+            w0 = fma(u, c.x, w0);
+            w1 = fma(u, c.y, w1);
+        }
+        a0 = fma(fma(u, w0, v0), va[s], a0);
+        a1 = fma(fma(u, w1, v1), va[s], a1);
     }
 #pragma unroll
     for (int s = 0; s < C; ++s) {
-        b0 = fma(fma(u, cb[s][1][0], cb[s][0][0]), vb[s], b0);
-        b1 = fma(fma(u, cb[s][1][1], cb[s][0][1]), vb[s], b1);
+        double w0, w1, v0, v1;
+        if (s < R) {
+            w0 = cb[s < R ? s : 0][1][0];
+            w1 = cb[s < R ? s : 0][1][1];
+            v0 = cb[s < R ? s : 0][0][0];
+            v1 = cb[s < R ? s : 0][0][1];
+        } else {
+            const double2 *more = high + (HI * C + (s - R) * 4 + 2) * kWave;
+            w0 = more[kWave].x;
+            w1 = more[kWave].y;
+            v0 = more[0].x;
+            v1 = more[0].y;
+        }
+        if constexpr (HI >= 2) {
+            const double2 c = high[(C + s) * kWave];
+            w0 = fma(u, c.x, w0);
+            w1 = fma(u, c.y, w1);
+        }
+        b0 = fma(fma(u, w0, v0), vb[s], b0);
+        b1 = fma(fma(u, w1, v1), vb[s], b1);
     }
     return sum_pair(fma(f, b0, a0), fma(f, b1, a1), sixteen);
 }
@@ -139,7 +193,7 @@ exponential(const double (&ca)[C][2][2], const double (&cb)[C][2][2],
 // M is kRun, kStore (a run that keeps every exponential's input and factor) or
 // kBack: the cotangents of an integrated readout in reverse, with transposed
 // matrices and the factors that kStore left.
-template <int C, bool FILL, int M>
+template <int C, bool FILL, int M, int HI>
 __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
                                          double *fbuf, const double *obs,
                                          const ssmx_series_block &blk,
@@ -154,18 +208,32 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
     const double *t = p.table + blk.table + lane;
     const int32_t *col = p.columns + blk.columns + lane;
     // [column][order][row of the pair]
-    double ca[C][2][2], cb[C][2][2];
+    constexpr int R = C < kRegSlots ? C : kRegSlots;
+    double ca[R][2][2], cb[R][2][2];
     lds_double *xa[C], *xb[C];
 #pragma unroll
-    for (int s = 0; s < C; ++s) {
+    for (int s = 0; s < R; ++s)
 #pragma unroll
         for (int o = 0; o < 4; ++o) {
             ca[s][o / 2][o % 2] = t[(s * 4 + o) * kWave];
-            cb[s][o / 2][o % 2] = t[((C + s) * 4 + o) * kWave];
+            cb[s][o / 2][o % 2] = t[((R + s) * 4 + o) * kWave];
         }
+#pragma unroll
+    for (int s = 0; s < C; ++s) {
         xa[s] = (lds_double *)xbuf + col[s * kWave];
         xb[s] = (lds_double *)xbuf + col[(C + s) * kWave];
     }
+    // the wavefront's own part of LDS, behind those of the ones before
+    constexpr int kHigh = HI * C + 4 * (C - R);
+    int before_me = 0;
+    if constexpr (HI > 0 || kRegSlots < kMaxSlots)
+        for (int k = 0; k < wave; ++k)
+            before_me += high_columns(p.blocks[k].slots, HI);
+    double2 *high = high_orders + before_me * kWave + lane;
+    const double2 *from = (const double2 *)(t - lane + R * 8 * kWave) + lane;
+#pragma unroll
+    for (int s = 0; s < kHigh; ++s)
+        high[s * kWave] = from[s * kWave];
     const double half_h = 0.5 * d.h;
     double x = 0.0, source = 0.0;
     if constexpr (M == kBack) {
@@ -198,8 +266,8 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
             for (int j = 0; j < J; ++j) {
                 if (leader)
                     store[(step * J + j) * p.pad] = x;
-                x += exponential<C>(ca, cb, xa, xb, j == 0 ? 0 : kMaxRows,
-                                    fc[j], sixteen);
+                x += exponential<C, HI>(ca, cb, xa, xb, j == 0 ? 0 : kMaxRows,
+                                        high, fc[j], sixteen);
                 // readouts after the step before and before this one
                 if (j == J - 1)
                     x = fma(step == 0 ? half_h : d.h, source, x);
@@ -249,7 +317,8 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
                 const int to = j == 1 ? kMaxRows : 0;
                 if (M == kStore && leader)
                     store[(step * J + j) * p.pad] = x;
-                x += exponential<C>(ca, cb, xa, xb, from, fc[j], sixteen);
+                x += exponential<C, HI>(ca, cb, xa, xb, from, high, fc[j],
+                                        sixteen);
                 if (leader)
                     xbuf[to + row] = x;
                 __syncthreads();
@@ -276,7 +345,7 @@ __device__ __forceinline__ void run_wave(const WSParams &p, double *xbuf,
     }
 }
 
-template <int C, int M>
+template <int C, int M, int HI>
 __device__ __forceinline__ void run_class(const WSParams &p, double *xbuf,
                                           double *fbuf, const double *obs,
                                           const ssmx_series_block &blk,
@@ -284,14 +353,14 @@ __device__ __forceinline__ void run_class(const WSParams &p, double *xbuf,
                                           bool fill)
 {
     if constexpr (M == kBack)
-        run_wave<C, false, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+        run_wave<C, false, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
     else if (fill)
-        run_wave<C, true, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+        run_wave<C, true, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
     else
-        run_wave<C, false, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
+        run_wave<C, false, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst);
 }
 
-template <int M>
+template <int M, int HI>
 __global__ __launch_bounds__(kWave *kMaxWaves)
 __attribute__((amdgpu_waves_per_eu(3))) void series_wide_kernel(WSParams p)
 {
@@ -317,16 +386,19 @@ __attribute__((amdgpu_waves_per_eu(3))) void series_wide_kernel(WSParams p)
     // every wavefront meets the same barriers whatever its class
     switch (blk.slots) {
     case 4:
-        run_class<4, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<4, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
         break;
     case 5:
-        run_class<5, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<5, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
         break;
     case 6:
-        run_class<6, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<6, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        break;
+    case 7:
+        run_class<7, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
         break;
     default:
-        run_class<7, M>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
+        run_class<8, M, HI>(p, xbuf, fbuf, obs, blk, wave, lane, inst, fill);
     }
 }
 
@@ -335,7 +407,8 @@ int check(const ssmx_series_desc &d, int32_t n_blocks, const char *what)
     const bool full = (d.flags & SSMX_READ_FULL) != 0;
     if (d.n < 1 || d.n > SSMX_MAX_N_WIDE || d.rows < 1 ||
         d.rows > kMaxRows || d.n_inst < 1 || d.n_exp != 2 ||
-        d.n_node != 2 || d.da != 1 || d.db != 1 || d.fine < 1 ||
+        d.n_node != 2 || d.da < 1 || d.da > 2 || d.db < 1 || d.db > d.da ||
+        d.fine < 1 ||
         d.n_out < 0 || d.wave_group < 1 || d.gen < 0 ||
         d.gen >= SSMX_MAX_GEN || !(d.h > 0.0) || !(d.dt > 0.0) ||
         (d.flags & ~(SSMX_READ_FULL | SSMX_READ_INTEGRAL)) != 0 ||
@@ -349,20 +422,45 @@ int check(const ssmx_series_desc &d, int32_t n_blocks, const char *what)
     if (n_blocks < 1 || n_blocks > kMaxWaves)
         return set_error(SSMX_EINVAL, "%d wavefronts outside 1..%d",
                          n_blocks, kMaxWaves);
+    if (d.na < 0 || d.na * kColumnBytes > kHighBytes)
+        return set_error(SSMX_EINVAL, "%d columns of coefficients exceed the "
+                         "LDS", d.na);
     return SSMX_OK;
 }
 
-template <int M>
+template <int M, int HI>
 int launch(const WSParams &p, int n_blocks, void *stream, const char *what)
 {
-    hipLaunchKernelGGL(series_wide_kernel<M>, dim3(p.d.n_inst),
-                       dim3(kWave * n_blocks), 0,
-                       static_cast<hipStream_t>(stream), p);
-    const hipError_t e = hipGetLastError();
+    const size_t bytes = (size_t)p.d.na * kColumnBytes;
+    hipError_t e = hipSuccess;
+    if (bytes > 0)
+        e = hipFuncSetAttribute(
+            reinterpret_cast<const void *>(series_wide_kernel<M, HI>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL((series_wide_kernel<M, HI>), dim3(p.d.n_inst),
+                           dim3(kWave * n_blocks), bytes,
+                           static_cast<hipStream_t>(stream), p);
+        e = hipGetLastError();
+    }
     if (e != hipSuccess)
         return set_error(SSMX_ELAUNCH, "%s launch: %s", what,
                          hipGetErrorString(e));
     return SSMX_OK;
+}
+
+template <int M>
+int launch_orders(const WSParams &p, int n_blocks, void *stream,
+                  const char *what)
+{
+    switch (p.d.da - 1 + p.d.db - 1) {
+    case 0:
+        return launch<M, 0>(p, n_blocks, stream, what);
+    case 1:
+        return launch<M, 1>(p, n_blocks, stream, what);
+    default:
+        return launch<M, 2>(p, n_blocks, stream, what);
+    }
 }
 
 }  // namespace
@@ -401,8 +499,8 @@ extern "C" int ssmx_propagate_series_wide(
     p.store = store;
     p.factors = factors;
     p.pad = (desc->rows + 15) / 16 * 16;
-    return store ? launch<kStore>(p, n_blocks, stream, "wide series")
-                 : launch<kRun>(p, n_blocks, stream, "wide series");
+    return store ? launch_orders<kStore>(p, n_blocks, stream, "wide series")
+                 : launch_orders<kRun>(p, n_blocks, stream, "wide series");
 }
 
 extern "C" int ssmx_series_wide_adjoint(
@@ -435,5 +533,5 @@ extern "C" int ssmx_series_wide_adjoint(
     p.out = lambda_out;
     p.store = store;
     p.pad = (desc->rows + 15) / 16 * 16;
-    return launch<kBack>(p, n_blocks, stream, "wide series adjoint");
+    return launch_orders<kBack>(p, n_blocks, stream, "wide series adjoint");
 }

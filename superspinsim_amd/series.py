@@ -158,6 +158,34 @@ def coefficient_matrices(terms, drive, orders, extended=False):
     return total if extended else [m.astype(_f64) for m in total]
 
 
+def chebyshev(mats, F):
+    """Chebyshev coefficients in f / F of sum_k f^k E_k."""
+    out = [np.zeros_like(mats[0]) for _ in mats]
+    for k, m in enumerate(mats):
+        power = np.zeros(k + 1)
+        power[k] = F ** k
+        for j, c in enumerate(np.polynomial.chebyshev.poly2cheb(power)):
+            if c:
+                out[j] += c * m
+    return out
+
+
+def economised(mats, da, db, F):
+    """E_k with the Chebyshev polynomials of the orders that (da, db) leave
+    out taken off, so that the kept ones represent the truncated Chebyshev
+    series."""
+    kept = [m.copy() for m in mats]
+    cheb = chebyshev(mats, F)
+    for j in _dropped(len(mats), da, db):
+        unit = np.zeros(j + 1)
+        unit[j] = 1.0
+        for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(unit)):
+            # (an underflown power: its order is zero as well)
+            if c and F ** k:
+                kept[k] -= (c / F ** k) * cheb[j]
+    return kept
+
+
 class SeriesModel:
     """E_k and row layout of one (constant, drive) pair at one step size.
 
@@ -233,6 +261,14 @@ class SeriesModel:
         return self.n_sectors <= 2 and \
             max(s.size for s in self.members) <= 11
 
+    def flops(self, plan):
+        """FP64 operations of one exponential: a multiply-add per order and
+        entry of the sectors, two per row."""
+        own = np.array([s.size for s in self.members])
+        opp = np.where(self.opposite >= 0, own[self.opposite], 0)
+        return int(2 * (own * (own * (plan[0] + 1) + opp * (plan[1] + 1) +
+                               2)).sum())
+
     def plan(self, drive_max, tol):
         """(da, db, F) for drives |c(t)| <= ``drive_max``, or None.
 
@@ -243,8 +279,7 @@ class SeriesModel:
         """
         F = self.h * self.weight * float(drive_max)
         worst = np.max([[np.abs(c).sum(axis=0).max() for c in cs]
-                        for cs in (self._chebyshev(es, F)
-                                   for es in self.sets)], axis=0)
+                        for cs in (chebyshev(es, F) for es in self.sets)], axis=0)
         if not np.all(np.isfinite(worst)):
             return None
         for da, db in ORDERS:
@@ -254,36 +289,9 @@ class SeriesModel:
                 return da, db, F
         return None
 
-    @staticmethod
-    def _chebyshev(mats, F):
-        """Chebyshev coefficients in f / F of sum_k f^k E_k."""
-        out = [np.zeros_like(mats[0]) for _ in mats]
-        for k, m in enumerate(mats):
-            power = np.zeros(k + 1)
-            power[k] = F ** k
-            for j, c in enumerate(np.polynomial.chebyshev.poly2cheb(power)):
-                if c:
-                    out[j] += c * m
-        return out
-
     def matrices(self, da, db, F):
-        """The kept E_k of every set, with the Chebyshev polynomials of the
-        orders left out taken off (so that they represent the truncated
-        Chebyshev series)."""
-        out = []
-        for mats in self.sets:
-            kept = [m.copy() for m in mats]
-            cheb = self._chebyshev(mats, F)
-            for j in _dropped(len(mats), da, db):
-                unit = np.zeros(j + 1)
-                unit[j] = 1.0
-                for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(
-                        unit)):
-                    # (an underflown power: its order is zero as well)
-                    if c and F ** k:
-                        kept[k] -= (c / F ** k) * cheb[j]
-            out.append(kept)
-        return out
+        """The kept E_k of every set (``economised``)."""
+        return [economised(mats, da, db, F) for mats in self.sets]
 
     def tables(self, da, db, F):
         """Device (layout, table) of the kernel's rows."""

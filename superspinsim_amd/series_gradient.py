@@ -11,7 +11,7 @@ import numpy as np
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 from superspinsim_amd.series import (
-    SeriesModel, lane_entries, lane_table, reachable)
+    SeriesModel, chebyshev, lane_entries, lane_table, reachable)
 
 _f64 = np.float64
 
@@ -105,7 +105,7 @@ class SeriesGradient:
         polynomials of f / F cut there; None if more than ``tol`` of a
         direction is cut off."""
         count = dmats.shape[0]
-        cheb = SeriesModel._chebyshev(list(dmats), F)
+        cheb = chebyshev(list(dmats), F)
         size = np.array([np.abs(c).sum(axis=1).max(axis=1) for c in cheb])
         if size.shape[1] and np.any(
                 size[ORDERS:].sum(axis=0) + size[-1] > tol * size.max(axis=0)):

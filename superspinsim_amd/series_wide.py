@@ -9,70 +9,90 @@ pairs over 8 or 16 lanes each.
 """
 
 import ctypes
+import math
 
 import numpy as np
 
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 from superspinsim_amd.series import (
-    MAX_NORM, SeriesModel, _dropped, coefficient_matrices, split_sectors)
+    ORDERS, _dropped, chebyshev, economised, split_sectors)
 
 _f64 = np.float64
 
 #: the kernel's limits: rows, wavefronts, columns per lane
-MAX_ROWS, MAX_WAVES, MIN_SLOTS, MAX_SLOTS = 256, 12, 4, 7
-#: orders kept (even 0, 2; odd 1, 3) and computed, which bounds the rest
-DA, DB, TOP = 1, 1, 4
+MAX_ROWS, MAX_WAVES, MIN_SLOTS, MAX_SLOTS = 256, 12, 4, 8
+#: highest 1-norm of h w C (beyond, the E_k fill in past the kernel's limits)
+MAX_NORM = 1.0
+#: highest order computed for the first of ORDERS, and for the others
+TOP = (4, 6)
+#: columns per lane whose orders 0..3 registers hold; KB of LDS for the other
+#: coefficients (one KB per column and order, for both rows of the pairs)
+REG_SLOTS, LDS_COLUMNS = 7, 150
 #: share of the tolerance that left-out entries may take, per column
 SHARE = 1.0 / 64.0
 
 
 def wide_coefficients(terms, drive, orders):
     """``coefficient_matrices`` where the extended products of every term
-    take a second (171 states): those of degree one and two are summed in
-    extended precision, the others in doubles.
+    take a second (171 states): those up to a degree d are summed in extended
+    precision, the others in doubles.
 
-    For a constant part of 1-norm c <= 1/4 the terms from degree three on
-    are c^3 / 6 of it, so that their rounding (some 10 ulp) stays a tenth of
-    the rounding of the result.  Larger ones take the extended products.
+    For a constant part of 1-norm c the terms beyond degree d are
+    c^d / (d + 1)! of it; d is the first where that is below 1/96 (2 for
+    c <= 1/4), so that their rounding (some 10 ulp) stays a tenth of the
+    rounding of the result.
     """
     const = sum(np.asarray(m, dtype=np.longdouble) * np.longdouble(s)
                 for m, s in terms)
     n = const.shape[0]
     norm = float(np.abs(const).sum(axis=0).max(initial=0.0))
-    if not norm <= 0.25:
-        return coefficient_matrices(terms, drive, orders)
     drive = np.asarray(drive, dtype=_f64)
-    rows = [(c, const[r, c]) for r, c in
-            ((r, np.flatnonzero(const[r])) for r in range(n))]
-    drows = [(c, drive[r, c]) for r, c in
-             ((r, np.flatnonzero(drive[r])) for r in range(n))]
+    exact, size = 2, norm ** 2 / 6.0
+    while size > 1.0 / 96.0:
+        exact += 1
+        size *= norm / (exact + 1)
 
-    def times(lists, mat):
-        return np.stack([v @ mat[c] for c, v in lists])
+    def lists(mat):
+        return [(c, mat[r, c]) for r, c in
+                ((r, np.flatnonzero(mat[r])) for r in range(n))]
 
-    first = [const, drive.astype(np.longdouble)]
-    half = np.longdouble(0.5)
-    second = [times(rows, const) * half,
-              (times(drows, const) + times(rows, first[1])) * half,
-              times(drows, first[1]) * half]
-    zero = np.zeros((n, n), dtype=np.longdouble)
-    total = [(first + [zero] * orders)[k] + (second + [zero] * orders)[k]
-             for k in range(orders + 1)]
-    term = np.zeros((orders + 1, n, n))
-    for k in range(min(orders, 2) + 1):
-        term[k] = second[k]
+    def times(rows, mat):
+        return np.stack([v @ mat[c] for c, v in rows])
+
+    rows, drows = lists(const), lists(drive)
+    # orders above the degree are zero
+    term = [const, drive.astype(np.longdouble)][:orders + 1]
+    total = list(term)
+    for t in range(2, exact + 1):
+        new = [times(rows, m) for m in term]
+        for k, m in enumerate(term[:orders]):
+            v = times(drows, m)
+            if k + 1 < len(new):
+                new[k + 1] += v
+            else:
+                new.append(v)
+        term = [m / t for m in new]
+        total = [m + term[k] if k < len(total) else term[k]
+                 for k, m in enumerate(total + term[len(total):])]
+    last = np.zeros((orders + 1, n, n))
+    for k, m in enumerate(term):
+        last[k] = m
     small = np.zeros((orders + 1, n, n))
     c64 = const.astype(_f64)
-    bound, t = 1.0, 2
-    while bound > 1e-24 or t <= orders + 2:
+    bound, t = 1.0, exact
+    while bound > 1e-18 or t <= orders + 2:
         t += 1
-        bound *= norm / max(t - orders, 1)
-        new = c64 @ term
-        new[1:] += drive @ term[:-1]
-        term = new / t
-        small += term
-    return [(m + s).astype(_f64) for m, s in zip(total, small)]
+        # an order's terms go like norm^(t - k) / (t - k)! of its first
+        bound = norm ** max(t - orders, 0) / math.factorial(
+            max(t - orders, 0))
+        new = c64 @ last
+        new[1:] += drive @ last[:-1]
+        last = new / t
+        small += last
+    return [(total[k] + small[k] if k < len(total) else
+             small[k].astype(np.longdouble)).astype(_f64)
+            for k in range(orders + 1)]
 
 
 def pair_rows(pattern, sector):
@@ -125,45 +145,59 @@ class WideModel:
         self.size = int(np.bincount(self.sector).max())
         self.weight = float(np.abs(weights).sum(axis=1).max())
         self.nnz = int(np.count_nonzero((const != 0) | (drive != 0)))
-        self.mats = wide_coefficients(terms, drive, TOP)
+        self.mats = []
+        self._point = terms, drive
+        self.drive_norm = float(np.abs(drive).sum(axis=0).max())
         return self
 
     def plan(self, drive_max, tol):
         """(da, db, F, budget) for drives |c(t)| <= ``drive_max``, or None;
         the bound of ``SeriesModel.plan`` with the left-out entries added."""
         F = self.h * self.weight * float(drive_max)
-        worst = [np.abs(c).sum(axis=0).max()
-                 for c in SeriesModel._chebyshev(self.mats, F)]
-        if not np.all(np.isfinite(worst)):
-            return None
         budget = SHARE * tol
-        if not 8.0 * (budget + worst[-1] + sum(
-                worst[k] for k in _dropped(TOP + 1, DA, DB))) <= tol:
-            return None
-        plan = DA, DB, F, budget
-        return None if self.layout(plan) is None else plan
+        # (drives that the first orders may not do for: all at once)
+        small = (F * self.drive_norm) ** 4 / 24.0 <= tol
+        for da, db in ORDERS:
+            top = TOP[0] if small and (da, db) == ORDERS[0] else TOP[1]
+            if len(self.mats) <= top:
+                self.mats = wide_coefficients(*self._point, top)
+            worst = [np.abs(c).sum(axis=0).max()
+                     for c in chebyshev(self.mats, F)]
+            if not np.all(np.isfinite(worst)):
+                return None
+            if 8.0 * (budget + worst[-1] + sum(
+                    worst[k] for k in _dropped(len(worst), da, db))) <= tol:
+                plan = da, db, F, budget
+                return None if self.layout(plan) is None else plan
+        return None
+
+    def flops(self, plan):
+        """FP64 operations of one exponential: a multiply-add per order and
+        kept entry, two per row."""
+        even, odd = self.entries
+        return int(2 * (even * (plan[0] + 1) + odd * (plan[1] + 1) +
+                        2 * self.n))
 
     def layout(self, plan):
-        """Device (blocks, states, columns, table) of the kernel, or None
-        where the rows don't fit it."""
+        """Device (blocks, states, columns, table) of the kernel and its
+        columns in LDS; None where the rows don't fit it."""
         if self._layout is None or self._layout[0] != plan:
-            arrays = self._arrays(*plan[2:])
-            self._layout = (plan, None if arrays is None else
-                            tuple(device_tensor(a) for a in arrays))
+            self._layout = plan, self._staged(self._arrays(*plan))
         return self._layout[1]
 
     def transposed(self, plan):
-        """``layout`` of the transposed matrices, on the host."""
-        return self._arrays(*plan[2:], transpose=True)
+        """``layout`` of the transposed matrices (not kept)."""
+        return self._staged(self._arrays(*plan, transpose=True))
 
-    def _arrays(self, F, budget, transpose=False):
-        kept = [m.copy() for m in self.mats[:4]]
-        # the dropped order's Chebyshev polynomial taken off
-        # (T_4 = 8 u^4 - 8 u^2 + 1: its lower coefficients stay with E_0, E_2)
-        top = F ** 4 / 8.0 * self.mats[4]
-        if F ** 2 > 0.0:
-            kept[0] -= top
-            kept[2] += (8.0 / F ** 2) * top
+    @staticmethod
+    def _staged(arrays):
+        return None if arrays is None else tuple(
+            device_tensor(a) for a in arrays[:-1]) + arrays[-1:]
+
+    def _arrays(self, da, db, F, budget, transpose=False):
+        kept = economised(self.mats, da, db, F)
+        kept = [kept[k] for k in range(2 * max(da, db) + 2)
+                if k <= (2 * db + 1 if k % 2 else 2 * da)]
         if transpose:
             kept = [np.ascontiguousarray(m.T) for m in kept]
         size = sum(F ** k * np.abs(m) for k, m in enumerate(kept))
@@ -172,6 +206,8 @@ class WideModel:
         np.put_along_axis(keep, order, np.cumsum(np.take_along_axis(
             size, order, axis=0), axis=0) >= budget, axis=0)
         same = self.sector[:, None] == self.sector[None, :]
+        self.entries = (np.count_nonzero(keep & same),
+                        np.count_nonzero(keep & ~same))
         pairs = pair_rows(keep, self.sector)
         cols = []
         for a, b in pairs:
@@ -181,7 +217,12 @@ class WideModel:
         widest = np.array([max(o.size, p.size) for o, p in cols])
         rank = np.argsort(-widest, kind="stable")
         waves = self._waves(widest[rank])
+        # orders above 3 and columns beyond the registers' lie in LDS
+        high = da - 1 + db - 1
         if waves is None:
+            return None
+        in_lds = sum(high * s + 4 * max(0, s - REG_SLOTS) for _, s in waves)
+        if in_lds > LDS_COLUMNS:
             return None
         pos = self.pos
         blocks = np.zeros((len(waves), 4), dtype=np.int32)
@@ -193,6 +234,7 @@ class WideModel:
             blocks[w] = slots, lanes, done, tabled
             c = np.zeros((2 * slots, 64), dtype=np.int32)
             t = np.zeros((2 * slots, 4, 64))
+            hi = np.zeros((high, slots, 64, 2))
             for g in range(64 // lanes):
                 if first + g >= len(pairs):
                     break
@@ -210,32 +252,46 @@ class WideModel:
                     lane = mine.ravel()[e % lanes]
                     c[slot, lane] = pos[cols[p][part]]
                     for i, r in enumerate(pairs[p]):
+                        if r < 0:
+                            continue
+                        use = keep[r, cols[p][part]]
                         for o in (0, 1):
-                            if r >= 0:
-                                t[slot, 2 * o + i, lane] = \
-                                    kept[2 * o + part][r, cols[p][part]] * \
-                                    keep[r, cols[p][part]]
+                            t[slot, 2 * o + i, lane] = \
+                                kept[2 * o + part][r, cols[p][part]] * use
+                        if high > part:
+                            hi[part, e // lanes, lane, i] = \
+                                kept[4 + part][r, cols[p][part]] * use
             first += 64 // lanes
             done += c.size
-            tabled += t.size
+            parts = [t[:slots][:REG_SLOTS], t[slots:][:REG_SLOTS], hi]
+            if slots > REG_SLOTS:
+                # [column][own 0, 2, opposite 1, 3][lane][row]
+                rest = np.stack([t[REG_SLOTS:slots],
+                                 t[slots + REG_SLOTS:]], axis=1)
+                parts.append(rest.reshape(-1, 2, 2, 2, 64).transpose(
+                    0, 1, 2, 4, 3))
             columns.append(c.ravel())
-            table.append(t.ravel())
-        return blocks, states, np.concatenate(columns), np.concatenate(table)
+            table += [part.ravel() for part in parts]
+            tabled += sum(part.size for part in parts)
+        return blocks, states, np.concatenate(columns), \
+            np.concatenate(table), in_lds
 
     @staticmethod
     def _waves(widest):
         """[(lanes per pair, columns per lane)] of the wavefronts for pairs
-        sorted by width: as few 16-lane ones as leave the others within
-        the kernel's columns per lane."""
-        for wide in range(MAX_WAVES + 1):
-            out, i = [], 0
-            while i < widest.size:
-                lanes = 16 if len(out) < wide else 8
-                slots = -(-int(widest[i]) // lanes)
-                out.append((lanes, max(slots, MIN_SLOTS)))
-                i += 64 // lanes
-            if len(out) <= MAX_WAVES and max(s for _, s in out) <= MAX_SLOTS:
-                return out
+        sorted by width: as few 16-lane ones as leave the others within the
+        registers' columns per lane, or else within the kernel's."""
+        for most in (REG_SLOTS, MAX_SLOTS):
+            for wide in range(MAX_WAVES + 1):
+                out, i = [], 0
+                while i < widest.size:
+                    lanes = 16 if len(out) < wide else 8
+                    slots = -(-int(widest[i]) // lanes)
+                    out.append((lanes, max(slots, MIN_SLOTS)))
+                    i += 64 // lanes
+                if len(out) <= MAX_WAVES and \
+                        max(s for _, s in out) <= most:
+                    return out
         return None
 
 
@@ -255,7 +311,7 @@ class WideRun:
         if read != "full" and not 1 <= n_obs <= _lib.MAX_OBS:
             raise ValueError(f"{n_obs} readout rows outside 1.."
                              f"{_lib.MAX_OBS}")
-        self.blocks, lane_states, self.columns, self.table = \
+        self.blocks, lane_states, self.columns, self.table, in_lds = \
             model.layout(plan)
         # the kernel's state index is the caller's
         index = device_tensor(np.asarray(states).astype(np.int32))
@@ -272,7 +328,8 @@ class WideRun:
             n=n, rows=model.n, n_inst=n_inst, members=1,
             n_exp=weights.shape[0], n_node=weights.shape[1], fine=fine,
             n_out=n_out, n_obs=n_obs, flags=flags, gen=gen, wave_group=1,
-            da=plan[0], db=plan[1], h=dt / fine, t0=t0, dt=dt)
+            na=in_lds, da=plan[0], db=plan[1], h=dt / fine, t0=t0,
+            dt=dt)
         shape = {"full": (n_inst, n_out, n), "obs": (n_inst, n_out, n_obs),
                  "integral": (n_inst, n_obs)}[read]
         self.out = torch.empty(shape, dtype=torch.float64, device="cuda")

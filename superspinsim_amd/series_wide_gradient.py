@@ -109,17 +109,16 @@ class WideGradient:
     def _staged(layout, index):
         if layout is None:
             return None
-        blocks, states, columns, table = layout
+        blocks, states, columns, table, in_lds = layout
         states = _torch().stack(
             [states[..., 0], index[states[..., 1].long()]], dim=-1)
-        return blocks, states, columns, table
+        return blocks, states, columns, table, in_lds
 
     def _back(self):
         """Tables of the transposed matrices (None where they don't fit)."""
         if self.back is None:
-            arrays = self.model.transposed(self.plan)
-            self.back = None if arrays is None else self._staged(
-                tuple(device_tensor(a) for a in arrays), self.index)
+            self.back = self._staged(self.model.transposed(self.plan),
+                                     self.index)
         return self.back
 
     def _derivatives(self, a, g, da, terms, drive_max):
@@ -144,15 +143,15 @@ class WideGradient:
         """Inputs and cotangents of every exponential."""
         return 2, n_inst, steps, J, self.npad
 
-    def _desc(self, problem, n_inst):
+    def _desc(self, problem, n_inst, in_lds):
         J, S = self.d_w.shape
         return _lib.SeriesDesc(
             n=problem.rho0.shape[-1], rows=self.model.n, n_inst=n_inst,
             members=1, n_exp=J, n_node=S, fine=problem.F,
             n_out=problem.n_out, n_obs=problem.obs.shape[0],
             flags=_lib.SSMX_READ_INTEGRAL, gen=self.gen, wave_group=1,
-            da=self.plan[0], db=self.plan[1], h=problem.dt / problem.F,
-            t0=problem.t0, dt=problem.dt)
+            na=in_lds, da=self.plan[0], db=self.plan[1],
+            h=problem.dt / problem.F, t0=problem.t0, dt=problem.dt)
 
     def forward(self, problem, state, rho0, store):
         """Integrated readouts (n_inst, n_obs); ``store`` keeps the inputs
@@ -170,9 +169,9 @@ class WideGradient:
                                       device="cuda")
             state["factors"] = factors
         d_rho, d_obs = device_tensor(rho0), device_tensor(problem.obs)
-        blocks, states, columns, table = self.tables
+        blocks, states, columns, table, in_lds = self.tables
         _lib.check(_lib.load().ssmx_propagate_series_wide(
-            ctypes.byref(self._desc(problem, n_inst)), _ptr(blocks),
+            ctypes.byref(self._desc(problem, n_inst, in_lds)), _ptr(blocks),
             blocks.shape[0], _ptr(states), _ptr(columns), _ptr(table),
             _ptr(self.d_w), _ptr(self.d_nodes), _ptr(state["d_waves"]),
             _ptr(state["d_segs"]), _ptr(d_rho), _ptr(d_obs), _ptr(out),
@@ -191,9 +190,9 @@ class WideGradient:
             lam.zero_()
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         lib = _lib.load()
-        blocks, states, columns, table = self._back()
+        blocks, states, columns, table, in_lds = self._back()
         _lib.check(lib.ssmx_series_wide_adjoint(
-            ctypes.byref(self._desc(problem, n_inst)), _ptr(blocks),
+            ctypes.byref(self._desc(problem, n_inst, in_lds)), _ptr(blocks),
             blocks.shape[0], _ptr(states), _ptr(columns), _ptr(table),
             _ptr(factors), _ptr(d_obs), _ptr(seed), _ptr(store[1]),
             _ptr(lam), stream))

@@ -635,7 +635,8 @@ class BatchSimulator:
                     taylor=m, substeps=s, slots=2 * model.size,
                     nnz=model.nnz, active=program, n_out=N,
                     steps=N * self.F, n=self.n, packed=run.k,
-                    involved=model.n, series=plan[:2])
+                    involved=model.n, series=plan[:2],
+                    flops=model.flops(plan))
                 return run
             if sub is not self:
                 run = sub._prepare_taylor(
@@ -822,7 +823,8 @@ class BatchSimulator:
             m, s = self.taylor_plan(waves, active, const, program, time_step)
             self.last_plan = dict(
                 taylor=m, substeps=s, slots=2 * model.size, nnz=model.nnz,
-                active=program, n=n, packed=k, involved=n, series=plan[:2])
+                active=program, n=n, packed=k, involved=n, series=plan[:2],
+                flops=model.flops(plan))
         else:
             members = [w for w in shifted for _ in range(n)]
             saved = self.pack
@@ -857,9 +859,12 @@ class BatchSimulator:
 
         J exponentials, each: assembly 2 K nnz (+ h scaling n), and s m
         Taylor terms of one sparse product (2 nnz) plus scale and add
-        (2 n); rotating frame adds the 2x2-block step (4 n).
+        (2 n); rotating frame adds the 2x2-block step (4 n).  Runs of the
+        series in the drive: the series' operations.
         """
         p = plan or self.last_plan
+        if "flops" in p:
+            return self.weights.shape[0] * p["flops"]
         J = self.weights.shape[0]
         K = len(p["active"]) * (self.nodes.size if self.rotating else 1)
         nnz, n = p["nnz"], p["n"]

@@ -76,15 +76,16 @@ def test_derivatives_equal_numpy(gpu, n, thetas, orders):
         assert err <= 1e-14 * np.max(np.abs(want[k])), k
 
 
-@pytest.mark.parametrize("points,outputs,fine,two", [
-    (3, 5, 61, True), (1, 1, 3, False), (2, 2, 100, False)])
-def test_wide_gradient_equals_frechet(gpu, points, outputs, fine, two):
+@pytest.mark.parametrize("points,outputs,fine,two,rabi", [
+    (3, 5, 61, True, 0.5e6), (1, 1, 3, False, 0.5e6),
+    (2, 2, 100, False, 0.5e6), (9, 3, 40, True, 3e6)])
+def test_wide_gradient_equals_frechet(gpu, points, outputs, fine, two, rabi):
     """As for the 7-level models: each side is exact to its truncation
     relative to each exponential, a few 1e-12 of a gradient plus the
     cancellation floor 1e-12 F / theta_scale."""
     wl = configs.odmr21(1, use_incoherent=True)
     h = 20e-12
-    b1 = configs.drive_amplitude(0.5e6)
+    b1 = configs.drive_amplitude(rabi)
     rng = np.random.default_rng(points)
 
     def waveforms(amps):

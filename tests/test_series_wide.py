@@ -36,25 +36,39 @@ def _model(n, block, norm=0.15, spread=0):
     return const, drive / np.abs(drive).sum(axis=0).max()
 
 
-@pytest.mark.parametrize("n,block,spread,lanes,slots", [
-    (65, 65, 0, 8, 5), (112, 112, 0, 8, 7), (150, 10, 3, 16, 5),
-    (192, 8, 0, 8, 4)])
+@pytest.mark.parametrize("n,block,spread,lanes,slots,amp,orders", [
+    (65, 65, 0, 8, 5, 1e7, (1, 1)), (112, 112, 0, 8, 7, 1e7, (1, 1)),
+    (150, 10, 3, 16, 5, 1e7, (1, 1)), (192, 8, 0, 8, 4, 1e7, (1, 1)),
+    (112, 112, 0, 8, 7, 1e8, (2, 1)), (65, 65, 0, 8, 5, 5e8, (2, 2)),
+    (150, 10, 3, 16, 5, 5e8, (2, 2)), (120, 120, 0, 8, 8, 1e8, (2, 1))])
 def test_layout_holds_the_matrices(monkeypatch, n, block, spread, lanes,
-                                   slots):
+                                   slots, amp, orders):
     monkeypatch.setattr(series_wide, "device_tensor", lambda a: a)
     const, drive = _model(n, block, spread=spread)
     _, weights, _ = quadratures.scheme(2)
     model = WideModel.build(const, drive, weights, H)
-    plan = model.plan(1e7, 1e-16)
+    plan = model.plan(amp, 1e-16)
     F = plan[2]
-    blocks, states, columns, table = model.layout(plan)
+    assert plan[:2] == orders
+    high = sum(orders) - 2
+    blocks, states, columns, table, in_lds = model.layout(plan)
     assert tuple(blocks[0, :2]) == (slots, lanes)
-    kept = [np.zeros((n, n)) for _ in range(4)]
+    assert in_lds == sum(high * s + 4 * max(0, s - 7)
+                         for s in blocks[:, 0])
+    kept = [np.zeros((n, n)) for _ in range(6)]
     where = {int(p): int(s) for p, s in states.reshape(-1, 2) if p >= 0}
     assert sorted(where.values()) == list(range(n))
     for w, (c, width, at, tat) in enumerate(blocks):
         col = columns[at:at + 2 * c * 64].reshape(2 * c, 64)
-        tab = table[tat:tat + 2 * c * 256].reshape(2 * c, 4, 64)
+        r = min(c, 7)
+        held = table[tat:tat + 2 * r * 256].reshape(2, r, 4, 64)
+        tat += 2 * r * 256
+        hi = table[tat:][:high * c * 128].reshape(high * c, 64, 2)
+        tat += high * c * 128
+        rest = table[tat:][:(c - r) * 512].reshape(c - r, 2, 2, 64, 2)
+        tab = np.concatenate([np.concatenate([held[part], rest[
+            :, part].transpose(0, 1, 3, 2).reshape(c - r, 4, 64)])
+            for part in (0, 1)])
         for lane in range(64):
             first = lane % 32 - lane % 32 % (width // 2)
             for i in (0, 1):
@@ -65,12 +79,16 @@ def test_layout_holds_the_matrices(monkeypatch, n, block, spread, lanes,
                             kept[2 * o + e // c][row, where[
                                 int(col[e, lane])]] += tab[e, 2 * o + i,
                                                            lane]
+                    if e < high * c:
+                        kept[4 + e // c][row, where[int(col[e, lane])]] += \
+                            hi[e, lane, i]
                 if p < 0:
                     assert not np.any(tab[:, i::2, lane])
+                    assert not np.any(hi[:, lane, i])
     # against the whole series at the ends and inside: what is left out
     # stays below the tolerance (half an ulp of the sums' largest
     # coefficient, 0.15, on top: 1.4e-17 per entry, n / 2 of them a column)
-    whole = coefficient_matrices([(const, 0.5 * H)], drive, 7, extended=True)
+    whole = coefficient_matrices([(const, 0.5 * H)], drive, 9, extended=True)
     for f in (0.0, 0.37 * F, -F):
         got = sum(np.longdouble(f) ** k * m for k, m in enumerate(kept))
         want = sum(np.longdouble(f) ** k * m for k, m in enumerate(whole))
@@ -97,8 +115,10 @@ def test_uncovered_models_are_refused(monkeypatch):
         w = quadratures.scheme(exps)[1]
         assert WideModel.build(*_model(n, 10), w, H) is None
     # more pairs than the wavefronts hold; rows of more columns than the
-    # lanes; a drive so large that order four counts
-    for n, block, amp in ((193, 8, 1e7), (190, 190, 1e7), (70, 70, 1e10)):
+    # lanes; a drive so large that order six counts; rows whose orders above
+    # three exceed the LDS
+    for n, block, amp in ((193, 8, 1e7), (190, 190, 1e7), (70, 70, 1e10),
+                          (192, 100, 5e8)):
         model = WideModel.build(*_model(n, block), weights, H)
         assert model.plan(amp, 1e-16) is None
     const, drive = _model(70, 10)
@@ -107,12 +127,20 @@ def test_uncovered_models_are_refused(monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,block,spread,norm,points,fine,read", [
-    (65, 65, 0, 0.15, 1, 7, "obs"), (112, 112, 0, 1.5, 3, 33, "full"),
-    (150, 10, 3, 0.15, 5, 1, "integral"), (192, 8, 0, 0.15, 2, 40, "obs"),
-    (171, 0, 0, 0.0, 3, 16, "integral"), (441, 0, 0, 0.0, 2, 31, "full")])
+@pytest.mark.parametrize("n,block,spread,norm,points,fine,read,scale,orders", [
+    (65, 65, 0, 0.15, 1, 7, "obs", 1, (1, 1)),
+    (112, 112, 0, 0.9, 3, 33, "full", 1, (1, 1)),
+    (150, 10, 3, 0.15, 5, 1, "integral", 1, (1, 1)),
+    (192, 8, 0, 0.15, 2, 40, "obs", 1, (1, 1)),
+    (171, 0, 0, 0.0, 3, 16, "integral", 1, (1, 1)),
+    (441, 0, 0, 0.0, 2, 31, "full", 1, (1, 1)),
+    (112, 112, 0, 0.15, 3, 20, "obs", 10, (2, 1)),
+    (150, 10, 3, 0.15, 2, 33, "integral", 50, (2, 2)),
+    (120, 120, 0, 0.15, 2, 9, "full", 1, (1, 1)),
+    (171, 0, 0, 0.0, 2, 16, "obs", 6, (2, 1)),
+    (65, 65, 0, 0.15, 3, 21, "full", 50, (2, 2))])
 def test_wide_series_equals_taylor(gpu, n, block, spread, norm, points, fine,
-                                   read):
+                                   read, scale, orders):
     """Both propagate the same exponentials to 1e-16; over 600 steps they
     differ by rounding, an ulp of the state per exponential at most
     (1200 x 1.1e-16 = 1.3e-13, times the few units by which the random
@@ -129,6 +157,7 @@ def test_wide_series_equals_taylor(gpu, n, block, spread, norm, points, fine,
         gens, rho, obs = wl.generators, wl.rho0, wl.obs
         base = [1.0, 0.0, 0.0, 0.0, wl.excitation]
         f0, amp = 2.87e9, configs.drive_amplitude(5e5)
+    amp *= scale
     waves = []
     for k in range(points):
         w = Waveform(len(base), base=base)
@@ -145,7 +174,7 @@ def test_wide_series_equals_taylor(gpu, n, block, spread, norm, points, fine,
     obs = None if read == "full" else obs
     print(f"{n} states x {points}, {read}", flush=True)
     got = sim.run(*args, obs=obs, read=read).cpu().numpy()
-    assert sim.last_plan["series"] == (1, 1), sim.last_plan
+    assert sim.last_plan["series"] == orders, sim.last_plan
     want = sim.run(*args, obs=obs, read=read, taylor=17).cpu().numpy()
     assert got.shape == want.shape
     err = np.max(np.abs(got - want)) / np.max(np.abs(want))
