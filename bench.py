@@ -13,13 +13,14 @@ per-instance inputs uploaded from pinned host memory before each launch.
 The gradient leg runs the 1024-point version of the sweep with a
 200-segment microwave amplitude: a forward that keeps every exponential's
 input in HBM, then the reverse run of the cotangents and the parameter
-moments, for the squared error against targets simulated at
-parameters perturbed by up to 2 %; the ratio is (forward with stored inputs
-+ backward) / plain forward, wall time.
+moments, for the squared error against targets simulated at parameters
+perturbed by up to 2 %; the ratio is (forward with stored inputs + backward)
+/ plain forward, wall time.
 
 The protocol leg runs 16384 pulsed Ramsey / Hahn-echo protocols of 58k-742k
 steps in one persistent work-queue launch (driven stretches step by step,
-waits by powers of their exponential; replayed from a HIP graph) and reports propagator steps/s over the whole batch.
+waits by powers of their exponential; replayed from a HIP graph) and reports
+propagator steps/s over the whole batch.
 
 The hyperfine leg runs the 21-level NV + 14N sweep (512 points, 250,000
 steps each, fluorescence every 2 ns) at n = 441 and at n = 171 through the
@@ -34,7 +35,6 @@ Prints one JSON line (rank 0, N = 1 GPU).
 
 import argparse
 import json
-import math
 import os
 import sys
 import time
@@ -49,7 +49,7 @@ PEAK_HBM_GBS = 8000.0
 # from rocprofv3 FETCH_SIZE / WRITE_SIZE passes scaled by a 1 GiB copy
 # (fetch x2.0, write x1.0); the summary is kept with the profiles.
 MEASURED_TRAFFIC = {
-    ("odmr7-nv-n49", 4096, 99900): (1320.9 * 2.0 + 35238.0 * 1.0) * 1024,
+    ("odmr7-nv-n49", 4096, 99900): (1427.0 * 2.0 + 32101.3 * 1.0) * 1024,
 }
 
 

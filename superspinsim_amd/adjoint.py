@@ -366,7 +366,7 @@ class GradientProblem:
             if series is not None and grad_gen not in (-1, series.gen):
                 series = None
             if series is None and grad_gen < 0:
-                series = WideGradient.build(*point)
+                series = WideGradient.build(*point, derivatives)
         state = GradientState(
             theta=theta, amplitudes=amplitudes, program=program,
             derivatives=bool(derivatives), series=series,

@@ -401,7 +401,8 @@ __attribute__((amdgpu_waves_per_eu(2))) void series_row_kernel(SParams p)
 
 // Sweeps of one instance per wavefront (Halves): fewer instructions per
 // step than two instances on a wavefront, for launches that do not fill the
-// SIMDs (64 points of the 7-level sweep: 344 ns a step in series_row_kernel).
+// SIMDs (64 points of the 7-level sweep: 300 ns a step, 344 in
+// series_row_kernel).
 // With p.store every exponential's input is kept for the adjoint: at J = 2
 // half 0 of the wavefront's 64 doubles per step holds the input of
 // exponential 1 and half 1 that of exponential 0, one coalesced store.

@@ -279,7 +279,8 @@ class SeriesModel:
         """
         F = self.h * self.weight * float(drive_max)
         worst = np.max([[np.abs(c).sum(axis=0).max() for c in cs]
-                        for cs in (chebyshev(es, F) for es in self.sets)], axis=0)
+                        for cs in (chebyshev(es, F)
+                                   for es in self.sets)], axis=0)
         if not np.all(np.isfinite(worst)):
             return None
         for da, db in ORDERS:
@@ -294,7 +295,7 @@ class SeriesModel:
         return [economised(mats, da, db, F) for mats in self.sets]
 
     def tables(self, da, db, F):
-        """Device (layout, table) of the kernel's rows."""
+        """(layout, on the host; device table) of the kernel's rows."""
         key = (da, db, F)
         if self._tables is None or self._tables[0] != key:
             n, size = self.n, self.size
@@ -318,7 +319,7 @@ class SeriesModel:
                     for a in range(db + 1):
                         table[e, own_w + a:own_w + opp.size * (db + 1):
                               db + 1, r] = mats[2 * a + 1][state, opp]
-            self._tables = (key, device_tensor(layout), device_tensor(table))
+            self._tables = (key, layout, device_tensor(table))
         return self._tables[1:]
 
     def lane_tables(self, da, db, F, states):
@@ -406,7 +407,7 @@ class SeriesRun:
             raise ValueError(f"{n_obs} readout rows outside 1.."
                              f"{_lib.MAX_OBS}")
         # a launch that leaves SIMDs idle spreads each instance over a whole
-        # wavefront: 64 points of the 7-level sweep 344 -> 270 ns a step;
+        # wavefront: 64 points of the 7-level sweep 344 -> 300 ns a step;
         # from two wavefronts per SIMD on, two instances to one are quicker
         self.whole = members == 1 and model.one_pair() and \
             weights.shape[0] <= 2 and n_inst <= simd_count()
@@ -416,9 +417,9 @@ class SeriesRun:
         else:
             layout, self.table = model.tables(*plan)
             # the kernel's state index is the caller's
-            self.layout = layout.clone()
-            self.layout[:, 3] = device_tensor(
-                states[model.order].astype(np.int32))
+            layout = layout.copy()
+            layout[:, 3] = states[model.order]
+            self.layout = device_tensor(layout)
             where = np.full(n, -1, dtype=np.int32)
             where[states] = model.pos
             self.d_where = device_tensor(where)

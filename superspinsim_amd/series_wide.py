@@ -179,8 +179,9 @@ class WideModel:
                         2 * self.n))
 
     def layout(self, plan):
-        """Device (blocks, states, columns, table) of the kernel and its
-        columns in LDS; None where the rows don't fit it."""
+        """(blocks, states, columns, table) of the kernel, on the device but
+        for the states, and its columns in LDS; None where the rows don't
+        fit it."""
         if self._layout is None or self._layout[0] != plan:
             self._layout = plan, self._staged(self._arrays(*plan))
         return self._layout[1]
@@ -191,8 +192,11 @@ class WideModel:
 
     @staticmethod
     def _staged(arrays):
-        return None if arrays is None else tuple(
-            device_tensor(a) for a in arrays[:-1]) + arrays[-1:]
+        if arrays is None:
+            return None
+        blocks, states, columns, table, in_lds = arrays
+        return device_tensor(blocks), states, device_tensor(columns), \
+            device_tensor(table), in_lds
 
     def _arrays(self, da, db, F, budget, transpose=False):
         kept = economised(self.mats, da, db, F)
@@ -295,6 +299,13 @@ class WideModel:
         return None
 
 
+def own_states(lane_states, states):
+    """``lane_states`` of a layout with the caller's state indices."""
+    out = lane_states.copy()
+    out[..., 1] = np.asarray(states)[lane_states[..., 1]]
+    return out
+
+
 class WideRun:
     """Staged inputs of one run through ``ssmx_propagate_series_wide``;
     arguments as ``SeriesRun``."""
@@ -313,10 +324,7 @@ class WideRun:
                              f"{_lib.MAX_OBS}")
         self.blocks, lane_states, self.columns, self.table, in_lds = \
             model.layout(plan)
-        # the kernel's state index is the caller's
-        index = device_tensor(np.asarray(states).astype(np.int32))
-        self.states = torch.stack(
-            [lane_states[..., 0], index[lane_states[..., 1].long()]], dim=-1)
+        self.states = device_tensor(own_states(lane_states, states))
         self.d_w, self.d_nodes = device_tensor(weights), device_tensor(nodes)
         self.d_rho0, self.d_waves, self.d_segs = (
             device_tensor(np.ascontiguousarray(rho0, dtype=_f64)), d_waves,

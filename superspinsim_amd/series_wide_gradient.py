@@ -14,7 +14,7 @@ import numpy as np
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 from superspinsim_amd.series import reachable
-from superspinsim_amd.series_wide import WideModel
+from superspinsim_amd.series_wide import WideModel, own_states
 
 _f64 = np.float64
 
@@ -43,8 +43,9 @@ class WideGradient:
 
     @classmethod
     def build(cls, sim, const, program, waves, dconst, rho0, obs, h, tol,
-              adjoint_tol):
-        """Arguments as ``SeriesGradient.build``."""
+              adjoint_tol, derivatives):
+        """Arguments as ``SeriesGradient.build``; ``derivatives`` unset: no
+        backward will follow."""
         varying = [g for g in program if g is not None]
         if len(varying) != 1 or None not in program or sim.rotating or \
                 sim.n <= _lib.MAX_N:
@@ -86,14 +87,13 @@ class WideGradient:
         self.npad = -(-model.n // 16) * 16
         self.d_w, self.d_nodes = (device_tensor(sim.weights),
                                   device_tensor(sim.nodes))
-        index = device_tensor(states.astype(np.int32))
-        self.tables = self._staged(model.layout(plan), index)
-        self.index, self.back = index, None
+        self.tables = self._staged(model.layout(plan), states)
+        self.back = None
         dc = dconst[:, at[0], at[1]]
         self.n_theta = dc.shape[0]
+        if derivatives and self._back() is None:
+            return None
         if self.n_theta:
-            if self._back() is None:
-                return None
             order = np.argsort(model.pos)
             rows = np.ix_(order, order)
             terms, size = 4, 1.0
@@ -106,19 +106,18 @@ class WideGradient:
         return self
 
     @staticmethod
-    def _staged(layout, index):
+    def _staged(layout, states):
         if layout is None:
             return None
-        blocks, states, columns, table, in_lds = layout
-        states = _torch().stack(
-            [states[..., 0], index[states[..., 1].long()]], dim=-1)
-        return blocks, states, columns, table, in_lds
+        blocks, lane_states, columns, table, in_lds = layout
+        return blocks, device_tensor(own_states(lane_states, states)), \
+            columns, table, in_lds
 
     def _back(self):
         """Tables of the transposed matrices (None where they don't fit)."""
         if self.back is None:
             self.back = self._staged(self.model.transposed(self.plan),
-                                     self.index)
+                                     self.states)
         return self.back
 
     def _derivatives(self, a, g, da, terms, drive_max):
@@ -137,6 +136,8 @@ class WideGradient:
         _lib.check(_lib.load().ssmx_series_derivatives(
             n, da.shape[0], terms, self.orders, drive_max, *args, _ptr(out),
             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        # (a backward may run on another stream than the setup)
+        torch.cuda.current_stream().synchronize()
         return out
 
     def store_shape(self, n_inst, steps, J):
@@ -200,7 +201,8 @@ class WideGradient:
         if g_theta is not None and self.n_theta:
             work = torch.empty(
                 (n_inst, lib.ssmx_series_moment_groups(
-                    self.model.n, self.orders), self.n_theta), dtype=torch.float64, device="cuda")
+                    self.model.n, self.orders), self.n_theta),
+                dtype=torch.float64, device="cuda")
             _lib.check(lib.ssmx_series_moments(
                 self.model.n, n_inst, exps, self.orders, self.n_theta,
                 _ptr(store[0]), _ptr(store[1]), _ptr(factors),

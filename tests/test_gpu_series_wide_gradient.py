@@ -11,7 +11,7 @@ from superspinsim_amd import _lib, configs
 from superspinsim_amd.adjoint import GradientProblem
 from superspinsim_amd.propagator import _ptr, device_tensor
 from superspinsim_amd.series_gradient import derivative_matrices
-from superspinsim_amd.series_wide_gradient import WideGradient, row_lists
+from superspinsim_amd.series_wide_gradient import WideGradient
 from superspinsim_amd.sweep import Waveform
 
 pytestmark = pytest.mark.gpu
