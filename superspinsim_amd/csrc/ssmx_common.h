@@ -85,6 +85,21 @@ __device__ __forceinline__ void wave_exchange()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The next entry of a work queue for the whole wavefront: lane 0 takes it
+// from `counter`, every lane gets it.  The convergent barrier in front keeps
+// this test of lane 0 apart from any such test before it: in a loop whose
+// body ends with one (a result stored by lane 0), the compiler otherwise joins
+// the two across the back edge, and the other lanes go round without lane 0
+// for ever, with the entry 0 they start from.
+__device__ __forceinline__ int next_entry(int32_t *counter, int lane)
+{
+    __builtin_amdgcn_wave_barrier();
+    int entry = 0;
+    if (lane == 0)
+        entry = atomicAdd(counter, 1);
+    return __builtin_amdgcn_readfirstlane(entry);
+}
+
 // Padding column of an unused slot s of lane r: r itself for even s, its
 // partner for odd s (the row's own aligned pair); the slot's value is 0.
 __device__ __forceinline__ int pad_column(int s, int lane)

@@ -28,6 +28,7 @@ using ssmx::keep_branch;
 using ssmx::kUnrolledMax;
 using ssmx::kUnrolledTaylor;
 using ssmx::kWave;
+using ssmx::next_entry;
 using ssmx::node_time;
 using ssmx::pad_column;
 using ssmx::fetched_pairs;
@@ -243,23 +244,17 @@ __device__ __forceinline__ void queue_loop(const QParams &p,
             if (step >= k_from)
                 xint = fma(half_h, x_prev + x, xint);
         }
+        // lane o writes readout o
         const double v0 = wave_sum(obs0 * xint);
-        if (lane == 0)
-            p.out[(size_t)inst * d.n_obs] = v0;
-        if (d.n_obs > 1) {
-            const double v1 = wave_sum(obs1 * xint);
-            if (lane == 0)
-                p.out[(size_t)inst * d.n_obs + 1] = v1;
-        }
+        const double v1 = d.n_obs > 1 ? wave_sum(obs1 * xint) : 0.0;
+        if (lane < d.n_obs)
+            p.out[(size_t)inst * d.n_obs + lane] = lane == 0 ? v0 : v1;
     };
 
     // Every pass takes one queue entry; the counter only grows, so every
     // wavefront leaves the loop once the n_inst entries are handed out.
     for (;;) {
-        int q = 0;
-        if (lane == 0)
-            q = atomicAdd(p.counter, 1);
-        q = __builtin_amdgcn_readfirstlane(q);
+        const int q = next_entry(p.counter, lane);
         if (q >= d.n_inst)
             break;
         const int inst = p.order[q];

@@ -607,12 +607,8 @@ __global__ __launch_bounds__(kWave * 8) __attribute__((
     if (entry >= p.n_waves)
         return;
     for (;;) {
-        if (p.counter) {
-            int got = 0;
-            if (lane == 0)
-                got = atomicAdd(p.counter, 1);
-            entry = __builtin_amdgcn_readfirstlane(got);
-        }
+        if (p.counter)
+            entry = ssmx::next_entry(p.counter, lane);
         if (entry >= d.n_inst)
             return;
         const int inst = __builtin_amdgcn_readfirstlane(p.order[entry]);
@@ -681,17 +677,17 @@ __global__ __launch_bounds__(kWave * 8) __attribute__((
                 done += steps;
             }
         }
-        for (int o = 0; o < d.n_obs; ++o) {
-            double v = (o == 0 ? ob0 : ob1) * xint;
+        // (the first half's lanes; lane o writes readout o)
+        double v0 = ob0 * xint, v1 = ob1 * xint;
 #pragma unroll
-            for (int off = 16; off > 0; off >>= 1)
-                v += __shfl_xor(v, off, kWave);
-            if (lane == 0)
-                p.out[(size_t)inst * d.n_obs + o] = v;
+        for (int off = 16; off > 0; off >>= 1) {
+            v0 += __shfl_xor(v0, off, kWave);
+            v1 += __shfl_xor(v1, off, kWave);
         }
-        if (!p.counter) {
+        if (lane < d.n_obs)
+            p.out[(size_t)inst * d.n_obs + lane] = lane == 0 ? v0 : v1;
+        if (!p.counter)
             entry += p.n_waves;
-        }
     }
 }
 
