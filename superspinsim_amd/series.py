@@ -354,7 +354,6 @@ def lane_entries(model, transposed=False):
     own, opp = [], []
     pair = [model.members[0], model.members[1]
             if model.n_sectors > 1 else np.zeros(0, dtype=np.int64)]
-    linked = model.n_sectors > 1 and model.opposite[0] == 1
     for lane in range(64):
         half, row, i = lane // 32, (lane // 16) % 2, lane % 16
         mine, other = pair[row], pair[1 - row]
@@ -365,8 +364,8 @@ def lane_entries(model, transposed=False):
             if i < mine.size and k < mine.size:
                 own.append((s, lane, mine[k], mine[i]) if transposed else
                            (s, lane, mine[i], mine[k]))
-            if not linked:
-                continue
+            # (tables of sectors that the drive leaves apart hold zeros there,
+            # but a parameter's derivative may couple them)
             if transposed and i < mine.size and k < other.size:
                 opp.append((s, lane, other[k], mine[i]))
             if not transposed and i < other.size and k < mine.size:

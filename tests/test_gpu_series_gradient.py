@@ -89,3 +89,38 @@ def test_series_gradient_equals_frechet(gpu, exps, incoherent, points,
     e = np.max(np.abs(a["lambda"] - b["lambda"])) / \
         np.max(np.abs(b["lambda"]))
     assert e <= 1e-12
+
+
+def test_parameter_that_joins_what_the_drive_does_not(gpu):
+    """State 1, which is read, gets theta times state 0: at theta = 0 its
+    derivative is (exp(-a t) - exp(-b t)) / (b - a), summed by the
+    trapezoid rule as the readout.  The truncation of an exponential's
+    derivative, 1e-12 of it, adds up over the exponentials a state has seen:
+    a weighted mean of them, so the bar is 1e-12 with the rounding of 1,000
+    steps (1e-13) below it."""
+    a, b, h, steps = 1e8, 3e8, 20e-12, 1000
+    drive = np.zeros((4, 4))
+    drive[2, 3] = drive[3, 2] = 1e9
+
+    def generators(theta):
+        const = np.diag([-a, -b, -1e8, -2e8])
+        const[1, 0] = theta[0]
+        return np.array([const, drive])
+
+    def waveforms(amps):
+        w = Waveform(2, base=[1.0, 0.0])
+        w.tone(1, 1e-3, 1e9)
+        return [w, w]
+
+    problem = GradientProblem(
+        generators, waveforms, np.eye(4)[0], np.eye(4)[1], 0.0,
+        steps * h * (1 + 1e-9), 10 * h, 10, 2, theta_scale=[1e8])
+    out, state = problem.forward([0.0], [])
+    assert state["by_series"] and state["series"].model.n == 2
+    got = problem.backward(state, np.ones((2, 1)))["theta"].cpu().numpy()
+    t = h * np.arange(steps + 1)
+    s = (np.exp(-a * t) - np.exp(-b * t)) / (b - a)
+    want = 0.5 * h * np.sum(s[:-1] + s[1:])
+    print(f"{np.max(np.abs(got / want - 1)):.1e}", flush=True)
+    assert np.all(out.cpu().numpy() == 0)
+    assert np.max(np.abs(got / want - 1)) <= 1e-12

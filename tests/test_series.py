@@ -152,3 +152,29 @@ def test_derivative_matrices_match_differences():
             want = (up[k] - down[k]) / 2e-5
             assert np.max(np.abs(got[k, i] - want)) <= \
                 1e-9 * np.max(np.abs(want))
+
+
+def test_derivatives_between_sectors_the_drive_does_not_join(monkeypatch):
+    """A parameter may couple two sectors that the drive leaves apart: its
+    dE_0 is h dC to first order, in the lane of the column, at the row's
+    slot of the opposite sector."""
+    from superspinsim_amd import series, series_gradient
+    from superspinsim_amd.sweep import BatchSimulator, Waveform
+    for module in (series, series_gradient):
+        monkeypatch.setattr(module, "device_tensor", np.asarray)
+    const = np.diag([-1e8, -2e8, -3e8, -4e8])
+    drive = np.zeros((4, 4))
+    drive[2, 3] = drive[3, 2] = 1e9
+    w = Waveform(2, base=[1.0, 0.0])
+    w.tone(1, 1e-3, 1e9)
+    sim = BatchSimulator(np.array([const, drive]), layout="plain")
+    active, fixed, program = sim.program([w])
+    dconst = np.zeros((1, 4, 4))
+    dconst[0, 1, 0] = 1.0
+    found = series_gradient.SeriesGradient.build(
+        sim, fixed, program, [w], dconst, np.eye(4)[:1], np.eye(4)[1:2], H,
+        1e-16, 1e-12)
+    assert found is not None and found.n_theta == 1
+    assert found.model.n_sectors == 2
+    scale = H * sim.weights[0].sum()
+    assert np.max(np.abs(found.d_dtable)) == pytest.approx(scale, rel=0.01)
