@@ -14,6 +14,7 @@ fills the coherences between the orbital blocks).
 """
 
 import ctypes
+import math
 
 import numpy as np
 
@@ -170,6 +171,19 @@ def chebyshev(mats, F):
     return out
 
 
+def scaled_powers(j, F):
+    """(k, coefficient of f^k) of the Chebyshev polynomial T_j(f / F).
+
+    Powers of F so small that the coefficient overflows are left out: the
+    order-j part of a series at that F, which it would multiply, has
+    underflowed to zero."""
+    unit = np.zeros(j + 1)
+    unit[j] = 1.0
+    for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(unit)):
+        if c and F ** k and math.isfinite(float(c) / F ** k):
+            yield k, c / F ** k
+
+
 def economised(mats, da, db, F):
     """E_k with the Chebyshev polynomials of the orders that (da, db) leave
     out taken off, so that the kept ones represent the truncated Chebyshev
@@ -177,12 +191,8 @@ def economised(mats, da, db, F):
     kept = [m.copy() for m in mats]
     cheb = chebyshev(mats, F)
     for j in _dropped(len(mats), da, db):
-        unit = np.zeros(j + 1)
-        unit[j] = 1.0
-        for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(unit)):
-            # (an underflown power: its order is zero as well)
-            if c and F ** k:
-                kept[k] -= (c / F ** k) * cheb[j]
+        for k, c in scaled_powers(j, F):
+            kept[k] -= c * cheb[j]
     return kept
 
 

@@ -11,7 +11,8 @@ import numpy as np
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 from superspinsim_amd.series import (
-    SeriesModel, chebyshev, lane_entries, lane_table, reachable)
+    SeriesModel, chebyshev, lane_entries, lane_table, reachable,
+    scaled_powers)
 
 _f64 = np.float64
 
@@ -112,12 +113,9 @@ class SeriesGradient:
             return None
         kept = [m.copy() for m in dmats[:ORDERS]]
         for j in range(ORDERS, count):
-            unit = np.zeros(j + 1)
-            unit[j] = 1.0
-            for k, c in enumerate(np.polynomial.chebyshev.cheb2poly(
-                    unit)[:ORDERS]):
-                if c and F ** k:
-                    kept[k] -= (c / F ** k) * cheb[j]
+            for k, c in scaled_powers(j, F):
+                if k < ORDERS:
+                    kept[k] -= c * cheb[j]
         return kept
 
     def store_shape(self, n_inst, steps, J):

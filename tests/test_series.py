@@ -178,3 +178,22 @@ def test_derivatives_between_sectors_the_drive_does_not_join(monkeypatch):
     assert found.model.n_sectors == 2
     scale = H * sim.weights[0].sum()
     assert np.max(np.abs(found.d_dtable)) == pytest.approx(scale, rel=0.01)
+
+
+@pytest.mark.parametrize("drive_max", [1e-95, 1e-148, 1e-155, 1e-300])
+def test_negligible_drives_leave_finite_matrices(drive_max):
+    """Powers of the largest drive that underflow, or whose inverse
+    overflows: the kept orders are those of the power series."""
+    from superspinsim_amd.series_gradient import SeriesGradient
+    wl = configs.odmr7(1, use_incoherent=True)
+    const, drive = _pair(wl)
+    _, weights, _ = quadratures.scheme(2)
+    model = SeriesModel.build(const, drive, weights, H)
+    plan = model.plan(drive_max, 1e-16)
+    assert plan is not None and plan[:2] == (1, 1)
+    kept, = model.matrices(*plan)
+    for k in range(4):
+        assert np.array_equal(kept[k], model.sets[0][k]), k
+    dmats = np.array(model.sets[0])[:, None]
+    for k, m in enumerate(SeriesGradient._kept(dmats, plan[2], 1e-12)):
+        assert np.array_equal(m[0], model.sets[0][k]), k
