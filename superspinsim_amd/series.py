@@ -160,14 +160,16 @@ def coefficient_matrices(terms, drive, orders, extended=False):
 
 
 def chebyshev(mats, F):
-    """Chebyshev coefficients in f / F of sum_k f^k E_k."""
+    """Chebyshev coefficients in f / F of sum_k f^k E_k (not finite where a
+    power of F is not)."""
     out = [np.zeros_like(mats[0]) for _ in mats]
-    for k, m in enumerate(mats):
-        power = np.zeros(k + 1)
-        power[k] = F ** k
-        for j, c in enumerate(np.polynomial.chebyshev.poly2cheb(power)):
-            if c:
-                out[j] += c * m
+    with np.errstate(over="ignore", invalid="ignore"):
+        for k, m in enumerate(mats):
+            power = np.zeros(k + 1)
+            power[k] = _f64(F) ** k
+            for j, c in enumerate(np.polynomial.chebyshev.poly2cheb(power)):
+                if c:
+                    out[j] += c * m
     return out
 
 

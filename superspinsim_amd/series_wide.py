@@ -156,7 +156,8 @@ class WideModel:
         F = self.h * self.weight * float(drive_max)
         budget = SHARE * tol
         # (drives that the first orders may not do for: all at once)
-        small = (F * self.drive_norm) ** 4 / 24.0 <= tol
+        b = F * self.drive_norm
+        small = b <= 1.0 and b ** 4 / 24.0 <= tol
         for da, db in ORDERS:
             top = TOP[0] if small and (da, db) == ORDERS[0] else TOP[1]
             if len(self.mats) <= top:

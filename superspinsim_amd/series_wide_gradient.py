@@ -73,6 +73,8 @@ class WideGradient:
         # where the quarter of the fourth that Chebyshev polynomials leave is
         # below the tolerance (a quarter less of the moments' work)
         b = plan[2] * float(np.abs(g).sum(axis=0).max())
+        if not b <= 1.0:
+            return None
         spread = math.exp(b + 2.0 * norm)
         if b ** 3 / 24.0 * spread <= adjoint_tol:
             orders = 3

@@ -197,3 +197,26 @@ def test_negligible_drives_leave_finite_matrices(drive_max):
     dmats = np.array(model.sets[0])[:, None]
     for k, m in enumerate(SeriesGradient._kept(dmats, plan[2], 1e-12)):
         assert np.array_equal(m[0], model.sets[0][k]), k
+
+
+@pytest.mark.parametrize("drive_max", [1e60, 1e300, np.inf])
+def test_drives_beyond_the_number_range_are_refused(drive_max):
+    """No plan (the Taylor path then refuses the run by its own error)."""
+    from superspinsim_amd.series_wide import WideModel
+    from superspinsim_amd.sweep import BatchSimulator, Waveform
+    wl = configs.odmr7(1, use_incoherent=True)
+    const, drive = _pair(wl)
+    _, weights, _ = quadratures.scheme(2)
+    model = SeriesModel.build(const, drive, weights, H)
+    assert model.plan(drive_max, 1e-16) is None
+    pairs = np.kron(np.eye(35), [[0.0, 1e9], [1e9, 0.0]])
+    wide = WideModel.build(np.diag(np.full(70, -1e8)), pairs, weights, H)
+    assert wide.plan(drive_max, 1e-16) is None
+    w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, wl.excitation])
+    w.tone(1, drive_max, 2.8e9)
+    sim = BatchSimulator(wl.generators, 2, 20)
+    point = sim.program([w])
+    assert sim.series_plan([w], *point[1:], 4e-10) is None
+    if np.isfinite(drive_max):
+        with pytest.raises(ValueError, match="no Taylor plan"):
+            sim.taylor_plan([w], *point, 4e-10)
