@@ -10,9 +10,12 @@ workgroup) and the Taylor plan of a ``ProtocolBatch``:
 * wavefronts per workgroup 1, 2, 4 or 8 (generator values are staged once
   per workgroup in LDS; more wavefronts share one copy).
 
+A batch that runs as series in the drive (``ProtocolBatch.series``) has no
+Taylor plan to choose: only the wavefronts per workgroup are tried.
+
 Each candidate runs on a trial copy of the batch: its longest instances (one
 grid's worth), truncated to ``trial_steps`` steps, timed with HIP events on
-the launch stream.  Results are cached per device and problem shape in
+the launch stream.  Results are cached per device, path and problem shape in
 ``$XDG_CACHE_HOME/superspinsim_amd/autotune.json`` (default ``~/.cache``).
 """
 
@@ -73,11 +76,18 @@ def plan_candidates(batch, samples):
 
 
 def problem_key(batch):
-    torch = _torch()
-    prop = batch.prop
-    name = torch.cuda.get_device_properties(0).name
-    return "|".join(str(v) for v in (
-        name, prop.n, prop.ell.slots, prop.K, prop.J, prop.S, prop.ell.nnz,
+    """Cache key: the device, the path (a choice made for one kernel says
+    nothing about the other) and the problem's shape."""
+    name = _torch().cuda.get_device_properties(0).name
+    if batch.series is not None:
+        model, plan = batch.series.model, batch.series.plan
+        J, S = batch.sim.weights.shape
+        shape = ("series", model.n, plan[0], plan[1], len(model.sets), J, S)
+    else:
+        prop = batch.prop
+        shape = ("taylor", prop.n, prop.ell.slots, prop.K, prop.J, prop.S,
+                 prop.ell.nnz)
+    return "|".join(str(v) for v in (name,) + shape + (
         batch.tolerance, batch.n_obs))
 
 
@@ -115,6 +125,8 @@ def tune(batch, trial_steps=20000, repeats=2, use_cache=True, verbose=False):
     trial_steps_arr = np.where(mask, trial_steps_arr, 0)
     batch.d_steps.copy_(torch.from_numpy(trial_steps_arr))
     batch.d_read_from.copy_(torch.from_numpy(trial_read))
+    if batch.series is not None:
+        batch.series.cut(trial_steps_arr)
     results = []
     try:
         for m, s in plans:
@@ -142,6 +154,8 @@ def tune(batch, trial_steps=20000, repeats=2, use_cache=True, verbose=False):
         batch.n_waves, batch.waves_per_block = n_waves, wpb
         batch.taylor, batch.substeps = m, s
         torch.cuda.synchronize()
+        if batch.series is not None:
+            batch.series.cut()
     best = min(results, key=lambda r: r["ms"])
     choice = dict(waves_per_block=best["waves_per_block"],
                   taylor=best["taylor"], substeps=best["substeps"],

@@ -160,15 +160,36 @@ class ProtocolRuns:
         begin = np.zeros(n_inst + 1, dtype=np.int32)
         np.cumsum(np.bincount(inst, minlength=n_inst), out=begin[1:])
         self.d_begin = device_tensor(begin)
-        raw = rec.tobytes() or bytes(RUN_DTYPE.itemsize)
-        self.d_runs = _torch().from_numpy(
-            np.frombuffer(raw, dtype=np.uint8).copy()).to("cuda")
-        # a free run costs about as much as twenty steps per power
+        self._records, self._inst = rec, inst
+        self._d_whole = self.d_runs = self._staged(rec)
+        # in steps: a free run's powers as one figure whatever its length, a
+        # driven run's table on top of its steps
         cost = np.where(free, 40, count + 20)
         self.cost = np.bincount(inst, weights=cost, minlength=n_inst)
         self.model, self.plan, self.h = model, plan, h
         self.gen = program.index(drive) if drive is not None else 0
         return self
+
+    @staticmethod
+    def _staged(records):
+        raw = records.tobytes() or bytes(RUN_DTYPE.itemsize)
+        return _torch().from_numpy(
+            np.frombuffer(raw, dtype=np.uint8).copy()).to("cuda")
+
+    @staticmethod
+    def cut_records(records, inst, steps):
+        """Run records that end after the first ``steps[i]`` steps of
+        instance i; runs behind them stay with no steps."""
+        out = records.copy()
+        out["count"] = np.clip(np.asarray(steps)[inst] - out["first"], 0,
+                               out["count"])
+        return out
+
+    def cut(self, steps=None):
+        """Launch only the first ``steps[i]`` steps of instance i from here
+        on; None: all of them again."""
+        self.d_runs = self._d_whole if steps is None else self._staged(
+            self.cut_records(self._records, self._inst, steps))
 
     @staticmethod
     def _layout(segs, base, drive, switched, nodes, steps, read_from, h):

@@ -1,0 +1,65 @@
+"""Protocol batches by either path (GPU): the series in the drive (a batch
+prepared without a Taylor plan) and the Taylor queue kernel (with one)."""
+
+import numpy as np
+import pytest
+
+from superspinsim_amd import autotune, configs
+
+pytestmark = pytest.mark.gpu
+
+H = 20e-12
+PATHS = [None, 11]
+
+
+@pytest.fixture(scope="module")
+def wl(gpu):
+    return configs.pulsed7(count=24, seed=5, t_p_range=(2e-9, 20e-9),
+                           tau_range=(10e-9, 100e-9), readout=50e-9)
+
+
+def _batch(wl, taylor, steps=None, **kw):
+    b = wl.batch().prepare(
+        wl.waves, wl.rho0, H, wl.steps if steps is None else steps,
+        wl.read_from, wl.obs, taylor=taylor, **kw)
+    assert (b.series is None) == (taylor is not None)
+    return b
+
+
+@pytest.mark.parametrize("taylor", PATHS)
+def test_tuning_trials_are_cut_and_paths_kept_apart(wl, taylor, tmp_path,
+                                                    monkeypatch):
+    monkeypatch.setenv("XDG_CACHE_HOME", str(tmp_path))
+    b = _batch(wl, taylor)
+    whole = b.run().cpu().numpy().copy()
+    # what the trials launch: 2,000 steps of every protocol
+    trials = []
+    launch = b.launch
+    monkeypatch.setattr(b, "launch", lambda *a, **k: (
+        launch(*a, **k), trials.append(b.out.cpu().numpy().copy()))[0])
+    choice = autotune.tune(b, trial_steps=2000, repeats=1)
+    assert not choice["cached"] and choice["trial_steps"] == 2000
+    plans = {(t["taylor"], t["substeps"]) for t in choice["trials"]}
+    assert (len(plans) == 1) == (taylor is None)
+    cut = _batch(wl, taylor, np.minimum(wl.steps, 2000)).run().cpu().numpy()
+    assert 0 < np.count_nonzero(cut) < cut.size
+    # (the Taylor trials have other degrees: 1e-10 as below)
+    bar = 0.0 if taylor is None else 1e-10 * np.max(cut)
+    assert trials and all(np.max(np.abs(t - cut)) <= bar for t in trials)
+    got = b.run().cpu().numpy()
+    assert np.max(np.abs(got - whole) / np.abs(whole)) < 1e-10
+    # the choice holds for this path only
+    assert autotune.tune(b, trial_steps=2000, repeats=1)["cached"]
+    other = _batch(wl, 11 if taylor is None else None)
+    assert not autotune.tune(other, trial_steps=2000, repeats=1)["cached"]
+
+
+def test_cut_series_batch_equals_fewer_steps(wl):
+    b = _batch(wl, None)
+    whole = b.run().cpu().numpy().copy()
+    steps = wl.steps - np.arange(len(wl.steps)) * 97
+    b.series.cut(steps)
+    got = b.run().cpu().numpy().copy()
+    assert np.array_equal(got, _batch(wl, None, steps).run().cpu().numpy())
+    b.series.cut()
+    assert np.array_equal(b.run().cpu().numpy(), whole)

@@ -9,7 +9,8 @@ import numpy as np
 import pytest
 
 from superspinsim_amd import configs, quadratures
-from superspinsim_amd.protocol_runs import ProtocolRuns, _padded, _times
+from superspinsim_amd.protocol_runs import (
+    RUN_DTYPE, ProtocolRuns, _padded, _times)
 from superspinsim_amd.sweep import Waveform
 
 H = 20e-12
@@ -80,3 +81,27 @@ def test_powers_equal_steps():
     assert np.max(np.abs(read @ x0 - xint)) < \
         256 * 1.2e-16 * np.abs(xint).max()
     assert np.max(np.abs(step @ step - np.eye(n) - powers[1][0])) < 1e-15
+
+
+def test_cut_runs_end_after_the_steps_asked_for():
+    rng = np.random.default_rng(5)
+    waves = _waves(rng, 9)
+    nodes, _, _ = quadratures.scheme(2)
+    steps = rng.integers(20, 70, 9)
+    segs = {g: _padded(waves, g) for g in (1, 4)}
+    base = np.array([w.base for w in waves])
+    first, count, read, _, _, inst = ProtocolRuns._layout(
+        segs, base, 1, [4], nodes, steps, np.zeros(9, np.int64), H)
+    rec = np.zeros(first.size, dtype=RUN_DTYPE)
+    rec["first"], rec["count"], rec["read"] = first, count, read
+    some = np.minimum(steps, rng.integers(0, 60, 9))
+    some[4] = 0
+    cut = ProtocolRuns.cut_records(rec, inst, some)
+    assert np.array_equal(np.bincount(inst, cut["count"], 9), some)
+    for k in range(9):
+        end = 0
+        for r in cut[(inst == k) & (cut["count"] > 0)]:
+            assert r["first"] == end
+            end += r["count"]
+    assert np.array_equal(rec["count"], count)
+    assert np.array_equal(cut[["first", "read"]], rec[["first", "read"]])
