@@ -309,7 +309,9 @@ class SeriesModel:
     def tables(self, da, db, F):
         """(layout, on the host; device table) of the kernel's rows."""
         key = (da, db, F)
-        if self._tables is None or self._tables[0] != key:
+        # (another thread may keep its own drive's in between)
+        kept = self._tables
+        if kept is None or kept[0] != key:
             n, size = self.n, self.size
             layout = np.zeros((n, 4), dtype=np.int32)
             own_w, opp_w = size * (da + 1), size * (db + 1)
@@ -331,8 +333,8 @@ class SeriesModel:
                     for a in range(db + 1):
                         table[e, own_w + a:own_w + opp.size * (db + 1):
                               db + 1, r] = mats[2 * a + 1][state, opp]
-            self._tables = (key, layout, device_tensor(table))
-        return self._tables[1:]
+            self._tables = kept = (key, layout, device_tensor(table))
+        return kept[1:]
 
     def lane_tables(self, da, db, F, states):
         """Device (state per lane, table) of one instance per wavefront;

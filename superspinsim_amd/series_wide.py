@@ -160,10 +160,13 @@ class WideModel:
         small = b <= 1.0 and b ** 4 / 24.0 <= tol
         for da, db in ORDERS:
             top = TOP[0] if small and (da, db) == ORDERS[0] else TOP[1]
-            if len(self.mats) <= top:
-                self.mats = wide_coefficients(*self._point, top)
-            worst = [np.abs(c).sum(axis=0).max()
-                     for c in chebyshev(self.mats, F)]
+            mats = self.mats
+            if len(mats) <= top:
+                mats = wide_coefficients(*self._point, top)
+                # (a thread with a larger drive may have kept more)
+                if len(mats) > len(self.mats):
+                    self.mats = mats
+            worst = [np.abs(c).sum(axis=0).max() for c in chebyshev(mats, F)]
             if not np.all(np.isfinite(worst)):
                 return None
             if 8.0 * (budget + worst[-1] + sum(
@@ -183,9 +186,11 @@ class WideModel:
         """(blocks, states, columns, table) of the kernel, on the device but
         for the states, and its columns in LDS; None where the rows don't
         fit it."""
-        if self._layout is None or self._layout[0] != plan:
-            self._layout = plan, self._staged(self._arrays(*plan))
-        return self._layout[1]
+        # (another thread may keep its own drive's in between)
+        kept = self._layout
+        if kept is None or kept[0] != plan:
+            self._layout = kept = plan, self._staged(self._arrays(*plan))
+        return kept[1]
 
     def transposed(self, plan):
         """``layout`` of the transposed matrices (not kept)."""

@@ -220,3 +220,46 @@ def test_drives_beyond_the_number_range_are_refused(drive_max):
     if np.isfinite(drive_max):
         with pytest.raises(ValueError, match="no Taylor plan"):
             sim.taylor_plan([w], *point, 4e-10)
+
+
+def test_tables_of_two_drives_at_once(monkeypatch):
+    """Another thread's drive between this one's tables being kept and
+    returned: each gets its own."""
+    from superspinsim_amd import series, series_wide
+    monkeypatch.setattr(series, "device_tensor", np.asarray)
+    monkeypatch.setattr(series_wide, "device_tensor", np.asarray)
+    _, weights, _ = quadratures.scheme(2)
+    wl = configs.odmr7(1, use_incoherent=True)
+    pairs = np.kron(np.eye(35), [[0.0, 1e9], [1e9, 0.0]])
+
+    def racing(base, kept, call):
+        class Racing(base):
+            def __setattr__(self, name, value):
+                super().__setattr__(name, value)
+                if name == kept and getattr(self, "other", None):
+                    other, self.other = self.other, None
+                    call(self, other)
+        return Racing
+
+    narrow = racing(SeriesModel, "_tables", lambda m, p: m.tables(*p))
+    model = narrow.build(*_pair(wl), weights, H)
+    plans = [model.plan(configs.drive_amplitude(r), 1e-16)
+             for r in (5e5, 3e6)]
+    model.other = plans[1]
+    got = model.tables(*plans[0])
+    assert model.other is None
+    assert np.array_equal(got[1], SeriesModel.build(
+        *_pair(wl), weights, H).tables(*plans[0])[1])
+
+    wide = racing(series_wide.WideModel, "_layout",
+                  lambda m, p: m.layout(p))
+    args = np.diag(np.full(70, -1e8)), pairs, weights, H
+    plans = [series_wide.WideModel.build(*args).plan(d, 1e-16)
+             for d in (1e-7, 1e-5)]
+    model = wide.build(*args)
+    model.plan(1e-5, 1e-16)
+    model._layout, model.other = None, plans[1]
+    got = model.layout(plans[0])
+    assert model.other is None
+    assert np.array_equal(got[3], model._staged(
+        model._arrays(*plans[0]))[3])
