@@ -34,6 +34,15 @@ def device_tensor(array, dtype=None):
     return t.to("cuda")
 
 
+def record_use(*tensors):
+    """The current stream uses ``tensors`` that another one may have staged
+    and whose owner may drop them: their memory is not handed out again
+    before the work enqueued so far is done."""
+    stream = _torch().cuda.current_stream()
+    for t in tensors:
+        t.record_stream(stream)
+
+
 def _ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 

@@ -19,7 +19,8 @@ import math
 import numpy as np
 
 from superspinsim_amd import _lib
-from superspinsim_amd.propagator import _ptr, _torch, device_tensor
+from superspinsim_amd.propagator import (
+    _ptr, _torch, device_tensor, record_use)
 
 _f64 = np.float64
 
@@ -473,6 +474,7 @@ class SeriesRun:
             _ptr(self.table), _ptr(self.d_w), _ptr(self.d_nodes),
             _ptr(self.d_waves), _ptr(self.d_segs), _ptr(self.d_rho0),
             _ptr(self.d_obs), _ptr(self.out), ctypes.c_void_p(stream)))
+        record_use(self.table)          # shared by the model's runs
         return self.out
 
     def result(self):

@@ -14,7 +14,8 @@ import math
 import numpy as np
 
 from superspinsim_amd import _lib
-from superspinsim_amd.propagator import _ptr, _torch, device_tensor
+from superspinsim_amd.propagator import (
+    _ptr, _torch, device_tensor, record_use)
 from superspinsim_amd.series import (
     ORDERS, _dropped, chebyshev, economised, split_sectors)
 
@@ -358,6 +359,8 @@ class WideRun:
             _ptr(self.d_waves), _ptr(self.d_segs), _ptr(self.d_rho0),
             _ptr(self.d_obs), _ptr(self.out), None, None, ctypes.c_void_p(
                 _torch().cuda.current_stream().cuda_stream)))
+        # (shared by the model's runs)
+        record_use(self.blocks, self.columns, self.table)
         return self.out
 
     def result(self):

@@ -252,3 +252,33 @@ def test_chunked_series_equals_run(gpu, name, exps, read):
     # node times counted from a chunk's start move by rounding: 4e-24 s in
     # phases of 2e10 rad/s, far below the state's own rounding
     assert err <= SAME
+
+
+@pytest.mark.parametrize("name,points", [("nv7", 2100), ("nv21c", 3)])
+def test_tables_outlive_a_launch_on_another_stream(gpu, name, points):
+    """Tables staged on one stream, used on another, and dropped by the
+    model for the next drive's before that launch has started."""
+    import torch
+    wl = configs.odmr21(1, use_incoherent=True) if name == "nv21c" else \
+        _model(name)
+    sim = BatchSimulator(wl.generators, 2, 10)
+    args = (wl.rho0, 0.0, 3 * 2e-10 * (1 + 1e-9), 2e-10, wl.obs)
+    first, next_ = (_waves(wl, points, rabi) for rabi in (3e5, 4e5))
+    want = sim.run(first, *args).cpu().numpy()
+    assert "series" in sim.last_plan
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        run = sim.prepare(first, *args)
+        torch.cuda._sleep(50_000_000)
+        run.launch()
+    sizes = [t.numel() for t in vars(run).values()
+             if isinstance(t, torch.Tensor) and t.dtype == torch.float64]
+    rest = [t for k, t in vars(run).items()
+            if k not in ("blocks", "columns", "table")]
+    out = run.out
+    del run
+    sim.run(next_, *args)           # the model keeps these tables instead
+    fill = [torch.full((n,), np.nan, dtype=torch.float64, device="cuda")
+            for n in sizes for _ in range(4)]
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), want), (len(rest), len(fill))
