@@ -525,7 +525,7 @@ class BatchSimulator:
                 tolerance=self.tolerance, layout=self.layout,
                 pack=self.pack)
         sub = self._reduced_cache[key]
-        sub.tolerance, sub.pack = self.tolerance, self.pack
+        sub.tolerance, sub.pack, sub.F = self.tolerance, self.pack, self.F
         return sub
 
     def involved(self, active, rho0, obs=None):

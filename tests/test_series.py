@@ -263,3 +263,12 @@ def test_tables_of_two_drives_at_once(monkeypatch):
     assert model.other is None
     assert np.array_equal(got[3], model._staged(
         model._arrays(*plans[0]))[3])
+
+
+def test_reduced_simulator_follows_the_fine_divisions():
+    from superspinsim_amd.sweep import BatchSimulator
+    sim = BatchSimulator(configs.odmr7(1).generators, 2, 20)
+    states = np.arange(5)
+    assert sim._reduced(states).F == 20
+    sim.F = 40
+    assert sim._reduced(states).F == 40
