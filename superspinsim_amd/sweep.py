@@ -32,6 +32,10 @@ from superspinsim_amd.series_wide import WideModel, WideRun
 _f64 = np.float64
 
 
+#: series models (constants and step) a simulator keeps, the last used ones:
+#: up to 2 MB each on the host and 0.4 MB on the device at 192 states
+MAX_MODELS = 64
+
 _NO_ROWS = np.zeros((0, 5), dtype=_f64)
 _NO_PARAMS = np.zeros(0, dtype=np.int64)
 _NO_DPARAMS = np.zeros(0, dtype=_f64)
@@ -551,14 +555,19 @@ class BatchSimulator:
             return None
         h = time_step / self.F
         key = (tuple(varying), tuple(sorted(const.items())), h)
-        if key not in self._series_cache:
+        cache = self._series_cache
+        try:
+            model = cache.pop(key)
+        except KeyError:
             drive = self.gens[varying[0]] if varying else \
                 np.zeros((self.n, self.n))
             build = SeriesModel.build if self.n <= _lib.MAX_N else \
                 WideModel.build
-            self._series_cache[key] = build(
-                self.folded(const), drive, self.weights, h)
-        model = self._series_cache[key]
+            model = build(self.folded(const), drive, self.weights, h)
+        # the last used at the end
+        cache[key] = model
+        for old in list(cache)[:-MAX_MODELS]:
+            cache.pop(old, None)
         if model is None:
             return None
         drive_max = max(w.abs_max()[varying[0]] for w in waves) \

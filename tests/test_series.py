@@ -272,3 +272,23 @@ def test_reduced_simulator_follows_the_fine_divisions():
     assert sim._reduced(states).F == 20
     sim.F = 40
     assert sim._reduced(states).F == 40
+
+
+def test_simulator_keeps_the_last_models():
+    from superspinsim_amd import sweep
+    wl = configs.odmr3(1)
+    sim = sweep.BatchSimulator(wl.generators, 2, 20)
+
+    def plan(k):
+        w = sweep.Waveform(5, base=[1.0, 0.0, 0.0, 0.0, 1e-3 * (k + 1)])
+        w.tone(1, wl.b1, 2.8e9)
+        return sim.series_plan([w], *sim.program([w])[1:], 1e-9)[0]
+
+    first = plan(0)
+    second = plan(1)
+    for k in range(2, sweep.MAX_MODELS):
+        plan(k)
+    assert plan(0) is first             # used again: stays
+    plan(sweep.MAX_MODELS)
+    assert len(sim._series_cache) == sweep.MAX_MODELS
+    assert plan(0) is first and plan(1) is not second
