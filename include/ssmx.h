@@ -341,7 +341,7 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
 
 /*
  * ssmx_propagate_series for models of more rows than a wavefront (at most
- * 256), one workgroup of n_blocks (at most 12) wavefronts per instance;
+ * 192), one workgroup of n_blocks (at most 12) wavefronts per instance;
  * n_exp = n_node = 2, (da, db) = (1, 1), (2, 1) or (2, 2); na the sum over the
  * wavefronts of (da + db - 2) slots + 4 max(0, slots - 7), the KB of LDS for
  * the coefficients that registers don't hold (at most 150); members, nb,
@@ -354,9 +354,9 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
  * coefficient 0). Lanes below 32 keep the pair's first row, the others the
  * second.
  * blocks   ssmx_series_block [n_blocks]
- * states   int32 [n_blocks][64][2]: the lane's row (0..255, -1 idle) and its
+ * states   int32 [n_blocks][64][2]: the lane's row (0..191, -1 idle) and its
  *          state index (idle lanes 0)
- * columns  int32 from blocks[b].columns: [2 slots][64] rows (0..255) of the
+ * columns  int32 from blocks[b].columns: [2 slots][64] rows (0..191) of the
  *          own-sector columns, then of the opposite ones
  * table    double from blocks[b].table, r = min(slots, 7):
  *          [2 r][4][64], entry 2 o + i of the first r own-sector columns, then

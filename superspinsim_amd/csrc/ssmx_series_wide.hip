@@ -44,7 +44,7 @@ using ssmx::quad_perm;
 using ssmx::set_error;
 
 constexpr int kMaxWaves = 12;
-constexpr int kMaxRows = 256;
+constexpr int kMaxRows = 16 * kMaxWaves;    // eight pairs a wavefront
 // LDS for the coefficients that registers don't hold, and for one column of them
 constexpr int kHighBytes = 150 * 1024;
 constexpr int kColumnBytes = kWave * sizeof(double2);

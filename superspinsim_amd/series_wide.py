@@ -1,4 +1,4 @@
-"""The series in the drive for models of 65 to 256 states
+"""The series in the drive for models of 65 to 192 states
 (``ssmx_propagate_series_wide``): matrices, layout and launch.
 
 The E_k of a model this size are sparse where its couplings are nearly
@@ -21,8 +21,11 @@ from superspinsim_amd.series import (
 
 _f64 = np.float64
 
-#: the kernel's limits: rows, wavefronts, columns per lane
-MAX_ROWS, MAX_WAVES, MIN_SLOTS, MAX_SLOTS = 256, 12, 4, 8
+#: the kernel's limits: rows (eight pairs in each wavefront), wavefronts,
+#: columns per lane
+MAX_ROWS, MAX_WAVES, MIN_SLOTS, MAX_SLOTS = 192, 12, 4, 8
+#: rows of a model beyond which none is built (up to here it has no plan)
+MAX_STATES = 256
 #: highest 1-norm of h w C (beyond, the E_k fill in past the kernel's limits)
 MAX_NORM = 1.0
 #: highest order computed for the first of ORDERS, and for the others
@@ -117,8 +120,8 @@ def pair_rows(pattern, sector):
 
 
 class WideModel:
-    """E_k of one (constant, drive) pair of 65..256 states at one step size;
-    ``build`` returns None where the kernel does not apply."""
+    """E_k of one (constant, drive) pair of 65..192 states at one step size;
+    ``build`` or ``plan`` returns None where the kernel does not apply."""
 
     def __init__(self):
         self._layout = None         # the last drive's
@@ -127,7 +130,7 @@ class WideModel:
     def build(cls, const, drive, weights, h):
         n = const.shape[0]
         sums = weights.sum(axis=1)
-        if not _lib.MAX_N < n <= MAX_ROWS or weights.shape != (2, 2) or \
+        if not _lib.MAX_N < n <= MAX_STATES or weights.shape != (2, 2) or \
                 not np.allclose(sums[0], sums[1], rtol=1e-15, atol=1e-16):
             return None
         terms = [(const, h * float(sums[0]))]
@@ -154,6 +157,8 @@ class WideModel:
     def plan(self, drive_max, tol):
         """(da, db, F, budget) for drives |c(t)| <= ``drive_max``, or None;
         the bound of ``SeriesModel.plan`` with the left-out entries added."""
+        if self.n > MAX_ROWS:
+            return None
         F = self.h * self.weight * float(drive_max)
         budget = SHARE * tol
         # (drives that the first orders may not do for: all at once)

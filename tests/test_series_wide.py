@@ -180,3 +180,9 @@ def test_wide_series_equals_taylor(gpu, n, block, spread, norm, points, fine,
     err = np.max(np.abs(got - want)) / np.max(np.abs(want))
     print(f"  {err:.1e}")
     assert err <= 1e-12
+
+
+def test_models_beyond_the_kernels_rows_cost_no_matrices():
+    _, weights, _ = quadratures.scheme(2)
+    model = WideModel.build(*_model(193, 8), weights, H)
+    assert model.plan(1e7, 1e-16) is None and len(model.mats) == 0
