@@ -485,6 +485,8 @@ extern "C" int ssmx_propagate_series_wide(
         return set_error(SSMX_EINVAL, "null required pointer");
     WSParams p{};
     p.d = *desc;
+    if (desc->flags & SSMX_READ_FULL)
+        p.d.n_obs = 0;          // no readout rows to stage
     p.blocks = blocks;
     p.states = states;
     p.columns = columns;
@@ -515,7 +517,7 @@ extern "C" int ssmx_series_wide_adjoint(
     const int rc = check(*desc, n_blocks, "wide series adjoint");
     if (rc != SSMX_OK)
         return rc;
-    if (desc->n_out < 1 || desc->n_obs < 1)
+    if (desc->n_out < 1 || desc->n_obs < 1 || desc->n_obs > SSMX_MAX_OBS)
         return set_error(SSMX_EINVAL, "wide series adjoint: n_out=%d, "
                          "n_obs=%d", desc->n_out, desc->n_obs);
     if (!blocks || !states || !columns || !table || !factors || !obs ||

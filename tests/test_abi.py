@@ -245,3 +245,19 @@ def test_chunk_null_pointers_are_rejected(lib):
     d = _cdesc()
     assert lib.ssmx_chunk_combine(ctypes.byref(d), *([None] * 5)) == -1
     assert b"null" in lib.ssmx_last_error()
+
+
+@pytest.mark.parametrize("flags", [0, _lib.SSMX_READ_FULL,
+                                   _lib.SSMX_READ_INTEGRAL])
+@pytest.mark.parametrize("bad", [dict(n_obs=3), dict(rows=193), dict(da=3),
+                                 dict(n_exp=1), dict(na=151), dict(h=0.0)])
+def test_invalid_wide_adjoint_descriptor_is_rejected(lib, flags, bad):
+    base = dict(n=200, rows=100, n_inst=1, members=1, n_exp=2, n_node=2,
+                fine=1, n_out=1, n_obs=1, flags=flags, gen=1, wave_group=1,
+                na=0, da=1, db=1, h=1e-11, t0=0.0, dt=1e-11)
+    base.update(bad)
+    d = _lib.SeriesDesc(**base)
+    dummy = ctypes.c_void_p(8)
+    assert lib.ssmx_series_wide_adjoint(
+        ctypes.byref(d), dummy, 3, *([dummy] * 9)) == -1
+    assert lib.ssmx_last_error().decode()

@@ -186,3 +186,14 @@ def test_models_beyond_the_kernels_rows_cost_no_matrices():
     _, weights, _ = quadratures.scheme(2)
     model = WideModel.build(*_model(193, 8), weights, H)
     assert model.plan(1e7, 1e-16) is None and len(model.mats) == 0
+
+
+@pytest.mark.gpu
+def test_full_states_whatever_the_count_of_readout_rows(gpu):
+    """READ_FULL has no readout rows: the descriptor's count is not used."""
+    wl = configs.odmr21(1, use_incoherent=True)
+    sim = BatchSimulator(wl.generators, 2, 10)
+    run = sim.prepare(wl.waveforms(), wl.rho0, 0.0, 1e-9, 2e-10, read="full")
+    want = run.launch().cpu().numpy().copy()
+    run.desc.n_obs = 40
+    assert np.array_equal(run.launch().cpu().numpy(), want)
