@@ -453,22 +453,29 @@ class GradientProblem:
     # ------------------------------------------------------------------
     def forward(self, theta, amplitudes, state=None):
         """(F (n_inst, n_obs) device tensor, state for ``backward``)."""
-        torch = _torch()
         if state is None:
             state = self.setup(theta, amplitudes)
         n_inst = state["n_inst"]
         rho0 = np.atleast_2d(self.rho0)
         if rho0.shape[0] == 1 and n_inst > 1:
             rho0 = np.repeat(rho0, n_inst, axis=0)
+        return self._forward(state, rho0)
+
+    def _forward(self, state, rho0):
+        torch = _torch()
+        n_inst = state["n_inst"]
         total = self.n_out * self.F
         P = (total + self.K - 1) // self.K
         series = state.get("series")
-        if series is not None and rho0.shape[0] == n_inst and total > 0:
+        # (rho0 and obs may be others than at setup)
+        if series is not None and rho0.shape[0] == n_inst and total > 0 and \
+                series.reach.covers(self.obs, rho0):
             store = self._series_store(state, series, total)
             if store is not False:
                 out = series.forward(self, state, rho0, store)
                 state.update(ckpt=store, inputs=store, n_ckpt=P,
-                             stored=store is not None, by_series=True)
+                             stored=store is not None, by_series=True,
+                             rho0=rho0.copy())
                 return out, state
         state["by_series"] = False
         prop = state["prop"]
@@ -550,6 +557,10 @@ class GradientProblem:
                              "use forward(theta, amplitudes) for gradients")
         torch = _torch()
         n_inst = state["n_inst"]
+        if state.get("by_series") and \
+                not state["series"].reach.covers(self.obs):
+            # rows that the stored run does not serve, set since
+            self._forward(state, state["rho0"])
         seed = torch.as_tensor(seed, dtype=torch.float64).to("cuda")
         seed = seed.reshape(n_inst, self.obs.shape[0]).contiguous()
         n_theta = int(state["n_theta"])

@@ -60,6 +60,29 @@ def reachable(pattern, rho0, obs=None):
     return np.flatnonzero(keep)
 
 
+class Reach:
+    """States that gradients involve: what the run reaches from ``rho0`` and
+    what the readout ``obs`` depends on (a parameter may join one to the
+    other)."""
+
+    def __init__(self, pattern, rho0, obs):
+        n = pattern.shape[0]
+        self.ahead, self.behind = np.zeros((2, n), dtype=bool)
+        self.ahead[reachable(pattern, rho0)] = True
+        self.behind[reachable(pattern.T, obs)] = True
+        self.states = np.flatnonzero(self.ahead | self.behind)
+
+    def covers(self, obs, rho0=None):
+        """Whether other rows (and initial states) involve no further
+        ones."""
+        def within(rows, mask):
+            return rows.shape[-1] == mask.size and \
+                not np.any(rows[:, ~mask] != 0)
+
+        return within(obs, self.behind) and \
+            (rho0 is None or within(rho0, self.ahead))
+
+
 def split_sectors(const, drive):
     """(sector of each state, opposite sector of each sector) or None.
 

@@ -11,8 +11,7 @@ import numpy as np
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 from superspinsim_amd.series import (
-    SeriesModel, chebyshev, lane_entries, lane_table, reachable,
-    scaled_powers)
+    Reach, SeriesModel, chebyshev, lane_entries, lane_table, scaled_powers)
 
 _f64 = np.float64
 
@@ -59,11 +58,8 @@ class SeriesGradient:
             return None
         folded, drive = sim.folded(const), sim.gens[varying[0]]
         pattern = (folded != 0) | (drive != 0)
-        # a gradient needs the states the run reaches and those the readout
-        # depends on: a parameter may join one to the other
-        forward = reachable(pattern, rho0)
-        back = reachable(pattern.T, np.atleast_2d(obs))
-        states = np.union1d(forward, back)
+        reach = Reach(pattern, rho0, np.atleast_2d(obs))
+        states = reach.states
         if states.size == 0 or states.size > _lib.MAX_N:
             return None
         at = np.ix_(states, states)
@@ -77,6 +73,7 @@ class SeriesGradient:
         self = cls()
         da, db, F = plan
         self.model, self.plan, self.states, self.h = model, plan, states, h
+        self.reach = reach
         self.gen = program.index(varying[0])
         self.d_lanes, self.d_table = model.lane_tables(*plan, states)
         _, own, opp = lane_entries(model, transposed=True)

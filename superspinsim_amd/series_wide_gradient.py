@@ -13,7 +13,7 @@ import numpy as np
 
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
-from superspinsim_amd.series import reachable
+from superspinsim_amd.series import Reach
 from superspinsim_amd.series_wide import WideModel, own_states
 
 _f64 = np.float64
@@ -52,10 +52,8 @@ class WideGradient:
             return None
         folded, drive = sim.folded(const), sim.gens[varying[0]]
         pattern = (folded != 0) | (drive != 0)
-        # what the run reaches and what the readout depends on: a parameter
-        # may join one to the other
-        states = np.union1d(reachable(pattern, rho0),
-                            reachable(pattern.T, np.atleast_2d(obs)))
+        reach = Reach(pattern, rho0, np.atleast_2d(obs))
+        states = reach.states
         if not _lib.MAX_N < states.size <= MAX_ROWS:
             return None
         at = np.ix_(states, states)
@@ -84,6 +82,7 @@ class WideGradient:
             return None
         self = cls()
         self.model, self.plan, self.states = model, plan, states
+        self.reach = reach
         self.orders = orders
         self.gen = program.index(varying[0])
         self.npad = -(-model.n // 16) * 16

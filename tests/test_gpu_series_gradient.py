@@ -124,3 +124,47 @@ def test_parameter_that_joins_what_the_drive_does_not(gpu):
     print(f"{np.max(np.abs(got / want - 1)):.1e}", flush=True)
     assert np.all(out.cpu().numpy() == 0)
     assert np.max(np.abs(got / want - 1)) <= 1e-12
+
+
+def test_states_and_rows_set_after_setup(gpu):
+    """A point set up for one initial state and readout serves any other,
+    through the Taylor path where they involve further states: as a point
+    set up for them, to the bars above."""
+    problem, theta, amps, seeds = _problem(2, False, 2, 4, 20, 3e6, True,
+                                           False)
+    n = problem.rho0.size
+    state = problem.setup(theta, amps)
+    out, _ = problem.forward(theta, amps, state)
+    assert state["by_series"]
+    first = out.cpu().numpy().copy()
+    reach = state["series"].reach
+    rng = np.random.default_rng(0)
+    rho, obs = rng.standard_normal((2, n))
+    rho[reach.ahead], obs[reach.behind] = problem.rho0[reach.ahead], 0.3
+
+    def gradients(st):
+        out, st = problem.forward(theta, amps, st)
+        back = problem.backward(st, seeds, lambda_out=True)
+        return out.cpu().numpy(), [back[k].cpu().numpy() for k in (
+            "theta", "amplitudes", "lambda")], st["by_series"]
+
+    saved = problem.rho0, problem.obs
+    for new in ((rho, saved[1]), (saved[0], obs[None]), (rho, obs[None])):
+        problem.rho0, problem.obs = new
+        got = gradients(state)
+        want = gradients(problem.setup(theta, amps))
+        assert not got[2]
+        assert np.max(np.abs(got[0] - want[0])) <= \
+            1e-12 * np.max(np.abs(want[0]))
+        for a, b in zip(got[1], want[1]):
+            size = np.max(np.abs(b), axis=0) if a.ndim == 2 else \
+                np.max(np.abs(b))
+            assert np.all(np.abs(a - b) <= 1e-10 * size + 1e-300)
+    # rows set between the two directions
+    problem.rho0, problem.obs = saved
+    out, _ = problem.forward(theta, amps, state)
+    assert state["by_series"] and np.array_equal(out.cpu().numpy(), first)
+    problem.obs = obs[None]
+    got = problem.backward(state, seeds)["theta"].cpu().numpy()
+    want = gradients(problem.setup(theta, amps))[1][0]
+    assert np.all(np.abs(got - want) <= 1e-10 * np.max(np.abs(want), axis=0))

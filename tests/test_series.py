@@ -292,3 +292,19 @@ def test_simulator_keeps_the_last_models():
     plan(sweep.MAX_MODELS)
     assert len(sim._series_cache) == sweep.MAX_MODELS
     assert plan(0) is first and plan(1) is not second
+
+
+def test_reach_covers_what_stays_within_it():
+    from superspinsim_amd.series import Reach
+    wl = configs.odmr7(1)
+    const, drive = _pair(wl)
+    reach = Reach((const != 0) | (drive != 0), wl.rho0[None], wl.obs)
+    assert 0 < reach.states.size < wl.n
+    rho = np.where(reach.ahead, 0.5, 0.0)[None]
+    obs = np.where(reach.behind, 0.5, 0.0)[None]
+    assert reach.covers(obs) and reach.covers(obs, rho)
+    for k in np.flatnonzero(~reach.ahead):
+        assert not reach.covers(obs, rho + np.eye(wl.n)[k])
+    for k in np.flatnonzero(~reach.behind):
+        assert not reach.covers(obs + np.eye(wl.n)[k])
+    assert not reach.covers(obs, rho[:, 1:]) and not reach.covers(obs[:, 1:])
