@@ -525,7 +525,11 @@ class GradientProblem:
         free += torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
         if 8 * math.prod(shape) > 0.8 * free:
             return False
-        return torch.empty(shape, dtype=torch.float64, device="cuda")
+        try:
+            return torch.empty(shape, dtype=torch.float64, device="cuda")
+        except torch.cuda.OutOfMemoryError:
+            # (memory the allocator holds may be in pieces)
+            return False
 
     def adjoint_desc(self, state):
         prop = state["prop"]

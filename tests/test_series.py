@@ -308,3 +308,27 @@ def test_reach_covers_what_stays_within_it():
     for k in np.flatnonzero(~reach.behind):
         assert not reach.covers(obs + np.eye(wl.n)[k])
     assert not reach.covers(obs, rho[:, 1:]) and not reach.covers(obs[:, 1:])
+
+
+def test_gradient_store_that_cannot_be_had(monkeypatch):
+    """Free memory in pieces: the checkpointed path, not an error."""
+    import torch
+    from superspinsim_amd import adjoint
+
+    class Series:
+        d_w = np.zeros((2, 2))
+        store_shape = staticmethod(lambda *a: a)
+
+    def empty(*args, **kw):
+        raise torch.cuda.OutOfMemoryError("in pieces")
+
+    problem = adjoint.GradientProblem(None, None, np.eye(4)[0], np.eye(4)[1],
+                                      0.0, 1e-9, 1e-10)
+    state = adjoint.GradientState(derivatives=True, n_inst=3)
+    monkeypatch.setattr(adjoint, "_torch", lambda: torch)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda: (1 << 30,) * 2)
+    for name in ("memory_reserved", "memory_allocated"):
+        monkeypatch.setattr(torch.cuda, name, lambda: 0)
+    monkeypatch.setattr(torch, "empty", empty)
+    assert problem._series_store(state, Series, 10) is False
+    assert problem._series_store(state, Series, 1 << 40) is False
