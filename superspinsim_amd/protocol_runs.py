@@ -16,7 +16,8 @@ import numpy as np
 from superspinsim_amd import _lib
 from superspinsim_amd.propagator import _ptr, _torch, device_tensor
 from superspinsim_amd.series import (
-    SeriesModel, coefficient_matrices, lane_entries, lane_table)
+    SeriesModel, coefficient_matrices, coefficient_stacks, lane_entries,
+    lane_table)
 
 _f64 = np.float64
 
@@ -101,29 +102,45 @@ class ProtocolRuns:
             return None
         folded = sim.folded(const)
         weights = sim.weights
-        sets, where, pure = [], [], []
-        for row in kinds:
+        # (kinds that no run steps through need no tables, only powers; the
+        # sets of equal terms are one: a switch's two edges in a step share
+        # theirs)
+        stepped = np.zeros(kinds.shape[0], dtype=bool)
+        stepped[index[driven]] = True
+        sets, idle, where, pure = {}, [], [], []
+        for row, steps_on in zip(kinds, stepped):
             v = row.reshape(S, -1)              # (node, switched)
             same = bool(np.all(v == v[0]))
             pure.append(same)
             ids = []
             for j in range(1 if same else J):
-                terms = [(folded, h * float(weights[j].sum()))]
-                for k, g in enumerate(switched):
-                    scale = float(weights[j].sum()) * v[0, k] if same else \
-                        float(weights[j] @ v[:, k])
-                    if scale != 0:
-                        terms.append((sim.gens[g], h * scale))
-                ids.append(len(sets))
-                sets.append(terms)
+                scales = (h * float(weights[j].sum()),) + tuple(
+                    h * (float(weights[j].sum()) * v[0, k] if same else
+                         float(weights[j] @ v[:, k]))
+                    for k in range(len(switched)))
+                if same and not steps_on:
+                    idle.append(scales)
+                    ids.append(0)
+                else:
+                    ids.append(sets.setdefault(scales, len(sets)))
             where.append((ids[0], ids[-1]))
+        if not sets:
+            sets[idle.pop()] = 0
+
+        def terms_of(scales):
+            return [(folded, scales[0])] + [
+                (sim.gens[g], s) for g, s in zip(switched, scales[1:])
+                if s != 0]
+
         sums = weights.sum(axis=1)
         if not np.allclose(sums, sums[::-1], rtol=1e-15, atol=1e-16):
             return None
         gen = sim.gens[drive] if drive is not None else \
             np.zeros((sim.n, sim.n))
-        model = SeriesModel.of_sets(sets, gen, weights, h)
-        if model is None or not model.one_pair():
+        model = SeriesModel.of_sets(
+            [terms_of(v) for v in sets], gen, weights, h,
+            also=[terms_of(v) for v in idle], pair=True)
+        if model is None:
             return None
         plan = model.plan(drive_max_of(drive), tolerance)
         if plan is None:
@@ -148,14 +165,16 @@ class ProtocolRuns:
             [lane_table(m, own, opp, plan[0], plan[1])
              for m in model.matrices(*plan)]))
         powers = np.zeros((max(used.size, 1), max(levels, 1), 2, 6, 64))
-        for k in used:
-            v = kinds[k].reshape(S, -1)[0] if switched else []
-            terms = [(folded, h)] + [(sim.gens[g], h * float(x))
-                                     for g, x in zip(switched, v)]
-            for b, (step, read_mat) in enumerate(
-                    cls._powers(terms, sim.n, h, levels)):
-                powers[power_of[int(k)], b, 0] = cls._own(step, own)
-                powers[power_of[int(k)], b, 1] = cls._own(read_mat, own)
+        if used.size:
+            undriven = coefficient_stacks(
+                [terms_of((h,) + tuple(h * kinds[k].reshape(S, -1)[0]))
+                 for k in used], np.zeros((sim.n, sim.n)), 0,
+                extended=True)[0]
+            for p, d in enumerate(undriven):
+                for b, (step, read_mat) in enumerate(
+                        cls._squares(d, h, levels)):
+                    powers[p, b, 0] = cls._own(step, own)
+                    powers[p, b, 1] = cls._own(read_mat, own)
         self.d_powers = device_tensor(powers)
         begin = np.zeros(n_inst + 1, dtype=np.int32)
         np.cumsum(np.bincount(inst, minlength=n_inst), out=begin[1:])
@@ -240,14 +259,18 @@ class ProtocolRuns:
         out[own[:, 0], own[:, 1]] = mat[own[:, 2], own[:, 3]]
         return out
 
+    @classmethod
+    def _powers(cls, terms, n, h, levels):
+        """``_squares`` of E = exp(sum of terms)."""
+        return cls._squares(coefficient_matrices(
+            terms, np.zeros((n, n)), 0, extended=True)[0], h, levels)
+
     @staticmethod
-    def _powers(terms, n, h, levels):
+    def _squares(d, h, levels):
         """(E^(2^b) - I, (h/2) sum_{k<2^b} (E^k + E^(k+1))), b < levels, of
-        E = exp(sum of terms), squared up in extended precision."""
-        d = coefficient_matrices(terms, np.zeros((n, n)), 0,
-                                 extended=True)[0]
+        E = I + d, squared up in extended precision."""
         half = np.longdouble(h) / 2
-        read = half * (2 * np.eye(n, dtype=np.longdouble) + d)
+        read = half * (2 * np.eye(d.shape[0], dtype=np.longdouble) + d)
         for _ in range(levels):
             yield d.astype(_f64), read.astype(_f64)
             read = 2 * read + read @ d

@@ -129,17 +129,64 @@ def _dropped(count, da, db):
             if k > (2 * da if k % 2 == 0 else 2 * db + 1)]
 
 
-def _sparse(mat):
-    """(columns, values) lists, slot by slot, of a matrix's rows."""
-    width = int(np.max(np.count_nonzero(mat, axis=1), initial=0))
-    n = mat.shape[0]
+def _sparse(mats):
+    """(columns, values [..., slot, row]), slot by slot, of the rows of
+    ``mats`` (..., n, n) over their common pattern."""
+    n = mats.shape[-1]
+    pattern = np.any(mats.reshape(-1, n, n) != 0, axis=0)
+    width = int(np.max(np.count_nonzero(pattern, axis=1), initial=0))
     cols = np.zeros((width, n), dtype=np.int64)
-    vals = np.zeros((width, n), dtype=np.longdouble)
+    vals = np.zeros(mats.shape[:-2] + (width, n), dtype=np.longdouble)
     for r in range(n):
-        c = np.flatnonzero(mat[r])
+        c = np.flatnonzero(pattern[r])
         cols[:c.size, r] = c
-        vals[:c.size, r] = mat[r, c]
+        vals[..., :c.size, r] = mats[..., r, c]
     return cols, vals
+
+
+def coefficient_stacks(sets, drive, orders, extended=False):
+    """``coefficient_matrices`` of every element of ``sets`` (terms) at once:
+    per order one array (sets, n, n).
+
+    A set's values are those it has alone; together they take half as long
+    as one by one (19 states)."""
+    const = np.stack([sum(np.asarray(m, dtype=np.longdouble) *
+                          np.longdouble(s) for m, s in terms)
+                      for terms in sets])
+    n = const.shape[-1]
+    cc, cv = _sparse(const)
+    dc, dv = _sparse(np.asarray(drive, dtype=_f64))
+
+    def times(cols, vals, mat):
+        out = np.zeros_like(mat)
+        for k, c in enumerate(cols):
+            out += vals[..., k, :, None] * mat[:, c]
+        return out
+
+    # terms of order t in const fall like norm^t / t!, drive orders add to t
+    count = np.zeros(len(sets), dtype=np.int64)
+    for e, norm in enumerate(np.abs(const).sum(axis=-2).max(
+            axis=-1, initial=0.0).astype(_f64)):
+        bound, t = 1.0, 0
+        while bound > 1e-24 or t <= orders + 2:
+            t += 1
+            bound *= norm / max(t - orders, 1)
+        count[e] = t
+    zero = np.zeros_like(const)
+    term = [zero + np.eye(n, dtype=np.longdouble)] + [zero] * orders
+    total = [zero.copy() for _ in range(orders + 1)]
+    for t in range(1, count.max() + 1):
+        new = []
+        for k in range(orders + 1):
+            v = times(cc, cv, term[k])
+            if k:
+                v += times(dc, dv, term[k - 1])
+            new.append(v / t)
+        term = new
+        on = slice(None) if count.min() >= t else count >= t
+        for k in range(orders + 1):
+            total[k][on] += term[k][on]
+    return total if extended else [m.astype(_f64) for m in total]
 
 
 def coefficient_matrices(terms, drive, orders, extended=False):
@@ -150,37 +197,8 @@ def coefficient_matrices(terms, drive, orders, extended=False):
     rounded once (not at all with ``extended``): the same E_k act at every
     step, so their rounding would not average out.
     """
-    const = sum(np.asarray(m, dtype=np.longdouble) * np.longdouble(s)
-                for m, s in terms)
-    n = const.shape[0]
-    cc, cv = _sparse(const)
-    dc, dv = _sparse(np.asarray(drive, dtype=_f64))
-
-    def times(cols, vals, mat):
-        out = np.zeros_like(mat)
-        for c, v in zip(cols, vals):
-            out += v[:, None] * mat[c]
-        return out
-
-    zero = np.zeros((n, n), dtype=np.longdouble)
-    term = [np.eye(n, dtype=np.longdouble)] + [zero] * orders
-    total = [zero.copy() for _ in range(orders + 1)]
-    norm = float(np.abs(const).sum(axis=0).max(initial=0.0))
-    bound, t = 1.0, 0
-    # terms of order t in const fall like norm^t / t!, drive orders add to t
-    while bound > 1e-24 or t <= orders + 2:
-        t += 1
-        bound *= norm / max(t - orders, 1)
-        new = []
-        for k in range(orders + 1):
-            v = times(cc, cv, term[k])
-            if k:
-                v += times(dc, dv, term[k - 1])
-            new.append(v / t)
-        term = new
-        for k in range(orders + 1):
-            total[k] += term[k]
-    return total if extended else [m.astype(_f64) for m in total]
+    return [m[0] for m in coefficient_stacks([terms], drive, orders,
+                                             extended)]
 
 
 def chebyshev(mats, F):
@@ -249,14 +267,16 @@ class SeriesModel:
         return self
 
     @classmethod
-    def of_sets(cls, sets, drive, weights, h):
+    def of_sets(cls, sets, drive, weights, h, also=(), pair=False):
         """Model with one set of matrices per element of ``sets`` (terms of
-        ``coefficient_matrices``) on common sectors."""
+        ``coefficient_matrices``) on sectors common to them and to ``also``
+        (terms whose matrices are not needed).  ``pair``: None where
+        ``one_pair`` does not hold."""
         n = drive.shape[0]
         if n > _lib.MAX_N:
             return None
         pattern = np.zeros((n, n))
-        for terms in sets:
+        for terms in list(sets) + list(also):
             norm = sum(abs(s) * np.abs(m).sum(axis=0).max()
                        for m, s in terms)
             if not norm <= MAX_NORM:
@@ -278,9 +298,6 @@ class SeriesModel:
         self.n_sectors = counts.size
         self.weight = float(np.abs(weights).sum(axis=1).max())
         self.nnz = int(np.count_nonzero((pattern != 0) | (drive != 0)))
-        top = 2 * ORDERS[-1][0] + 3
-        self.sets = [coefficient_matrices(terms, drive, top)
-                     for terms in sets]
         order = np.argsort(sector, kind="stable")
         self.members = [order[np.searchsorted(sector[order], k):
                               np.searchsorted(sector[order], k, "right")]
@@ -289,6 +306,11 @@ class SeriesModel:
         for k, states in enumerate(self.members):
             pos[states] = k * self.pad + np.arange(states.size)
         self.pos, self.order = pos, order
+        if pair and not self.one_pair():
+            return None
+        top = 2 * ORDERS[-1][0] + 3
+        self.stacks = coefficient_stacks(sets, drive, top)
+        self.sets = [[m[e] for m in self.stacks] for e in range(len(sets))]
         return self
 
     def one_pair(self):
@@ -314,9 +336,8 @@ class SeriesModel:
         ``tol`` with the Taylor plans' margin (a factor of 8).
         """
         F = self.h * self.weight * float(drive_max)
-        worst = np.max([[np.abs(c).sum(axis=0).max() for c in cs]
-                        for cs in (chebyshev(es, F)
-                                   for es in self.sets)], axis=0)
+        worst = np.array([np.abs(c).sum(axis=-2).max()
+                          for c in chebyshev(self.stacks, F)])
         if not np.all(np.isfinite(worst)):
             return None
         for da, db in ORDERS:
@@ -328,7 +349,8 @@ class SeriesModel:
 
     def matrices(self, da, db, F):
         """The kept E_k of every set (``economised``)."""
-        return [economised(mats, da, db, F) for mats in self.sets]
+        kept = economised(self.stacks, da, db, F)
+        return [[m[e] for m in kept] for e in range(len(self.sets))]
 
     def tables(self, da, db, F):
         """(layout, on the host; device table) of the kernel's rows."""

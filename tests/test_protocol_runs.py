@@ -105,3 +105,38 @@ def test_cut_runs_end_after_the_steps_asked_for():
             end += r["count"]
     assert np.array_equal(rec["count"], count)
     assert np.array_equal(cut[["first", "read"]], rec[["first", "read"]])
+
+
+def test_tables_of_many_switch_values(monkeypatch):
+    """As many tables as differ and are stepped through, each as its terms
+    alone give it."""
+    from superspinsim_amd import protocol_runs, series
+    from superspinsim_amd.sweep import BatchSimulator
+    monkeypatch.setattr(protocol_runs, "device_tensor", np.array)
+    monkeypatch.setattr(ProtocolRuns, "_staged", staticmethod(np.copy))
+    wl = configs.odmr7(1, use_incoherent=True)
+    waves, steps = [], []
+    for k in range(5):
+        w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, 0.0])
+        w.add(1, 0.0, 3.1e-10, 1e-4, 2e10)
+        w.add(4, 5.05e-10, 9.4e-10, 0.01 * (k + 1))     # edges within steps
+        waves.append(w)
+        steps.append(60)
+    sim = BatchSimulator(wl.generators, 2)
+    _, const, program = sim.program(waves)
+    runs = ProtocolRuns.build(sim, waves, const, program, np.array(steps),
+                              np.zeros(5, np.int64), H,
+                              lambda g: waves[0].abs_max()[g], 1e-16)
+    table, rec = runs.d_table, runs.d_runs
+    # the dark one, and per value one edge's pair (the other's swapped)
+    assert len(np.unique(table.reshape(len(table), -1), axis=0)) == \
+        len(table) == 11
+    stepped = rec[rec["kind"] != protocol_runs.FREE]
+    assert set(stepped["set0"]) | set(stepped["set1"]) == set(range(11))
+    assert len(runs.d_powers) == 6
+    alone = series.coefficient_matrices(
+        [(sim.folded(const), 0.5 * H)], wl.generators[1], 7)
+    driven = rec[rec["kind"] == protocol_runs.DRIVEN]
+    assert np.unique(driven["set0"]).size == 1
+    for k, m in enumerate(alone):
+        assert np.array_equal(runs.model.sets[driven["set0"][0]][k], m)
