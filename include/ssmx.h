@@ -106,9 +106,12 @@ typedef struct ssmx_propagate_desc {
                          row (exchanged by DPP instead of ds_bpermute) */
     int32_t ckpt_every; /* K > 0: state_out receives checkpoints (the state
                            before steps 0, K, 2K, ...); 0: the final state */
-    int32_t reserved;   /* ssmx_propagate, table mode, n <= 64: instances in a
-                           row that share one coefficient table (0 = 1);
-                           else 0 */
+    union {
+        int32_t coef_group; /* ssmx_propagate, table mode, n <= 64:
+                               instances in a row that share one coefficient
+                               table (0 = 1); else 0 */
+        int32_t reserved;   /* its name up to version 103 (then always 0) */
+    };
     int64_t coef_inst_stride; /* table mode: doubles between instances (or
                                  groups); 0 = one table for all */
     double h;         /* propagator step dt / F (s) */
@@ -218,7 +221,11 @@ typedef struct ssmx_series_desc {
     int32_t flags;      /* SSMX_READ_FULL, SSMX_READ_INTEGRAL or 0 */
     int32_t gen;        /* driven generator's index in ssmx_wave */
     int32_t wave_group; /* instances that share one waveform, >= 1 */
-    int32_t na, da;     /* own-sector components and highest even order / 2 */
+    union {
+        int32_t na;         /* own-sector components */
+        int32_t lds_columns; /* wide entries: KB of LDS for coefficients */
+    };
+    int32_t da;         /* highest even order / 2 */
     int32_t nb, db;     /* opposite components, (highest odd order - 1) / 2 */
     int32_t sector;     /* LDS doubles per sector, even, >= na and nb */
     int32_t sectors;    /* sectors per member */
@@ -342,7 +349,7 @@ int ssmx_series_adjoint(const ssmx_series_desc *desc, const int32_t *lanes,
 /*
  * ssmx_propagate_series for models of more rows than a wavefront (at most
  * 192), one workgroup of n_blocks (at most 12) wavefronts per instance;
- * n_exp = n_node = 2, (da, db) = (1, 1), (2, 1) or (2, 2); na the sum over the
+ * n_exp = n_node = 2, (da, db) = (1, 1), (2, 1) or (2, 2); lds_columns the sum over the
  * wavefronts of (da + db - 2) slots + 4 max(0, slots - 7), the KB of LDS for
  * the coefficients that registers don't hold (at most 150); members, nb,
  * sector fields unused.
@@ -710,7 +717,8 @@ int ssmx_adjoint(const ssmx_adjoint_desc *desc, const int32_t *ell_col,
 /* Message of the last failure on this thread ("" if none). */
 const char *ssmx_last_error(void);
 
-/* ABI version (major * 100 + minor). */
+/* ABI version (major * 100 + minor).  104: the series entries, coefficient
+ * tables shared by groups of instances (coef_group, before a reserved field). */
 int ssmx_version(void);
 
 /* Number of HIP devices visible, or a negative code. */

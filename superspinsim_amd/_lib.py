@@ -44,7 +44,7 @@ class PropagateDesc(ctypes.Structure):
         ("taylor", ctypes.c_int32), ("substeps", ctypes.c_int32),
         ("n_obs", ctypes.c_int32), ("flags", ctypes.c_int32),
         ("first_out", ctypes.c_int32), ("partner", ctypes.c_int32),
-        ("ckpt_every", ctypes.c_int32), ("reserved", ctypes.c_int32),
+        ("ckpt_every", ctypes.c_int32), ("coef_group", ctypes.c_int32),
         ("coef_inst_stride", ctypes.c_int64),
         ("h", ctypes.c_double), ("t0", ctypes.c_double),
         ("dt", ctypes.c_double),
@@ -98,6 +98,10 @@ class SeriesDesc(ctypes.Structure):
         "n_obs", "flags", "gen", "wave_group", "na", "da", "nb", "db",
         "sector", "sectors", "sector_rows", "reserved")] + [
             (f, ctypes.c_double) for f in ("h", "t0", "dt")]
+
+
+#: the name of ``na`` in the wide entries
+SeriesDesc.lds_columns = SeriesDesc.na
 
 
 class Segment(ctypes.Structure):

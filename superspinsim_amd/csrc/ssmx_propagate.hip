@@ -236,8 +236,9 @@ __device__ __forceinline__ void propagate_instance(const Params &p,
     if (wave_mode)
         q.waves = p.waves + inst;
     else
-        q.coef = p.coef + (size_t)(d.reserved > 1 ? inst / d.reserved : inst) *
-                              d.coef_inst_stride;
+        q.coef = p.coef +
+                 (size_t)(d.coef_group > 1 ? inst / d.coef_group : inst) *
+                     d.coef_inst_stride;
 
     // Lane t holds 1/t: the Taylor recursion broadcasts it with readlane
     // (a scalar memory load or a division would sit in the dependent
@@ -692,12 +693,12 @@ int validate(const ssmx_propagate_desc *d)
         return set_error(SSMX_EINVAL, "partner flag must be 0 or 1");
     if (d->ckpt_every < 0)
         return set_error(SSMX_EINVAL, "ckpt_every=%d < 0", d->ckpt_every);
-    if (d->reserved < 0 ||
-        (d->reserved > 1 &&
+    if (d->coef_group < 0 ||
+        (d->coef_group > 1 &&
          (d->n > SSMX_MAX_N || (d->flags & SSMX_COEF_WAVE))))
-        return set_error(SSMX_EINVAL, "reserved=%d: tables shared by groups "
+        return set_error(SSMX_EINVAL, "coef_group=%d: tables shared by groups "
                          "of instances need n <= 64 and table mode",
-                         d->reserved);
+                         d->coef_group);
     if (d->n > SSMX_MAX_N) {
         // one row per thread: at most 32 slots, and the staged generator
         // values plus one instance's two 512-row exchange buffers within
@@ -731,7 +732,7 @@ int ssmx_wide_propagate(const ssmx_propagate_desc *desc,
 
 extern "C" {
 
-int ssmx_version(void) { return 103; }
+int ssmx_version(void) { return 104; }
 
 const char *ssmx_last_error(void) { return ssmx::error_buffer(); }
 

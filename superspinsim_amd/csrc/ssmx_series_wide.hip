@@ -422,16 +422,16 @@ int check(const ssmx_series_desc &d, int32_t n_blocks, const char *what)
     if (n_blocks < 1 || n_blocks > kMaxWaves)
         return set_error(SSMX_EINVAL, "%d wavefronts outside 1..%d",
                          n_blocks, kMaxWaves);
-    if (d.na < 0 || d.na * kColumnBytes > kHighBytes)
+    if (d.lds_columns < 0 || d.lds_columns * kColumnBytes > kHighBytes)
         return set_error(SSMX_EINVAL, "%d columns of coefficients exceed the "
-                         "LDS", d.na);
+                         "LDS", d.lds_columns);
     return SSMX_OK;
 }
 
 template <int M, int HI>
 int launch(const WSParams &p, int n_blocks, void *stream, const char *what)
 {
-    const size_t bytes = (size_t)p.d.na * kColumnBytes;
+    const size_t bytes = (size_t)p.d.lds_columns * kColumnBytes;
     hipError_t e = hipSuccess;
     if (bytes > 0)
         e = hipFuncSetAttribute(

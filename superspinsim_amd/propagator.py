@@ -1044,7 +1044,7 @@ class Propagator:
             taylor=int(taylor), substeps=int(substeps), n_obs=max(n_obs, 1),
             flags=flags, first_out=int(first_out),
             partner=1 if self.ell.partner else 0,
-            ckpt_every=int(ckpt_every), reserved=int(coef_group),
+            ckpt_every=int(ckpt_every), coef_group=int(coef_group),
             coef_inst_stride=int(coef_inst_stride), h=float(h),
             t0=float(t0), dt=float(dt))
         obs_rows = None

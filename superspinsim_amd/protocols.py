@@ -181,7 +181,7 @@ class ProtocolBatch:
             n=prop.n, n_inst=self.n_inst, n_gen=prop.K, slots=prop.ell.slots,
             n_exp=prop.J, n_node=prop.S, fine=1, n_out=0,
             taylor=self.taylor, substeps=self.substeps, n_obs=self.n_obs,
-            flags=flags, first_out=0, partner=1, ckpt_every=0, reserved=0,
+            flags=flags, first_out=0, partner=1, ckpt_every=0, coef_group=0,
             coef_inst_stride=0, h=self.h, t0=0.0, dt=self.h)
 
     def launch(self, stream=None):

@@ -348,7 +348,7 @@ class WideRun:
             n=n, rows=model.n, n_inst=n_inst, members=1,
             n_exp=weights.shape[0], n_node=weights.shape[1], fine=fine,
             n_out=n_out, n_obs=n_obs, flags=flags, gen=gen, wave_group=1,
-            na=in_lds, da=plan[0], db=plan[1], h=dt / fine, t0=t0,
+            lds_columns=in_lds, da=plan[0], db=plan[1], h=dt / fine, t0=t0,
             dt=dt)
         shape = {"full": (n_inst, n_out, n), "obs": (n_inst, n_out, n_obs),
                  "integral": (n_inst, n_obs)}[read]

@@ -152,7 +152,7 @@ class WideGradient:
             members=1, n_exp=J, n_node=S, fine=problem.F,
             n_out=problem.n_out, n_obs=problem.obs.shape[0],
             flags=_lib.SSMX_READ_INTEGRAL, gen=self.gen, wave_group=1,
-            na=in_lds, da=self.plan[0], db=self.plan[1],
+            lds_columns=in_lds, da=self.plan[0], db=self.plan[1],
             h=problem.dt / problem.F, t0=problem.t0, dt=problem.dt)
 
     def forward(self, problem, state, rho0, store):

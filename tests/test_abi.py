@@ -261,3 +261,35 @@ def test_invalid_wide_adjoint_descriptor_is_rejected(lib, flags, bad):
     assert lib.ssmx_series_wide_adjoint(
         ctypes.byref(d), dummy, 3, *([dummy] * 9)) == -1
     assert lib.ssmx_last_error().decode()
+
+
+def test_second_names_of_fields(tmp_path):
+    """Fields of two meanings have a name for each, at one offset."""
+    probe = tmp_path / "probe.c"
+    probe.write_text(r'''
+#include <stddef.h>
+#include <stdio.h>
+#include "ssmx.h"
+int main(void) {
+  printf("%zu %zu %zu %zu %zu\n", offsetof(ssmx_series_desc, na),
+         offsetof(ssmx_series_desc, lds_columns),
+         offsetof(ssmx_series_desc, da),
+         offsetof(ssmx_propagate_desc, coef_group),
+         offsetof(ssmx_propagate_desc, reserved));
+  return 0;
+}
+''')
+    exe = str(tmp_path / "probe")
+    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), "-o", exe,
+                    str(probe)], check=True)
+    na, lds, da, group, reserved = map(int, subprocess.run(
+        [exe], capture_output=True, text=True, check=True).stdout.split())
+    D = _lib.SeriesDesc
+    assert (D.na.offset, D.lds_columns.offset, D.da.offset) == (na, lds, da)
+    assert na == lds and group == reserved == \
+        _lib.PropagateDesc.coef_group.offset
+    assert _lib.SeriesDesc(lds_columns=7).na == 7
+
+
+def test_version_of_the_series_entries(lib):
+    assert lib.ssmx_version() >= 104
