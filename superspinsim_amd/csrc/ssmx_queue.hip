@@ -244,11 +244,14 @@ __device__ __forceinline__ void queue_loop(const QParams &p,
             if (step >= k_from)
                 xint = fma(half_h, x_prev + x, xint);
         }
-        // lane o writes readout o
         const double v0 = wave_sum(obs0 * xint);
-        const double v1 = d.n_obs > 1 ? wave_sum(obs1 * xint) : 0.0;
-        if (lane < d.n_obs)
-            p.out[(size_t)inst * d.n_obs + lane] = lane == 0 ? v0 : v1;
+        if (lane == 0)
+            p.out[(size_t)inst * d.n_obs] = v0;
+        if (d.n_obs > 1) {
+            const double v1 = wave_sum(obs1 * xint);
+            if (lane == 0)
+                p.out[(size_t)inst * d.n_obs + 1] = v1;
+        }
     };
 
     // Every pass takes one queue entry; the counter only grows, so every
