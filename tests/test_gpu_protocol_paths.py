@@ -63,3 +63,53 @@ def test_cut_series_batch_equals_fewer_steps(wl):
     assert np.array_equal(got, _batch(wl, None, steps).run().cpu().numpy())
     b.series.cut()
     assert np.array_equal(b.run().cpu().numpy(), whole)
+
+
+def _result(b):
+    return b.out.cpu().numpy()[:, 0].copy()
+
+
+@pytest.mark.parametrize("taylor", PATHS)
+def test_grid_graph_and_stream_do_not_change_results(wl, taylor):
+    import torch
+    b = _batch(wl, taylor)
+    want = b.run().cpu().numpy()[:, 0].copy()
+    assert np.all(want != 0)
+    for n_waves, wpb in ((1, 1), (5, 2), (7, 8)):
+        got = _batch(wl, taylor, n_waves=n_waves, waves_per_block=wpb)
+        got.run()
+        assert np.array_equal(_result(got), want), (n_waves, wpb)
+    b.out.fill_(np.nan)
+    b.launch_noalloc()
+    assert np.array_equal(_result(b), want)
+    b.capture()
+    scratch = torch.ones(1 << 20, dtype=torch.float64, device="cuda")
+    for _ in range(3):
+        scratch.mul_(1.5)               # unrelated eager work
+        torch.cuda.synchronize()
+        b.out.fill_(np.nan)
+        b.graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(_result(b), want)
+        assert int(b.counter.item()) == len(wl.waves) + b.n_waves
+    side = torch.cuda.Stream()
+    for _ in range(2):
+        b.out.fill_(np.nan)
+        side.wait_stream(torch.cuda.current_stream())
+        b.launch(stream=side.cuda_stream)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        assert np.array_equal(_result(b), want)
+
+
+def test_paths_agree_and_a_plan_set_later_changes_the_path(wl):
+    """The Taylor plan set on a prepared series batch launches the Taylor
+    queue; both within 1e-12 (9,355 steps, an ulp each at most)."""
+    b = _batch(wl, None)
+    series = b.run().cpu().numpy()[:, 0].copy()
+    b.taylor = 13
+    taylor = b.run().cpu().numpy()[:, 0].copy()
+    assert np.array_equal(taylor, _batch(wl, 13).run().cpu().numpy()[:, 0])
+    assert np.max(np.abs(series - taylor) / np.abs(taylor)) <= 1e-12
+    b.taylor = b.plan_default[0]
+    assert np.array_equal(b.run().cpu().numpy()[:, 0], series)
