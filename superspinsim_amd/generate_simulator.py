@@ -347,23 +347,23 @@ def generate_simulator(
             N, F, mats.shape[-1], J=weights.shape[0], products=m * s,
             matrices=mats.shape[0] if not use_rotating else
             mats.shape[0] * mats.shape[1], pairs=use_rotating)
+        states = None
         if split is not None:
-            states = _chunked_states(mats, weights, nodes, use_rotating, eig,
-                                     coef, x0, h, m, s, N, F, split)
-            return time, _finish(states, n, rho_flat, vmap, use_hermitian,
-                                 hilbert, use_rotating, vectors_real,
-                                 inv_vectors_real, use_kernel,
-                                 image_projection, use_unitary, elimination,
-                                 duplication)
-        prop = propagator()
-        d_rho = device_tensor(x0)
-        d_coef = device_tensor(coef)
-        out = prop.run(n_inst=n_inst, fine=F, n_out=N, h=h, t0=time_start,
-                       dt=time_step, rho0=d_rho, coef=d_coef,
-                       coef_inst_stride=0, taylor=m, substeps=s,
-                       read="full")
-        torch.cuda.synchronize()
-        states = out.cpu().numpy()                           # (I, N, n)
+            try:
+                states = _chunked_states(mats, weights, nodes, use_rotating,
+                                         eig, coef, x0, h, m, s, N, F, split)
+            except torch.cuda.OutOfMemoryError:
+                pass            # one wavefront keeps no propagators
+        if states is None:
+            prop = propagator()
+            d_rho = device_tensor(x0)
+            d_coef = device_tensor(coef)
+            out = prop.run(n_inst=n_inst, fine=F, n_out=N, h=h, t0=time_start,
+                           dt=time_step, rho0=d_rho, coef=d_coef,
+                           coef_inst_stride=0, taylor=m, substeps=s,
+                           read="full")
+            torch.cuda.synchronize()
+            states = out.cpu().numpy()                       # (I, N, n)
         return time, _finish(states, n, rho_flat, vmap, use_hermitian,
                              hilbert, use_rotating, vectors_real,
                              inv_vectors_real, use_kernel, image_projection,

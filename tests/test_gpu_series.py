@@ -282,3 +282,31 @@ def test_tables_outlive_a_launch_on_another_stream(gpu, name, points):
             for n in sizes for _ in range(4)]
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy(), want), (len(rest), len(fill))
+
+
+def test_drop_in_without_room_for_chunks(gpu, monkeypatch):
+    """Chunk propagators that cannot be allocated: one wavefront, the same
+    states."""
+    import torch
+    gs = importlib.import_module("superspinsim_amd.generate_simulator")
+
+    def sampler(t, row):
+        row[0], row[1] = 1.0, np.sin(2e9 * t)
+
+    rng = np.random.default_rng(1)
+    gens = rng.standard_normal((2, 4, 4)) * 1e8 - 4e8 * np.eye(4)
+    vmap = np.array([(0, 0, 0), (0, 1, 0), (0, 1, 1), (1, 1, 0)])
+    sim = gs.generate_simulator(sampler, gens, vmap,
+                                number_of_fine_divisions=30)
+    args = (rng.standard_normal((2, 2)), 0.0, 20 * 6e-10, 6e-10)
+    tried = []
+
+    def full(*a, **kw):
+        tried.append(1)
+        raise torch.cuda.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(gs, "_chunked_states", full)
+    got = sim(*args)[1]
+    assert tried
+    monkeypatch.setattr(gs, "time_chunks", lambda *a, **k: None)
+    assert np.array_equal(got, sim(*args)[1])
