@@ -15,12 +15,13 @@ The gradient leg runs the 1024-point version of the sweep with a
 input in HBM, then the reverse run of the cotangents and the parameter
 moments, for the squared error against targets simulated at parameters
 perturbed by up to 2 %; the ratio is (forward with stored inputs + backward)
-/ plain forward, wall time.
+/ plain forward, wall time, gradients and plain forwards each in a row.
 
 The protocol leg runs 16384 pulsed Ramsey / Hahn-echo protocols of 58k-742k
 steps in one persistent work-queue launch (driven stretches step by step,
 waits by powers of their exponential; replayed from a HIP graph) and reports
-propagator steps/s over the whole batch.
+steps of protocol time per second over the whole batch (``steps_per_s``) and
+the steps executed one by one among them (``steps_driven``).
 
 The hyperfine leg runs the 21-level NV + 14N sweep (512 points, 250,000
 steps each, fluorescence every 2 ns) at n = 441 and at n = 171 through the
@@ -192,11 +193,19 @@ def adjoint_leg(args):
     plain()
     grad()
     torch.cuda.synchronize()
+    # plain forwards among themselves, gradients among themselves: a launch of
+    # one wavefront per SIMD that follows the adjoint's takes half as long
+    # again (some SIMDs get two, others none), whichever forward it is
     times = {"forward": [], "forward_ckpt": [], "backward": []}
+    plain()
     for _ in range(args.adjoint_steps):
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         plain()
+        torch.cuda.synchronize()
+        times["forward"].append(time.perf_counter() - t0)
+    grad()
+    for _ in range(args.adjoint_steps):
         torch.cuda.synchronize()
         t1 = time.perf_counter()
         out, st = pb.forward(wl.theta, wl.amplitudes, state)
@@ -205,7 +214,6 @@ def adjoint_leg(args):
         res = pb.backward(st, 2.0 * (out - target))
         torch.cuda.synchronize()
         t3 = time.perf_counter()
-        times["forward"].append(t1 - t0)
         times["forward_ckpt"].append(t2 - t1)
         times["backward"].append(t3 - t2)
     med = {k: float(np.median(v)) for k, v in times.items()}
@@ -272,6 +280,8 @@ def protocol_leg(args):
         "workload": wl.name,
         "protocols": batch.n_inst,
         "steps_total": total,
+        "steps_driven": total if batch.series is None else
+        batch.series.driven_steps(),
         "steps_min": int(wl.steps.min()),
         "steps_max": int(wl.steps.max()),
         "readout": "integrated fluorescence over the final 1 us window",

@@ -189,6 +189,11 @@ class ProtocolRuns:
         self.gen = program.index(drive) if drive is not None else 0
         return self
 
+    def driven_steps(self):
+        """Steps launched one by one (those of free runs are powers)."""
+        rec = self._records
+        return int(rec["count"][rec["kind"] != FREE].sum())
+
     @staticmethod
     def _staged(records):
         raw = records.tobytes() or bytes(RUN_DTYPE.itemsize)
