@@ -578,10 +578,12 @@ class BatchSimulator:
     def series_members(self, n_inst, rows):
         """Instances per wavefront of a series run.
 
-        A SIMD's time goes with the wavefronts it holds, each costing the
-        same whatever its lanes do, so the smallest count that minimises the
-        wavefronts on the fullest SIMD (4096 instances of 19 rows: 2 per
-        wavefront, 2 wavefronts per SIMD)."""
+        The smallest count that minimises the wavefronts on the fullest
+        SIMD: a second one there costs half a step's time again, more than
+        the lanes of another instance do.  ns a step at 19 rows: 2,048
+        points two per wavefront 397, three (through LDS) 448; 2,500 points
+        (two wavefronts to a SIMD, or one) 630 and 450; 4,096 points 635 and
+        685; 6,000 points 905 and 750."""
         limit = min(_lib.MAX_N // rows, _lib.MAX_N // self.weights.shape[0])
         if not self.pack or n_inst < 2:
             return 1
