@@ -433,10 +433,11 @@ int launch(const WSParams &p, int n_blocks, void *stream, const char *what)
 {
     const size_t bytes = (size_t)p.d.lds_columns * kColumnBytes;
     hipError_t e = hipSuccess;
+    // (one limit for every launch: another thread may launch with more)
     if (bytes > 0)
         e = hipFuncSetAttribute(
             reinterpret_cast<const void *>(series_wide_kernel<M, HI>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+            hipFuncAttributeMaxDynamicSharedMemorySize, kHighBytes);
     if (e == hipSuccess) {
         hipLaunchKernelGGL((series_wide_kernel<M, HI>), dim3(p.d.n_inst),
                            dim3(kWave * n_blocks), bytes,

@@ -197,3 +197,49 @@ def test_full_states_whatever_the_count_of_readout_rows(gpu):
     want = run.launch().cpu().numpy().copy()
     run.desc.n_obs = 40
     assert np.array_equal(run.launch().cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+def test_launches_of_two_lds_sizes_at_once(gpu):
+    """Two threads launch one kernel with different parts of LDS, each on its
+    own stream, 300 times."""
+    import threading
+
+    import torch
+    runs = []
+    wl = configs.odmr21(1, use_incoherent=True)
+    for scale, gens, rho, obs, base in (
+            (6, wl.generators, wl.rho0, wl.obs,
+             [1.0, 0.0, 0.0, 0.0, wl.excitation]),
+            (10, np.stack(_model(112, 112)), np.ones((1, 112)) / 112,
+             np.ones((1, 112)), [1.0, 0.0])):
+        w = Waveform(len(base), base=base)
+        amp = configs.drive_amplitude(5e5) if len(base) == 5 else 1e7
+        w.tone(1, scale * amp, 2.87e9)
+        sim = BatchSimulator(gens, 2, 3)
+        run = sim.prepare([w], rho, 0.0, 3 * 6e-11 * (1 + 1e-9), 6e-11,
+                          obs=obs)
+        assert sim.last_plan["series"] == (2, 1)
+        runs.append((run, run.launch().cpu().numpy().copy()))
+    sizes = [run.desc.lds_columns for run, _ in runs]
+    assert 0 < min(sizes) < max(sizes)
+    failed = []
+
+    def go(run, want):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(300):
+                    run.launch()
+                torch.cuda.current_stream().synchronize()
+            if not np.array_equal(run.out.cpu().numpy(), want):
+                failed.append(run)
+        except Exception as error:      # the thread's own
+            failed.append(error)
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=go, args=r) for r in runs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not failed, failed
