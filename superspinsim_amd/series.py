@@ -160,7 +160,9 @@ def coefficient_stacks(sets, drive, orders, extended=False):
     def times(cols, vals, mat):
         out = np.zeros_like(mat)
         for k, c in enumerate(cols):
-            out += vals[..., k, :, None] * mat[:, c]
+            part = mat.take(c, axis=1)
+            part *= vals[..., k, :, None]
+            out += part
         return out
 
     # terms of order t in const fall like norm^t / t!, drive orders add to t
