@@ -310,3 +310,30 @@ def test_drop_in_without_room_for_chunks(gpu, monkeypatch):
     assert tried
     monkeypatch.setattr(gs, "time_chunks", lambda *a, **k: None)
     assert np.array_equal(got, sim(*args)[1])
+
+
+@pytest.mark.parametrize("name,points,read", [
+    ("nv7", 3, "full"), ("nv7", 2100, "obs"), ("nv3", 2100, "full"),
+    ("nv21c", 3, "full")])
+def test_launch_in_a_graph(gpu, name, points, read):
+    """Every kernel's launch captured and replayed, with eager launches and
+    another drive's tables between."""
+    import torch
+    wl = configs.odmr21(1, use_incoherent=True) if name == "nv21c" else \
+        _model(name)
+    sim = BatchSimulator(wl.generators, 2, 10)
+    obs = None if read == "full" else wl.obs
+    args = (wl.rho0, 0.0, 3 * 2e-10 * (1 + 1e-9), 2e-10, obs, read)
+    first, next_ = (_waves(wl, points, rabi) for rabi in (3e5, 4e5))
+    run = sim.prepare(first, *args)
+    assert "series" in sim.last_plan
+    want = run.launch().cpu().numpy().copy()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run.launch()
+    for _ in range(3):
+        sim.run(next_, *args)
+        run.out.fill_(np.nan)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(run.out.cpu().numpy(), want)
