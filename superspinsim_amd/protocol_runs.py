@@ -92,6 +92,8 @@ class ProtocolRuns:
             return None
         self = cls()
         first, count, read, values, driven, inst = runs
+        if first.size == 0:
+            return None             # no protocol has a step
         # sets: the switch values at every node, alike or not
         flat = values.reshape(values.shape[0], -1)
         kinds, index = (np.unique(flat, axis=0, return_inverse=True)

@@ -113,3 +113,12 @@ def test_paths_agree_and_a_plan_set_later_changes_the_path(wl):
     assert np.max(np.abs(series - taylor) / np.abs(taylor)) <= 1e-12
     b.taylor = b.plan_default[0]
     assert np.array_equal(b.run().cpu().numpy()[:, 0], series)
+
+
+def test_protocols_of_no_steps(wl):
+    from superspinsim_amd.protocols import ProtocolBatch
+    none = np.zeros(len(wl.waves), dtype=np.int64)
+    b = ProtocolBatch(wl.generators, 2).prepare(
+        wl.waves, wl.rho0, H, none, none, wl.obs)
+    b.out.fill_(np.nan)
+    assert np.all(b.run().cpu().numpy() == 0)

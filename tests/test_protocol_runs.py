@@ -140,3 +140,19 @@ def test_tables_of_many_switch_values(monkeypatch):
     assert np.unique(driven["set0"]).size == 1
     for k, m in enumerate(alone):
         assert np.array_equal(runs.model.sets[driven["set0"][0]][k], m)
+
+
+@pytest.mark.parametrize("switched", [False, True])
+def test_batch_of_no_steps(switched):
+    """Protocols of no steps at all are left to the Taylor queue."""
+    from superspinsim_amd.sweep import BatchSimulator
+    wl = configs.odmr7(1, use_incoherent=True)
+    w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, 0.0])
+    w.add(1, 0.0, 1e-9, 1e-4, 2e10)
+    if switched:
+        w.add(4, 1e-9, 2e-9, 0.01)
+    sim = BatchSimulator(wl.generators, 2)
+    _, const, program = sim.program([w, w])
+    assert ProtocolRuns.build(
+        sim, [w, w], const, program, np.zeros(2, np.int64),
+        np.zeros(2, np.int64), H, lambda g: w.abs_max()[g], 1e-16) is None
