@@ -329,8 +329,9 @@ int ssmx_propagate_series_wave(const ssmx_series_desc *desc,
  *          (s (da + 1) + k) is E_2k[row s of the half's][lane's component],
  *          row s in the lane's sector, then (s (db + 1) + k)
  *          E_(2k+1)[row s][lane's component], row s in the opposite sector
- * dtable   double [n_theta][2][6][4][64]: d E_k / d theta, k = 0..3, at the
- *          same rows and columns, own sector then opposite sector
+ * dtable   double [n_theta][6 (5 + 4)][64]: d E_k / d theta at the same rows
+ *          and columns: entry (5 s + k), k = 0..4, own sector, then
+ *          (4 s + k), k = 0..3, opposite sector
  * store    the forward's
  * seed     double [n_inst * n_obs] dLoss/dF; obs double [n_obs * n]
  * grad_theta  double [n_inst * n_theta]; grad_seg double [records],
@@ -416,7 +417,7 @@ int ssmx_series_wide_adjoint(const ssmx_series_desc *desc,
                              double *lambda_out, void *stream);
 
 /*
- * dE_k, k < orders (3 or 4), of exp(A + f G) = sum f^k E_k in n_theta
+ * dE_k, k < orders (3 to 5), of exp(A + f G) = sum f^k E_k in n_theta
  * directions dA, to `terms` terms of the exponential's series; n at most 192.
  * With three orders the fourth is economised: for |f| <= drive_max it is
  * taken as the linear term that leaves a quarter of it.
@@ -434,7 +435,7 @@ int ssmx_series_derivatives(int32_t n, int32_t n_theta, int32_t terms,
 
 /*
  * grad_theta[inst][theta] = sum over the instance's `exps` exponentials and
- * k < orders (3 or 4) of f^k mu^T dE_k y.
+ * k < orders (3 to 5) of f^k mu^T dE_k y.
  * y, mu    double [n_inst][exps][npad] inputs and cotangents of the results
  * factors  double [n_inst][exps]
  * dtable   as ssmx_series_derivatives' out

@@ -362,7 +362,7 @@ class GradientProblem:
             point = (sim, const, program, waves, dconst,
                      np.atleast_2d(self.rho0), self.obs, h, self.tolerance,
                      self.adjoint_tolerance)
-            series = SeriesGradient.build(*point)
+            series = SeriesGradient.build(*point, derivatives)
             if series is not None and grad_gen not in (-1, series.gen):
                 series = None
             if series is None and grad_gen < 0:

@@ -8,9 +8,11 @@
 // The derivative with respect to the parameters of the constant matrix is
 // therefore a contraction of a few moments sum f^k mu y^T, summed over all
 // steps in registers, with dE_k / dtheta, formed once on the host: no Frechet
-// chain per exponential. Orders 0..3 are kept for every entry (parameters that
-// break the model's parity enter E_k at the other parity), which the host
-// allows only where the rest is below the adjoint's tolerance.
+// chain per exponential. Orders 0..4 are kept for entries within a sector, 0..3
+// for those between the two (every order in both: parameters that break the
+// model's parity enter E_k at the other parity), which the host allows only
+// where the rest is below the adjoint's tolerance beside the first order that
+// a parameter can act through.
 //
 // One instance per wavefront, both halves holding the cotangent (Halves): a
 // lane owns a column s, i.e. component s of y and of the new cotangent, and
@@ -18,10 +20,12 @@
 // opposite sector's after one exchange of rows). The same broadcasts feed the
 // product with E_k^T, the derivative in f and the moments.
 //
-// What bounds it: VALU issue, about 130 instructions per exponential of which
-// 48 are moments and 24 the derivative in f. 512 points x 25,000 steps, 9
-// parameters and 50 amplitudes: 33 ms after a forward run of 8.6; the Frechet
-// chain of adjoint_kernel took 88 after a forward run of 51.
+// What bounds it: VALU issue, about 136 instructions per exponential of which
+// 54 are moments and 24 the derivative in f. 512 points x 25,000 steps, 9
+// parameters and 50 amplitudes: 33.6 ms after a forward run of 8.7; the Frechet
+// chain of adjoint_kernel took 88 after a forward run of 51. (Without order 4
+// within the sectors 32.9, and what a parameter does through the drive alone
+// was off by up to 1e-9.)
 #include "ssmx_series_dev.h"
 
 namespace {
@@ -36,7 +40,8 @@ using ssmx::swap_pair;
 using ssmx::swap_rows;
 using ssmx::wave_exchange;
 
-constexpr int kOrders = 4;      // moments of orders 0..3
+// orders of the moments within a sector and between sectors
+constexpr int kOwn = 5, kOpp = 4;
 
 struct AParams {
     ssmx_series_desc d;
@@ -89,11 +94,29 @@ __device__ __forceinline__ void bcast_two(double &a, double xa,
 }
 
 // m[s][k] += z[k] x(lane s), s < N.
-template <int K0, int N>
-__device__ __forceinline__ void bcast_moments(double (*m)[kOrders], double x,
-                                              const double (&z)[kOrders])
+template <int K0, int N, int O>
+__device__ __forceinline__ void bcast_moments(double (*m)[O], double x,
+                                              const double (&z)[kOwn])
 {
-    if constexpr (N >= 1) {
+    if constexpr (N >= 1 && O == 5) {
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %5, %6 row_newbcast:%11 row_mask:0xf "
+            "bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %5, %7 row_newbcast:%11 row_mask:0xf "
+            "bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %5, %8 row_newbcast:%11 row_mask:0xf "
+            "bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %5, %9 row_newbcast:%11 row_mask:0xf "
+            "bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %4, %5, %10 row_newbcast:%11 row_mask:0xf "
+            "bank_mask:0xf"
+            : "+v"(m[0][0]), "+v"(m[0][1]), "+v"(m[0][2]), "+v"(m[0][3]),
+              "+v"(m[0][4])
+            : "v"(x), "v"(z[0]), "v"(z[1]), "v"(z[2]), "v"(z[3]), "v"(z[4]),
+              "n"(K0));
+        bcast_moments<K0 + 1, N - 1>(m + 1, x, z);
+    } else if constexpr (N >= 1) {
+        static_assert(O == 4, "moments of four or five orders");
         asm("s_nop 1\n\t"
             "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%9 row_mask:0xf "
             "bank_mask:0xf\n\t"
@@ -199,12 +222,16 @@ __attribute__((amdgpu_waves_per_eu(1))) void series_adjoint_kernel(AParams p)
             cb[s][o] =
                 p.table[(S * (DA + 1) + s * (DB + 1) + o) * kWave + lane];
     }
-    double mown[S][kOrders], mopp[S][kOrders];
+    double mown[S][kOwn], mopp[S][kOpp];
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+    for (int s = 0; s < S; ++s) {
 #pragma unroll
-        for (int k = 0; k < kOrders; ++k)
-            mown[s][k] = mopp[s][k] = 0.0;
+        for (int k = 0; k < kOwn; ++k)
+            mown[s][k] = 0.0;
+#pragma unroll
+        for (int k = 0; k < kOpp; ++k)
+            mopp[s][k] = 0.0;
+    }
     double source = 0.0;
     if (has)
         for (int o = 0; o < d.n_obs; ++o)
@@ -324,11 +351,12 @@ __attribute__((amdgpu_waves_per_eu(1))) void series_adjoint_kernel(AParams p)
                         acc = fma(abuf[e], g1, acc);
                     }
                 }
-                double z[kOrders];
+                double z[kOwn];
                 z[0] = y[j];
                 z[1] = f * y[j];
                 z[2] = u * y[j];
                 z[3] = u * z[1];
+                z[4] = u * z[2];
                 bcast_moments<0, S>(mown, ms, z);
                 bcast_moments<0, S>(mopp, mo, z);
                 lambda += ssmx::sum_halves(fma(f, yb, ya));
@@ -346,16 +374,18 @@ __attribute__((amdgpu_waves_per_eu(1))) void series_adjoint_kernel(AParams p)
     if (grad)
         flush(-1);
     for (int i = 0; i < p.n_theta; ++i) {
-        const double *t = p.dtable + (size_t)i * 2 * S * kOrders * kWave;
+        const double *t =
+            p.dtable + (size_t)i * S * (kOwn + kOpp) * kWave + lane;
         double v = 0.0;
 #pragma unroll
-        for (int s = 0; s < S; ++s)
+        for (int s = 0; s < S; ++s) {
 #pragma unroll
-            for (int k = 0; k < kOrders; ++k) {
-                v = fma(mown[s][k], t[(s * kOrders + k) * kWave + lane], v);
-                v = fma(mopp[s][k],
-                        t[((S + s) * kOrders + k) * kWave + lane], v);
-            }
+            for (int k = 0; k < kOwn; ++k)
+                v = fma(mown[s][k], t[(s * kOwn + k) * kWave], v);
+#pragma unroll
+            for (int k = 0; k < kOpp; ++k)
+                v = fma(mopp[s][k], t[(S * kOwn + s * kOpp + k) * kWave], v);
+        }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1)
             v += __shfl_xor(v, off, kWave);

@@ -329,13 +329,15 @@ class SeriesModel:
         return int(2 * (own * (own * (plan[0] + 1) + opp * (plan[1] + 1) +
                                2)).sum())
 
-    def plan(self, drive_max, tol):
+    def plan(self, drive_max, tol, slope=None):
         """(da, db, F) for drives |c(t)| <= ``drive_max``, or None.
 
         F bounds the factors |f| and the kept orders are those of the
         series in Chebyshev polynomials of f / F, whose order k is 2^(k-1)
         smaller than the power series': what is left out must stay below
-        ``tol`` with the Taylor plans' margin (a factor of 8).
+        ``tol`` with the Taylor plans' margin (a factor of 8).  With
+        ``slope`` the derivative in f is used as well: of what is left out,
+        it must stay below that share of the lowest even and odd order's.
         """
         F = self.h * self.weight * float(drive_max)
         worst = np.array([np.abs(c).sum(axis=-2).max()
@@ -343,9 +345,15 @@ class SeriesModel:
         if not np.all(np.isfinite(worst)):
             return None
         for da, db in ORDERS:
+            left = _dropped(worst.size, da, db)
             # (the orders beyond the last matrix are smaller than it)
-            if 8.0 * (worst[-1] + sum(worst[_dropped(worst.size, da, db)])) \
-                    <= tol:
+            if 8.0 * (worst[-1] + sum(worst[left])) > tol:
+                continue
+            # T_k' is k^2 at most, that of T_2 4, of T_1 1
+            if slope is None or all(
+                    sum(k * k * worst[k] for k in left if k % 2 == odd) <=
+                    slope * lead
+                    for odd, lead in ((0, 4 * worst[2]), (1, worst[1]))):
                 return da, db, F
         return None
 

@@ -15,8 +15,9 @@ from superspinsim_amd.series import (
 
 _f64 = np.float64
 
-#: moments of orders 0 .. ORDERS - 1 are kept by the kernel
-ORDERS = 4
+#: moments of orders 0 .. OWN - 1 are kept by the kernel within a sector, of
+#: 0 .. OPP - 1 between the two
+OWN, OPP = 5, 4
 
 
 def derivative_matrices(const, drive, dconst, orders):
@@ -49,9 +50,10 @@ class SeriesGradient:
 
     @classmethod
     def build(cls, sim, const, program, waves, dconst, rho0, obs, h, tol,
-              adjoint_tol):
+              adjoint_tol, derivatives=True):
         """``sim`` holds every state; ``dconst`` (directions, n, n) are the
-        derivatives of the folded constant matrix."""
+        derivatives of the folded constant matrix; ``derivatives`` unset: no
+        backward will follow."""
         varying = [g for g in program if g is not None]
         if len(varying) != 1 or None not in program or sim.rotating or \
                 sim.weights.shape[0] > 2:
@@ -67,7 +69,8 @@ class SeriesGradient:
         model = SeriesModel.build(c, g, sim.weights, h)
         if model is None or len(model.sets) != 1 or not model.one_pair():
             return None
-        plan = model.plan(max(w.abs_max()[varying[0]] for w in waves), tol)
+        plan = model.plan(max(w.abs_max()[varying[0]] for w in waves), tol,
+                          adjoint_tol if derivatives else None)
         if plan is None:
             return None
         self = cls()
@@ -83,37 +86,54 @@ class SeriesGradient:
         self.n_theta = dc.shape[0]
         scale = h * float(sim.weights[0].sum())
         dmats = derivative_matrices(scale * c, g, scale * dc, 7)
-        kept = cls._kept(dmats, F, adjoint_tol)
+        same = model.sector[:, None] == model.sector[None, :]
+        kept = cls._kept(dmats, F, adjoint_tol, same)
         if kept is None:
             return None
-        # [theta][own, opposite][slot][order][lane]
-        table = np.zeros((self.n_theta, 2, 6, ORDERS, 64))
-        for which, entries in enumerate((own, opp)):
+        # [theta][own: slot, order; opposite: slot, order][lane]
+        table = np.zeros((self.n_theta, 6 * (OWN + OPP), 64))
+        for entries, mats, first in ((own, kept[0], 0),
+                                     (opp, kept[1], 6 * OWN)):
             s, lane, row, col = entries.T
-            for k in range(ORDERS):
-                table[:, which, s, k, lane] = kept[k][:, row, col]
+            for k, m in enumerate(mats):
+                table[:, first + s * len(mats) + k, lane] = m[:, row, col]
         self.d_dtable = device_tensor(table)
         self.d_w, self.d_nodes = (device_tensor(sim.weights),
                                   device_tensor(sim.nodes))
         return self
 
     @staticmethod
-    def _kept(dmats, F, tol):
-        """Orders 0 .. ORDERS - 1 of the derivatives as series in Chebyshev
-        polynomials of f / F cut there; None if more than ``tol`` of a
-        direction is cut off."""
-        count = dmats.shape[0]
-        cheb = chebyshev(list(dmats), F)
-        size = np.array([np.abs(c).sum(axis=1).max(axis=1) for c in cheb])
-        if size.shape[1] and np.any(
-                size[ORDERS:].sum(axis=0) + size[-1] > tol * size.max(axis=0)):
-            return None
-        kept = [m.copy() for m in dmats[:ORDERS]]
-        for j in range(ORDERS, count):
-            for k, c in scaled_powers(j, F):
-                if k < ORDERS:
-                    kept[k] -= c * cheb[j]
-        return kept
+    def _kept(dmats, F, tol, same):
+        """(orders 0 .. OWN - 1 of the derivatives' entries within a sector,
+        0 .. OPP - 1 of those between sectors) as series in Chebyshev
+        polynomials of f / F cut there; None if more than ``tol`` of what a
+        direction can do is cut off.
+
+        What a parameter does through the drive alone is of second order
+        within a sector (a population made and unmade), however small
+        beside the undriven part: orders cut off are weighed against order 2
+        (even) and 1 (odd) there, between sectors against 0 and 1.
+        """
+        out = []
+        for part, orders in ((same, OWN), (~same, OPP)):
+            mats = list(dmats * part)
+            cheb = chebyshev(mats, F)
+            size = np.array([np.abs(c).sum(axis=1).max(axis=1, initial=0.0)
+                             for c in cheb])
+            for parity in (0, 1):
+                lead = size[1] if parity else \
+                    np.maximum(size[2], tol * size[0]) if orders == OWN \
+                    else size[0]
+                first = orders + (orders + parity) % 2
+                if np.any(size[first::2].sum(axis=0) > tol * lead):
+                    return None
+            kept = [m.copy() for m in mats[:orders]]
+            for j in range(orders, len(mats)):
+                for k, c in scaled_powers(j, F):
+                    if k < orders:
+                        kept[k] -= c * cheb[j]
+            out.append(kept)
+        return out
 
     def store_shape(self, n_inst, steps, J):
         """Inputs of every exponential."""

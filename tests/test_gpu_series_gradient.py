@@ -168,3 +168,32 @@ def test_states_and_rows_set_after_setup(gpu):
     got = problem.backward(state, seeds)["theta"].cpu().numpy()
     want = gradients(problem.setup(theta, amps))[1][0]
     assert np.all(np.abs(got - want) <= 1e-10 * np.max(np.abs(want), axis=0))
+
+
+@pytest.mark.parametrize("steps,b", [(3, 1.5e-4), (50, 1.5e-4), (3, 1.5e-3),
+                                     (50, 5e-6)])
+def test_amplitude_gradient_of_a_weak_rotation(gpu, steps, b):
+    """Two states that a constant drive rotates into each other, both
+    decaying: the read one is exp(-a t) cos(g c t), its derivative in c
+    -g t exp(-a t) sin(g c t), of second order in the drive.  1e-12 as
+    asked for, of the derivative itself (b is half a step's angle)."""
+    a, h, g = 1e8, 20e-12, 1e9
+    c = b / (0.5 * h * g)
+    drive = np.array([[0.0, -g], [g, 0.0]])
+
+    def waveforms(amps):
+        w = Waveform(2, base=[1.0, 0.0])
+        w.add(1, 0.0, 1.0, amps[0], param=0, dparam=1.0)
+        return [w, w, w]
+
+    problem = GradientProblem(
+        lambda th: np.array([np.diag([-a, -a]), drive]), waveforms,
+        np.eye(2)[0], np.eye(2)[0], 0.0, steps * h * (1 + 1e-9), h, 1, 2)
+    out, state = problem.forward([], [c])
+    assert state["by_series"]
+    got = problem.backward(state, np.ones((3, 1)))["amplitudes"].cpu().numpy()
+    t = h * np.arange(steps + 1)
+    s = -3 * g * t * np.exp(-a * t) * np.sin(g * c * t)
+    want = 0.5 * h * np.sum(s[:-1] + s[1:])
+    print(f"{got[0] / want - 1:.1e}", flush=True)
+    assert abs(got[0] / want - 1) <= 1e-12

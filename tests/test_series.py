@@ -195,8 +195,11 @@ def test_negligible_drives_leave_finite_matrices(drive_max):
     for k in range(4):
         assert np.array_equal(kept[k], model.sets[0][k]), k
     dmats = np.array(model.sets[0])[:, None]
-    for k, m in enumerate(SeriesGradient._kept(dmats, plan[2], 1e-12)):
-        assert np.array_equal(m[0], model.sets[0][k]), k
+    same = model.sector[:, None] == model.sector[None, :]
+    for part, mats in zip((same, ~same), SeriesGradient._kept(
+            dmats, plan[2], 1e-12, same)):
+        for k, m in enumerate(mats):
+            assert np.array_equal(m[0], model.sets[0][k] * part), k
 
 
 @pytest.mark.parametrize("drive_max", [1e60, 1e300, np.inf])
@@ -332,3 +335,37 @@ def test_gradient_store_that_cannot_be_had(monkeypatch):
     monkeypatch.setattr(torch, "empty", empty)
     assert problem._series_store(state, Series, 10) is False
     assert problem._series_store(state, Series, 1 << 40) is False
+
+
+@pytest.mark.parametrize("rabi", [5e5, 3e6])
+def test_kept_derivatives_of_each_order_the_drive_brings(rabi):
+    """What is cut off is small beside the lowest even and odd orders that a
+    parameter can act through (1e-12), not only beside the whole: random
+    directions within and between the sectors."""
+    from superspinsim_amd.series_gradient import (
+        SeriesGradient, derivative_matrices)
+    wl = configs.odmr7(1, use_incoherent=True)
+    const, drive = _pair(wl)
+    _, weights, _ = quadratures.scheme(2)
+    model = SeriesModel.build(const, drive, weights, H)
+    F = model.plan(configs.drive_amplitude(rabi), 1e-16, 1e-12)[2]
+    scale = H * weights[0].sum()
+    same = model.sector[:, None] == model.sector[None, :]
+    rng = np.random.default_rng(1)
+    dirs = rng.standard_normal((4, wl.n, wl.n)) * 1e-3
+    dirs[:2] *= same
+    dirs[2:] *= ~same
+    full = derivative_matrices(scale * const, drive, dirs, 9)
+    kept = SeriesGradient._kept(full[:8], F, 1e-12, same)
+    for f in F * np.array([1e-3, 0.3, -1.0]):
+        for part, mats, even in ((same, kept[0], 2), (~same, kept[1], 0)):
+            for odd, lead in ((0, even), (1, 1)):
+                got = sum(f ** k * m for k, m in enumerate(mats)
+                          if k % 2 == odd)
+                want = sum(f ** k * m for k, m in enumerate(full)
+                           if k % 2 == odd) * part
+                for g, w, first in zip(got, want, full[lead] * part):
+                    size = np.max(np.abs(F ** lead * first))
+                    # (rounding of order 0, which may be far larger)
+                    noise = 1e-15 * np.max(np.abs(w))
+                    assert np.max(np.abs(g - w)) <= 1e-12 * size + noise
