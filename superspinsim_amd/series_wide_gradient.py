@@ -20,6 +20,8 @@ _f64 = np.float64
 
 #: rows of the moment kernel
 MAX_ROWS = 192
+#: shares of the run's left-out entries that gradients try to leave out
+FINER = (1e-1, 1.0)
 
 
 def row_lists(mats):
@@ -88,12 +90,14 @@ class WideGradient:
         self.npad = -(-model.n // 16) * 16
         self.d_w, self.d_nodes = (device_tensor(sim.weights),
                                   device_tensor(sim.nodes))
-        self.tables = self._staged(model.layout(plan), states)
-        self.back = None
         dc = dconst[:, at[0], at[1]]
         self.n_theta = dc.shape[0]
-        if derivatives and self._back() is None:
-            return None
+        if derivatives:
+            self._stage_both()
+            if self.back is None:
+                return None
+        else:
+            self.tables = self._staged(model.layout(plan), states)
         if self.n_theta:
             order = np.argsort(model.pos)
             rows = np.ix_(order, order)
@@ -114,12 +118,20 @@ class WideGradient:
         return blocks, device_tensor(own_states(lane_states, states)), \
             columns, table, in_lds
 
-    def _back(self):
-        """Tables of the transposed matrices (None where they don't fit)."""
-        if self.back is None:
-            self.back = self._staged(self.model.transposed(self.plan),
-                                     self.states)
-        return self.back
+    def _stage_both(self):
+        """Tables of the matrices and of their transposes (``back``: None
+        where these don't fit), with as much of them as the kernel's columns
+        hold in steps of ten: a gradient may hang on entries that the run
+        itself is free to leave out."""
+        da, db, F, budget = self.plan
+        for share in FINER:
+            self.plan = da, db, F, share * budget
+            self.tables = self._staged(self.model.layout(self.plan),
+                                       self.states)
+            self.back = None if self.tables is None else self._staged(
+                self.model.transposed(self.plan), self.states)
+            if self.back is not None:
+                return
 
     def _derivatives(self, a, g, da, terms, drive_max):
         """d E_k in every direction, by row position."""
@@ -192,7 +204,7 @@ class WideGradient:
             lam.zero_()
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         lib = _lib.load()
-        blocks, states, columns, table, in_lds = self._back()
+        blocks, states, columns, table, in_lds = self.back
         _lib.check(lib.ssmx_series_wide_adjoint(
             ctypes.byref(self._desc(problem, n_inst, in_lds)), _ptr(blocks),
             blocks.shape[0], _ptr(states), _ptr(columns), _ptr(table),

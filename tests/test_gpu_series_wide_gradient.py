@@ -126,3 +126,35 @@ def test_wide_gradient_equals_frechet(gpu, points, outputs, fine, two, rabi):
     e = np.max(np.abs(a["lambda"] - b["lambda"])) / \
         np.max(np.abs(b["lambda"]))
     assert e <= 1e-12
+
+
+@pytest.mark.parametrize("steps", [3, 40])
+def test_small_gradients_of_short_runs(gpu, steps):
+    """Each parameter beside its own size, however small: the quadrupole's
+    gradient hangs on entries of 1e-18 of the E_k over a few steps.  Against
+    extended precision the Frechet chain is good to 4e-10 there."""
+    wl = configs.odmr21(1, use_incoherent=True)
+    b1 = configs.drive_amplitude(5e5)
+
+    def waveforms(amps):
+        w = Waveform(5, base=[1.0, 0.0, 0.0, 0.0, wl.excitation])
+        w.tone(1, b1, 2.8695e9)
+        return [w]
+
+    res = {}
+    for store in ("auto", False):
+        problem = GradientProblem(
+            lambda th: configs.nv21_generators(th, use_incoherent=True),
+            waveforms, wl.rho0, wl.obs, 0.0, steps * 20e-12 * (1 + 1e-9),
+            20e-12, 1, 2, 300, theta_scale=configs.THETA21_SCALE,
+            store_inputs=store)
+        out, state = problem.forward(configs.nv21_theta0(), [])
+        assert state["by_series"] == bool(store)
+        res[store] = problem.backward(state, np.ones((1, 1)))[
+            "theta"].cpu().numpy()[0]
+    names = np.array(configs.THETA21_NAMES)
+    for name in ("D_gs", "radiative", "isc_pm", "quadrupole", "A_par",
+                 "A_perp"):
+        a, b = (r[names == name][0] for r in (res["auto"], res[False]))
+        print(f"{name} {a / b - 1:.1e}", flush=True)
+        assert abs(a / b - 1) <= 1e-9, name
